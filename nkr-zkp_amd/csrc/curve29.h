@@ -15,7 +15,7 @@
 //   ZZ3 = ZZ PP, ZZZ3 = ZZZ PPP                                    < 2p
 // so the invariant holds without a single reduction.  PP and RR are
 // squarings (fp29_sqr: the symmetric partial products once).  A product's inputs stay
-// below a*b < 2^261 p (fp29_mul).  The exceptional cases (P = 0: the base
+// below a*b < 145 p^2 (fp29_mul).  The exceptional cases (P = 0: the base
 // equals the accumulator, or its negation) take the canonical 32-bit path.
 // Every result is the same field element as xyzz_add_affine's, so the
 // canonical outputs are bit-identical.
@@ -157,17 +157,17 @@ NKR_HD Xyzz29<P> xyzz29_add(const Xyzz29<P> &a, const Xyzz29<P> &b)
 // each output component one Montgomery reduction of a sum of two (or, for
 // Y3, four) partial products (fp29_mul_add): (a b)_0 = a0 b0 + a1 (Kp - b1),
 // (a b)_1 = a0 b1 + a1 b0 -- the multiply-adds of Karatsuba's three products
-// without its five additions of sums, and with input bounds up to A*B = 84
-// (components below A p and B p; 2AB + 2AK below 2^261/p^2 = 169.28 p^2,
-// K the multiple of p that negates b1), outputs below 2p.  Squares use
-// (a0 + a1)(a0 - a1) and a0 (2 a1), inputs below 6.5p.
+// without its five additions of sums, for components below A p and B p with
+// A (B + K) at most 145 (K the multiple of p that negates b1), outputs below
+// 2p.  Squares use
+// (a0 + a1)(a0 - a1) and a0 (2 a1), inputs below 6p.
 //   accumulator  X below 8p, Y, ZZ, ZZZ below 2p; infinity is ZZ = 0 exactly
 //   base         x2, y2 below 32p (fp29_from_mont, no reduction)
 // madd-2008-s, the sequence of xyzz29_add_affine:
 //   U2 = x2 ZZ, S2 = y2 ZZZ (32p x 2p: 2 * 64 = 128)         below 2p
 //   P = U2 + 8p - X, R = S2 + 2p - Y, each reduced by 4p      below 6p
-//   PP = P^2, RR = R^2 ((12p)^2 = 144: c0 < 1.86p; c1 = P0 (2 P1)
-//        72: < 1.43p)                                         below 2p
+//   PP = P^2, RR = R^2 ((12p)^2 = 144: c0 < 2p; c1 = P0 (2 P1)
+//        72: < 1.57p)                                         below 2p
 //   PPP = P PP, Q = X PP, ZZ3 = ZZ PP (at most 8p x 2p)       below 2p
 //   X3 = (RR + 2p - PPP) + 4p - 2Q                            below 8p
 //   Y3 = R (Q + 8p - X3) + Y (2p - PPP): per component one
@@ -193,8 +193,8 @@ NKR_HD fq2_t fq2_29_to(const Fq2_29<P> &a)
     return {fp29_to_mont(a.c0), fp29_to_mont(a.c1)};
 }
 
-// a * b; components below A p and B p with A*B <= 84 and b1 <= KB p,
-// A*(B + KB) <= 169: components below 2p.
+// a * b; components below A p and B p with b1 <= KB p and 2 A B and
+// A*(B + KB) at most 145: components below 2p.
 template <class P, uint32_t KB>
 NKR_HD Fq2_29<P> fq2_29_mul(const Fq2_29<P> &a, const Fq2_29<P> &b)
 {
@@ -202,7 +202,7 @@ NKR_HD Fq2_29<P> fq2_29_mul(const Fq2_29<P> &a, const Fq2_29<P> &b)
     return {fp29_mul_add(a.c0, b.c0, a.c1, nb1), fp29_mul_add(a.c0, b.c1, a.c1, b.c0)};
 }
 
-// a^2, components below 6.5p: c0 below 1.86p, c1 below 1.43p.
+// a^2, components below 6p: c0 below 2p, c1 below 1.57p.
 template <class P, uint32_t KA>
 NKR_HD Fq2_29<P> fq2_29_sqr(const Fq2_29<P> &a)
 {

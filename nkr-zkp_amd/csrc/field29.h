@@ -127,31 +127,15 @@ NKR_HD void fp29_opaque(Fp29<P> &x)
 #endif
 }
 
-// Could x (below k_max * p, k_max <= 16) be 0 mod p?  A necessary condition
-// on the low limb only: x = j*p for some j < k_max.  Exact answers come from
-// fp29_to_mont(x).is_zero().
-template <class P>
-struct P29LowMultiples {
-    uint32_t v[16];
-};
-
-template <class P>
-constexpr P29LowMultiples<P> p29_low_multiples()
-{
-    P29LowMultiples<P> r{};
-    for (uint32_t j = 0; j < 16; ++j) r.v[j] = P29<P>::times(j).l[0];
-    return r;
-}
-
+// Could x (below KMax * p) be 0 mod p?  A necessary condition on the low limb
+// only: x = j*p for some j < KMax, so j = x p^-1 mod 2^29 must come out below
+// KMax.  (As KMax comparisons with the low limbs of j*p it compiled into a
+// tree of divergent branches, about 180 scalar instructions of every bucket
+// addition.)  Exact answers come from fp29_to_mont(x).is_zero().
 template <class P, uint32_t KMax>
 NKR_HD bool fp29_may_be_zero(const Fp29<P> &x)
 {
-    static_assert(KMax <= 16, "at most 16 multiples of p");
-    constexpr P29LowMultiples<P> lm = p29_low_multiples<P>();
-    bool any = false;
-#pragma unroll
-    for (uint32_t j = 0; j < KMax; ++j) any = any || x.l[0] == lm.v[j];
-    return any;
+    return ((0u - x.l[0] * P29<P>::inv()) & kMask29) < KMax;
 }
 
 }  // namespace nkr
