@@ -22,12 +22,15 @@
 //         resident waves, which take pieces by grid stride;
 //      2. fold: buckets left with more than 64 partial sums (skewed digit
 //         distributions, e.g. witnesses that are mostly 0 or 1) are folded
-//         4:1 until they are not; other buckets are untouched;
-//      3. complete: 1..16 lanes per bucket (about 8 partials per lane),
-//         strided partial sums then a shuffle tree, give the bucket sums S_m;
+//         64:1, a wave per sum, until they are not; others are untouched;
+//      3. complete: 1..16 lane groups per bucket, strided partial sums then
+//         a shuffle tree, give the bucket sums S_m;
 //      4. bit planes: a log-depth tree merges bucket blocks into
 //         U_j = sum over m with bit j of S_m (c points per job), several
 //         levels per launch inside LDS.
+//    Stages 2-4 are chains of additions with few in flight, so each addition
+//    is shared by a group of lanes (coop29.h); which buckets need what is
+//    planned from the schedules in one launch before the accumulation.
 //    The host combines sum_j 2^j U_j (c doublings) and normalises.
 // The reference computes the same sums with libff multi_exp<BDLO12>
 // (third_party/.../libff/algebra/scalar_multiplication/multiexp.tcc:165-282);
@@ -225,25 +228,26 @@ public:
     // next run reallocates what it needs).
     uint64_t device_bytes() const
     {
-        uint64_t b = complete_base_.bytes() + class_count_.bytes() + class_list_.bytes() + jobs_dev_.bytes() +
-                     thread_base_dev_.bytes() + pool_.bytes() + sums_.bytes() + reg_start_.bytes() +
-                     reg_count_.bytes() + fold_start_.bytes();
-        return b + tree_[0].bytes() + tree_[1].bytes();
+        return seg_base_.bytes() + seg_count_.bytes() + class_count_.bytes() + class_list_.bytes() +
+               jobs_dev_.bytes() + piece_base_.bytes() + pool_.bytes() + sums_.bytes() + reg_start_.bytes() +
+               reg_count_.bytes() + recs_.bytes() + state_.bytes() + tree_[0].bytes() + tree_[1].bytes();
     }
     void release_device()
     {
-        complete_base_.release();
+        seg_base_.release();
+        seg_count_.release();
         class_count_.release();
         class_list_.release();
         jobs_dev_.release();
-        thread_base_dev_.release();
+        piece_base_.release();
         pool_.release();
         sums_.release();
         tree_[0].release();
         tree_[1].release();
         reg_start_.release();
         reg_count_.release();
-        fold_start_.release();
+        recs_.release();
+        state_.release();
         key_.clear();  // the layout cache refers to the released buffers
     }
 
@@ -253,17 +257,17 @@ public:
 private:
     void layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream);
     std::vector<const void *> key_;
-    uint32_t fold_levels_ = 0;
-    std::vector<uint64_t> fold_cap_;  // largest partial count of any job at each fold level
-    uint64_t thread_total_ = 0;
-    uint64_t complete_bound_ = 0;  // completion lanes at most
-    DeviceBuffer<uint32_t> complete_base_, class_count_, class_list_;
-    std::vector<uint64_t> thread_base_;
-    DeviceBuffer<uint8_t> jobs_dev_;
-    DeviceBuffer<uint32_t> thread_base_dev_;
+    uint32_t fold_levels_ = 0;     // 4:1 levels the largest possible bucket needs
+    uint32_t fold_base_[kMaxFoldLevels / 3] = {};  // where each fold launch's outputs start in pool_
+    uint64_t fold_cap_[kMaxFoldLevels / 3] = {};   // and their largest number
+    uint64_t rec_cap_ = 0;                         // fold records of one launch at most
+    uint64_t piece_bound_ = 0;                     // level-0 pieces of all jobs at most
+    uint64_t complete_bound_ = 0;                  // completion lanes at most
+    DeviceBuffer<uint32_t> seg_base_, seg_count_, class_count_, class_list_, piece_base_;
+    DeviceBuffer<uint8_t> jobs_dev_, recs_, state_;
     PinnedStaging<uint8_t> jobs_stage_;
     DeviceBuffer<partial_t<F>> pool_, sums_, tree_[2];
-    DeviceBuffer<uint32_t> reg_start_, reg_count_, fold_start_;
+    DeviceBuffer<uint32_t> reg_start_, reg_count_;
 };
 
 // Host: sum_j 2^j U_j, then the reference's affine form (Z = 1, or (0, 1, 0)).

@@ -1,6 +1,7 @@
 // Pippenger MSM kernels for gfx950 (see msm.h for the design).
 #include "msm.h"
 
+#include "coop29.h"
 #include "curve29.h"
 
 #include <algorithm>
@@ -21,16 +22,35 @@ constexpr uint32_t kSortMinPerBlock = 256;
 constexpr uint32_t kSortThreads = 1024;
 // Column scan tile: 64 buckets x kScanGroups row groups per workgroup.
 constexpr uint32_t kScanGroups = 16;
-// LDS per tree workgroup (two buffers of 2^h blocks): 64 KiB for G1 (two
-// workgroups per CU); 32 KiB for G2, whose trees run beside the main
-// stream's transforms and histograms and must leave them room on the CU.
+// LDS per tree workgroup (two buffers of 2^h blocks): two workgroups per CU.
+constexpr size_t kTreeLds = 64 * 1024;
+constexpr uint32_t kTreeThreads = 256;
+// Completion classes: 1, 2, 4, 8 or 16 lane groups per bucket (G2: up to 8,
+// the groups of one wave).
+constexpr uint32_t kCompleteClasses = 5;
+// Partial sums one wave folds into one: three 4:1 levels at once.
+constexpr uint32_t kFoldLevelsPerLaunch = 3;
+constexpr uint32_t kFoldSpan = 64;
+static_assert(kFoldSpan == kMsmFoldIn * kMsmFoldIn * kMsmFoldIn && kFoldSpan <= kMsmCompleteMax, "fold span");
+constexpr uint32_t kMaxFoldLaunches = kMaxFoldLevels / kFoldLevelsPerLaunch;
+// Lane groups of an addition per wave (coop29.h).
 template <class F>
-constexpr size_t tree_lds_bytes()
-{
-    return std::is_same<F, fq2_t>::value ? 32 * 1024 : 64 * 1024;
-}
-// Completion lane classes (1, 2, 4, 8 lanes per bucket).
-constexpr uint32_t kCompleteClasses = 4;
+constexpr uint32_t kWaveGroups = 64 / Coop<F>::kLanes;
+
+// One bucket to fold at one level: its partials at pool[src .. src + cnt)
+// become ceil(cnt / kFoldSpan) sums, the level's outputs `start` ...
+struct FoldRec {
+    uint32_t start, src, cnt;
+};
+
+// A batch's reduction plan on the device (k_reduce_plan).  `ticket` and
+// `fold_ctr` are zero between launches; fold_count holds their last values.
+struct ReduceState {
+    uint32_t ticket;
+    uint32_t pad;
+    unsigned long long fold_ctr[kMaxFoldLaunches];  // records << 32 | outputs
+    unsigned long long fold_count[kMaxFoldLaunches];
+};
 
 template <class F>
 struct JobDev {
@@ -38,31 +58,16 @@ struct JobDev {
     const uint32_t *sorted;
     const uint32_t *bucket_start;  // B + 1
     const uint32_t *piece_start;   // B + 1
-    const uint32_t *piece_max;     // largest level-0 piece count of any bucket
     const uint32_t *piece_len;     // entries per level-0 piece (chosen on the device)
-    partial_t<F> *pool;            // partial sums (level 0 region, then fold levels)
-    uint32_t *reg_start;           // B: where bucket k's partials live in `pool`
+    uint32_t *reg_start;           // B: where bucket k's partials to complete live in the pool
     uint32_t *reg_count;           // B
-    uint32_t *fold_start;          // B + 1
     partial_t<F> *sums;            // B: S_{k+1}
     partial_t<F> *tree[2];         // B each
     Xyzz<F> *planes;               // c (canonical)
+    uint32_t pool_off;             // the job's level-0 partials start here in the pool
     uint32_t B, c;
-    uint32_t list_off;                    // this job's completion lists start at 4 * list_off
-    uint32_t level_base[kMaxFoldLevels];  // where each fold level's partials start in `pool`
+    uint32_t list_off;  // this job's completion lists start at kCompleteClasses * list_off
 };
-
-// Sum of two partial sums, and a partial sum as a canonical bit plane.
-__device__ __forceinline__ Xyzz29<FqParams> partial_add(const Xyzz29<FqParams> &a, const Xyzz29<FqParams> &b)
-{
-    return xyzz29_add(a, b);
-}
-__device__ __forceinline__ Xyzz2_29<FqParams> partial_add(const Xyzz2_29<FqParams> &a, const Xyzz2_29<FqParams> &b)
-{
-    return xyzz2_29_add(a, b);
-}
-__device__ __forceinline__ Xyzz<fq_t> partial_plane(const Xyzz29<FqParams> &a) { return xyzz29_to(a); }
-__device__ __forceinline__ Xyzz<fq2_t> partial_plane(const Xyzz2_29<FqParams> &a) { return xyzz2_29_to(a); }
 
 // ------------------------------------------------------------ digit recoding
 // Signed c-bit digits of an integer scalar (< 2^254): d_w in [-2^(c-1), 2^(c-1)],
@@ -383,43 +388,111 @@ __global__ __launch_bounds__(kSortThreads) void k_scatter_batch(const SortJob *_
                   jb.bucket_start, jb.block_count, jb.sorted);
 }
 
-template <class F>
-__global__ __launch_bounds__(256) void k_regions_init(const JobDev<F> *__restrict__ jobs,
-                                                      uint32_t *__restrict__ class_count)
+// Exclusive prefix of f(0) .. f(len - 1) into out[0 .. len], by one workgroup
+// (whole waves).
+template <class Fn>
+__device__ void group_prefix(uint32_t len, uint32_t *__restrict__ out, Fn f)
 {
-    const JobDev<F> &jb = jobs[blockIdx.y];
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < kCompleteClasses) class_count[kCompleteClasses * blockIdx.y + k] = 0;
-    if (k >= jb.B) return;
-    jb.reg_start[k] = jb.piece_start[k];
-    jb.reg_count[k] = jb.piece_start[k + 1] - jb.piece_start[k];
+    __shared__ uint32_t wave_sum[16];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    uint32_t base = 0;
+    for (uint32_t k0 = 0; k0 < len; k0 += blockDim.x) {
+        const uint32_t k = k0 + threadIdx.x;
+        const uint32_t v = k < len ? f(k) : 0u;
+        uint32_t incl = v;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)incl, off);
+            if (lane >= (uint32_t)off) incl += y;
+        }
+        if (lane == 63) wave_sum[wave] = incl;
+        __syncthreads();
+        uint32_t run = base;
+        for (uint32_t w = 0; w < waves; ++w) {
+            if (w < wave) run += wave_sum[w];
+            base += wave_sum[w];
+        }
+        if (k < len) out[k] = run + incl - v;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[len] = base;
 }
 
-// piece_base[j] = level-0 pieces of jobs before j (as scheduled on the
-// device), piece_base[J] = all of them.  One workgroup.
+// The reduction plan of a batch, from the schedules' piece splits alone: one
+// launch before the accumulation instead of six small ones after it.
+//   * a bucket with more than kMsmCompleteMax partials gets a fold record per
+//     level that brings it below (kFoldSpan : 1 each); any bucket's final
+//     partials become reg_start / reg_count;
+//   * completion classes: a bucket with m partials is completed by 2^c lane
+//     groups, the smallest c with m <= serial << c (the host's serial target
+//     is short where the launch leaves the chip idle and long where every
+//     lane group has several buckets); an empty bucket's sum is infinity;
+//   * the last workgroup to finish turns the counts into offsets:
+//     piece_base[j] = level-0 pieces of the jobs before j, seg_base[s] = lanes
+//     of the completion segments before s = kCompleteClasses * j + c, each
+//     padded to whole waves, and clears the counters for the next launch.
 template <class F>
-__global__ __launch_bounds__(1024) void k_piece_scan(const JobDev<F> *__restrict__ jobs, uint32_t J,
-                                                     uint32_t *__restrict__ piece_base)
+__global__ __launch_bounds__(256) void k_reduce_plan(const JobDev<F> *__restrict__ jobs, uint32_t J,
+                                                     uint32_t max_class, uint32_t serial,
+                                                     ReduceState *__restrict__ st, FoldRec *__restrict__ recs,
+                                                     uint32_t rec_cap, const uint32_t *__restrict__ fold_base,
+                                                     uint32_t *__restrict__ class_count,
+                                                     uint32_t *__restrict__ class_list,
+                                                     uint32_t *__restrict__ piece_base,
+                                                     uint32_t *__restrict__ seg_count,
+                                                     uint32_t *__restrict__ seg_base)
 {
-    __shared__ uint32_t part[1024];
-    const uint32_t per = (J + blockDim.x - 1) / blockDim.x;
-    const uint32_t beg = min(J, threadIdx.x * per), end = min(J, beg + per);
-    uint32_t sum = 0;
-    for (uint32_t j = beg; j < end; ++j) sum += jobs[j].piece_start[jobs[j].B];
-    part[threadIdx.x] = sum;
+    const uint32_t j = blockIdx.y;
+    const JobDev<F> &jb = jobs[j];
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t m = 0;
+    if (k < jb.B) {
+        uint32_t src = jb.pool_off + jb.piece_start[k];
+        m = jb.piece_start[k + 1] - jb.piece_start[k];
+        for (uint32_t L = 0; m > kMsmCompleteMax; ++L) {
+            const uint32_t n = (m + kFoldSpan - 1) / kFoldSpan;
+            const unsigned long long at = atomicAdd(&st->fold_ctr[L], (1ull << 32) | n);
+            const uint32_t start = (uint32_t)at;
+            recs[(size_t)L * rec_cap + (uint32_t)(at >> 32)] = FoldRec{start, src, m};
+            src = fold_base[L] + start;
+            m = n;
+        }
+        jb.reg_start[k] = src;
+        jb.reg_count[k] = m;
+        if (m == 0) jb.sums[k] = partial_t<F>::infinity();
+    }
+    // one atomic per wave and class: a ballot ranks the lanes
+    uint32_t c = 0;
+    while (c < max_class && (serial << c) < m) ++c;
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t *list = class_list + (size_t)jb.list_off * kCompleteClasses;
+    for (uint32_t cc = 0; cc <= max_class; ++cc) {
+        const bool mine = m > 0 && c == cc;
+        const uint64_t mask = __ballot(mine);
+        if (mask == 0) continue;
+        const uint32_t leader = (uint32_t)__ffsll((unsigned long long)mask) - 1u;
+        uint32_t first = 0;
+        if (lane == leader) first = atomicAdd(&class_count[kCompleteClasses * j + cc], (uint32_t)__popcll(mask));
+        first = (uint32_t)__shfl((int)first, (int)leader);
+        if (mine) list[(size_t)cc * jb.B + first + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = k;
+    }
+
+    __shared__ uint32_t last;
     __syncthreads();
-    for (uint32_t off = 1; off < blockDim.x; off <<= 1) {
-        const uint32_t t = threadIdx.x >= off ? part[threadIdx.x - off] : 0u;
-        __syncthreads();
-        part[threadIdx.x] += t;
-        __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence();
+        last = atomicAdd(&st->ticket, 1u) + 1u == gridDim.x * gridDim.y ? 1u : 0u;
     }
-    uint32_t run = part[threadIdx.x] - sum;
-    for (uint32_t j = beg; j < end; ++j) {
-        piece_base[j] = run;
-        run += jobs[j].piece_start[jobs[j].B];
-    }
-    if (threadIdx.x == blockDim.x - 1) piece_base[J] = part[threadIdx.x];
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    group_prefix(J, piece_base, [&](uint32_t i) { return jobs[i].piece_start[jobs[i].B]; });
+    group_prefix(kCompleteClasses * J, seg_base, [&](uint32_t s) {
+        const uint32_t n = atomicExch(&class_count[s], 0u);
+        seg_count[s] = n;
+        return ((n * Coop<F>::kLanes << (s % kCompleteClasses)) + 63u) & ~63u;
+    });
+    if (threadIdx.x < kMaxFoldLaunches) st->fold_count[threadIdx.x] = atomicExch(&st->fold_ctr[threadIdx.x], 0ull);
+    if (threadIdx.x == 0) st->ticket = 0;
 }
 
 // The G2 accumulator of one lane with X and ZZ in registers and Y and ZZZ in
@@ -479,7 +552,8 @@ struct Xyzz2_29Lds {
 // covers every piece).
 template <class F>
 __device__ __forceinline__ void accumulate_body(const JobDev<F> *__restrict__ jobs,
-                                                const uint32_t *__restrict__ piece_base, uint32_t J)
+                                                const uint32_t *__restrict__ piece_base, uint32_t J,
+                                                partial_t<F> *__restrict__ pool)
 {
     const uint32_t total = piece_base[J];
 #pragma unroll 1
@@ -536,15 +610,17 @@ __device__ __forceinline__ void accumulate_body(const JobDev<F> *__restrict__ jo
             }
             acc = acc29;
         }
-        jb.pool[p] = acc;
+        pool[jb.pool_off + p] = acc;
     }
 }
 
+// G1: at most 168 registers, three waves per SIMD.
 template <class F>
-__global__ __launch_bounds__(256) void k_accumulate(const JobDev<F> *__restrict__ jobs,
-                                                    const uint32_t *__restrict__ piece_base, uint32_t J)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_accumulate(const JobDev<F> *__restrict__ jobs,
+                                                    const uint32_t *__restrict__ piece_base, uint32_t J,
+                                                    partial_t<F> *__restrict__ pool)
 {
-    accumulate_body<F>(jobs, piece_base, J);
+    accumulate_body<F>(jobs, piece_base, J, pool);
 }
 
 // The G2 addition's working set exceeds 256 registers, which would leave one
@@ -554,162 +630,94 @@ __global__ __launch_bounds__(256) void k_accumulate(const JobDev<F> *__restrict_
 // workgroup) the spills fall from 280 to 80 bytes per lane.
 template <>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_accumulate<fq2_t>(
-    const JobDev<fq2_t> *__restrict__ jobs, const uint32_t *__restrict__ piece_base, uint32_t J)
+    const JobDev<fq2_t> *__restrict__ jobs, const uint32_t *__restrict__ piece_base, uint32_t J,
+    partial_t<fq2_t> *__restrict__ pool)
 {
-    accumulate_body<fq2_t>(jobs, piece_base, J);
+    accumulate_body<fq2_t>(jobs, piece_base, J, pool);
 }
 
-// Fold level L: buckets with more than kMsmCompleteMax partials get
-// ceil(count / kMsmFoldIn) new partials written at pool[level_base[L] ...].
+// Sum over the lane groups of aligned runs of `groups` groups: every group of
+// a run ends with its run's sum.
 template <class F>
-// 256 threads (one wave per SIMD): on the side stream this launch runs beside
-// a resident-sized accumulation on the main stream, and a smaller workgroup
-// needs less free room on a CU to start.
-__global__ __launch_bounds__(256) void k_fold_scan(const JobDev<F> *__restrict__ jobs)
+__device__ __forceinline__ Coop<F> coop_reduce(Coop<F> acc, uint32_t groups)
 {
-    const JobDev<F> &jb = jobs[blockIdx.x];
-    if (*jb.piece_max <= kMsmCompleteMax) return;  // no skewed bucket: nothing to fold
-    block_scan(jb.reg_count, jb.B, 3, kMsmFoldIn, kMsmCompleteMax, jb.fold_start);
+#pragma unroll 1
+    for (uint32_t off = groups >> 1; off >= 1; off >>= 1) acc = coop_add(acc, coop_shfl_xor(acc, off));
+    return acc;
 }
 
+// pool[src + i] for i = first, first + step, ... < cnt, summed by one lane
+// group (infinity when there is none); the next partial is loaded before the
+// addition that precedes it.
 template <class F>
-__global__ __launch_bounds__(256) void k_fold(const JobDev<F> *__restrict__ jobs, uint32_t L)
+__device__ __forceinline__ Coop<F> coop_sum(const partial_t<F> *__restrict__ pool, uint32_t src, uint32_t cnt,
+                                            uint32_t first, uint32_t step)
 {
-    const JobDev<F> &jb = jobs[blockIdx.y];
-    if (*jb.piece_max <= kMsmCompleteMax) return;
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= jb.fold_start[jb.B]) return;
-    const uint32_t k = find_segment(jb.fold_start, jb.B, p);
-    const uint32_t q = p - jb.fold_start[k];
-    const uint32_t beg = jb.reg_start[k] + q * kMsmFoldIn;
-    const uint32_t end = min(beg + kMsmFoldIn, jb.reg_start[k] + jb.reg_count[k]);
-    partial_t<F> acc = jb.pool[beg];
-    for (uint32_t e = beg + 1; e < end; ++e) acc = partial_add(acc, jb.pool[e]);
-    jb.pool[jb.level_base[L] + p] = acc;
+    Coop<F> acc = first < cnt ? coop_load<F>(pool, (size_t)src + first) : Coop<F>::infinity();
+    uint32_t i = first + step;
+    Coop<F> next = i < cnt ? coop_load<F>(pool, (size_t)src + i) : Coop<F>::infinity();
+#pragma unroll 1
+    while (i < cnt) {
+        const Coop<F> cur = next;
+        i += step;
+        if (i < cnt) next = coop_load<F>(pool, (size_t)src + i);
+        acc = coop_add(acc, cur);
+    }
+    return acc;
 }
 
+// Fold launch L: a wave sums up to kFoldSpan partials of one record into one
+// output; 7 (G1) or 10 (G2) additions deep.
 template <class F>
-__global__ __launch_bounds__(256) void k_fold_retarget(const JobDev<F> *__restrict__ jobs, uint32_t L)
+__global__ __launch_bounds__(256) void k_fold(const ReduceState *__restrict__ st, const FoldRec *__restrict__ recs,
+                                              uint32_t L, uint32_t out_base, partial_t<F> *__restrict__ pool)
 {
-    const JobDev<F> &jb = jobs[blockIdx.y];
-    if (*jb.piece_max <= kMsmCompleteMax) return;
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= jb.B) return;
-    if (jb.reg_count[k] > kMsmCompleteMax) {
-        jb.reg_start[k] = jb.level_base[L] + jb.fold_start[k];
-        jb.reg_count[k] = jb.fold_start[k + 1] - jb.fold_start[k];
+    const unsigned long long n = st->fold_count[L];
+    const uint32_t total = (uint32_t)n, nrec = (uint32_t)(n >> 32);
+    const uint32_t group = (threadIdx.x & 63u) / Coop<F>::kLanes;
+#pragma unroll 1
+    for (uint32_t t = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64; t < total;
+         t += gridDim.x * (blockDim.x / 64)) {
+        uint32_t lo = 0, hi = nrec;  // the last record with start <= t
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (recs[mid].start <= t)
+                lo = mid;
+            else
+                hi = mid;
+        }
+        const FoldRec r = recs[lo];
+        const uint32_t off = (t - r.start) * kFoldSpan;
+        const uint32_t cnt = min(kFoldSpan, r.cnt - off);
+        const Coop<F> acc =
+            coop_reduce(coop_sum<F>(pool, r.src + off, cnt, group, kWaveGroups<F>), kWaveGroups<F>);
+        if (group == 0) coop_store<F>(pool, (size_t)out_base + t, acc);
     }
 }
 
-template <class T>
-__device__ __forceinline__ T shfl_xor_point(const T &p, int mask)
-{
-    T r;
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(&p);
-    uint32_t *dst = reinterpret_cast<uint32_t *>(&r);
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(T) / 4); ++i) dst[i] = (uint32_t)__shfl_xor((int)src[i], mask, 16);
-    return r;
-}
-
-// Completion classes: a bucket with m partials (m <= kMsmCompleteMax = 64
-// after folding) is summed by L = nextpow2(ceil(m / 8)) lanes (1, 2, 4 or 8:
-// at most 8 serial additions, then log2 L shuffle levels), so light buckets
-// do not drag idle lanes through a shuffle tree sized for the heaviest one.
-// Class c = log2 L; segment 4j + c lists job j's buckets of class c.
-__device__ __forceinline__ uint32_t complete_class(uint32_t m, uint32_t max_class)
-{
-    uint32_t c = 0;
-    while (c < max_class && (8u << c) < m) ++c;
-    return c;
-}
-
-// Buckets with no partial get S = infinity here; the others are appended to
-// their class list (one atomic per wave and class: a ballot ranks the lanes).
-template <class F>
-__global__ __launch_bounds__(256) void k_classify(const JobDev<F> *__restrict__ jobs, uint32_t max_class,
-                                                  uint32_t *__restrict__ class_count,
-                                                  uint32_t *__restrict__ class_list)
-{
-    const uint32_t j = blockIdx.y;
-    const JobDev<F> &jb = jobs[j];
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool in = k < jb.B;
-    const uint32_t m = in ? jb.reg_count[k] : 0u;
-    if (in && m == 0) jb.sums[k] = partial_t<F>::infinity();
-    const uint32_t c = complete_class(m, max_class);
-    const uint32_t lane = threadIdx.x & 63u;
-    uint32_t *list = class_list + (size_t)jb.list_off * kCompleteClasses;
-    for (uint32_t cc = 0; cc <= max_class; ++cc) {
-        const bool mine = in && m > 0 && c == cc;
-        const uint64_t mask = __ballot(mine);
-        if (mask == 0) continue;
-        const uint32_t leader = (uint32_t)__ffsll((unsigned long long)mask) - 1u;
-        uint32_t first = 0;
-        if (lane == leader) first = atomicAdd(&class_count[kCompleteClasses * j + cc], (uint32_t)__popcll(mask));
-        first = (uint32_t)__shfl((int)first, (int)leader);
-        if (mine) list[(size_t)cc * jb.B + first + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = k;
-    }
-}
-
-// Lane offsets of the completion segments: segment s = 4j + c takes
-// count * 2^c lanes, padded to whole waves (every wave completes buckets of
-// one segment, in aligned groups of 2^c lanes).  One workgroup.
-__global__ __launch_bounds__(1024) void k_complete_scan(const uint32_t *__restrict__ class_count, uint32_t S,
-                                                        uint32_t *__restrict__ base)
-{
-    __shared__ uint32_t part[1024];
-    auto span = [&](uint32_t s) -> uint32_t {
-        return ((class_count[s] << (s % kCompleteClasses)) + 63u) & ~63u;
-    };
-    const uint32_t per = (S + blockDim.x - 1) / blockDim.x;
-    const uint32_t beg = min(S, threadIdx.x * per), end = min(S, beg + per);
-    uint32_t sum = 0;
-    for (uint32_t s = beg; s < end; ++s) sum += span(s);
-    part[threadIdx.x] = sum;
-    __syncthreads();
-    for (uint32_t off = 1; off < blockDim.x; off <<= 1) {
-        const uint32_t t = threadIdx.x >= off ? part[threadIdx.x - off] : 0u;
-        __syncthreads();
-        part[threadIdx.x] += t;
-        __syncthreads();
-    }
-    uint32_t run = part[threadIdx.x] - sum;
-    for (uint32_t s = beg; s < end; ++s) {
-        base[s] = run;
-        run += span(s);
-    }
-    if (threadIdx.x == blockDim.x - 1) base[S] = part[threadIdx.x];
-}
-
-// Bucket completion: the 2^c lanes of a class-c bucket stride over its
+// Bucket completion: the 2^c lane groups of a class-c bucket stride over its
 // partials, then a shuffle tree of c levels; grid-stride over all segments.
 template <class F>
 __global__ __launch_bounds__(256) void k_complete(const JobDev<F> *__restrict__ jobs,
-                                                  const uint32_t *__restrict__ class_count,
+                                                  const partial_t<F> *__restrict__ pool,
+                                                  const uint32_t *__restrict__ seg_count,
                                                   const uint32_t *__restrict__ class_list,
-                                                  const uint32_t *__restrict__ base, uint32_t S)
+                                                  const uint32_t *__restrict__ seg_base, uint32_t S)
 {
-    const uint32_t total = base[S];
+    const uint32_t total = seg_base[S];
 #pragma unroll 1
     for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < total; g += gridDim.x * blockDim.x) {
-        const uint32_t s = find_segment(base, S, g);
+        const uint32_t s = find_segment(seg_base, S, g);
         const uint32_t j = s / kCompleteClasses, c = s % kCompleteClasses;
         const JobDev<F> &jb = jobs[j];
-        const uint32_t local = g - base[s];
-        const uint32_t idx = local >> c, lane = local & ((1u << c) - 1u);
-        const bool live = idx < class_count[s];
+        const uint32_t local = (g - seg_base[s]) / Coop<F>::kLanes;
+        const uint32_t idx = local >> c, group = local & ((1u << c) - 1u);
+        const bool live = idx < seg_count[s];
         const uint32_t k =
             live ? class_list[(size_t)jb.list_off * kCompleteClasses + (size_t)c * jb.B + idx] : 0u;
-        partial_t<F> acc = partial_t<F>::infinity();
-        if (live) {
-            const uint32_t start = jb.reg_start[k];
-            const uint32_t cnt = jb.reg_count[k];
-            for (uint32_t i = lane; i < cnt; i += (1u << c)) acc = partial_add(acc, jb.pool[start + i]);
-        }
-        for (uint32_t off = (1u << c) >> 1; off >= 1; off >>= 1)
-            acc = partial_add(acc, shfl_xor_point(acc, (int)off));
-        if (live && lane == 0) jb.sums[k] = acc;
+        Coop<F> acc = coop_sum<F>(pool, live ? jb.reg_start[k] : 0u, live ? jb.reg_count[k] : 0u, group, 1u << c);
+        acc = coop_reduce(acc, 1u << c);
+        if (live && group == 0) coop_store<F>(jb.sums, k, acc);
     }
 }
 
@@ -721,14 +729,15 @@ __global__ __launch_bounds__(256) void k_complete(const JobDev<F> *__restrict__ 
 // bit planes U_e, and U_{c-1} = S_B (bucket B = 2^(c-1) alone has bit c-1).
 //
 // One launch runs up to h levels from level t0: a workgroup loads 2^h
-// level-t0 blocks of one job into LDS and merges them level by level with a
-// barrier in between (one addition of latency per level, no launch or
-// global round trip), then stores the merged block to the other global
-// tree buffer (`src` names the one it reads).  Jobs whose tree ends earlier
-// run fewer levels; jobs already done return.
+// level-t0 blocks of one job into LDS and merges them level by level, a lane
+// group per addition, with a barrier in between (one addition of latency per
+// level, no launch or global round trip), then stores the merged block to the
+// other global tree buffer (`src` names the one it reads).  Jobs whose tree
+// ends earlier run fewer levels; jobs already done return.  LDS accesses are
+// one component (9 words, an odd stride) per lane: no bank conflicts.
 template <class F>
-__global__ __launch_bounds__(256) void k_tree_lds(const JobDev<F> *__restrict__ jobs, uint32_t t0, uint32_t h,
-                                                  uint32_t src)
+__global__ __launch_bounds__(kTreeThreads) void k_tree_lds(const JobDev<F> *__restrict__ jobs, uint32_t t0,
+                                                           uint32_t h, uint32_t src)
 {
     extern __shared__ uint8_t tree_lds[];
     const JobDev<F> &jb = jobs[blockIdx.y];
@@ -738,15 +747,17 @@ __global__ __launch_bounds__(256) void k_tree_lds(const JobDev<F> *__restrict__ 
     const uint32_t cap = (1u << h) * (t0 + 1);
     partial_t<F> *buf[2] = {reinterpret_cast<partial_t<F> *>(tree_lds),
                             reinterpret_cast<partial_t<F> *>(tree_lds) + cap};
+    const uint32_t group = threadIdx.x / Coop<F>::kLanes, groups = blockDim.x / Coop<F>::kLanes;
 
     const uint32_t nin = (1u << lv) * (t0 + 1);
-    const uint32_t blk0 = blockIdx.x << lv;
-    for (uint32_t idx = threadIdx.x; idx < nin; idx += blockDim.x) {
-        const uint32_t blk = blk0 + idx / (t0 + 1), ent = idx % (t0 + 1);
-        if (t0 == 0)
-            buf[0][idx] = blk == 0 ? partial_t<F>::infinity() : jb.sums[blk - 1];
-        else
-            buf[0][idx] = jb.tree[src][(size_t)blk * (t0 + 1) + ent];
+    const uint32_t first = (blockIdx.x << lv) * (t0 + 1);
+    for (uint32_t idx = group; idx < nin; idx += groups) {
+        Coop<F> v = Coop<F>::infinity();
+        if (t0 != 0)
+            v = coop_load<F>(jb.tree[src], first + idx);
+        else if (first + idx != 0)
+            v = coop_load<F>(jb.sums, first + idx - 1);
+        coop_store<F>(buf[0], idx, v);
     }
     __syncthreads();
     for (uint32_t s = 0; s < lv; ++s) {
@@ -754,30 +765,27 @@ __global__ __launch_bounds__(256) void k_tree_lds(const JobDev<F> *__restrict__ 
         const bool last = (t + 1 == jb.c - 1);
         const partial_t<F> *in = buf[s & 1];
         partial_t<F> *out = buf[(s + 1) & 1];
-        const uint32_t nout = (1u << (lv - s - 1)) * E;
-        for (uint32_t idx = threadIdx.x; idx < nout; idx += blockDim.x) {
-            const uint32_t b = idx / E, e = idx % E;
-            const partial_t<F> *l = in + (size_t)(2 * b) * (t + 1);
-            const partial_t<F> *r = l + (t + 1);
-            // one addition site for every lane: the P_e and T merges do not
-            // diverge into two serial additions
-            const uint32_t q = e < t ? e : t;
-            partial_t<F> o = partial_add(l[q], r[q]);
-            if (e == t)
-                o = r[t];
-            else if (e > t && last)
-                o = jb.sums[jb.B - 1];
-            if (last)
-                jb.planes[e] = partial_plane(o);
-            else
-                out[idx] = o;
+        const uint32_t adds = (1u << (lv - s - 1)) * (t + 1);
+        for (uint32_t idx = group; idx < adds; idx += groups) {
+            const uint32_t b = idx / (t + 1), e = idx % (t + 1);
+            const Coop<F> l = coop_load<F>(in, (size_t)(2 * b) * (t + 1) + e);
+            const Coop<F> r = coop_load<F>(in, (size_t)(2 * b + 1) * (t + 1) + e);
+            const bool top = e == t;  // T: the sum goes behind P_t, which is r itself
+            const Coop<F> o = last && top ? coop_load<F>(jb.sums, jb.B - 1) : coop_add(l, r);
+            if (last) {
+                coop_store_plane<F>(jb.planes + (top ? t + 1 : e), o);
+                if (top) coop_store_plane<F>(jb.planes + t, r);
+            } else {
+                coop_store<F>(out, (size_t)b * E + (top ? t + 1 : e), o);
+                if (top) coop_store<F>(out, (size_t)b * E + t, r);
+            }
         }
         __syncthreads();
     }
     const uint32_t t1 = t0 + lv;
     if (t1 < jb.c - 1)
-        for (uint32_t e = threadIdx.x; e <= t1; e += blockDim.x)
-            jb.tree[src ^ 1u][(size_t)blockIdx.x * (t1 + 1) + e] = buf[lv & 1][e];
+        for (uint32_t e = group; e <= t1; e += groups)
+            coop_store<F>(jb.tree[src ^ 1u], (size_t)blockIdx.x * (t1 + 1) + e, coop_load<F>(buf[lv & 1], e));
 }
 
 // Base preparation: normalise the reference-layout Jacobian point and store
@@ -849,15 +857,28 @@ uint64_t msm_schedule_bytes(const MsmPlan &p)
     return p.max_entries() * 4 + (uint64_t)p.B * 4 * 3 + blocks * p.B * 4 + 32;
 }
 
+// Partial sums of all fold launches: a launch turns more than kMsmCompleteMax
+// partials of a bucket into ceil(m / kFoldSpan), fewer than m / 32.
+static uint64_t fold_outputs(uint64_t pieces) { return pieces / 32 + 1; }
+static uint64_t fold_outputs_total(uint64_t pieces)
+{
+    uint64_t sum = 0;
+    for (uint32_t L = 0; L < kMaxFoldLaunches; ++L) sum += pieces = fold_outputs(pieces);
+    return sum;
+}
+// Fold records of one launch: buckets with more than kMsmCompleteMax partials.
+static uint64_t fold_records(uint64_t pieces) { return pieces / (kMsmCompleteMax + 1) + 1; }
+
 template <class F>
 uint64_t msm_job_bytes(const MsmPlan &p)
 {
-    const uint64_t total = msm_partial_capacity(p, p.max_pieces(msm_target_pieces_log()), nullptr, nullptr);
-    // partial sums; per bucket: sums and two tree levels, region start,
-    // count and fold start, the completion class lists; the bit planes; and
+    const uint64_t pieces = p.max_pieces(msm_target_pieces_log());
+    // partial sums; per bucket: sums and two tree levels, region start and
+    // count, the completion class lists; fold records; the bit planes; and
     // the job's fixed records (job table, class counters, piece offsets)
-    return total * sizeof(partial_t<F>) + (uint64_t)p.B * (3 * sizeof(partial_t<F>) + 12 + 4 * kCompleteClasses) +
-           p.c * sizeof(Xyzz<F>) + 1024;
+    return (pieces + fold_outputs_total(pieces)) * sizeof(partial_t<F>) +
+           (uint64_t)p.B * (3 * sizeof(partial_t<F>) + 8 + 4 * kCompleteClasses) +
+           fold_records(pieces) * kMaxFoldLaunches * sizeof(FoldRec) + p.c * sizeof(Xyzz<F>) + 1024;
 }
 
 template <class F>
@@ -1038,43 +1059,44 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
     std::vector<const void *> key = layout_key(jobs);
     if (key == key_) return;
     const uint32_t J = (uint32_t)jobs.size();
-    // Per job, sized by its own plan: the partial-sum pool (level-0 pieces,
-    // then each fold level's worst case) and the per-bucket arrays.
-    std::vector<uint64_t> pool_off(J + 1, 0), b_off(J + 1, 0), b1_off(J + 1, 0);
-    std::vector<std::array<uint32_t, kMaxFoldLevels>> level_base(J);
+    // Per job, sized by its own plan: its level-0 partials in the pool, then
+    // the fold launches' outputs of all jobs; and the per-bucket arrays.
+    std::vector<uint64_t> pool_off(J + 1, 0), b_off(J + 1, 0);
     fold_levels_ = 0;
-    fold_cap_.assign(kMaxFoldLevels, 0);
-    thread_base_.assign(J + 1, 0);
     for (uint32_t j = 0; j < J; ++j) {
         const MsmPlan &p = jobs[j].sched->plan();
         NKR_REQUIRE(jobs[j].bases->plan().n == p.n && jobs[j].bases->plan().c == p.c,
                     "MSM bases and schedule disagree");
         const uint64_t pieces = job_max_pieces(jobs[j]);
-        thread_base_[j + 1] = thread_base_[j] + pieces;
-        uint64_t lb[kMaxFoldLevels], lc[kMaxFoldLevels];
         uint32_t levels = 0;
-        const uint64_t base = msm_partial_capacity(p, pieces, &levels, lb, lc);
-        NKR_REQUIRE(base < (1ull << 32), "MSM partial pool exceeds 32-bit indexing");
-        for (uint32_t L = 0; L < kMaxFoldLevels; ++L) {
-            level_base[j][L] = (uint32_t)lb[L];
-            fold_cap_[L] = std::max<uint64_t>(fold_cap_[L], lc[L]);
-        }
+        (void)msm_partial_capacity(p, pieces, &levels, nullptr);
         fold_levels_ = std::max(fold_levels_, levels);
-        pool_off[j + 1] = pool_off[j] + base;
+        pool_off[j + 1] = pool_off[j] + pieces;
         b_off[j + 1] = b_off[j] + p.B;
-        b1_off[j + 1] = b1_off[j] + p.B + 1;
     }
+    piece_bound_ = pool_off[J];
+    uint64_t at = piece_bound_, outs = piece_bound_;
+    for (uint32_t L = 0; L < kMaxFoldLaunches; ++L) {
+        fold_base_[L] = (uint32_t)at;
+        outs = fold_outputs(outs);
+        fold_cap_[L] = outs;
+        at += outs;
+    }
+    NKR_REQUIRE(at < (1ull << 32), "MSM partial pool exceeds 32-bit indexing");
+    rec_cap_ = fold_records(piece_bound_);
     // grow-only: a batch whose composition changes from call to call reuses them
-    pool_.ensure(pool_off[J]);
+    pool_.ensure(at);
     sums_.ensure(b_off[J]);
     tree_[0].ensure(b_off[J]);
     tree_[1].ensure(b_off[J]);
     reg_start_.ensure(b_off[J]);
     reg_count_.ensure(b_off[J]);
-    fold_start_.ensure(b1_off[J]);
 
     static_assert(std::is_trivially_copyable<JobDev<F>>::value, "job records are raw-copied");
-    JobDev<F> *host = reinterpret_cast<JobDev<F> *>(jobs_stage_.reuse(sizeof(JobDev<F>) * J));
+    const size_t jobs_bytes = (sizeof(JobDev<F>) * J + 15) & ~size_t(15);
+    const size_t table_bytes = jobs_bytes + sizeof(fold_base_);
+    uint8_t *st = jobs_stage_.reuse(table_bytes);
+    JobDev<F> *host = reinterpret_cast<JobDev<F> *>(st);
     for (uint32_t j = 0; j < J; ++j) {
         const MsmJob<F> &jb = jobs[j];
         JobDev<F> &d = host[j];
@@ -1082,33 +1104,37 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
         d.sorted = jb.sched->sorted_.get();
         d.bucket_start = jb.sched->bucket_start_.get();
         d.piece_start = job_piece_start(jb);
-        d.piece_max = job_counters(jb) + 2;
         d.piece_len = job_counters(jb) + 3;
-        d.pool = pool_.get() + pool_off[j];
         d.reg_start = reg_start_.get() + b_off[j];
         d.reg_count = reg_count_.get() + b_off[j];
-        d.fold_start = fold_start_.get() + b1_off[j];
         d.sums = sums_.get() + b_off[j];
         d.tree[0] = tree_[0].get() + b_off[j];
         d.tree[1] = tree_[1].get() + b_off[j];
         d.planes = jb.planes;
+        d.pool_off = (uint32_t)pool_off[j];
         d.B = jb.sched->plan().B;
         d.c = jb.sched->plan().c;
         d.list_off = (uint32_t)b_off[j];
-        for (uint32_t L = 0; L < kMaxFoldLevels; ++L) d.level_base[L] = level_base[j][L];
     }
-    thread_total_ = thread_base_[J];
-    // completion lanes: at most 8 per bucket, plus each segment's padding
+    std::memcpy(st + jobs_bytes, fold_base_, sizeof(fold_base_));
+    // completion lanes: a bucket's lane groups, plus each segment's padding
     complete_bound_ = 0;
-    for (uint32_t j = 0; j < J; ++j) complete_bound_ += (uint64_t)host[j].B * 8 + kCompleteClasses * 64;
-    NKR_REQUIRE(complete_bound_ < (1ull << 32) && thread_total_ < (1ull << 32),
-                "MSM batch too large for 32-bit work indices");
-    complete_base_.ensure(kCompleteClasses * J + 1);
+    for (uint32_t j = 0; j < J; ++j)
+        complete_bound_ += (uint64_t)host[j].B * 64 + kCompleteClasses * 64;
+    NKR_REQUIRE(complete_bound_ < (1ull << 32), "MSM batch too large for 32-bit work indices");
+    seg_base_.ensure(kCompleteClasses * J + 1);
+    seg_count_.ensure(kCompleteClasses * J);
     class_count_.ensure(kCompleteClasses * J);
     class_list_.ensure(kCompleteClasses * b_off[J]);
-    jobs_dev_.ensure(sizeof(JobDev<F>) * J);
-    thread_base_dev_.ensure(J + 1);  // actual piece offsets, filled on the device per run
-    NKR_HIP(hipMemcpyAsync(jobs_dev_.get(), host, sizeof(JobDev<F>) * J, hipMemcpyHostToDevice, stream));
+    recs_.ensure(rec_cap_ * kMaxFoldLaunches * sizeof(FoldRec));
+    state_.ensure(sizeof(ReduceState));
+    jobs_dev_.ensure(table_bytes);
+    piece_base_.ensure(J + 1);  // filled on the device per run
+    // k_reduce_plan leaves its counters cleared; new buffers start so (never
+    // inside a captured graph, which reuses the layout of an eager run)
+    NKR_HIP(hipMemsetAsync(class_count_.get(), 0, class_count_.bytes(), stream));
+    NKR_HIP(hipMemsetAsync(state_.get(), 0, sizeof(ReduceState), stream));
+    NKR_HIP(hipMemcpyAsync(jobs_dev_.get(), st, table_bytes, hipMemcpyHostToDevice, stream));
     jobs_stage_.uploaded(stream);
     key_ = key;
 }
@@ -1125,11 +1151,35 @@ void MsmBatch<F>::run(const std::vector<MsmJob<F>> &jobs, hipStream_t stream, St
         Bmax = std::max(Bmax, jb.sched->plan().B);
         cmax = std::max(cmax, jb.sched->plan().c);
     }
-    const JobDev<F> *jd = reinterpret_cast<const JobDev<F> *>(jobs_dev_.get());
+    const uint8_t *table = jobs_dev_.get();
+    const JobDev<F> *jd = reinterpret_cast<const JobDev<F> *>(table);
+    const uint32_t *fold_base_dev =
+        reinterpret_cast<const uint32_t *>(table + ((sizeof(JobDev<F>) * J + 15) & ~size_t(15)));
+    ReduceState *state = reinterpret_cast<ReduceState *>(state_.get());
+    FoldRec *recs = reinterpret_cast<FoldRec *>(recs_.get());
 
-    k_regions_init<F><<<dim3(div_up(Bmax, 256), J), 256, 0, stream>>>(jd, class_count_.get());
-    NKR_LAUNCH_CHECK();
-    k_piece_scan<F><<<1, 1024, 0, stream>>>(jd, J, thread_base_dev_.get());
+    // A launch that fails half way leaves the plan's counters unknown: the
+    // next run lays the batch out again.
+    struct Relayout {
+        std::vector<const void *> *key;
+        ~Relayout()
+        {
+            if (key) key->clear();
+        }
+    } relayout{&key_};
+
+    // Completion: as many lane groups per bucket as leave each about `serial`
+    // partials.  One addition deep per group while the launch would not fill
+    // the chip's 65536 lanes twice, then longer runs (idle groups in the
+    // shuffle levels are the price of short ones).
+    uint32_t max_class = 0;
+    while ((2u << max_class) <= std::min(msm_complete_lanes_cap(), kWaveGroups<F>)) ++max_class;
+    const uint64_t lanes = piece_bound_ * Coop<F>::kLanes;
+    const uint32_t serial = (uint32_t)std::min<uint64_t>(16, std::max<uint64_t>(1, lanes / (2 * 65536)));
+    const uint32_t S = kCompleteClasses * J;
+    k_reduce_plan<F><<<dim3(div_up(Bmax, 256), J), 256, 0, stream>>>(
+        jd, J, max_class, serial, state, recs, (uint32_t)rec_cap_, fold_base_dev, class_count_.get(),
+        class_list_.get(), piece_base_.get(), seg_count_.get(), seg_base_.get());
     NKR_LAUNCH_CHECK();
     // the accumulation stage brackets exactly the k_accumulate launch
     const int acc_stage = std::is_same<F, fq2_t>::value ? kStageAccumulateG2 : kStageAccumulate;
@@ -1141,64 +1191,56 @@ void MsmBatch<F>::run(const std::vector<MsmJob<F>> &jobs, hipStream_t stream, St
     // as they free up instead of waiting for the whole launch (dense 2^20
     // Poseidon-style proof 12.0 -> 11.2 ms and 64-proof mix 33.5-34.0 ->
     // 31.2-32.4 ms with the witness in HBM, on MI355X).
-    const uint64_t blocks = div_up(thread_total_, kAccThreads);
-    k_accumulate<F><<<(uint32_t)std::max<uint64_t>(blocks, 1), kAccThreads, 0, stream>>>(jd, thread_base_dev_.get(), J);
+    const uint64_t blocks = div_up(piece_bound_, kAccThreads);
+    k_accumulate<F><<<(uint32_t)std::max<uint64_t>(blocks, 1), kAccThreads, 0, stream>>>(jd, piece_base_.get(), J,
+                                                                                        pool_.get());
     NKR_LAUNCH_CHECK();
     if (timer) {
         timer->end(acc_stage, stream);
         timer->begin(kStageFold, stream);
     }
-    // Fold levels the largest bucket of any job needs: read from the host
+    // Fold launches the largest bucket of any job needs: read from the host
     // copy of the schedules' counters.  The accumulation is already queued,
     // so this wait overlaps the GPU's work instead of stalling it.
-    uint32_t folds = 0;
+    uint32_t levels = 0;
     if (graph) {
-        folds = fold_levels_;
+        levels = fold_levels_;
     } else {
         for (const auto &jb : jobs) {
             const uint64_t cnt = (jb.alt ? jb.sched->alt_totals_host() : jb.sched->totals_host())[2];
-            folds = std::max(folds, msm_fold_levels(cnt));
+            levels = std::max(levels, msm_fold_levels(cnt));
         }
     }
-    NKR_REQUIRE(folds <= fold_levels_, "MSM bucket exceeds the partial-sum capacity");
-    for (uint32_t L = 0; L < folds; ++L) {
-        k_fold_scan<F><<<J, 256, 0, stream>>>(jd);
-        NKR_LAUNCH_CHECK();
-        k_fold<F><<<dim3(div_up(fold_cap_[L], 256), J), 256, 0, stream>>>(jd, L);
-        NKR_LAUNCH_CHECK();
-        k_fold_retarget<F><<<dim3(div_up(Bmax, 256), J), 256, 0, stream>>>(jd, L);
+    NKR_REQUIRE(levels <= fold_levels_, "MSM bucket exceeds the partial-sum capacity");
+    for (uint32_t L = 0; L * kFoldLevelsPerLaunch < levels; ++L) {
+        const uint64_t blocks = std::min<uint64_t>(div_up(fold_cap_[L], 4), 1024);
+        k_fold<F><<<(uint32_t)blocks, 256, 0, stream>>>(state, recs + (size_t)L * rec_cap_, L, fold_base_[L],
+                                                      pool_.get());
         NKR_LAUNCH_CHECK();
     }
-    uint32_t max_class = 0;
-    while (max_class + 1 < kCompleteClasses && (2u << max_class) <= msm_complete_lanes_cap()) ++max_class;
-    k_classify<F><<<dim3(div_up(Bmax, 256), J), 256, 0, stream>>>(jd, max_class, class_count_.get(),
-                                                                   class_list_.get());
-    NKR_LAUNCH_CHECK();
-    const uint32_t S = kCompleteClasses * J;
-    k_complete_scan<<<1, 1024, 0, stream>>>(class_count_.get(), S, complete_base_.get());
-    NKR_LAUNCH_CHECK();
     {
         const uint64_t blocks = std::min<uint64_t>(div_up(complete_bound_, 256), resident_blocks<k_complete<F>>());
         k_complete<F><<<(uint32_t)std::max<uint64_t>(blocks, 1), 256, 0, stream>>>(
-            jd, class_count_.get(), class_list_.get(), complete_base_.get(), S);
+            jd, pool_.get(), seg_count_.get(), class_list_.get(), seg_base_.get(), S);
     }
     NKR_LAUNCH_CHECK();
     // bit-plane tree: as many levels per launch as two LDS buffers of 2^h
-    // level-t blocks allow; a workgroup has as many lanes as its widest
-    // level has merges (whole waves, at most 256), so no idle wave holds a
-    // SIMD's registers
+    // level-t blocks allow; a workgroup has a lane group per addition of its
+    // widest level (whole waves, at most kTreeThreads)
     for (uint32_t t = 0, src = 0; t + 1 <= cmax - 1; src ^= 1u) {
         uint32_t h = 1;
-        while (t + h < cmax - 1 && 2 * (size_t(2) << h) * (t + 1) * sizeof(partial_t<F>) <= tree_lds_bytes<F>())
-            ++h;
+        while (t + h < cmax - 1 && 2 * (size_t(2) << h) * (t + 1) * sizeof(partial_t<F>) <= kTreeLds) ++h;
         const size_t lds = 2 * (size_t(1) << h) * (t + 1) * sizeof(partial_t<F>);
-        const uint32_t widest = (1u << (h - 1)) * (t + 2);
-        const uint32_t lanes = std::min<uint32_t>(256, (uint32_t)div_up(widest, 64) * 64);
+        uint32_t widest = 0;
+        for (uint32_t s = 0; s < h; ++s) widest = std::max(widest, (1u << (h - 1 - s)) * (t + s + 1));
+        const uint32_t lanes =
+            std::min<uint32_t>(kTreeThreads, (uint32_t)div_up(widest * Coop<F>::kLanes, 64) * 64);
         k_tree_lds<F><<<dim3(Bmax >> (t + h), J), lanes, lds, stream>>>(jd, t, h, src);
         NKR_LAUNCH_CHECK();
         t += h;
     }
     if (timer) timer->end(kStageFold, stream);
+    relayout.key = nullptr;
 }
 
 template <class F>
