@@ -99,7 +99,8 @@ int nkr_g16_ctx_create(const nkr_g16_circuit *circuit, const nkr_g16_pk *pk, int
  *   ntt_radix_log        2 or 3: register radix of the transform rounds
  *   ntt_split_policy     1 + policy: 1 balanced passes, 2 full last pass
  *   msm_target_pieces_log  2^k accumulation pieces per MSM launch, 12..24
- *   witness_g1_piece_min   shortest piece of the witness G1 MSMs, 1..64 */
+ *   witness_g1_piece_min   shortest piece of the G1 MSMs (the witness ones and
+ *                          H share a launch), 1..64 */
 typedef struct {
     uint32_t witness_window_bits, h_window_bits;
     uint32_t ntt_lds_log, ntt_radix_log, ntt_split_policy;
@@ -323,12 +324,12 @@ int nkr_fr_ntt_dev_noalloc(void *data_dev, uint32_t log_n, int kind, void *strea
  * measurement. */
 int nkr_ntt_set_shape(uint32_t lds_log, uint32_t radix_log, uint32_t split_policy);
 
-/* MSM tuning knobs for every MSM run afterwards: the accumulation splits
- * each bucket's entries into pieces summed by one thread, with the piece
- * length chosen on the device so that a vector has about 2^target_pieces_log
- * pieces (10 .. 22); at most complete_lanes_cap lanes (1, 2, 4, 8 or 16)
- * then sum one bucket's pieces.  Set while no proof runs.  Results do not
- * depend on either; the defaults (19, 16) are chosen by measurement. */
+/* MSM tuning knobs for every MSM run afterwards: the accumulation splits the
+ * sorted entries of a launch evenly over 2^target_pieces_log threads (10 ..
+ * 22); at most complete_lanes_cap lane groups (1, 2, 4, 8 or 16) then sum one
+ * bucket's partial sums.  Set while no proof runs.  Results do not depend on
+ * either; unset, the library picks the threads by the number of entries and
+ * up to 16 lane groups, chosen by measurement. */
 int nkr_msm_set_shape(uint32_t target_pieces_log, uint32_t complete_lanes_cap);
 
 /* y = M * z for one CSR matrix (host memory). */

@@ -41,11 +41,7 @@ void parallel_for(size_t n, Fn fn)
 
 size_t align16(size_t x) { return (x + 15) & ~size_t(15); }
 
-constexpr uint32_t kBatchPiece = 32;
-
 }  // namespace
-
-MsmPlan batch_plan(const MsmPlan &plan) { return plan.with_piece(kBatchPiece); }
 
 BatchProver::BatchProver(int device) : device_(device)
 {
@@ -229,7 +225,7 @@ void BatchProver::prove(const std::vector<BatchItem> &items)
             for (size_t i = 0; i < K; ++i) {
                 Groth16Prover &g = *items[i].ctx;
                 Slot &sl = *slots_[i];
-                wsorts.push_back({&sl.wsched, sl.z.get(), batch_plan(g.wplan_)});
+                wsorts.push_back({&sl.wsched, sl.z.get(), g.wplan_});
                 g2jobs.push_back({&g.b2_, &sl.wsched, planes_2_.get() + p2_off[i]});
             }
             sort_w_.build(wsorts, stream2_, graph);
@@ -297,7 +293,7 @@ void BatchProver::prove(const std::vector<BatchItem> &items)
         for (size_t i = 0; i < K; ++i) {
             Groth16Prover &g = *items[i].ctx;
             Slot &sl = *slots_[i];
-            hsorts.push_back({&sl.hsched, sl.pa.get(), batch_plan(g.hplan_)});
+            hsorts.push_back({&sl.hsched, sl.pa.get(), g.hplan_});
         }
         sort_h_.build(hsorts, stream_, graph);
         NKR_HIP(hipStreamWaitEvent(stream_, ev_wsched_, 0));

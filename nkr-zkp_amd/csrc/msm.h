@@ -17,9 +17,9 @@
 //  * Several MSMs run as one batch ("jobs"): every stage below is a single
 //    launch over all jobs, so the latency of each reduction level is paid
 //    once per batch, not once per MSM.
-//      1. accumulate: one thread sums a piece of 4..64 entries of one bucket
-//         (mixed affine additions into XYZZ); the launch holds only the
-//         resident waves, which take pieces by grid stride;
+//      1. accumulate: every lane sums an equally long run of the sorted
+//         entries, one partial sum per bucket it meets (mixed affine
+//         additions into XYZZ);
 //      2. fold: buckets left with more than 64 partial sums (skewed digit
 //         distributions, e.g. witnesses that are mostly 0 or 1) are folded
 //         64:1, a wave per sum, until they are not; others are untouched;
@@ -47,11 +47,14 @@
 
 namespace nkr {
 
-// Process-wide MSM tuning knobs: the target piece count (2^target_log, 10 ..
-// 22) and the most lanes that complete one bucket (1 .. 16, a power of two).
-// Set them before proving, not while proofs run.
+// Process-wide MSM tuning knobs: the accumulation lanes of a launch
+// (2^target_log, 10 .. 22; until it is set, MsmLanes' own) and the most lane
+// groups that complete one bucket (1 .. 16, a power of two).  Set them before
+// proving, not while proofs run.
 void msm_set_shape(uint32_t target_pieces_log, uint32_t complete_lanes_cap);
-uint32_t msm_target_pieces_log();
+// The lanes of a group's launches: its own rule, or 2^target_log, or (0) the
+// process-wide setting.
+MsmLanes msm_lanes(bool g2, uint32_t target_log = 0, uint32_t piece_min = 1);
 uint32_t msm_complete_lanes_cap();
 
 // Device bytes of one schedule (MsmSchedule) and of one MSM job's partial
@@ -86,79 +89,37 @@ public:
     // Sizes the buffers for `plan`; returns the scalars per sort workgroup.
     uint32_t prepare(const MsmPlan &plan);
     const MsmPlan &plan() const { return plan_; }
-    uint64_t max_pieces() const { return plan_.max_pieces(target_log_); }
-    // Device counters: [0] entries (non-zero digits), [1] level-0 pieces,
-    // [2] largest piece count of a bucket, [3] piece length.
+    // Device counter: entries (non-zero digits).
     const uint32_t *totals() const { return bucket_start_.get() + plan_.B; }
-    // The same four counters on the host; blocks until the sort that writes
-    // them has run.
-    const uint32_t *totals_host() const
-    {
-        host_stage_->wait();
-        return host_totals_;
-    }
     // Sort workgroups for n scalars (each histograms a contiguous slice).
     static uint32_t sort_blocks(uint32_t n);
-
-    // A second split of the same sorted entries into pieces of at least
-    // `piece_lo` entries (chosen on the device as in build, within
-    // [piece_lo, max(piece_lo, plan piece_hi)]), computed by the next builds:
-    // one scalar vector feeds MSMs in different groups, and a G1 MSM
-    // completes its buckets faster from fewer, longer pieces while the G2
-    // MSM, at one wave per SIMD, needs the short ones.  0 turns it off.
-    // Jobs select it with MsmJob::alt.
-    void set_alt_pieces(uint32_t piece_lo) { alt_piece_lo_ = piece_lo; }
-    // 2^target_log level-0 pieces per build instead of the process-wide
-    // setting (0 restores it).
-    void set_target_log(uint32_t target_log) { target_override_ = target_log; }
-    uint64_t alt_max_pieces() const
-    {
-        NKR_REQUIRE(alt_piece_lo_ > 0, "an MSM job reads the second piece split of a schedule that has none");
-        MsmPlan p = plan_;
-        p.piece_lo = alt_piece_lo_;
-        p.piece_hi = std::max(alt_piece_lo_, p.piece_hi);
-        return p.max_pieces(target_log_);
-    }
-    const uint32_t *alt_totals_host() const
-    {
-        NKR_REQUIRE(alt_piece_lo_ > 0, "an MSM job reads the second piece split of a schedule that has none");
-        return totals_host() + 4;
-    }
 
     // Device bytes held, and their release (the next prepare reallocates).
     uint64_t device_bytes() const
     {
-        return sorted_.bytes() + count_.bytes() + bucket_start_.bytes() + piece_start_.bytes() +
-               block_count_.bytes() + alt_piece_start_.bytes();
+        return sorted_.bytes() + bucket_start_.bytes() + in_tile_.bytes() + tile_total_.bytes() +
+               block_count_.bytes();
     }
     void release_device()
     {
         sorted_.release();
-        count_.release();
         bucket_start_.release();
-        piece_start_.release();
+        in_tile_.release();
+        tile_total_.release();
         block_count_.release();
-        alt_piece_start_.release();
     }
 
     MsmPlan plan_;
     uint32_t blocks_ = 0;
-    uint32_t target_log_ = kMsmTargetPiecesLog;  // as of the last prepare
     DeviceBuffer<uint32_t> sorted_;        // entries: sign << 31 | (w * n + i)
-    DeviceBuffer<uint32_t> count_;         // per bucket (B)
-    DeviceBuffer<uint32_t> bucket_start_;  // B + 1, then the totals above, then the second split's
-    DeviceBuffer<uint32_t> piece_start_;   // B + 1
+    DeviceBuffer<uint32_t> bucket_start_;  // B + 1, the last the entry count
+    DeviceBuffer<uint32_t> in_tile_;       // B: bucket starts within 64-bucket tiles
+    DeviceBuffer<uint32_t> tile_total_;    // entries of each tile
     DeviceBuffer<uint32_t> block_count_;   // blocks x B: per-workgroup counts, then offsets
-    PinnedStaging<uint32_t> own_totals_;   // host copy of the counters (build)
-    uint32_t alt_piece_lo_ = 0;
-    uint32_t target_override_ = 0;
-    DeviceBuffer<uint32_t> alt_piece_start_;  // B + 1 (its counters follow the first split's)
-    const uint32_t *host_totals_ = nullptr;
-    const PinnedStaging<uint32_t> *host_stage_ = nullptr;
 };
 
-// Many schedules with one launch per sort phase (zero, histogram, scan,
-// scatter) instead of four launches per schedule.  Same result as
+// Many schedules with one launch per sort phase (histogram, scan, scatter)
+// instead of three launches per schedule.  Same result as
 // MsmSchedule::build for each of them.
 class MsmScheduleBatch {
 public:
@@ -168,23 +129,16 @@ public:
         MsmPlan plan;
     };
     // graph: the launches are being captured into a graph that is replayed
-    // later, so nothing here may wait for or read device results on the host
-    // (the schedules' counters are not copied back and no staging event is
+    // later, so nothing here may wait on the host (no staging event is
     // recorded; the caller synchronises its streams before the staging
     // buffers are written again).
     void build(const std::vector<Item> &items, hipStream_t stream, bool graph = false);
-    uint64_t device_bytes() const { return table_.bytes() + totals_dev_.bytes(); }
-    void release_device()
-    {
-        table_.release();
-        totals_dev_.release();
-    }
+    uint64_t device_bytes() const { return table_.bytes(); }
+    void release_device() { table_.release(); }
 
 private:
     PinnedStaging<uint8_t> stage_;
     DeviceBuffer<uint8_t> table_;
-    DeviceBuffer<uint32_t> totals_dev_;
-    PinnedStaging<uint32_t> totals_host_;
 };
 
 // The form of the partial sums between the accumulation and the bit planes:
@@ -211,17 +165,20 @@ struct MsmJob {
     const MsmBases<F> *bases;
     const MsmSchedule *sched;
     Xyzz<F> *planes;   // device output: c points U_0 .. U_{c-1}
-    bool alt = false;  // use the schedule's second piece split (set_alt_pieces)
 };
 
 // Runs a batch of MSMs of one group (all with the same window width).
 template <class F>
 class MsmBatch {
 public:
-    // graph: as MsmScheduleBatch::build; the fold levels are then launched
-    // for the largest bucket the partial-sum capacity allows (levels a batch
-    // does not need find nothing to fold) instead of for the counters read
-    // back from the schedules.
+    // The lanes of the batch's accumulations (msm_lanes), instead of the
+    // process-wide setting as of each layout.
+    void set_lanes(const MsmLanes &lanes)
+    {
+        own_lanes_ = lanes;
+        have_lanes_ = true;
+    }
+    // graph: as MsmScheduleBatch::build.
     void run(const std::vector<MsmJob<F>> &jobs, hipStream_t stream, StageTimer *timer = nullptr,
              bool graph = false);
     // Device bytes held by the batch's work buffers, and their release (the
@@ -229,7 +186,7 @@ public:
     uint64_t device_bytes() const
     {
         return seg_base_.bytes() + seg_count_.bytes() + class_count_.bytes() + class_list_.bytes() +
-               jobs_dev_.bytes() + piece_base_.bytes() + pool_.bytes() + sums_.bytes() + reg_start_.bytes() +
+               jobs_dev_.bytes() + lane_base_.bytes() + pool_.bytes() + sums_.bytes() + reg_start_.bytes() +
                reg_count_.bytes() + recs_.bytes() + state_.bytes() + tree_[0].bytes() + tree_[1].bytes();
     }
     void release_device()
@@ -239,7 +196,7 @@ public:
         class_count_.release();
         class_list_.release();
         jobs_dev_.release();
-        piece_base_.release();
+        lane_base_.release();
         pool_.release();
         sums_.release();
         tree_[0].release();
@@ -261,9 +218,12 @@ private:
     uint32_t fold_base_[kMaxFoldLevels / 3] = {};  // where each fold launch's outputs start in pool_
     uint64_t fold_cap_[kMaxFoldLevels / 3] = {};   // and their largest number
     uint64_t rec_cap_ = 0;                         // fold records of one launch at most
-    uint64_t piece_bound_ = 0;                     // level-0 pieces of all jobs at most
+    uint64_t lane_bound_ = 0;                      // accumulation lanes of all jobs at most
+    uint64_t bucket_total_ = 0;                    // buckets of all jobs
+    MsmLanes lanes_{}, own_lanes_{};               // lanes_: as of the layout
+    bool have_lanes_ = false;
     uint64_t complete_bound_ = 0;                  // completion lanes at most
-    DeviceBuffer<uint32_t> seg_base_, seg_count_, class_count_, class_list_, piece_base_;
+    DeviceBuffer<uint32_t> seg_base_, seg_count_, class_count_, class_list_, lane_base_;
     DeviceBuffer<uint8_t> jobs_dev_, recs_, state_;
     PinnedStaging<uint8_t> jobs_stage_;
     DeviceBuffer<partial_t<F>> pool_, sums_, tree_[2];

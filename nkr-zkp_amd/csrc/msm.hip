@@ -32,6 +32,10 @@ constexpr uint32_t kCompleteClasses = 5;
 constexpr uint32_t kFoldLevelsPerLaunch = 3;
 constexpr uint32_t kFoldSpan = 64;
 static_assert(kFoldSpan == kMsmFoldIn * kMsmFoldIn * kMsmFoldIn && kFoldSpan <= kMsmCompleteMax, "fold span");
+// Partials of a bucket that are completed without a fold: 8 lane groups sum
+// this many in fewer additions of latency than a fold and a completion.
+constexpr uint32_t kDirectMax = 128;
+constexpr uint32_t kPlanThreads = 1024;
 constexpr uint32_t kMaxFoldLaunches = kMaxFoldLevels / kFoldLevelsPerLaunch;
 // Lane groups of an addition per wave (coop29.h).
 template <class F>
@@ -47,7 +51,7 @@ struct FoldRec {
 // `fold_ctr` are zero between launches; fold_count holds their last values.
 struct ReduceState {
     uint32_t ticket;
-    uint32_t pad;
+    uint32_t piece;  // entries per accumulation lane
     unsigned long long fold_ctr[kMaxFoldLaunches];  // records << 32 | outputs
     unsigned long long fold_count[kMaxFoldLaunches];
 };
@@ -57,16 +61,13 @@ struct JobDev {
     const Affine<F> *bases;
     const uint32_t *sorted;
     const uint32_t *bucket_start;  // B + 1
-    const uint32_t *piece_start;   // B + 1
-    const uint32_t *piece_len;     // entries per level-0 piece (chosen on the device)
     uint32_t *reg_start;           // B: where bucket k's partials to complete live in the pool
     uint32_t *reg_count;           // B
     partial_t<F> *sums;            // B: S_{k+1}
     partial_t<F> *tree[2];         // B each
     Xyzz<F> *planes;               // c (canonical)
-    uint32_t pool_off;             // the job's level-0 partials start here in the pool
     uint32_t B, c;
-    uint32_t list_off;  // this job's completion lists start at kCompleteClasses * list_off
+    uint32_t b_off;  // buckets of the jobs before this one
 };
 
 // ------------------------------------------------------------ digit recoding
@@ -131,263 +132,6 @@ __device__ __forceinline__ void hist_block(uint32_t *hist, const fr_t *__restric
     for (uint32_t k = threadIdx.x; k < B; k += blockDim.x) row[k] = hist[k];
 }
 
-// Column scan of the count matrix for buckets [k0, k0 + 64): row b of
-// block_count becomes the offset of workgroup b's entries inside each
-// bucket (the sum of the rows above it) and count[k] the column total.
-// 64 x kScanGroups threads: each row group sums its rows, the groups'
-// sums are scanned in LDS, then each group rewrites its rows as offsets.
-__device__ __forceinline__ void colscan_tile(uint32_t *__restrict__ block_count, uint32_t blocks, uint32_t B,
-                                            uint32_t k0, uint32_t *__restrict__ count)
-{
-    __shared__ uint32_t part[kScanGroups][64];
-    const uint32_t kk = threadIdx.x & 63u, g = threadIdx.x >> 6;
-    const uint32_t k = k0 + kk;
-    const uint32_t rows = (blocks + kScanGroups - 1) / kScanGroups;
-    const uint32_t r0 = min(blocks, g * rows), r1 = min(blocks, r0 + rows);
-    uint32_t sum = 0;
-    if (k < B)
-        for (uint32_t r = r0; r < r1; ++r) sum += block_count[(size_t)r * B + k];
-    part[g][kk] = sum;
-    __syncthreads();
-    uint32_t run = 0;
-    for (uint32_t h = 0; h < g; ++h) run += part[h][kk];
-    if (k < B) {
-        for (uint32_t r = r0; r < r1; ++r) {
-            uint32_t *p = block_count + (size_t)r * B + k;
-            const uint32_t v = *p;
-            *p = run;
-            run += v;
-        }
-        if (g == kScanGroups - 1) count[k] = run;
-    }
-}
-
-__device__ __forceinline__ void scatter_block(uint32_t *cursor, const fr_t *__restrict__ scalars, uint32_t n,
-                                             uint32_t c, uint32_t W, uint32_t B, uint32_t per_block, uint32_t b,
-                                             const uint32_t *__restrict__ bucket_start,
-                                             const uint32_t *__restrict__ block_off, uint32_t *__restrict__ sorted)
-{
-    const uint32_t *row = block_off + (size_t)b * B;
-    for (uint32_t k = threadIdx.x; k < B; k += blockDim.x) cursor[k] = bucket_start[k] + row[k];
-    __syncthreads();
-    const uint32_t beg = b * per_block;
-    const uint32_t end = min(n, beg + per_block);
-    for (uint32_t i = beg + threadIdx.x; i < end; i += blockDim.x) {
-        const fr_t s = fp_from_mont(scalars[i]);
-        for_each_digit(s, c, W, [&](uint32_t w, int32_t d) {
-            const uint32_t m = (uint32_t)(d < 0 ? -d : d);
-            const uint32_t pos = atomicAdd(&cursor[m - 1], 1u);
-            sorted[pos] = (d < 0 ? 0x80000000u : 0u) | (w * n + i);
-        });
-    }
-}
-
-__global__ __launch_bounds__(kSortThreads) void k_hist(const fr_t *__restrict__ scalars, uint32_t n, uint32_t c,
-                                                       uint32_t W, uint32_t B, uint32_t per_block,
-                                                       uint32_t *__restrict__ block_count)
-{
-    extern __shared__ uint32_t lds[];
-    hist_block(lds, scalars, n, c, W, B, per_block, blockIdx.x, block_count);
-}
-
-__global__ __launch_bounds__(64 * kScanGroups) void k_colscan(uint32_t *__restrict__ block_count, uint32_t blocks,
-                                                              uint32_t B, uint32_t *__restrict__ count)
-{
-    colscan_tile(block_count, blocks, B, blockIdx.x * 64, count);
-}
-
-__global__ __launch_bounds__(kSortThreads) void k_scatter(const fr_t *__restrict__ scalars, uint32_t n, uint32_t c,
-                                                          uint32_t W, uint32_t B, uint32_t per_block,
-                                                          const uint32_t *__restrict__ bucket_start,
-                                                          const uint32_t *__restrict__ block_off,
-                                                          uint32_t *__restrict__ sorted)
-{
-    extern __shared__ uint32_t lds[];
-    scatter_block(lds, scalars, n, c, W, B, per_block, blockIdx.x, bucket_start, block_off, sorted);
-}
-
-
-// Exclusive prefix of `len` (<= kMsmMaxBuckets) values into out[0..len]
-// within one workgroup; returns the total.  The values are staged in LDS
-// with coalesced loads, each thread scans a run of `per` of them, and the
-// runs' sums are scanned across the workgroup.  Runs sit at an odd LDS
-// stride, so the threads of a wave walking their runs hit distinct banks.
-//   mode 0: v[k] = src[k]
-//   mode 2: v[k] = ceil(src[k] / T)
-//   mode 3: v[k] = src[k] > lim ? ceil(src[k] / T) : 0
-__device__ uint32_t block_scan(const uint32_t *__restrict__ src, uint32_t len, uint32_t mode, uint32_t T,
-                               uint32_t lim, uint32_t *__restrict__ out, uint32_t *__restrict__ max_out = nullptr)
-{
-    __shared__ uint32_t vals[kMsmMaxBuckets + 1024];
-    __shared__ uint32_t part[1024];
-    __shared__ uint32_t pmax;
-    const uint32_t per = (len + blockDim.x - 1) / blockDim.x;
-    const uint32_t stride = per | 1u;
-    auto at = [&](uint32_t k) -> uint32_t { return (k / per) * stride + k % per; };
-    if (threadIdx.x == 0) pmax = 0;
-    for (uint32_t k = threadIdx.x; k < len; k += blockDim.x) {
-        const uint32_t x = src[k];
-        vals[at(k)] = mode == 0 ? x : (mode == 2 || x > lim) ? (x + T - 1) / T : 0u;
-    }
-    __syncthreads();
-    const uint32_t beg = min(len, threadIdx.x * per);
-    const uint32_t end = min(len, beg + per);
-    uint32_t *run_vals = vals + threadIdx.x * stride;
-    uint32_t sum = 0, mx = 0;
-    for (uint32_t k = 0; k < end - beg; ++k) {
-        const uint32_t v = run_vals[k];
-        sum += v;
-        mx = max(mx, v);
-    }
-    if (max_out && mx) atomicMax(&pmax, mx);
-    // the runs' sums scanned across the workgroup: within each wave by
-    // shuffles, then the waves' totals by the first wave (two barriers)
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
-    uint32_t incl = sum;
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)incl, off);
-        if (lane >= (uint32_t)off) incl += y;
-    }
-    if (lane == 63) part[wave] = incl;
-    __syncthreads();
-    if (wave == 0) {
-        uint32_t w = lane < waves ? part[lane] : 0u;
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y = (uint32_t)__shfl_up((int)w, off);
-            if (lane >= (uint32_t)off) w += y;
-        }
-        if (lane < waves) part[lane] = w;
-    }
-    __syncthreads();
-    uint32_t run = (wave ? part[wave - 1] : 0u) + incl - sum;
-    for (uint32_t k = 0; k < end - beg; ++k) {
-        const uint32_t v = run_vals[k];
-        run_vals[k] = run;
-        run += v;
-    }
-    __syncthreads();
-    for (uint32_t k = threadIdx.x; k < len; k += blockDim.x) out[k] = vals[at(k)];
-    const uint32_t total = part[waves - 1];
-    if (threadIdx.x == 0) {
-        out[len] = total;
-        if (max_out) *max_out = pmax;
-    }
-    __syncthreads();
-    return total;
-}
-
-// Bucket starts (prefix of counts), the piece length for the number of
-// entries, and level-0 piece starts (prefix of ceil(count / piece)):
-// bucket_start[B + 1] = pieces, [B + 2] = largest piece count of a bucket,
-// [B + 3] = piece length.
-__device__ void schedule_scan(const uint32_t *__restrict__ count, uint32_t B, uint32_t piece_lo, uint32_t piece_hi,
-                              uint32_t target_log, uint32_t *__restrict__ bucket_start,
-                              uint32_t *__restrict__ piece_start)
-{
-    const uint32_t entries = block_scan(count, B, 0, 1, 0, bucket_start);
-    const uint32_t q = entries >> target_log;
-    // Longer pieces also while an average bucket would be left with more
-    // than kMsmCompleteMax partials: small MSMs (few entries against the
-    // piece target) then complete without fold levels.  Longer pieces only
-    // lower the piece count, so the host's max_pieces bound still holds.
-    uint32_t piece = piece_lo;
-    while (piece < piece_hi && (2 * piece <= q || (uint64_t)piece * B * kMsmCompleteMax < entries)) piece <<= 1;
-    const uint32_t pieces = block_scan(count, B, 2, piece, 0, piece_start, bucket_start + B + 2);
-    if (threadIdx.x == 0) {
-        bucket_start[B + 1] = pieces;
-        bucket_start[B + 3] = piece;
-    }
-}
-
-// One schedule's bucket starts and piece split; with alt_lo > 0 also the
-// second split (pieces of at least alt_lo entries) into alt_piece_start and
-// the counters bucket_start[B + 4 .. B + 8).
-__global__ __launch_bounds__(1024) void k_schedule_scan(const uint32_t *__restrict__ count, uint32_t B,
-                                                        uint32_t piece_lo, uint32_t piece_hi, uint32_t target_log,
-                                                        uint32_t *__restrict__ bucket_start,
-                                                        uint32_t *__restrict__ piece_start, uint32_t alt_lo,
-                                                        uint32_t *__restrict__ alt_piece_start)
-{
-    schedule_scan(count, B, piece_lo, piece_hi, target_log, bucket_start, piece_start);
-    if (alt_lo == 0) return;
-    const uint32_t entries = bucket_start[B];
-    const uint32_t q = entries >> target_log;
-    const uint32_t hi = max(alt_lo, piece_hi);
-    uint32_t piece = alt_lo;
-    while (piece < hi && 2 * piece <= q) piece <<= 1;
-    uint32_t *ctr = bucket_start + B + 4;
-    const uint32_t pieces = block_scan(count, B, 2, piece, 0, alt_piece_start, ctr + 2);
-    if (threadIdx.x == 0) {
-        ctr[0] = entries;
-        ctr[1] = pieces;
-        ctr[3] = piece;
-    }
-}
-
-// Last index k in [0, len) with starts[k] <= p (starts[0] <= p < starts[len]).
-__device__ __forceinline__ uint32_t find_segment(const uint32_t *starts, uint32_t len, uint32_t p)
-{
-    uint32_t lo = 0, hi = len;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (starts[mid] <= p)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
-// One schedule of a batched sort.
-struct SortJob {
-    const fr_t *scalars;
-    uint32_t n, c, W, B, blocks, per_block, piece_lo, piece_hi, target_log;
-    uint32_t *count, *block_count, *bucket_start, *piece_start, *sorted;
-};
-
-// Workgroup blockIdx.x is sort block (blockIdx.x - block_off[j]) of job j.
-__global__ __launch_bounds__(kSortThreads) void k_hist_batch(const SortJob *__restrict__ jobs,
-                                                             const uint32_t *__restrict__ block_off, uint32_t J)
-{
-    extern __shared__ uint32_t lds[];
-    const uint32_t j = find_segment(block_off, J, blockIdx.x);
-    const SortJob &jb = jobs[j];
-    hist_block(lds, jb.scalars, jb.n, jb.c, jb.W, jb.B, jb.per_block, blockIdx.x - block_off[j], jb.block_count);
-}
-
-__global__ __launch_bounds__(64 * kScanGroups) void k_colscan_batch(const SortJob *__restrict__ jobs)
-{
-    const SortJob &jb = jobs[blockIdx.y];
-    if (blockIdx.x * 64 >= jb.B) return;
-    colscan_tile(jb.block_count, jb.blocks, jb.B, blockIdx.x * 64, jb.count);
-}
-
-__global__ __launch_bounds__(1024) void k_schedule_scan_batch(const SortJob *__restrict__ jobs)
-{
-    const SortJob &jb = jobs[blockIdx.x];
-    schedule_scan(jb.count, jb.B, jb.piece_lo, jb.piece_hi, jb.target_log, jb.bucket_start, jb.piece_start);
-}
-
-// out[4j + i] = schedule j's counter i (entries, pieces, largest piece count, piece length).
-__global__ __launch_bounds__(256) void k_gather_totals(const SortJob *__restrict__ jobs, uint32_t J,
-                                                       uint32_t *__restrict__ out)
-{
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= 4 * J) return;
-    const SortJob &jb = jobs[g >> 2];
-    out[g] = jb.bucket_start[jb.B + (g & 3u)];
-}
-
-__global__ __launch_bounds__(kSortThreads) void k_scatter_batch(const SortJob *__restrict__ jobs,
-                                                                const uint32_t *__restrict__ block_off, uint32_t J)
-{
-    extern __shared__ uint32_t lds[];
-    const uint32_t j = find_segment(block_off, J, blockIdx.x);
-    const SortJob &jb = jobs[j];
-    scatter_block(lds, jb.scalars, jb.n, jb.c, jb.W, jb.B, jb.per_block, blockIdx.x - block_off[j],
-                  jb.bucket_start, jb.block_count, jb.sorted);
-}
-
 // Exclusive prefix of f(0) .. f(len - 1) into out[0 .. len], by one workgroup
 // (whole waves).
 template <class Fn>
@@ -415,40 +159,223 @@ __device__ void group_prefix(uint32_t len, uint32_t *__restrict__ out, Fn f)
         __syncthreads();
     }
     if (threadIdx.x == 0) out[len] = base;
+    __syncthreads();
 }
 
-// The reduction plan of a batch, from the schedules' piece splits alone: one
-// launch before the accumulation instead of six small ones after it.
-//   * a bucket with more than kMsmCompleteMax partials gets a fold record per
+// Column scan of the count matrix for buckets [64 tile, 64 tile + 64): row b
+// of block_count becomes the offset of workgroup b's entries inside each
+// bucket (the sum of the rows above it), and the columns' totals the buckets'
+// starts within the tile (in_tile) and the tile's total; the scatter adds the
+// tiles' prefix.  64 x kScanGroups threads: each row group sums its rows, the
+// groups' sums are scanned in LDS, then each group rewrites its rows as
+// offsets, and the last group scans its totals.
+__device__ __forceinline__ void colscan_tile(uint32_t *__restrict__ block_count, uint32_t blocks, uint32_t B,
+                                            uint32_t tile, uint32_t *__restrict__ in_tile,
+                                            uint32_t *__restrict__ tile_total)
+{
+    __shared__ uint32_t part[kScanGroups][64];
+    const uint32_t kk = threadIdx.x & 63u, g = threadIdx.x >> 6;
+    const uint32_t k = tile * 64 + kk;
+    const uint32_t rows = (blocks + kScanGroups - 1) / kScanGroups;
+    const uint32_t r0 = min(blocks, g * rows), r1 = min(blocks, r0 + rows);
+    uint32_t sum = 0;
+    if (k < B)
+        for (uint32_t r = r0; r < r1; ++r) sum += block_count[(size_t)r * B + k];
+    part[g][kk] = sum;
+    __syncthreads();
+    uint32_t run = 0;
+    for (uint32_t h = 0; h < g; ++h) run += part[h][kk];
+    if (k < B) {
+        for (uint32_t r = r0; r < r1; ++r) {
+            uint32_t *p = block_count + (size_t)r * B + k;
+            const uint32_t v = *p;
+            *p = run;
+            run += v;
+        }
+    }
+    if (g == kScanGroups - 1) {
+        const uint32_t v = k < B ? run : 0u;
+        uint32_t incl = v;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)incl, off);
+            if (kk >= (uint32_t)off) incl += y;
+        }
+        if (k < B) in_tile[k] = incl - v;
+        if (kk == 63) tile_total[tile] = incl;
+    }
+}
+
+// Every workgroup scans the (at most kMsmMaxBuckets / 64) tile totals for its
+// own cursors, which costs less than a launch that would do it once; the
+// first one writes the bucket starts for the kernels after it.
+__device__ __forceinline__ void scatter_block(uint32_t *cursor, const fr_t *__restrict__ scalars, uint32_t n,
+                                             uint32_t c, uint32_t W, uint32_t B, uint32_t per_block, uint32_t b,
+                                             const uint32_t *__restrict__ in_tile,
+                                             const uint32_t *__restrict__ tile_total,
+                                             const uint32_t *__restrict__ block_off,
+                                             uint32_t *__restrict__ bucket_start, uint32_t *__restrict__ sorted)
+{
+    __shared__ uint32_t tile_base[kMsmMaxBuckets / 64 + 1];
+    group_prefix((B + 63) / 64, tile_base, [&](uint32_t t) { return tile_total[t]; });
+    const uint32_t *row = block_off + (size_t)b * B;
+    for (uint32_t k = threadIdx.x; k < B; k += blockDim.x) {
+        const uint32_t start = in_tile[k] + tile_base[k / 64];
+        cursor[k] = start + row[k];
+        if (b == 0) bucket_start[k] = start;
+    }
+    if (b == 0 && threadIdx.x == 0) bucket_start[B] = tile_base[(B + 63) / 64];
+    __syncthreads();
+    const uint32_t beg = b * per_block;
+    const uint32_t end = min(n, beg + per_block);
+    for (uint32_t i = beg + threadIdx.x; i < end; i += blockDim.x) {
+        const fr_t s = fp_from_mont(scalars[i]);
+        for_each_digit(s, c, W, [&](uint32_t w, int32_t d) {
+            const uint32_t m = (uint32_t)(d < 0 ? -d : d);
+            const uint32_t pos = atomicAdd(&cursor[m - 1], 1u);
+            sorted[pos] = (d < 0 ? 0x80000000u : 0u) | (w * n + i);
+        });
+    }
+}
+
+__global__ __launch_bounds__(kSortThreads) void k_hist(const fr_t *__restrict__ scalars, uint32_t n, uint32_t c,
+                                                       uint32_t W, uint32_t B, uint32_t per_block,
+                                                       uint32_t *__restrict__ block_count)
+{
+    extern __shared__ uint32_t lds[];
+    hist_block(lds, scalars, n, c, W, B, per_block, blockIdx.x, block_count);
+}
+
+__global__ __launch_bounds__(64 * kScanGroups) void k_colscan(uint32_t *__restrict__ block_count, uint32_t blocks,
+                                                              uint32_t B, uint32_t *__restrict__ in_tile,
+                                                              uint32_t *__restrict__ tile_total)
+{
+    colscan_tile(block_count, blocks, B, blockIdx.x, in_tile, tile_total);
+}
+
+__global__ __launch_bounds__(kSortThreads) void k_scatter(const fr_t *__restrict__ scalars, uint32_t n, uint32_t c,
+                                                          uint32_t W, uint32_t B, uint32_t per_block,
+                                                          const uint32_t *__restrict__ in_tile,
+                                                          const uint32_t *__restrict__ tile_total,
+                                                          const uint32_t *__restrict__ block_off,
+                                                          uint32_t *__restrict__ bucket_start,
+                                                          uint32_t *__restrict__ sorted)
+{
+    extern __shared__ uint32_t lds[];
+    scatter_block(lds, scalars, n, c, W, B, per_block, blockIdx.x, in_tile, tile_total, block_off, bucket_start,
+                  sorted);
+}
+
+// Last index k in [0, len) with starts[k] <= p (starts[0] <= p < starts[len]).
+__device__ __forceinline__ uint32_t find_segment(const uint32_t *starts, uint32_t len, uint32_t p)
+{
+    uint32_t lo = 0, hi = len;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (starts[mid] <= p)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+// One schedule of a batched sort.
+struct SortJob {
+    const fr_t *scalars;
+    uint32_t n, c, W, B, blocks, per_block;
+    uint32_t *block_count, *in_tile, *tile_total, *bucket_start, *sorted;
+};
+
+// Workgroup blockIdx.x is sort block (blockIdx.x - block_off[j]) of job j.
+__global__ __launch_bounds__(kSortThreads) void k_hist_batch(const SortJob *__restrict__ jobs,
+                                                             const uint32_t *__restrict__ block_off, uint32_t J)
+{
+    extern __shared__ uint32_t lds[];
+    const uint32_t j = find_segment(block_off, J, blockIdx.x);
+    const SortJob &jb = jobs[j];
+    hist_block(lds, jb.scalars, jb.n, jb.c, jb.W, jb.B, jb.per_block, blockIdx.x - block_off[j], jb.block_count);
+}
+
+__global__ __launch_bounds__(64 * kScanGroups) void k_colscan_batch(const SortJob *__restrict__ jobs)
+{
+    const SortJob &jb = jobs[blockIdx.y];
+    if (blockIdx.x * 64 >= jb.B) return;
+    colscan_tile(jb.block_count, jb.blocks, jb.B, blockIdx.x, jb.in_tile, jb.tile_total);
+}
+
+__global__ __launch_bounds__(kSortThreads) void k_scatter_batch(const SortJob *__restrict__ jobs,
+                                                                const uint32_t *__restrict__ block_off, uint32_t J)
+{
+    extern __shared__ uint32_t lds[];
+    const uint32_t j = find_segment(block_off, J, blockIdx.x);
+    const SortJob &jb = jobs[j];
+    scatter_block(lds, jb.scalars, jb.n, jb.c, jb.W, jb.B, jb.per_block, blockIdx.x - block_off[j], jb.in_tile,
+                  jb.tile_total, jb.block_count, jb.bucket_start, jb.sorted);
+}
+
+// Entries per accumulation lane for E entries in all (MsmLanes).
+__device__ __forceinline__ uint32_t piece_length(uint64_t E, const MsmLanes &r)
+{
+    uint32_t lanes = r.lanes[3];
+    for (int i = 2; i >= 0; --i)
+        if (E < r.below[i]) lanes = r.lanes[i];
+    return (uint32_t)max((uint64_t)r.piece_min, (E + lanes - 1) / lanes);
+}
+
+// The plan of a batch, from the schedules' bucket starts: one launch before
+// the accumulation instead of several small ones around it.
+//   * the accumulation gives every lane L consecutive entries of a job's
+//     sorted list, L = piece_length of all jobs' entries; a bucket of the
+//     entries [a, b) therefore gets a partial from each of the lanes a / L ..
+//     (b - 1) / L, and lane l's partial of bucket k is number l + k of the job
+//     (two lanes share a bucket, or one lane two buckets, never both), at
+//     lanes and buckets of the jobs before it in the pool;
+//   * a bucket with more than kDirectMax partials gets a fold record per
 //     level that brings it below (kFoldSpan : 1 each); any bucket's final
 //     partials become reg_start / reg_count;
 //   * completion classes: a bucket with m partials is completed by 2^c lane
-//     groups, the smallest c with m <= serial << c (the host's serial target
-//     is short where the launch leaves the chip idle and long where every
-//     lane group has several buckets); an empty bucket's sum is infinity;
+//     groups, the smallest c with m <= serial << c.  With the partials spread
+//     over the chip's lane groups a group has (lanes + buckets) / groups of
+//     them; half as many again keep most buckets in one group (the shuffle
+//     levels of more idle half of them or more), and only the longer ones
+//     take several.  An empty bucket's sum is infinity;
 //   * the last workgroup to finish turns the counts into offsets:
-//     piece_base[j] = level-0 pieces of the jobs before j, seg_base[s] = lanes
-//     of the completion segments before s = kCompleteClasses * j + c, each
-//     padded to whole waves, and clears the counters for the next launch.
+//     lane_base[j] = accumulation lanes of the jobs before j, seg_base[s] =
+//     lanes of the completion segments before s = kCompleteClasses * j + c,
+//     each padded to whole waves, and clears the counters for the next launch.
 template <class F>
-__global__ __launch_bounds__(256) void k_reduce_plan(const JobDev<F> *__restrict__ jobs, uint32_t J,
-                                                     uint32_t max_class, uint32_t serial,
+__global__ __launch_bounds__(kPlanThreads) void k_reduce_plan(const JobDev<F> *__restrict__ jobs, uint32_t J,
+                                                     MsmLanes rule, uint32_t buckets, uint32_t max_class,
                                                      ReduceState *__restrict__ st, FoldRec *__restrict__ recs,
                                                      uint32_t rec_cap, const uint32_t *__restrict__ fold_base,
                                                      uint32_t *__restrict__ class_count,
                                                      uint32_t *__restrict__ class_list,
-                                                     uint32_t *__restrict__ piece_base,
+                                                     uint32_t *__restrict__ lane_base,
                                                      uint32_t *__restrict__ seg_count,
                                                      uint32_t *__restrict__ seg_base)
 {
     const uint32_t j = blockIdx.y;
     const JobDev<F> &jb = jobs[j];
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ unsigned long long entries;
+    if (threadIdx.x == 0) entries = 0;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < J; i += blockDim.x)
+        atomicAdd(&entries, (unsigned long long)jobs[i].bucket_start[jobs[i].B]);
+    __syncthreads();
+    const uint32_t piece = piece_length(entries, rule);
+    __shared__ uint32_t lanes_before;
+    if (threadIdx.x == 0) lanes_before = 0;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < j; i += blockDim.x)
+        atomicAdd(&lanes_before, (jobs[i].bucket_start[jobs[i].B] + piece - 1) / piece);
+    __syncthreads();
     uint32_t m = 0;
     if (k < jb.B) {
-        uint32_t src = jb.pool_off + jb.piece_start[k];
-        m = jb.piece_start[k + 1] - jb.piece_start[k];
-        for (uint32_t L = 0; m > kMsmCompleteMax; ++L) {
+        const uint32_t beg = jb.bucket_start[k], end = jb.bucket_start[k + 1];
+        uint32_t src = lanes_before + jb.b_off + beg / piece + k;
+        if (beg < end) m = (end - 1) / piece - beg / piece + 1;
+        for (uint32_t L = 0; m > kDirectMax; ++L) {
             const uint32_t n = (m + kFoldSpan - 1) / kFoldSpan;
             const unsigned long long at = atomicAdd(&st->fold_ctr[L], (1ull << 32) | n);
             const uint32_t start = (uint32_t)at;
@@ -460,39 +387,53 @@ __global__ __launch_bounds__(256) void k_reduce_plan(const JobDev<F> *__restrict
         jb.reg_count[k] = m;
         if (m == 0) jb.sums[k] = partial_t<F>::infinity();
     }
-    // one atomic per wave and class: a ballot ranks the lanes
+    // one atomic per workgroup and class: ballots rank the lanes of a wave, and
+    // the waves' counts are scanned in LDS
+    __shared__ uint32_t count[kCompleteClasses][kPlanThreads / 64], list_at[kCompleteClasses];
+    constexpr uint32_t groups = 65536 / Coop<F>::kLanes;
+    const uint32_t serial = 1 + (uint32_t)(3 * (entries / piece + buckets) / (2 * groups));
     uint32_t c = 0;
     while (c < max_class && (serial << c) < m) ++c;
-    const uint32_t lane = threadIdx.x & 63u;
-    uint32_t *list = class_list + (size_t)jb.list_off * kCompleteClasses;
-    for (uint32_t cc = 0; cc <= max_class; ++cc) {
-        const bool mine = m > 0 && c == cc;
-        const uint64_t mask = __ballot(mine);
-        if (mask == 0) continue;
-        const uint32_t leader = (uint32_t)__ffsll((unsigned long long)mask) - 1u;
-        uint32_t first = 0;
-        if (lane == leader) first = atomicAdd(&class_count[kCompleteClasses * j + cc], (uint32_t)__popcll(mask));
-        first = (uint32_t)__shfl((int)first, (int)leader);
-        if (mine) list[(size_t)cc * jb.B + first + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = k;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    uint32_t rank = 0;
+    for (uint32_t cc = 0; cc < kCompleteClasses; ++cc) {
+        const uint64_t mask = __ballot(m > 0 && c == cc);
+        if (c == cc) rank = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+        if (lane == 0) count[cc][wave] = (uint32_t)__popcll(mask);
     }
+    __syncthreads();
+    if (threadIdx.x < kCompleteClasses) {
+        uint32_t sum = 0;
+        for (uint32_t w = 0; w < waves; ++w) {
+            const uint32_t n = count[threadIdx.x][w];
+            count[threadIdx.x][w] = sum;
+            sum += n;
+        }
+        if (sum) list_at[threadIdx.x] = atomicAdd(&class_count[kCompleteClasses * j + threadIdx.x], sum);
+    }
+    __syncthreads();
+    if (m > 0)
+        class_list[((size_t)jb.b_off * kCompleteClasses + (size_t)c * jb.B) + list_at[c] + count[c][wave] + rank] = k;
 
+    // The last workgroup reads what the others left in the counters, which are
+    // only touched by atomics; each of its own has returned here.
     __shared__ uint32_t last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) {
-        __threadfence();
         last = atomicAdd(&st->ticket, 1u) + 1u == gridDim.x * gridDim.y ? 1u : 0u;
+        if (last) st->ticket = 0;
     }
     __syncthreads();
     if (!last) return;
-    __threadfence();
-    group_prefix(J, piece_base, [&](uint32_t i) { return jobs[i].piece_start[jobs[i].B]; });
+    if (threadIdx.x == 0) st->piece = piece;
+    group_prefix(J, lane_base, [&](uint32_t i) { return (jobs[i].bucket_start[jobs[i].B] + piece - 1) / piece; });
     group_prefix(kCompleteClasses * J, seg_base, [&](uint32_t s) {
         const uint32_t n = atomicExch(&class_count[s], 0u);
         seg_count[s] = n;
         return ((n * Coop<F>::kLanes << (s % kCompleteClasses)) + 63u) & ~63u;
     });
     if (threadIdx.x < kMaxFoldLaunches) st->fold_count[threadIdx.x] = atomicExch(&st->fold_ctr[threadIdx.x], 0ull);
-    if (threadIdx.x == 0) st->ticket = 0;
 }
 
 // The G2 accumulator of one lane with X and ZZ in registers and Y and ZZZ in
@@ -547,80 +488,240 @@ struct Xyzz2_29Lds {
     __device__ Xyzz2_29<P> get() const { return {x, load(y), zz, load(zzz)}; }
 };
 
-// Level 0 over all jobs: a thread sums one piece of signed bases of one
-// bucket into one partial (the loop strides by the grid, so any grid size
-// covers every piece).
+// What a lane keeps of its run between the entries: in registers, or (Lds) in
+// a column of LDS words, read where it is used.  The G1 addition needs all
+// 168 registers that three waves per SIMD leave it, and a spilled one would
+// cost more than its reload: scratch loads return in order behind the direct
+// loads of the next base, so each addition would wait for that one's latency
+// (4.6 against 4.1 us per addition at two waves per SIMD).
+enum LaneWord { kBucket, kNextEnd, kSlot, kBuckets, kStarts, kStarts1, kSorted, kSorted1, kFirst, kLast, kBases, kBases1,
+                kLaneWords };
+template <bool Lds>
+struct LaneWords {
+    uint32_t w[kLaneWords];
+    __device__ LaneWords(uint32_t *) {}
+    __device__ uint32_t get(int i) const { return w[i]; }
+    __device__ void set(int i, uint32_t v) { w[i] = v; }
+};
+template <>
+struct LaneWords<true> {
+    lds_word_t *w;  // word i of the lane at w[i * kAccThreads]
+    __device__ LaneWords(uint32_t *lds) : w((lds_word_t *)(lds + threadIdx.x)) {}
+    __device__ uint32_t get(int i) const { return w[i * kAccThreads]; }
+    __device__ void set(int i, uint32_t v) { w[i * kAccThreads] = v; }
+};
+template <class T, bool Lds>
+__device__ __forceinline__ const T *lane_ptr(const LaneWords<Lds> &lw, int i)
+{
+    return reinterpret_cast<const T *>((uint64_t)lw.get(i + 1) << 32 | lw.get(i));
+}
+template <class T, bool Lds>
+__device__ __forceinline__ void set_lane_ptr(LaneWords<Lds> &lw, int i, const T *p)
+{
+    lw.set(i, (uint32_t)(uint64_t)p);
+    lw.set(i + 1, (uint32_t)((uint64_t)p >> 32));
+}
+
+// A lane's walk over its run of a job's sorted entries.
+template <bool Lds>
+struct RunCursor {
+    uint32_t e, e1;  // next entry, end of the run
+    uint32_t end;    // end of entry e's bucket
+    LaneWords<Lds> &lw;
+
+    // lane: of the job; lane0: lanes and buckets of the jobs before it
+    __device__ RunCursor(LaneWords<Lds> &words, const uint32_t *__restrict__ starts, uint32_t B, uint32_t lane0,
+                         uint32_t lane, uint32_t piece)
+        : lw(words)
+    {
+        e = lane * piece;
+        e1 = min(e + piece, starts[B]);
+        const uint32_t k = find_segment(starts, B, e);
+        end = starts[k + 1];
+        lw.set(kBucket, k);
+        lw.set(kNextEnd, starts[min(k + 2, B)]);  // loaded ahead
+        lw.set(kSlot, lane0 + lane + k);
+        lw.set(kBuckets, B);
+        set_lane_ptr(lw, kStarts, starts);
+    }
+    // where this lane's partial of the current bucket goes
+    __device__ __forceinline__ uint32_t slot() const { return lw.get(kSlot); }
+    // Past the last entry of the bucket: on to the bucket of entry e.
+    __device__ __forceinline__ void advance()
+    {
+        const uint32_t *starts = lane_ptr<uint32_t>(lw, kStarts);
+        const uint32_t B = lw.get(kBuckets), k0 = lw.get(kBucket);
+        uint32_t k = k0, next = lw.get(kNextEnd);
+        do {
+            ++k;
+            end = next;
+            next = starts[min(k + 2, B)];
+        } while (end == e);
+        lw.set(kBucket, k);
+        lw.set(kNextEnd, next);
+        lw.set(kSlot, lw.get(kSlot) + k - k0);
+    }
+};
+
+// The bases of a lane's run, one entry ahead of the additions.  They are
+// gathered (64 or 128 bytes anywhere in a gigabyte), so a load is microseconds
+// away, and neither holding the next base in registers (16 or 32 of them, a
+// wave per SIMD less) nor waiting for it behind three waves pays.  Instead a
+// lane's loads go straight to LDS while it adds: each 16-byte part of the
+// wave's 64 bases is one direct load, lane i's at part[i].  The sorted indices
+// come the same way, four at a time (one by one, a line of them would have
+// left the caches before its next use), in two blocks used in turn.
+//
+// A direct load writes at one LDS address for the whole wave plus the lane's
+// place, so the row must be the same for all lanes that load together.  The
+// lanes of a wave take their entries in step; the blocks are therefore counted
+// from each lane's first one, and those that go on to another block at the
+// same step go on to one of the same number.
+template <class F, bool Lds>
+struct BaseStream {
+    static constexpr uint32_t kParts = sizeof(Affine<F>) / sizeof(uint4);
+    static constexpr uint32_t kRows = kParts + 2;  // rows of 64 x 16 bytes per wave
+    uint4 (*rows)[64];                             // this wave's
+    LaneWords<Lds> &lw;
+    uint32_t v = 0;  // index of the base on its way
+
+    __device__ static void load(const uint4 *from, uint4 *row)
+    {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)from,
+                                         (__attribute__((address_space(3))) void *)row, 16, 0, 0);
+    }
+    // Direct loads so far have arrived / LDS reads so far are done.
+    __device__ static void arrived() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+    __device__ static void read_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+    // the run's block number t (counted in the list) of four indices
+    __device__ __forceinline__ void load_block(uint32_t t)
+    {
+        load(lane_ptr<uint4>(lw, kSorted) + min(t, lw.get(kLast)),
+             rows[kParts + __builtin_amdgcn_readfirstlane((t - lw.get(kFirst)) & 1u)]);
+    }
+    __device__ __forceinline__ uint32_t index(uint32_t e) const
+    {
+        const uint4 *block = &rows[kParts + (((e >> 2) - lw.get(kFirst)) & 1u)][threadIdx.x & 63u];
+        return reinterpret_cast<const uint32_t *>(block)[e & 3u];
+    }
+    __device__ __forceinline__ void load_base()
+    {
+        const uint4 *b = reinterpret_cast<const uint4 *>(lane_ptr<Affine<F>>(lw, kBases) + (v & kEntryMask));
+#pragma unroll
+        for (uint32_t k = 0; k < kParts; ++k) load(b + k, rows[k]);
+    }
+    // Starts the run at entry e of a list of `entries`.
+    __device__ BaseStream(uint4 (*wave_rows)[64], LaneWords<Lds> &words, const Affine<F> *bases,
+                          const uint32_t *sorted, uint32_t e, uint32_t entries)
+        : rows(wave_rows), lw(words)
+    {
+        set_lane_ptr(lw, kBases, bases);
+        set_lane_ptr(lw, kSorted, sorted);
+        lw.set(kFirst, e >> 2);
+        lw.set(kLast, (entries - 1) >> 2);
+        load_block(e >> 2);
+        load_block((e >> 2) + 1);
+        arrived();
+        v = index(e);
+        load_base();
+    }
+    // Entry e's base and sign.  The next entry's is on its way when this
+    // returns (at the end of the run, e + 1 = e1, entry e's again).
+    __device__ __forceinline__ Affine<F> take(uint32_t e, uint32_t e1, bool &negative)
+    {
+        Affine<F> P;
+        arrived();
+        uint4 *out = reinterpret_cast<uint4 *>(&P);
+#pragma unroll
+        for (uint32_t k = 0; k < kParts; ++k) out[k] = rows[k][threadIdx.x & 63u];
+        negative = v >> 31;
+        const bool more = e + 1 < e1;
+        v = index(more ? e + 1 : e);
+        read_done();
+        load_base();
+        if (more && ((e + 1) & 3u) == 0) load_block(((e + 1) >> 2) + 1);
+        return P;
+    }
+};
+
+// Accumulation over all jobs: a lane sums its run of L consecutive sorted
+// entries (k_reduce_plan) of signed bases into one partial per bucket it
+// meets.  Every lane has the same number of additions whatever the buckets'
+// sizes, so waves end together and a launch of resident size is even; the
+// store at a bucket's end costs a wave a few lanes' time once every bucket.
 template <class F>
 __device__ __forceinline__ void accumulate_body(const JobDev<F> *__restrict__ jobs,
-                                                const uint32_t *__restrict__ piece_base, uint32_t J,
-                                                partial_t<F> *__restrict__ pool)
+                                                const uint32_t *__restrict__ lane_base, uint32_t J,
+                                                const ReduceState *__restrict__ st, partial_t<F> *__restrict__ pool)
 {
-    const uint32_t total = piece_base[J];
+    constexpr bool kLds = !std::is_same<F, fq2_t>::value;
+    using Stream = BaseStream<F, kLds>;
+    __shared__ uint4 stage[kAccThreads / 64][Stream::kRows][64];
+    __shared__ uint32_t words[kLds ? kLaneWords * kAccThreads : 1];
+    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= lane_base[J]) return;
+    const uint32_t j = find_segment(lane_base, J, g);
+    const JobDev<F> &jb = jobs[j];
+    LaneWords<kLds> lw(words);
+    RunCursor<kLds> c(lw, jb.bucket_start, jb.B, lane_base[j] + jb.b_off, g - lane_base[j], st->piece);
+    Stream in(stage[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)], lw, jb.bases, jb.sorted, c.e,
+              jb.bucket_start[jb.B]);
+    if constexpr (std::is_same<F, fq2_t>::value) {
+        // G2: the accumulator in the reduced-radix form as for G1 (curve29.h,
+        // Fq2 bounds), stored in it; Y and ZZZ in LDS between their uses.
+        __shared__ uint32_t side[36 * kAccThreads];
+        Xyzz2_29Lds<FqParams> acc{Fq2_29<FqParams>{}, Fq2_29<FqParams>{}, (lds_word_t *)(side + threadIdx.x),
+                                  (lds_word_t *)(side + 18 * kAccThreads + threadIdx.x)};
+        acc.set(Xyzz2_29<FqParams>::infinity());
 #pragma unroll 1
-    for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < total; g += gridDim.x * blockDim.x) {
-        const uint32_t j = find_segment(piece_base, J, g);
-        const JobDev<F> &jb = jobs[j];
-        const uint32_t p = g - piece_base[j];
-        const uint32_t k = find_segment(jb.piece_start, jb.B, p);
-        const uint32_t q = p - jb.piece_start[k];
-        const uint32_t piece = *jb.piece_len;
-        const uint32_t beg = jb.bucket_start[k] + q * piece;
-        const uint32_t end = min(beg + piece, jb.bucket_start[k + 1]);
-        const Affine<F> *__restrict__ bases = jb.bases;
-        const uint32_t *__restrict__ sorted = jb.sorted;
-        partial_t<F> acc = partial_t<F>::infinity();
-        if constexpr (std::is_same<F, fq2_t>::value) {
-            // G2: the accumulator in the reduced-radix form as for G1
-            // (curve29.h, Fq2 bounds), stored in it; Y and ZZZ in LDS
-            // between their uses; no prefetch.
-            __shared__ uint32_t side[36 * kAccThreads];
-            Xyzz2_29Lds<FqParams> acc29{Fq2_29<FqParams>{}, Fq2_29<FqParams>{},
-                                        (lds_word_t *)(side + threadIdx.x),
-                                        (lds_word_t *)(side + 18 * kAccThreads + threadIdx.x)};
-            acc29.set(Xyzz2_29<FqParams>::infinity());
-#pragma unroll 1
-            for (uint32_t e = beg; e < end; ++e) {
-                const uint32_t v = sorted[e];
-                const Affine<F> P = bases[v & kEntryMask];
-                if (!affine_is_inf(P)) {
-                    const F y = (v >> 31) ? FieldOps<F>::neg(P.y) : P.y;
-                    xyzz2_29_madd<FqParams>(acc29, fq2_29_from<FqParams>(P.x), fq2_29_from<FqParams>(y));
-                }
+        for (; c.e < c.e1; ++c.e) {
+            if (c.e == c.end) {
+                pool[c.slot()] = acc.get();
+                acc.set(Xyzz2_29<FqParams>::infinity());
+                c.advance();
             }
-            acc = acc29.get();
-        } else if (beg < end) {
-            // G1: the accumulator stays in the reduced-radix form
-            // (curve29.h: one v_mad_u64_u32 per product term, no carries)
-            // for the whole piece and is stored in it; bases are converted
-            // as they arrive.  The next sorted index is
-            // fetched one entry ahead; the base itself is not (its 16
-            // registers cost more occupancy than its latency costs three
-            // resident waves, measured on MI355X).
-            Xyzz29<FqParams> acc29 = Xyzz29<FqParams>::infinity();
-            uint32_t v = sorted[beg];
-#pragma unroll 1
-            for (uint32_t e = beg; e < end; ++e) {
-                const Affine<F> P = bases[v & kEntryMask];
-                const uint32_t vn = e + 1 < end ? sorted[e + 1] : 0u;
-                if (!affine_is_inf(P)) {
-                    const F y = (v >> 31) ? FieldOps<F>::neg(P.y) : P.y;
-                    acc29 = xyzz29_add_affine(acc29, fp29_from_mont(P.x), fp29_from_mont(y));
-                }
-                v = vn;
+            bool negative;
+            const Affine<F> P = in.take(c.e, c.e1, negative);
+            if (!affine_is_inf(P)) {
+                const F y = negative ? FieldOps<F>::neg(P.y) : P.y;
+                xyzz2_29_madd<FqParams>(acc, fq2_29_from<FqParams>(P.x), fq2_29_from<FqParams>(y));
             }
-            acc = acc29;
         }
-        pool[jb.pool_off + p] = acc;
+        pool[c.slot()] = acc.get();
+    } else {
+        // G1: the accumulator stays in the reduced-radix form (curve29.h: one
+        // v_mad_u64_u32 per product term, no carries) for the whole run and is
+        // stored in it; bases are converted as they arrive.
+        Xyzz29<FqParams> acc = Xyzz29<FqParams>::infinity();
+#pragma unroll 1
+        for (; c.e < c.e1; ++c.e) {
+            if (c.e == c.end) {
+                pool[c.slot()] = acc;
+                acc = Xyzz29<FqParams>::infinity();
+                c.advance();
+            }
+            bool negative;
+            const Affine<F> P = in.take(c.e, c.e1, negative);
+            if (!affine_is_inf(P)) {
+                const F y = negative ? FieldOps<F>::neg(P.y) : P.y;
+                acc = xyzz29_add_affine(acc, fp29_from_mont(P.x), fp29_from_mont(y));
+            }
+        }
+        pool[c.slot()] = acc;
     }
+    // no direct load may be in flight when the workgroup gives its LDS back
+    Stream::arrived();
 }
 
 // G1: at most 168 registers, three waves per SIMD.
 template <class F>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_accumulate(const JobDev<F> *__restrict__ jobs,
-                                                    const uint32_t *__restrict__ piece_base, uint32_t J,
+                                                    const uint32_t *__restrict__ lane_base, uint32_t J,
+                                                    const ReduceState *__restrict__ st,
                                                     partial_t<F> *__restrict__ pool)
 {
-    accumulate_body<F>(jobs, piece_base, J, pool);
+    accumulate_body<F>(jobs, lane_base, J, st, pool);
 }
 
 // The G2 addition's working set exceeds 256 registers, which would leave one
@@ -630,10 +731,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 // workgroup) the spills fall from 280 to 80 bytes per lane.
 template <>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_accumulate<fq2_t>(
-    const JobDev<fq2_t> *__restrict__ jobs, const uint32_t *__restrict__ piece_base, uint32_t J,
-    partial_t<fq2_t> *__restrict__ pool)
+    const JobDev<fq2_t> *__restrict__ jobs, const uint32_t *__restrict__ lane_base, uint32_t J,
+    const ReduceState *__restrict__ st, partial_t<fq2_t> *__restrict__ pool)
 {
-    accumulate_body<fq2_t>(jobs, piece_base, J, pool);
+    accumulate_body<fq2_t>(jobs, lane_base, J, st, pool);
 }
 
 // Sum over the lane groups of aligned runs of `groups` groups: every group of
@@ -714,7 +815,7 @@ __global__ __launch_bounds__(256) void k_complete(const JobDev<F> *__restrict__ 
         const uint32_t idx = local >> c, group = local & ((1u << c) - 1u);
         const bool live = idx < seg_count[s];
         const uint32_t k =
-            live ? class_list[(size_t)jb.list_off * kCompleteClasses + (size_t)c * jb.B + idx] : 0u;
+            live ? class_list[(size_t)jb.b_off * kCompleteClasses + (size_t)c * jb.B + idx] : 0u;
         Coop<F> acc = coop_sum<F>(pool, live ? jb.reg_start[k] : 0u, live ? jb.reg_count[k] : 0u, group, 1u << c);
         acc = coop_reduce(acc, 1u << c);
         if (live && group == 0) coop_store<F>(jb.sums, k, acc);
@@ -828,7 +929,7 @@ uint64_t resident_blocks()
     return blocks;
 }
 
-uint32_t g_target_log = kMsmTargetPiecesLog;
+uint32_t g_target_log = 0;  // 0: the group's own lanes
 uint32_t g_lanes_cap = 16;
 
 }  // namespace
@@ -843,7 +944,16 @@ void msm_set_shape(uint32_t target_pieces_log, uint32_t complete_lanes_cap)
     g_lanes_cap = complete_lanes_cap;
 }
 
-uint32_t msm_target_pieces_log() { return g_target_log; }
+
+MsmLanes msm_lanes(bool g2, uint32_t target_log, uint32_t piece_min)
+{
+    MsmLanes r = g2 ? kMsmLanesG2 : kMsmLanesG1;
+    if (target_log == 0) target_log = g_target_log;
+    if (target_log)
+        for (uint32_t &l : r.lanes) l = 1u << target_log;
+    r.piece_min = std::max(1u, piece_min);
+    return r;
+}
 uint32_t msm_complete_lanes_cap() { return g_lanes_cap; }
 
 uint32_t MsmSchedule::sort_blocks(uint32_t n)
@@ -854,31 +964,26 @@ uint32_t MsmSchedule::sort_blocks(uint32_t n)
 uint64_t msm_schedule_bytes(const MsmPlan &p)
 {
     const uint64_t blocks = MsmSchedule::sort_blocks(p.n);
-    return p.max_entries() * 4 + (uint64_t)p.B * 4 * 3 + blocks * p.B * 4 + 32;
+    return p.max_entries() * 4 + (uint64_t)p.B * 4 * 2 + blocks * p.B * 4 + 32;
 }
 
 // Partial sums of all fold launches: a launch turns more than kMsmCompleteMax
 // partials of a bucket into ceil(m / kFoldSpan), fewer than m / 32.
-static uint64_t fold_outputs(uint64_t pieces) { return pieces / 32 + 1; }
-static uint64_t fold_outputs_total(uint64_t pieces)
-{
-    uint64_t sum = 0;
-    for (uint32_t L = 0; L < kMaxFoldLaunches; ++L) sum += pieces = fold_outputs(pieces);
-    return sum;
-}
+static uint64_t fold_outputs(uint64_t partials) { return partials / 32 + 1; }
 // Fold records of one launch: buckets with more than kMsmCompleteMax partials.
-static uint64_t fold_records(uint64_t pieces) { return pieces / (kMsmCompleteMax + 1) + 1; }
+static uint64_t fold_records(uint64_t partials) { return partials / (kMsmCompleteMax + 1) + 1; }
 
 template <class F>
 uint64_t msm_job_bytes(const MsmPlan &p)
 {
-    const uint64_t pieces = p.max_pieces(msm_target_pieces_log());
-    // partial sums; per bucket: sums and two tree levels, region start and
-    // count, the completion class lists; fold records; the bit planes; and
-    // the job's fixed records (job table, class counters, piece offsets)
-    return (pieces + fold_outputs_total(pieces)) * sizeof(partial_t<F>) +
+    const uint64_t partials = p.max_pieces(std::max(kMsmMaxLanesLog, g_target_log) - 1);
+    // partial sums and their folds; per bucket: sums and two tree levels,
+    // region start and count, the completion class lists; fold records; the
+    // bit planes; and the job's fixed records (job table, class counters, lane
+    // offsets)
+    return msm_partial_capacity(p, partials, nullptr, nullptr) * sizeof(partial_t<F>) +
            (uint64_t)p.B * (3 * sizeof(partial_t<F>) + 8 + 4 * kCompleteClasses) +
-           fold_records(pieces) * kMaxFoldLaunches * sizeof(FoldRec) + p.c * sizeof(Xyzz<F>) + 1024;
+           fold_records(partials) * kMaxFoldLaunches * sizeof(FoldRec) + p.c * sizeof(Xyzz<F>) + 1024;
 }
 
 template <class F>
@@ -914,15 +1019,13 @@ uint32_t MsmSchedule::prepare(const MsmPlan &plan)
 {
     allow_sort_lds();
     NKR_REQUIRE(plan.B <= kMsmMaxBuckets, "MSM window too wide for the bucket scans");
-    NKR_REQUIRE(plan.piece_lo >= 1 && plan.piece_lo <= plan.piece_hi, "MSM piece bounds");
     plan_ = plan;
-    target_log_ = target_override_ ? target_override_ : msm_target_pieces_log();
     const uint32_t n = plan.n, B = plan.B;
     blocks_ = sort_blocks(n);
-    sorted_.ensure((size_t)n * plan.W);
-    count_.ensure(B);
-    bucket_start_.ensure(B + 8);  // + the four counters of each piece split
-    piece_start_.ensure(B + 1);
+    sorted_.ensure(((size_t)n * plan.W + 3) & ~size_t(3));  // read in blocks of four
+    bucket_start_.ensure(B + 1);
+    in_tile_.ensure(B);
+    tile_total_.ensure(div_up(B, 64));
     block_count_.ensure((size_t)blocks_ * B);
     return div_up(n, blocks_);
 }
@@ -936,20 +1039,12 @@ void MsmSchedule::build(const fr_t *scalars_mont, const MsmPlan &plan, hipStream
     if (timer) timer->begin(kStageSort, stream);
     k_hist<<<blocks_, threads, lds, stream>>>(scalars_mont, n, plan.c, plan.W, B, per_block, block_count_.get());
     NKR_LAUNCH_CHECK();
-    k_colscan<<<div_up(B, 64), 64 * kScanGroups, 0, stream>>>(block_count_.get(), blocks_, B, count_.get());
+    k_colscan<<<div_up(B, 64), 64 * kScanGroups, 0, stream>>>(block_count_.get(), blocks_, B, in_tile_.get(),
+                                                              tile_total_.get());
     NKR_LAUNCH_CHECK();
-    if (alt_piece_lo_) alt_piece_start_.ensure(B + 1);
-    k_schedule_scan<<<1, 1024, 0, stream>>>(count_.get(), B, plan.piece_lo, plan.piece_hi, target_log_,
-                                            bucket_start_.get(), piece_start_.get(), alt_piece_lo_,
-                                            alt_piece_lo_ ? alt_piece_start_.get() : nullptr);
-    NKR_LAUNCH_CHECK();
-    uint32_t *th = own_totals_.reuse(8);
-    NKR_HIP(hipMemcpyAsync(th, bucket_start_.get() + B, 8 * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-    own_totals_.uploaded(stream);
-    host_totals_ = th;
-    host_stage_ = &own_totals_;
-    k_scatter<<<blocks_, threads, lds, stream>>>(scalars_mont, n, plan.c, plan.W, B, per_block,
-                                                 bucket_start_.get(), block_count_.get(), sorted_.get());
+    k_scatter<<<blocks_, threads, lds, stream>>>(scalars_mont, n, plan.c, plan.W, B, per_block, in_tile_.get(),
+                                                 tile_total_.get(), block_count_.get(), bucket_start_.get(),
+                                                 sorted_.get());
     NKR_LAUNCH_CHECK();
     if (timer) timer->end(kStageSort, stream);
 }
@@ -970,11 +1065,9 @@ void MsmScheduleBatch::build(const std::vector<Item> &items, hipStream_t stream,
     for (uint32_t j = 0; j < J; ++j) {
         MsmSchedule &s = *items[j].sched;
         const MsmPlan &p = items[j].plan;
-        NKR_REQUIRE(s.alt_piece_lo_ == 0, "batched schedules have one piece split");
         const uint32_t per_block = s.prepare(p);
-        jobs[j] = SortJob{items[j].scalars_mont, p.n, p.c, p.W, p.B, s.blocks_, per_block, p.piece_lo, p.piece_hi,
-                          s.target_log_, s.count_.get(), s.block_count_.get(), s.bucket_start_.get(), s.piece_start_.get(),
-                          s.sorted_.get()};
+        jobs[j] = SortJob{items[j].scalars_mont, p.n,  p.c, p.W, p.B, s.blocks_, per_block, s.block_count_.get(),
+                          s.in_tile_.get(), s.tile_total_.get(), s.bucket_start_.get(), s.sorted_.get()};
         off[j] = (uint32_t)blocks;
         blocks += s.blocks_;
         Bmax = std::max(Bmax, p.B);
@@ -991,45 +1084,8 @@ void MsmScheduleBatch::build(const std::vector<Item> &items, hipStream_t stream,
     NKR_LAUNCH_CHECK();
     k_colscan_batch<<<dim3(div_up(Bmax, 64), J), 64 * kScanGroups, 0, stream>>>(dj);
     NKR_LAUNCH_CHECK();
-    k_schedule_scan_batch<<<J, 1024, 0, stream>>>(dj);
-    NKR_LAUNCH_CHECK();
-    if (!graph) {
-        // every schedule's four counters to the host in one copy
-        totals_dev_.ensure(4 * J);
-        k_gather_totals<<<div_up(4 * J, 256), 256, 0, stream>>>(dj, J, totals_dev_.get());
-        NKR_LAUNCH_CHECK();
-        uint32_t *th = totals_host_.reuse(4 * J);
-        NKR_HIP(hipMemcpyAsync(th, totals_dev_.get(), 4 * J * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-        totals_host_.uploaded(stream);
-        for (uint32_t j = 0; j < J; ++j) {
-            items[j].sched->host_totals_ = th + 4 * j;
-            items[j].sched->host_stage_ = &totals_host_;
-        }
-    } else {
-        for (uint32_t j = 0; j < J; ++j) {
-            items[j].sched->host_totals_ = nullptr;
-            items[j].sched->host_stage_ = nullptr;
-        }
-    }
     k_scatter_batch<<<(uint32_t)blocks, threads, lds, stream>>>(dj, doff, J);
     NKR_LAUNCH_CHECK();
-}
-
-// The piece split a job reads: its schedule's own, or the second one.
-template <class F>
-static const uint32_t *job_counters(const MsmJob<F> &jb)
-{
-    return jb.sched->bucket_start_.get() + jb.sched->plan().B + (jb.alt ? 4 : 0);
-}
-template <class F>
-static const uint32_t *job_piece_start(const MsmJob<F> &jb)
-{
-    return jb.alt ? jb.sched->alt_piece_start_.get() : jb.sched->piece_start_.get();
-}
-template <class F>
-static uint64_t job_max_pieces(const MsmJob<F> &jb)
-{
-    return jb.alt ? jb.sched->alt_max_pieces() : jb.sched->max_pieces();
 }
 
 template <class F>
@@ -1040,9 +1096,9 @@ static std::vector<const void *> layout_key(const std::vector<MsmJob<F>> &jobs)
         key.push_back(jb.bases->data());
         key.push_back(jb.sched->sorted_.get());
         key.push_back(jb.sched->bucket_start_.get());
-        key.push_back(job_piece_start(jb));
         key.push_back(jb.planes);
-        key.push_back(reinterpret_cast<const void *>((uintptr_t)job_max_pieces(jb)));
+        key.push_back(reinterpret_cast<const void *>((uintptr_t)jb.sched->plan().max_entries()));
+        key.push_back(reinterpret_cast<const void *>((uintptr_t)jb.sched->plan().B));
     }
     return key;
 }
@@ -1057,25 +1113,25 @@ template <class F>
 void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
 {
     std::vector<const void *> key = layout_key(jobs);
-    if (key == key_) return;
+    const MsmLanes lanes = have_lanes_ ? own_lanes_ : msm_lanes(std::is_same<F, fq2_t>::value);
+    if (key == key_ && lanes == lanes_) return;
+    lanes_ = lanes;
     const uint32_t J = (uint32_t)jobs.size();
-    // Per job, sized by its own plan: its level-0 partials in the pool, then
-    // the fold launches' outputs of all jobs; and the per-bucket arrays.
-    std::vector<uint64_t> pool_off(J + 1, 0), b_off(J + 1, 0);
-    fold_levels_ = 0;
+    // The pool: a partial per lane and bucket of the launch (k_reduce_plan),
+    // then the fold launches' outputs of all jobs; and the per-bucket arrays.
+    std::vector<uint64_t> b_off(J + 1, 0);
+    uint64_t entries = 0;
+    const uint64_t max_lanes = *std::max_element(lanes_.lanes, lanes_.lanes + 4);
     for (uint32_t j = 0; j < J; ++j) {
         const MsmPlan &p = jobs[j].sched->plan();
         NKR_REQUIRE(jobs[j].bases->plan().n == p.n && jobs[j].bases->plan().c == p.c,
                     "MSM bases and schedule disagree");
-        const uint64_t pieces = job_max_pieces(jobs[j]);
-        uint32_t levels = 0;
-        (void)msm_partial_capacity(p, pieces, &levels, nullptr);
-        fold_levels_ = std::max(fold_levels_, levels);
-        pool_off[j + 1] = pool_off[j] + pieces;
+        entries += p.max_entries();
         b_off[j + 1] = b_off[j] + p.B;
     }
-    piece_bound_ = pool_off[J];
-    uint64_t at = piece_bound_, outs = piece_bound_;
+    lane_bound_ = std::min(entries, max_lanes) + J;
+    fold_levels_ = msm_fold_levels(std::min(entries, max_lanes) + 1);
+    uint64_t at = lane_bound_ + b_off[J], outs = at;
     for (uint32_t L = 0; L < kMaxFoldLaunches; ++L) {
         fold_base_[L] = (uint32_t)at;
         outs = fold_outputs(outs);
@@ -1083,7 +1139,8 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
         at += outs;
     }
     NKR_REQUIRE(at < (1ull << 32), "MSM partial pool exceeds 32-bit indexing");
-    rec_cap_ = fold_records(piece_bound_);
+    bucket_total_ = b_off[J];
+    rec_cap_ = fold_records(lane_bound_ + bucket_total_);
     // grow-only: a batch whose composition changes from call to call reuses them
     pool_.ensure(at);
     sums_.ensure(b_off[J]);
@@ -1103,18 +1160,15 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
         d.bases = jb.bases->data();
         d.sorted = jb.sched->sorted_.get();
         d.bucket_start = jb.sched->bucket_start_.get();
-        d.piece_start = job_piece_start(jb);
-        d.piece_len = job_counters(jb) + 3;
         d.reg_start = reg_start_.get() + b_off[j];
         d.reg_count = reg_count_.get() + b_off[j];
         d.sums = sums_.get() + b_off[j];
         d.tree[0] = tree_[0].get() + b_off[j];
         d.tree[1] = tree_[1].get() + b_off[j];
         d.planes = jb.planes;
-        d.pool_off = (uint32_t)pool_off[j];
         d.B = jb.sched->plan().B;
         d.c = jb.sched->plan().c;
-        d.list_off = (uint32_t)b_off[j];
+        d.b_off = (uint32_t)b_off[j];
     }
     std::memcpy(st + jobs_bytes, fold_base_, sizeof(fold_base_));
     // completion lanes: a bucket's lane groups, plus each segment's padding
@@ -1129,7 +1183,7 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
     recs_.ensure(rec_cap_ * kMaxFoldLaunches * sizeof(FoldRec));
     state_.ensure(sizeof(ReduceState));
     jobs_dev_.ensure(table_bytes);
-    piece_base_.ensure(J + 1);  // filled on the device per run
+    lane_base_.ensure(J + 1);  // filled on the device per run
     // k_reduce_plan leaves its counters cleared; new buffers start so (never
     // inside a captured graph, which reuses the layout of an eager run)
     NKR_HIP(hipMemsetAsync(class_count_.get(), 0, class_count_.bytes(), stream));
@@ -1168,51 +1222,28 @@ void MsmBatch<F>::run(const std::vector<MsmJob<F>> &jobs, hipStream_t stream, St
         }
     } relayout{&key_};
 
-    // Completion: as many lane groups per bucket as leave each about `serial`
-    // partials.  One addition deep per group while the launch would not fill
-    // the chip's 65536 lanes twice, then longer runs (idle groups in the
-    // shuffle levels are the price of short ones).
     uint32_t max_class = 0;
     while ((2u << max_class) <= std::min(msm_complete_lanes_cap(), kWaveGroups<F>)) ++max_class;
-    const uint64_t lanes = piece_bound_ * Coop<F>::kLanes;
-    const uint32_t serial = (uint32_t)std::min<uint64_t>(16, std::max<uint64_t>(1, lanes / (2 * 65536)));
     const uint32_t S = kCompleteClasses * J;
-    k_reduce_plan<F><<<dim3(div_up(Bmax, 256), J), 256, 0, stream>>>(
-        jd, J, max_class, serial, state, recs, (uint32_t)rec_cap_, fold_base_dev, class_count_.get(),
-        class_list_.get(), piece_base_.get(), seg_count_.get(), seg_base_.get());
+    const uint32_t plan_threads = std::min<uint32_t>(kPlanThreads, std::max<uint32_t>(256, (Bmax + 63) & ~63u));
+    k_reduce_plan<F><<<dim3(div_up(Bmax, plan_threads), J), plan_threads, 0, stream>>>(
+        jd, J, lanes_, (uint32_t)bucket_total_, max_class, state, recs, (uint32_t)rec_cap_, fold_base_dev, class_count_.get(),
+        class_list_.get(), lane_base_.get(), seg_count_.get(), seg_base_.get());
     NKR_LAUNCH_CHECK();
     // the accumulation stage brackets exactly the k_accumulate launch
     const int acc_stage = std::is_same<F, fq2_t>::value ? kStageAccumulateG2 : kStageAccumulate;
     if (timer) timer->begin(acc_stage, stream);
-    // One workgroup per kAccThreads pieces rather than a grid of resident
-    // size: the accumulation's workgroups then retire all along the launch,
-    // so the other stream's kernels (SpMV and transforms beside the G2
-    // accumulation, the G2 bucket reduction beside the G1 one) get CU slots
-    // as they free up instead of waiting for the whole launch (dense 2^20
-    // Poseidon-style proof 12.0 -> 11.2 ms and 64-proof mix 33.5-34.0 ->
-    // 31.2-32.4 ms with the witness in HBM, on MI355X).
-    const uint64_t blocks = div_up(piece_bound_, kAccThreads);
-    k_accumulate<F><<<(uint32_t)std::max<uint64_t>(blocks, 1), kAccThreads, 0, stream>>>(jd, piece_base_.get(), J,
-                                                                                        pool_.get());
+    k_accumulate<F><<<(uint32_t)div_up(lane_bound_, kAccThreads), kAccThreads, 0, stream>>>(
+        jd, lane_base_.get(), J, state, pool_.get());
     NKR_LAUNCH_CHECK();
     if (timer) {
         timer->end(acc_stage, stream);
         timer->begin(kStageFold, stream);
     }
-    // Fold launches the largest bucket of any job needs: read from the host
-    // copy of the schedules' counters.  The accumulation is already queued,
-    // so this wait overlaps the GPU's work instead of stalling it.
-    uint32_t levels = 0;
-    if (graph) {
-        levels = fold_levels_;
-    } else {
-        for (const auto &jb : jobs) {
-            const uint64_t cnt = (jb.alt ? jb.sched->alt_totals_host() : jb.sched->totals_host())[2];
-            levels = std::max(levels, msm_fold_levels(cnt));
-        }
-    }
-    NKR_REQUIRE(levels <= fold_levels_, "MSM bucket exceeds the partial-sum capacity");
-    for (uint32_t L = 0; L * kFoldLevelsPerLaunch < levels; ++L) {
+    // as many fold launches as one bucket with every lane's partial would
+    // need (2, or 3 beyond 2^18 lanes): an empty one costs less than the
+    // host's wait for the largest count
+    for (uint32_t L = 0; L * kFoldLevelsPerLaunch < fold_levels_; ++L) {
         const uint64_t blocks = std::min<uint64_t>(div_up(fold_cap_[L], 4), 1024);
         k_fold<F><<<(uint32_t)blocks, 256, 0, stream>>>(state, recs + (size_t)L * rec_cap_, L, fold_base_[L],
                                                       pool_.get());

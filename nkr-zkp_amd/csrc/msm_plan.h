@@ -10,19 +10,36 @@
 
 namespace nkr {
 
-// Largest accumulation piece, fold fan-in and the completion limit.  Small
-// MSMs use shorter pieces (down to kMsmPieceMin) so that the serial chain of
-// one thread, not the amount of work, stops dominating their latency.
-constexpr uint32_t kMsmPiece = 64;
-constexpr uint32_t kMsmPieceMin = 4;
+// Fold fan-in of one level and the completion limit.
 constexpr uint32_t kMsmFoldIn = 4;
 constexpr uint32_t kMsmCompleteMax = 64;
 constexpr uint32_t kMaxFoldLevels = 12;
-// The piece length is chosen on the device once the number of non-zero
-// digits E is known: the largest power of two <= E / 2^target_log,
-// clamped to [piece_lo, piece_hi], so a schedule has about 2^target_log
-// pieces (default 2^19: every resident accumulation thread busy).
-constexpr uint32_t kMsmTargetPiecesLog = 19;
+// Accumulation lanes.  A batch's E sorted entries (non-zero digits, known on
+// the device) are split evenly: each lane sums ceil(E / lanes) consecutive
+// ones, a serial chain, and leaves about one partial sum to the bucket
+// reduction, whose additions have a quarter (G2: an eighth) of the chip's
+// lanes' parallelism but only 2.5 us (3.8 us) of latency.  lanes[i] applies
+// while E is below below[i] (lanes[3] from below[2] on):
+//   one wave per SIMD (65536 lanes) while the chain is short: 4.6 us per
+//   addition at G1, 13 us at G2, with single entries at the smallest sizes;
+//   more waves (G1 up to three per SIMD, G2 two) once what they gain in
+//   throughput (G1 5.0 -> 4.0 us per wave and SIMD, G2 13 -> 12.2) is more
+//   than the reduction of their partials costs (10 and 29 us per 65536);
+//   two full rounds of those for the largest, whose last round then ends
+//   early where another stream's kernels took some of the slots.
+struct MsmLanes {
+    uint32_t lanes[4];
+    uint64_t below[3];
+    uint32_t piece_min;  // shortest run of a lane
+    bool operator==(const MsmLanes &o) const
+    {
+        return std::equal(lanes, lanes + 4, o.lanes) && std::equal(below, below + 3, o.below) &&
+               piece_min == o.piece_min;
+    }
+};
+constexpr MsmLanes kMsmLanesG1 = {{1u << 16, 2u << 16, 4u << 16, 6u << 16}, {1u << 22, 1u << 24, 1u << 25}, 1};
+constexpr MsmLanes kMsmLanesG2 = {{1u << 16, 1u << 16, 2u << 16, 4u << 16}, {1u << 19, 1u << 21, 1u << 23}, 1};
+constexpr uint32_t kMsmMaxLanesLog = 19;  // at least log2 of every lane count above
 // Largest bucket count (c <= 16): the histograms and bucket scans hold B
 // counts in one workgroup's LDS (128 KiB of gfx950's 160 KiB).
 constexpr uint32_t kMsmMaxBuckets = 1u << 15;
@@ -44,7 +61,7 @@ struct MsmPlan {
     uint32_t c = 0;         // window width in bits
     uint32_t W = 0;         // windows (signed digits), c*W >= 255
     uint32_t B = 0;         // buckets 1..B, B = 2^(c-1)
-    uint32_t piece_lo = 0;  // bounds of the accumulation piece length
+    uint32_t piece_lo = 0;  // bounds of the accumulation piece length (max_pieces)
     uint32_t piece_hi = 0;
 
     // ~3/4 log2 n bits (16 from 2^20 terms up), or c_override when non-zero.
@@ -74,10 +91,8 @@ struct MsmPlan {
         p.c = c;
         p.W = (255 + c - 1) / c;
         p.B = 1u << (c - 1);
-        // The piece length follows the actual number of non-zero digits
-        // (chosen on the device): sparse witnesses get short serial chains.
-        p.piece_lo = kMsmPieceMin;
-        p.piece_hi = kMsmPiece;
+        p.piece_lo = 1;
+        p.piece_hi = UINT32_MAX;
         NKR_REQUIRE((uint64_t)p.W * n < (1ull << 31), "MSM too large for 31-bit entry indices");
         return p;
     }
@@ -87,7 +102,7 @@ struct MsmPlan {
     uint64_t max_entries() const { return (uint64_t)n * W; }
     // Upper bound of level-0 pieces for any scalars when the device targets
     // 2^target_log pieces: the piece p it picks is piece_hi, or
-    // p > E / 2^(target_log + 1).  Every bucket may add one short piece.
+    // p >= E / 2^target_log.  Every bucket may add one short piece.
     uint64_t max_pieces(uint32_t target_log) const
     {
         NKR_REQUIRE(piece_lo >= 1 && piece_lo <= piece_hi, "MSM piece bounds must satisfy 1 <= lo <= hi");
@@ -95,14 +110,6 @@ struct MsmPlan {
         const uint64_t by_lo = max_entries() / piece_lo;
         const uint64_t by_target = std::max<uint64_t>(2ull << target_log, max_entries() / piece_hi);
         return std::min(by_lo, by_target) + B + 1;
-    }
-    // The same plan with a fixed piece length.
-    MsmPlan with_piece(uint32_t piece) const
-    {
-        NKR_REQUIRE(piece >= 1, "MSM piece length must be at least 1");
-        MsmPlan p = *this;
-        p.piece_lo = p.piece_hi = piece;
-        return p;
     }
 };
 

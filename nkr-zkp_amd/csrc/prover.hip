@@ -73,7 +73,7 @@ Groth16Prover::Groth16Prover(const nkr_g16_circuit &c, const nkr_g16_pk &pk, int
     NKR_REQUIRE(tn.ntt_split_policy <= 2, "tuning: NTT split policy must be 0 (default), 1 or 2");
     NKR_REQUIRE(tn.msm_target_pieces_log == 0 || (tn.msm_target_pieces_log >= 12 && tn.msm_target_pieces_log <= 24),
                 "tuning: MSM target pieces must be 2^12 .. 2^24");
-    NKR_REQUIRE(tn.witness_g1_piece_min <= kMsmPiece, "tuning: witness G1 piece minimum must be 0..64");
+    NKR_REQUIRE(tn.witness_g1_piece_min <= 64, "tuning: witness G1 piece minimum must be 0..64");
     // validate_circuit / validate_proving_key (protocols/groth16/common/src/protocol.cpp:9-67)
     check_circuit(c);
     NKR_REQUIRE(pk.a_query && pk.b_g1_query && pk.b_g2_query && pk.l_query && pk.h_query,
@@ -124,8 +124,10 @@ Groth16Prover::Groth16Prover(const nkr_g16_circuit &c, const nkr_g16_pk &pk, int
     wplan_ = MsmPlan::choose(cols_, tn.witness_window_bits);
     if (wplan_.c > 15) wplan_ = MsmPlan::choose(cols_, 15);
     hplan_ = MsmPlan::choose(rows_, tn.h_window_bits);
-    wsched_.set_target_log(tn.msm_target_pieces_log);
-    hsched_.set_target_log(tn.msm_target_pieces_log);
+    if (tn.msm_target_pieces_log || tn.witness_g1_piece_min) {
+        batch_g1_.set_lanes(msm_lanes(false, tn.msm_target_pieces_log, tn.witness_g1_piece_min));
+        batch_g2_.set_lanes(msm_lanes(true, tn.msm_target_pieces_log));
+    }
 
     {
         DeviceBuffer<g1_jac> tmp1(std::max(cols_, rows_));
@@ -185,11 +187,6 @@ Groth16Prover::Groth16Prover(const nkr_g16_circuit &c, const nkr_g16_pk &pk, int
     upload_ = std::make_unique<WitnessUpload>(cols_);
     NKR_HIP(hipStreamSynchronize(stream_));
     helpers_ = std::make_unique<HostHelpers>(2);
-    // The witness G1 MSMs read the schedule in pieces of at least 32 entries
-    // (a few partial sums per bucket to complete); bs2 keeps the short
-    // device-chosen pieces its one-wave-per-SIMD accumulation needs.
-    // Measured on the 2^20 prove: 4.13 -> 3.98 ms.
-    wsched_.set_alt_pieces(tn.witness_g1_piece_min ? tn.witness_g1_piece_min : 32);
     release_on_throw.armed = false;
 }
 
@@ -461,9 +458,9 @@ void Groth16Prover::run(const fr_t *z, void *raw_out, void *az, void *bz, void *
     // latency-bound reduction levels are paid once for all four.
     hsched_.build(pa_.get(), hplan_, s, t);
     NKR_HIP(hipStreamWaitEvent(s, ev_wsched_, 0));
-    batch_g1_.run({MsmJob<fq_t>{&a_, &wsched_, planes1_.get() + 0 * cw, true},
-                   MsmJob<fq_t>{&b1_, &wsched_, planes1_.get() + 1 * cw, true},
-                   MsmJob<fq_t>{&l_, &wsched_, planes1_.get() + 2 * cw, true},
+    batch_g1_.run({MsmJob<fq_t>{&a_, &wsched_, planes1_.get() + 0 * cw},
+                   MsmJob<fq_t>{&b1_, &wsched_, planes1_.get() + 1 * cw},
+                   MsmJob<fq_t>{&l_, &wsched_, planes1_.get() + 2 * cw},
                    MsmJob<fq_t>{&h_, &hsched_, planes1_.get() + 3 * cw}},
                   s, t);
     const size_t n1 = 3 * cw + hplan_.c;
