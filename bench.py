@@ -401,6 +401,8 @@ def main() -> int:
     stage_ms = (ctypes.c_double * len(STAGES))()
     counters = (ctypes.c_uint64 * 4)()
     N._check(N.lib().nkr_g16_profile_read(prover.h, stage_ms, counters))
+    entries_of = (ctypes.c_uint64 * 3)()
+    N._check(N.lib().nkr_g16_profile_entries(prover.h, entries_of))
     N._check(N.lib().nkr_g16_profile(prover.h, 0))
     stages = {k: round(stage_ms[i] / args.steps, 3) for i, k in enumerate(STAGES)}
     log(f"stages (device time per prove, overlapping streams) {stages}")
@@ -425,12 +427,14 @@ def main() -> int:
     # products).  The G2 accumulation (bs2: 128 B bases, 30 Fq products per
     # entry with 3-product Fq2 Karatsuba) is reported beside it.
     proves = max(1, counters[0])
-    e_w = counters[2] / proves          # witness schedule: 3 G1 MSMs + 1 G2 MSM
-    e_h = counters[3] / proves          # H schedule: 1 G1 MSM
+    e_w = entries_of[0] / proves        # witness schedule: ar and zk
+    e_b = entries_of[1] / proves        # the schedule of bs1 and bs2
+    e_h = entries_of[2] / proves        # H schedule
     g1_ms = stage_ms[4] / args.steps
     g2_ms = stage_ms[7] / args.steps
     kern = {}
-    for name, ms, entries, per_bytes, per_mul in (("g1", g1_ms, 3 * e_w + e_h, 68, 10), ("g2", g2_ms, e_w, 132, 30)):
+    for name, ms, entries, per_bytes, per_mul in (("g1", g1_ms, 2 * e_w + e_b + e_h, 68, 10),
+                                                  ("g2", g2_ms, e_b, 132, 30)):
         muls = entries * per_mul
         kern[name] = {"launch_ms": round(ms, 4), "entries": int(entries), "alg_fq_mul": int(muls),
                       "alg_bytes": int(entries * per_bytes),

@@ -220,11 +220,17 @@ int nkr_g16_server_destroy(nkr_g16_server *server);
  *   totals do not add up to the proof's latency.
  * counters[0] = proves timed, counters[1] = accumulation launches,
  * counters[2] = bucket entries (non-zero signed digits) of the witness
- * schedule, summed over proves (each is used by 3 G1 MSMs and the G2 MSM),
- * counters[3] = bucket entries of the H schedule (the fifth MSM). */
+ * schedule, summed over proves (each is used by ar and zk, and by bs1 and bs2
+ * unless they have a schedule of their own), counters[3] = bucket entries of
+ * the H schedule (the fifth MSM). */
 #define NKR_G16_STAGES 8
 int nkr_g16_profile(nkr_g16_ctx *ctx, int enable);
 int nkr_g16_profile_read(const nkr_g16_ctx *ctx, double *stage_ms, uint64_t *counters);
+/* entries[0], [1] and [2]: the bucket entries, over the same proves, of the
+ * schedules that ar and zk, bs1 and bs2, and H read.  bs1 and bs2 have one of
+ * their own, over the variables that occur in B, where that leaves out at
+ * least a quarter of the variables. */
+int nkr_g16_profile_entries(const nkr_g16_ctx *ctx, uint64_t *entries);
 
 /* check_witness (protocols/groth16/common/src/protocol.cpp:69-83): *ok = 1
  * when (A z) * (B z) = C z row by row.  Host arithmetic. */

@@ -76,7 +76,7 @@ private:
     void drop_graph() noexcept;
     struct Slot {
         DeviceBuffer<fr_t> z, pa, pb, pc;
-        MsmSchedule wsched, hsched;
+        MsmSchedule wsched, bsched, hsched;
     };
     int device_;
     hipStream_t stream_ = nullptr;   // SpMV, transforms, H schedules, G1 MSMs

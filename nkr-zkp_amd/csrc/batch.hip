@@ -107,7 +107,7 @@ uint64_t BatchProver::device_bytes() const
                  planes_2_.bytes();
     for (const auto &sl : slots_)
         b += sl->z.bytes() + sl->pa.bytes() + sl->pb.bytes() + sl->pc.bytes() + sl->wsched.device_bytes() +
-             sl->hsched.device_bytes();
+             sl->bsched.device_bytes() + sl->hsched.device_bytes();
     return b;
 }
 
@@ -164,9 +164,9 @@ void BatchProver::prove(const std::vector<BatchItem> &items)
         const Groth16Prover &g = *items[i].ctx;
         for (int m = 0; m < 3; ++m) max_long = std::max(max_long, g.views_[m].n_long);
         max_rows = std::max(max_rows, g.rows_);
-        pw_off[i + 1] = pw_off[i] + 3 * g.wplan_.c;
+        pw_off[i + 1] = pw_off[i] + g.planes_g1_witness();
         ph_off[i + 1] = ph_off[i] + g.hplan_.c;
-        p2_off[i + 1] = p2_off[i] + g.wplan_.c;
+        p2_off[i + 1] = p2_off[i] + g.bplan_.c;
     }
     planes_w_.ensure(pw_off[K]);
     planes_h_.ensure(ph_off[K]);
@@ -225,8 +225,9 @@ void BatchProver::prove(const std::vector<BatchItem> &items)
             for (size_t i = 0; i < K; ++i) {
                 Groth16Prover &g = *items[i].ctx;
                 Slot &sl = *slots_[i];
-                wsorts.push_back({&sl.wsched, sl.z.get(), g.wplan_});
-                g2jobs.push_back({&g.b2_, &sl.wsched, planes_2_.get() + p2_off[i]});
+                wsorts.push_back({&sl.wsched, sl.z.get(), nullptr, g.wplan_});
+                if (g.own_b_schedule()) wsorts.push_back({&sl.bsched, sl.z.get(), g.b_terms_.get(), g.bplan_});
+                g2jobs.push_back({&g.b2_, g.own_b_schedule() ? &sl.bsched : &sl.wsched, planes_2_.get() + p2_off[i]});
             }
             sort_w_.build(wsorts, stream2_, graph);
             NKR_HIP(hipEventRecord(ev_wsched_, stream2_));
@@ -293,7 +294,7 @@ void BatchProver::prove(const std::vector<BatchItem> &items)
         for (size_t i = 0; i < K; ++i) {
             Groth16Prover &g = *items[i].ctx;
             Slot &sl = *slots_[i];
-            hsorts.push_back({&sl.hsched, sl.pa.get(), g.hplan_});
+            hsorts.push_back({&sl.hsched, sl.pa.get(), nullptr, g.hplan_});
         }
         sort_h_.build(hsorts, stream_, graph);
         NKR_HIP(hipStreamWaitEvent(stream_, ev_wsched_, 0));
@@ -302,9 +303,9 @@ void BatchProver::prove(const std::vector<BatchItem> &items)
             Slot &sl = *slots_[i];
             const uint32_t cw = g.wplan_.c;
             Xyzz<fq_t> *pw = planes_w_.get() + pw_off[i];
-            g1jobs.push_back({&g.a_, &sl.wsched, pw + 0 * cw});
-            g1jobs.push_back({&g.b1_, &sl.wsched, pw + 1 * cw});
-            g1jobs.push_back({&g.l_, &sl.wsched, pw + 2 * cw});
+            g1jobs.push_back({&g.a_, &sl.wsched, pw});
+            g1jobs.push_back({&g.l_, &sl.wsched, pw + cw});
+            g1jobs.push_back({&g.b1_, g.own_b_schedule() ? &sl.bsched : &sl.wsched, pw + 2 * cw});
             g1jobs.push_back({&g.h_, &sl.hsched, planes_h_.get() + ph_off[i]});
         }
         batch_g1_.run(g1jobs, stream_, nullptr, graph);

@@ -418,6 +418,14 @@ int nkr_g16_profile_read(const nkr_g16_ctx *ctx, double *stage_ms, uint64_t *cou
     });
 }
 
+int nkr_g16_profile_entries(const nkr_g16_ctx *ctx, uint64_t *entries)
+{
+    return guarded([&] {
+        NKR_REQUIRE(ctx && entries, "null argument");
+        ctx->prover->profile_entries(entries);
+    });
+}
+
 int nkr_g16_blind(const nkr_g16_pk *pk, const void *raw, const void *r, const void *s, void *proof_out)
 {
     return guarded([&] {

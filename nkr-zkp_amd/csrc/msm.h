@@ -80,12 +80,19 @@ private:
     DeviceBuffer<Affine<F>> pts_;
 };
 
+// The terms i < n for which a[i] or b[i] (device arrays) is not infinity, in
+// order.  Synchronises the stream.
+void msm_finite_terms(const g1_jac *a, const g2_jac *b, uint32_t n, std::vector<uint32_t> &terms, hipStream_t stream);
+
 // Signed-digit recoding and bucket sort of one scalar vector; shared by every
 // MSM that uses the same scalars (the witness drives four of the five).
 // Entirely asynchronous on `stream`.
 class MsmSchedule {
 public:
-    void build(const fr_t *scalars_mont, const MsmPlan &plan, hipStream_t stream, StageTimer *timer = nullptr);
+    // pick: optional device list of plan.n scalar numbers; term i's scalar is
+    // then scalars_mont[pick[i]] (for bases prepared with the same list).
+    void build(const fr_t *scalars_mont, const uint32_t *pick, const MsmPlan &plan, hipStream_t stream,
+               StageTimer *timer = nullptr);
     // Sizes the buffers for `plan`; returns the scalars per sort workgroup.
     uint32_t prepare(const MsmPlan &plan);
     const MsmPlan &plan() const { return plan_; }
@@ -126,6 +133,7 @@ public:
     struct Item {
         MsmSchedule *sched;
         const fr_t *scalars_mont;
+        const uint32_t *pick;
         MsmPlan plan;
     };
     // graph: the launches are being captured into a graph that is replayed

@@ -112,8 +112,10 @@ __device__ __forceinline__ void for_each_digit(const fr_t &s, uint32_t c, uint32
 
 // Histogram of the bucket magnitudes of scalars [b * per_block, ...) in LDS,
 // written as row b of the (blocks x B) count matrix.
-__device__ __forceinline__ void hist_block(uint32_t *hist, const fr_t *__restrict__ scalars, uint32_t n, uint32_t c,
-                                          uint32_t W, uint32_t B, uint32_t per_block, uint32_t b,
+// Term i's scalar is scalars[pick[i]], or scalars[i] without a list.
+__device__ __forceinline__ void hist_block(uint32_t *hist, const fr_t *__restrict__ scalars,
+                                          const uint32_t *__restrict__ pick, uint32_t n, uint32_t c, uint32_t W,
+                                          uint32_t B, uint32_t per_block, uint32_t b,
                                           uint32_t *__restrict__ block_count)
 {
     for (uint32_t k = threadIdx.x; k < B; k += blockDim.x) hist[k] = 0;
@@ -121,7 +123,7 @@ __device__ __forceinline__ void hist_block(uint32_t *hist, const fr_t *__restric
     const uint32_t beg = b * per_block;
     const uint32_t end = min(n, beg + per_block);
     for (uint32_t i = beg + threadIdx.x; i < end; i += blockDim.x) {
-        const fr_t s = fp_from_mont(scalars[i]);
+        const fr_t s = fp_from_mont(scalars[pick ? pick[i] : i]);
         for_each_digit(s, c, W, [&](uint32_t, int32_t d) {
             const uint32_t m = (uint32_t)(d < 0 ? -d : d);
             atomicAdd(&hist[m - 1], 1u);
@@ -208,8 +210,9 @@ __device__ __forceinline__ void colscan_tile(uint32_t *__restrict__ block_count,
 // Every workgroup scans the (at most kMsmMaxBuckets / 64) tile totals for its
 // own cursors, which costs less than a launch that would do it once; the
 // first one writes the bucket starts for the kernels after it.
-__device__ __forceinline__ void scatter_block(uint32_t *cursor, const fr_t *__restrict__ scalars, uint32_t n,
-                                             uint32_t c, uint32_t W, uint32_t B, uint32_t per_block, uint32_t b,
+__device__ __forceinline__ void scatter_block(uint32_t *cursor, const fr_t *__restrict__ scalars,
+                                             const uint32_t *__restrict__ pick, uint32_t n, uint32_t c, uint32_t W,
+                                             uint32_t B, uint32_t per_block, uint32_t b,
                                              const uint32_t *__restrict__ in_tile,
                                              const uint32_t *__restrict__ tile_total,
                                              const uint32_t *__restrict__ block_off,
@@ -228,7 +231,7 @@ __device__ __forceinline__ void scatter_block(uint32_t *cursor, const fr_t *__re
     const uint32_t beg = b * per_block;
     const uint32_t end = min(n, beg + per_block);
     for (uint32_t i = beg + threadIdx.x; i < end; i += blockDim.x) {
-        const fr_t s = fp_from_mont(scalars[i]);
+        const fr_t s = fp_from_mont(scalars[pick ? pick[i] : i]);
         for_each_digit(s, c, W, [&](uint32_t w, int32_t d) {
             const uint32_t m = (uint32_t)(d < 0 ? -d : d);
             const uint32_t pos = atomicAdd(&cursor[m - 1], 1u);
@@ -237,12 +240,13 @@ __device__ __forceinline__ void scatter_block(uint32_t *cursor, const fr_t *__re
     }
 }
 
-__global__ __launch_bounds__(kSortThreads) void k_hist(const fr_t *__restrict__ scalars, uint32_t n, uint32_t c,
+__global__ __launch_bounds__(kSortThreads) void k_hist(const fr_t *__restrict__ scalars,
+                                                       const uint32_t *__restrict__ pick, uint32_t n, uint32_t c,
                                                        uint32_t W, uint32_t B, uint32_t per_block,
                                                        uint32_t *__restrict__ block_count)
 {
     extern __shared__ uint32_t lds[];
-    hist_block(lds, scalars, n, c, W, B, per_block, blockIdx.x, block_count);
+    hist_block(lds, scalars, pick, n, c, W, B, per_block, blockIdx.x, block_count);
 }
 
 __global__ __launch_bounds__(64 * kScanGroups) void k_colscan(uint32_t *__restrict__ block_count, uint32_t blocks,
@@ -252,7 +256,8 @@ __global__ __launch_bounds__(64 * kScanGroups) void k_colscan(uint32_t *__restri
     colscan_tile(block_count, blocks, B, blockIdx.x, in_tile, tile_total);
 }
 
-__global__ __launch_bounds__(kSortThreads) void k_scatter(const fr_t *__restrict__ scalars, uint32_t n, uint32_t c,
+__global__ __launch_bounds__(kSortThreads) void k_scatter(const fr_t *__restrict__ scalars,
+                                                          const uint32_t *__restrict__ pick, uint32_t n, uint32_t c,
                                                           uint32_t W, uint32_t B, uint32_t per_block,
                                                           const uint32_t *__restrict__ in_tile,
                                                           const uint32_t *__restrict__ tile_total,
@@ -261,7 +266,7 @@ __global__ __launch_bounds__(kSortThreads) void k_scatter(const fr_t *__restrict
                                                           uint32_t *__restrict__ sorted)
 {
     extern __shared__ uint32_t lds[];
-    scatter_block(lds, scalars, n, c, W, B, per_block, blockIdx.x, in_tile, tile_total, block_off, bucket_start,
+    scatter_block(lds, scalars, pick, n, c, W, B, per_block, blockIdx.x, in_tile, tile_total, block_off, bucket_start,
                   sorted);
 }
 
@@ -282,6 +287,7 @@ __device__ __forceinline__ uint32_t find_segment(const uint32_t *starts, uint32_
 // One schedule of a batched sort.
 struct SortJob {
     const fr_t *scalars;
+    const uint32_t *pick;
     uint32_t n, c, W, B, blocks, per_block;
     uint32_t *block_count, *in_tile, *tile_total, *bucket_start, *sorted;
 };
@@ -293,7 +299,7 @@ __global__ __launch_bounds__(kSortThreads) void k_hist_batch(const SortJob *__re
     extern __shared__ uint32_t lds[];
     const uint32_t j = find_segment(block_off, J, blockIdx.x);
     const SortJob &jb = jobs[j];
-    hist_block(lds, jb.scalars, jb.n, jb.c, jb.W, jb.B, jb.per_block, blockIdx.x - block_off[j], jb.block_count);
+    hist_block(lds, jb.scalars, jb.pick, jb.n, jb.c, jb.W, jb.B, jb.per_block, blockIdx.x - block_off[j], jb.block_count);
 }
 
 __global__ __launch_bounds__(64 * kScanGroups) void k_colscan_batch(const SortJob *__restrict__ jobs)
@@ -309,7 +315,7 @@ __global__ __launch_bounds__(kSortThreads) void k_scatter_batch(const SortJob *_
     extern __shared__ uint32_t lds[];
     const uint32_t j = find_segment(block_off, J, blockIdx.x);
     const SortJob &jb = jobs[j];
-    scatter_block(lds, jb.scalars, jb.n, jb.c, jb.W, jb.B, jb.per_block, blockIdx.x - block_off[j], jb.in_tile,
+    scatter_block(lds, jb.scalars, jb.pick, jb.n, jb.c, jb.W, jb.B, jb.per_block, blockIdx.x - block_off[j], jb.in_tile,
                   jb.tile_total, jb.block_count, jb.bucket_start, jb.sorted);
 }
 
@@ -889,6 +895,14 @@ __global__ __launch_bounds__(kTreeThreads) void k_tree_lds(const JobDev<F> *__re
             coop_store<F>(jb.tree[src ^ 1u], (size_t)blockIdx.x * (t1 + 1) + e, coop_load<F>(buf[lv & 1], e));
 }
 
+// finite[i] = 1 if a[i] or b[i] is not infinity.
+__global__ __launch_bounds__(256) void k_finite(const g1_jac *__restrict__ a, const g2_jac *__restrict__ b, uint32_t n,
+                                                uint8_t *__restrict__ finite)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) finite[i] = !a[i].Z.is_zero() || !b[i].Z.is_zero() ? 1 : 0;
+}
+
 // Base preparation: normalise the reference-layout Jacobian point and store
 // 2^(c*w) * P for every window w (affine, infinity flagged).
 template <class F>
@@ -986,6 +1000,19 @@ uint64_t msm_job_bytes(const MsmPlan &p)
            fold_records(partials) * kMaxFoldLaunches * sizeof(FoldRec) + p.c * sizeof(Xyzz<F>) + 1024;
 }
 
+void msm_finite_terms(const g1_jac *a, const g2_jac *b, uint32_t n, std::vector<uint32_t> &terms, hipStream_t stream)
+{
+    DeviceBuffer<uint8_t> dev(n);
+    std::vector<uint8_t> host(n);
+    k_finite<<<div_up(n, 256), 256, 0, stream>>>(a, b, n, dev.get());
+    NKR_LAUNCH_CHECK();
+    NKR_HIP(hipMemcpyAsync(host.data(), dev.get(), n, hipMemcpyDeviceToHost, stream));
+    NKR_HIP(hipStreamSynchronize(stream));
+    terms.clear();
+    for (uint32_t i = 0; i < n; ++i)
+        if (host[i]) terms.push_back(i);
+}
+
 template <class F>
 void MsmBases<F>::prepare(const Jacobian<F> *jacobian, const uint32_t *perm, const MsmPlan &plan,
                           hipStream_t stream)
@@ -1030,19 +1057,20 @@ uint32_t MsmSchedule::prepare(const MsmPlan &plan)
     return div_up(n, blocks_);
 }
 
-void MsmSchedule::build(const fr_t *scalars_mont, const MsmPlan &plan, hipStream_t stream, StageTimer *timer)
+void MsmSchedule::build(const fr_t *scalars_mont, const uint32_t *pick, const MsmPlan &plan, hipStream_t stream,
+                        StageTimer *timer)
 {
     const uint32_t per_block = prepare(plan);
     const uint32_t n = plan.n, B = plan.B;
     const size_t lds = (size_t)B * sizeof(uint32_t);
     const uint32_t threads = std::min<uint32_t>(kSortThreads, (per_block + 63) & ~63u);
     if (timer) timer->begin(kStageSort, stream);
-    k_hist<<<blocks_, threads, lds, stream>>>(scalars_mont, n, plan.c, plan.W, B, per_block, block_count_.get());
+    k_hist<<<blocks_, threads, lds, stream>>>(scalars_mont, pick, n, plan.c, plan.W, B, per_block, block_count_.get());
     NKR_LAUNCH_CHECK();
     k_colscan<<<div_up(B, 64), 64 * kScanGroups, 0, stream>>>(block_count_.get(), blocks_, B, in_tile_.get(),
                                                               tile_total_.get());
     NKR_LAUNCH_CHECK();
-    k_scatter<<<blocks_, threads, lds, stream>>>(scalars_mont, n, plan.c, plan.W, B, per_block, in_tile_.get(),
+    k_scatter<<<blocks_, threads, lds, stream>>>(scalars_mont, pick, n, plan.c, plan.W, B, per_block, in_tile_.get(),
                                                  tile_total_.get(), block_count_.get(), bucket_start_.get(),
                                                  sorted_.get());
     NKR_LAUNCH_CHECK();
@@ -1066,7 +1094,7 @@ void MsmScheduleBatch::build(const std::vector<Item> &items, hipStream_t stream,
         MsmSchedule &s = *items[j].sched;
         const MsmPlan &p = items[j].plan;
         const uint32_t per_block = s.prepare(p);
-        jobs[j] = SortJob{items[j].scalars_mont, p.n,  p.c, p.W, p.B, s.blocks_, per_block, s.block_count_.get(),
+        jobs[j] = SortJob{items[j].scalars_mont, items[j].pick, p.n, p.c, p.W, p.B, s.blocks_, per_block, s.block_count_.get(),
                           s.in_tile_.get(), s.tile_total_.get(), s.bucket_start_.get(), s.sorted_.get()};
         off[j] = (uint32_t)blocks;
         blocks += s.blocks_;
@@ -1303,7 +1331,7 @@ template <class F>
 Jacobian<F> MsmContext<F>::run(const fr_t *scalars_dev, hipStream_t stream)
 {
     const MsmPlan &plan = bases_.plan();
-    sched_.build(scalars_dev, plan, stream);
+    sched_.build(scalars_dev, nullptr, plan, stream);
     batch_.run({MsmJob<F>{&bases_, &sched_, planes_.get()}}, stream);
     std::vector<Xyzz<F>> host(plan.c);
     NKR_HIP(hipMemcpyAsync(host.data(), planes_.get(), plan.c * sizeof(Xyzz<F>), hipMemcpyDeviceToHost, stream));

@@ -48,6 +48,9 @@ public:
     static constexpr int kStages = 8;
     void set_profiling(bool on);
     void profile_read(double *stage_ms, uint64_t *counters) const;
+    // bucket entries since profiling was switched on: of the witness schedule
+    // (ar and zk), of bs1's and bs2's, of H's
+    void profile_entries(uint64_t *entries) const;
 
     uint64_t device_bytes() const;
     int device() const { return device_; }
@@ -57,7 +60,12 @@ public:
     uint32_t rows() const { return rows_; }
     uint32_t cols() const { return cols_; }
     const MsmPlan &witness_plan() const { return wplan_; }
+    // the plan of bs1 and bs2, and whether they have a schedule of their own
+    const MsmPlan &b_plan() const { return bplan_; }
+    bool own_b_schedule() const { return b_terms_.size() != 0; }
     const MsmPlan &h_plan() const { return hplan_; }
+    // bit planes of the G1 MSMs: ar, zk, bs1, then H
+    uint32_t planes_g1_witness() const { return 2 * wplan_.c + bplan_.c; }
 
 private:
     void release() noexcept;  // streams, events and pinned memory (destructor, failed constructor)
@@ -68,10 +76,17 @@ private:
     DeviceBuffer<fr_t> values_[3];
     CsrView views_[3];
     std::unique_ptr<NttDomain> domain_;
-    MsmPlan wplan_, hplan_;
+    MsmPlan wplan_, bplan_, hplan_;
+    // The B query (bs1 and bs2) without its points at infinity: most R1CS
+    // variables are in no row of B, and a point at infinity would still cost
+    // its digits' sort, its gather and, where another lane of the wave has a
+    // finite one, an addition.  Where at least a quarter of the points go, bs1
+    // and bs2 have a schedule of their own over the columns b_terms_; otherwise
+    // they read the witness schedule (bplan_ is wplan_).
+    DeviceBuffer<uint32_t> b_terms_;
     MsmBases<fq_t> a_, b1_, l_, h_;
     MsmBases<fq2_t> b2_;
-    MsmSchedule wsched_, hsched_;
+    MsmSchedule wsched_, bsched_, hsched_;
     MsmBatch<fq_t> batch_g1_;            // ar, bs1, zk and H as one batch
     MsmBatch<fq2_t> batch_g2_;
     hipStream_t stream2_ = nullptr;      // witness schedule and the G2 MSM, beside the NTT chain
@@ -95,8 +110,8 @@ private:
     };
     void run(const fr_t *z, void *raw_out, void *az, void *bz, void *cz, void *h, const BlindJob *blind = nullptr);
     BlindPre blind_pre(const fr_t &r, const fr_t &s) const;
-    // p1w: the bit planes of ar, bs1 and zk (3 x wplan c), p1h: those of H
-    // (hplan c), p2: those of bs2 (wplan c).
+    // p1w: the bit planes of ar and zk (wplan c each) and bs1 (bplan c), p1h:
+    // those of H (hplan c), p2: those of bs2 (bplan c).
     void finish(const Xyzz<fq_t> *p1w, const Xyzz<fq_t> *p1h, const Xyzz<fq2_t> *p2, const BlindJob *blind,
                 const BlindPre *pre, void *raw_out) const;
     // The two halves of finish: bs2 (and B) from the G2 planes, the rest from the G1 planes.
@@ -126,6 +141,7 @@ private:
     StageTimer timer_;
     double stage_ms_[kStages] = {};
     uint64_t counters_[4] = {};
+    uint64_t b_entries_ = 0;
 };
 
 // blind_proof (protocols/groth16/common/src/protocol.cpp:85-94) with given r, s.

@@ -131,12 +131,32 @@ Groth16Prover::Groth16Prover(const nkr_g16_circuit &c, const nkr_g16_pk &pk, int
 
     {
         DeviceBuffer<g1_jac> tmp1(std::max(cols_, rows_));
-        const void *g1_vecs[3] = {pk.a_query, pk.b_g1_query, pk.l_query};
-        MsmBases<fq_t> *g1_sets[3] = {&a_, &b1_, &l_};
-        for (int k = 0; k < 3; ++k) {
+        const void *g1_vecs[2] = {pk.a_query, pk.l_query};
+        MsmBases<fq_t> *g1_sets[2] = {&a_, &l_};
+        for (int k = 0; k < 2; ++k) {
             NKR_HIP(hipMemcpyAsync(tmp1.get(), g1_vecs[k], (size_t)cols_ * sizeof(g1_jac), hipMemcpyHostToDevice,
                                    stream_));
             g1_sets[k]->prepare(tmp1.get(), nullptr, wplan_, stream_);
+            NKR_HIP(hipStreamSynchronize(stream_));
+        }
+        {
+            DeviceBuffer<g2_jac> tmp2(cols_);
+            NKR_HIP(hipMemcpyAsync(tmp1.get(), pk.b_g1_query, (size_t)cols_ * sizeof(g1_jac), hipMemcpyHostToDevice,
+                                   stream_));
+            NKR_HIP(hipMemcpyAsync(tmp2.get(), pk.b_g2_query, (size_t)cols_ * sizeof(g2_jac), hipMemcpyHostToDevice,
+                                   stream_));
+            std::vector<uint32_t> terms;
+            msm_finite_terms(tmp1.get(), tmp2.get(), cols_, terms, stream_);
+            if (terms.empty()) terms.push_back(0);  // an MSM has at least one term
+            bplan_ = wplan_;
+            if (terms.size() <= cols_ - cols_ / 4) {
+                const uint32_t n = (uint32_t)terms.size();
+                bplan_ = MsmPlan::choose(n, tn.witness_window_bits);
+                if (bplan_.c > 15) bplan_ = MsmPlan::choose(n, 15);
+                upload(b_terms_, terms.data(), terms.size(), stream_);
+            }
+            b1_.prepare(tmp1.get(), b_terms_.get(), bplan_, stream_);
+            b2_.prepare(tmp2.get(), b_terms_.get(), bplan_, stream_);
             NKR_HIP(hipStreamSynchronize(stream_));
         }
         // H query in the basis of the quotient's coset evaluations (the prove
@@ -150,13 +170,6 @@ Groth16Prover::Groth16Prover(const nkr_g16_circuit &c, const nkr_g16_pk &pk, int
         DeviceBuffer<g1_jac> hq(rows_);
         h_query_coset_basis(tmp1.get(), *domain_, hq.get(), stream_);
         h_.prepare(hq.get(), dperm.get(), hplan_, stream_);
-        NKR_HIP(hipStreamSynchronize(stream_));
-    }
-    {
-        DeviceBuffer<g2_jac> tmp2(cols_);
-        NKR_HIP(hipMemcpyAsync(tmp2.get(), pk.b_g2_query, (size_t)cols_ * sizeof(g2_jac), hipMemcpyHostToDevice,
-                               stream_));
-        b2_.prepare(tmp2.get(), nullptr, wplan_, stream_);
         NKR_HIP(hipStreamSynchronize(stream_));
     }
 
@@ -182,8 +195,8 @@ Groth16Prover::Groth16Prover(const nkr_g16_circuit &c, const nkr_g16_pk &pk, int
     fr_t *const table[3] = {pa_.get(), pb_.get(), pc_.get()};
     poly_table_.allocate(3);
     NKR_HIP(hipMemcpyAsync(poly_table_.get(), table, sizeof(table), hipMemcpyHostToDevice, stream_));
-    planes1_.allocate(3 * wplan_.c + hplan_.c);
-    planes2_.allocate(wplan_.c);
+    planes1_.allocate(planes_g1_witness() + hplan_.c);
+    planes2_.allocate(bplan_.c);
     upload_ = std::make_unique<WitnessUpload>(cols_);
     NKR_HIP(hipStreamSynchronize(stream_));
     helpers_ = std::make_unique<HostHelpers>(2);
@@ -215,7 +228,7 @@ void Groth16Prover::release() noexcept
 
 uint64_t Groth16Prover::device_bytes() const
 {
-    uint64_t b = a_.bytes() + b1_.bytes() + l_.bytes() + h_.bytes() + b2_.bytes();
+    uint64_t b = a_.bytes() + b1_.bytes() + l_.bytes() + h_.bytes() + b2_.bytes() + b_terms_.bytes();
     for (int m = 0; m < 3; ++m) b += row_ptr_[m].bytes() + col_idx_[m].bytes() + values_[m].bytes();
     b += z_.bytes() + pa_.bytes() + pb_.bytes() + pc_.bytes();
     if (upload_) b += upload_->device_bytes();
@@ -242,6 +255,7 @@ void Groth16Prover::set_profiling(bool on)
     timer_.enable(on);
     for (double &v : stage_ms_) v = 0;
     for (uint64_t &v : counters_) v = 0;
+    b_entries_ = 0;
 }
 
 void Groth16Prover::profile_read(double *stage_ms, uint64_t *counters) const
@@ -263,6 +277,13 @@ void Groth16Prover::prove_blind(const void *witness, bool on_device, const fr_t 
     }
     const BlindJob job{r, s, proof_out};
     run(z, raw_out, nullptr, nullptr, nullptr, nullptr, &job);
+}
+
+void Groth16Prover::profile_entries(uint64_t *entries) const
+{
+    entries[0] = counters_[2];
+    entries[1] = b_entries_;
+    entries[2] = counters_[3];
 }
 
 // A0 = alpha_1 + r delta_1, B0 = beta_2 + s delta_2 and
@@ -294,11 +315,11 @@ void Groth16Prover::finish_serial(const Xyzz<fq_t> *p1w, const Xyzz<fq_t> *p1h, 
     // raw proof: ar, bs1, zk, qz (G1) and bs2 (G2); blinded: A, C (G1), B (G2)
     g1_xyzz g1[6];
     g2_xyzz g2[2];
-    g1[0] = msm_sum(p1w + 0 * cw, cw);
-    g1[1] = msm_sum(p1w + 1 * cw, cw);
-    g1[2] = msm_sum(p1w + 2 * cw, cw);
+    g1[0] = msm_sum(p1w, cw);
+    g1[1] = msm_sum(p1w + 2 * cw, bplan_.c);
+    g1[2] = msm_sum(p1w + cw, cw);
     g1[3] = msm_sum(p1h, hplan_.c);
-    g2[0] = msm_sum(p2, cw);
+    g2[0] = msm_sum(p2, bplan_.c);
     int n1 = 4, n2 = 1;
     if (blind) {
         g1[4] = xyzz_add(pre->A0, g1[0]);
@@ -327,7 +348,7 @@ void Groth16Prover::finish_serial(const Xyzz<fq_t> *p1w, const Xyzz<fq_t> *p1h, 
 void Groth16Prover::finish_g2(const Xyzz<fq2_t> *p2, const BlindJob *blind, const BlindPre *pre,
                               void *raw_out) const
 {
-    const g2_jac bs2 = msm_finish(p2, wplan_.c);
+    const g2_jac bs2 = msm_finish(p2, bplan_.c);
     std::memcpy(static_cast<uint8_t *>(raw_out) + 384, &bs2, 192);
     if (!blind) return;
     const g2_jac B = xyzz_to_jacobian_affine(xyzz_add(pre->B0, jacobian_to_xyzz(bs2)));
@@ -345,11 +366,11 @@ void Groth16Prover::finish_g1(const Xyzz<fq_t> *p1, const Xyzz<fq_t> *p1h, const
     g1_xyzz pts[6];
     g1_xyzz s_ar = g1_xyzz::infinity(), r_bs1 = g1_xyzz::infinity();
     auto part_zq = [&] {
-        pts[2] = msm_sum(p1 + 2 * cw, cw);
+        pts[2] = msm_sum(p1 + cw, cw);
         pts[3] = msm_sum(p1h, hplan_.c);
     };
     auto part_b = [&] {
-        pts[1] = msm_sum(p1 + 1 * cw, cw);
+        pts[1] = msm_sum(p1 + 2 * cw, bplan_.c);
         if (blind) r_bs1 = g1_mul_glv(pts[1], blind->r);
     };
     // the helpers' tasks refer to this frame: if anything below throws, the
@@ -370,7 +391,7 @@ void Groth16Prover::finish_g1(const Xyzz<fq_t> *p1, const Xyzz<fq_t> *p1h, const
         helpers->run(1, part_b);
         join.h = helpers;
     }
-    pts[0] = msm_sum(p1 + 0 * cw, cw);
+    pts[0] = msm_sum(p1, cw);
     if (blind) {
         pts[4] = xyzz_add(pre->A0, pts[0]);
         s_ar = g1_mul_glv(pts[0], blind->s);
@@ -443,27 +464,29 @@ void Groth16Prover::run(const fr_t *z, void *raw_out, void *az, void *bz, void *
         NKR_HIP(hipMemcpyAsync(h, pc_.get(), poly_bytes, hipMemcpyDeviceToHost, s));
     }
 
-    // The witness schedule and the G2 MSM (bs2) depend only on z: they run on
+    // The witness schedules and the G2 MSM (bs2) depend only on z: they run on
     // the side stream while the main stream computes H.
     NKR_HIP(hipStreamWaitEvent(stream2_, ev_start_, 0));
-    wsched_.build(z, wplan_, stream2_, t);
+    wsched_.build(z, nullptr, wplan_, stream2_, t);
+    MsmSchedule &bsched = own_b_schedule() ? bsched_ : wsched_;
+    if (own_b_schedule()) bsched_.build(z, b_terms_.get(), bplan_, stream2_, t);
     NKR_HIP(hipEventRecord(ev_wsched_, stream2_));
-    batch_g2_.run({MsmJob<fq2_t>{&b2_, &wsched_, planes2_.get()}}, stream2_, t);
-    Xyzz<fq2_t> *h2 = planes2_host_.reuse(cw);
-    NKR_HIP(hipMemcpyAsync(h2, planes2_.get(), cw * sizeof(Xyzz<fq2_t>), hipMemcpyDeviceToHost, stream2_));
+    batch_g2_.run({MsmJob<fq2_t>{&b2_, &bsched, planes2_.get()}}, stream2_, t);
+    Xyzz<fq2_t> *h2 = planes2_host_.reuse(bplan_.c);
+    NKR_HIP(hipMemcpyAsync(h2, planes2_.get(), bplan_.c * sizeof(Xyzz<fq2_t>), hipMemcpyDeviceToHost, stream2_));
     planes2_host_.uploaded(stream2_);
 
     // The G1 MSMs ar, bs1, zk (witness) and H as one batch on the main
     // stream: the witness pieces fill the H accumulation launch, and the
     // latency-bound reduction levels are paid once for all four.
-    hsched_.build(pa_.get(), hplan_, s, t);
+    hsched_.build(pa_.get(), nullptr, hplan_, s, t);
     NKR_HIP(hipStreamWaitEvent(s, ev_wsched_, 0));
-    batch_g1_.run({MsmJob<fq_t>{&a_, &wsched_, planes1_.get() + 0 * cw},
-                   MsmJob<fq_t>{&b1_, &wsched_, planes1_.get() + 1 * cw},
-                   MsmJob<fq_t>{&l_, &wsched_, planes1_.get() + 2 * cw},
-                   MsmJob<fq_t>{&h_, &hsched_, planes1_.get() + 3 * cw}},
+    batch_g1_.run({MsmJob<fq_t>{&a_, &wsched_, planes1_.get()},
+                   MsmJob<fq_t>{&l_, &wsched_, planes1_.get() + cw},
+                   MsmJob<fq_t>{&b1_, &bsched, planes1_.get() + 2 * cw},
+                   MsmJob<fq_t>{&h_, &hsched_, planes1_.get() + planes_g1_witness()}},
                   s, t);
-    const size_t n1 = 3 * cw + hplan_.c;
+    const size_t n1 = planes_g1_witness() + hplan_.c;
     Xyzz<fq_t> *h1 = planes1_host_.reuse(n1);
     NKR_HIP(hipMemcpyAsync(h1, planes1_.get(), n1 * sizeof(Xyzz<fq_t>), hipMemcpyDeviceToHost, s));
     planes1_host_.uploaded(s);
@@ -479,7 +502,7 @@ void Groth16Prover::run(const fr_t *z, void *raw_out, void *az, void *bz, void *
     host_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - host0).count();
     planes1_host_.wait();
     host0 = std::chrono::steady_clock::now();
-    finish_g1(h1, h1 + 3 * cw, blind, blind ? &pre : nullptr, raw_out, helpers_.get());
+    finish_g1(h1, h1 + planes_g1_witness(), blind, blind ? &pre : nullptr, raw_out, helpers_.get());
     host_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - host0).count();
 
     if (t) {
@@ -489,10 +512,12 @@ void Groth16Prover::run(const fr_t *z, void *raw_out, void *az, void *bz, void *
         stage_ms_[6] += host_ms;
         counters_[0] += 1;
         counters_[1] += 2;  // k_accumulate launches: G1 batch (witness and H), G2
-        uint32_t tw = 0, th = 0;
+        uint32_t tw = 0, tb = 0, th = 0;
         NKR_HIP(hipMemcpy(&tw, wsched_.totals(), sizeof(tw), hipMemcpyDeviceToHost));
+        NKR_HIP(hipMemcpy(&tb, bsched.totals(), sizeof(tb), hipMemcpyDeviceToHost));
         NKR_HIP(hipMemcpy(&th, hsched_.totals(), sizeof(th), hipMemcpyDeviceToHost));
         counters_[2] += tw;
+        b_entries_ += tb;
         counters_[3] += th;
     }
 }

@@ -13,10 +13,12 @@ uint64_t Server::request_bytes(const Groth16Prover &g)
     // offsets and chunk entry
     const uint64_t packed = (uint64_t)g.cols() * sizeof(fr_t) + ((uint64_t)g.cols() / 64 + 1) * 20 +
                             ((uint64_t)g.cols() / WitnessUpload::kChunk + 1) * sizeof(WitnessBatchUpload::Chunk) + 16;
-    const MsmPlan &w = g.witness_plan(), &h = g.h_plan();
-    const uint64_t planes = (3ull * w.c + h.c) * sizeof(Xyzz<fq_t>) + (uint64_t)w.c * sizeof(Xyzz<fq2_t>);
-    return polys + packed + planes + msm_schedule_bytes(w) + msm_schedule_bytes(h) + 3 * msm_job_bytes<fq_t>(w) +
-           msm_job_bytes<fq_t>(h) + msm_job_bytes<fq2_t>(w);
+    const MsmPlan &w = g.witness_plan(), &b = g.b_plan(), &h = g.h_plan();
+    const uint64_t planes =
+        (uint64_t)(g.planes_g1_witness() + h.c) * sizeof(Xyzz<fq_t>) + (uint64_t)b.c * sizeof(Xyzz<fq2_t>);
+    const uint64_t own_b = g.own_b_schedule() ? msm_schedule_bytes(b) : 0;
+    return polys + packed + planes + msm_schedule_bytes(w) + own_b + msm_schedule_bytes(h) +
+           2 * msm_job_bytes<fq_t>(w) + msm_job_bytes<fq_t>(b) + msm_job_bytes<fq_t>(h) + msm_job_bytes<fq2_t>(b);
 }
 
 Server::Server(int device, uint32_t workers, uint32_t max_batch, uint64_t work_budget_bytes)
