@@ -14,6 +14,8 @@
 // (FixedBaseMul); the pairing runs on the host.
 #include "keygen.h"
 
+#include "block_inverse.h"
+
 #include <cstring>
 #include <vector>
 
@@ -28,17 +30,19 @@ namespace nkr {
 
 namespace {
 
-// L_i(t) = Z(t)/N * w^i / (t - w^i), w a primitive N-th root of unity.
-__global__ void k_lagrange(fr_t *out, fr_t omega, fr_t t, fr_t zt_over_n, uint32_t n)
+// L_i(t) = Z(t)/N * w^i / (t - w^i), w a primitive N-th root of unity (an
+// inversion per workgroup).
+__global__ __launch_bounds__(256) void k_lagrange(fr_t *out, fr_t omega, fr_t t, fr_t zt_over_n, uint32_t n)
 {
+    __shared__ fr_t node[2 * 256];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
     fr_t w = fr_t::one(), sq = omega;
     for (uint32_t e = i; e; e >>= 1) {
         if (e & 1) w = fp_mul(w, sq);
         sq = fp_sqr(sq);
     }
-    out[i] = fp_mul(fp_mul(zt_over_n, w), fp_inv(fp_sub(t, w)));
+    const fr_t inv = block_inverse<256>(i < n ? fp_sub(t, w) : fr_t::one(), node);
+    if (i < n) out[i] = fp_mul(fp_mul(zt_over_n, w), inv);
 }
 
 __global__ void k_query_scalars(const fr_t *at, const fr_t *bt, const fr_t *ct, fr_t *l, fr_t *ic, uint32_t cols,
@@ -108,6 +112,14 @@ struct StreamGuard {
     ~StreamGuard()
     {
         if (s) (void)hipStreamDestroy(s);
+    }
+};
+
+struct EventGuard {
+    hipEvent_t e = nullptr;
+    ~EventGuard()
+    {
+        if (e) (void)hipEventDestroy(e);
     }
 };
 
@@ -193,44 +205,62 @@ void groth16_keygen(const nkr_g16_circuit &c, const Trapdoors &td, int device, c
     k_h_scalars<<<div_up(n, 256), 256, 0, s>>>(h.get(), td.t, fp_mul(zt, delta_inv), n);
     NKR_LAUNCH_CHECK();
 
-    // fixed-base multiples of the generators
-    const FixedBaseMul<fq_t> fb1(g1_generator(), s);
-    const FixedBaseMul<fq2_t> fb2(g2_generator(), s);
-    const uint64_t big = std::max<uint64_t>(cols, n);
-    DeviceBuffer<g1_jac> out1(big);
-    DeviceBuffer<g2_jac> out2(cols);
-    struct G1Query {
-        const fr_t *scalars;
-        uint64_t count;
-        void *dst;
-    };
-    const G1Query g1q[5] = {{at.get(), cols, pk.a_query},
-                            {bt.get(), cols, pk.b_g1_query},
-                            {l.get(), cols, pk.l_query},
-                            {h.get(), n, pk.h_query},
-                            {ic.get(), pub + 1ull, vk.ic}};
-    for (const G1Query &q : g1q) {
-        fb1.run(q.scalars, q.count, out1.get(), s);
-        NKR_HIP(hipMemcpyAsync(q.dst, out1.get(), q.count * sizeof(g1_jac), hipMemcpyDeviceToHost, s));
-        NKR_HIP(hipStreamSynchronize(s));  // out1 is reused by the next query
-    }
-    fb2.run(bt.get(), cols, out2.get(), s);
-    NKR_HIP(hipMemcpyAsync(pk.b_g2_query, out2.get(), cols * sizeof(g2_jac), hipMemcpyDeviceToHost, s));
-
-    // alpha, beta, delta in G1; beta, delta, gamma in G2
+    // fixed-base multiples of the generators: every G1 scalar (the queries, ic,
+    // and alpha, beta, delta) in one launch, every G2 scalar (the B query,
+    // beta, delta, gamma) in one beside it on a second stream, since each is
+    // bound by its chain of additions and inversion, not by their number
+    const uint64_t n1 = 3ull * cols + n + (pub + 1) + 3, n2 = cols + 3ull;
+    const uint64_t o_b = cols, o_l = 2ull * cols, o_h = 3ull * cols, o_ic = o_h + n, o_k1 = o_ic + pub + 1;
+    DeviceBuffer<fr_t> s1(n1), s2(n2);
+    DeviceBuffer<g1_jac> out1(n1);
+    DeviceBuffer<g2_jac> out2(n2);
     const fr_t k1[3] = {td.alpha, td.beta, td.delta}, k2[3] = {td.beta, td.delta, td.gamma};
-    DeviceBuffer<fr_t> kd(6);
-    NKR_HIP(hipMemcpyAsync(kd.get(), k1, sizeof(k1), hipMemcpyHostToDevice, s));
-    NKR_HIP(hipMemcpyAsync(kd.get() + 3, k2, sizeof(k2), hipMemcpyHostToDevice, s));
-    DeviceBuffer<g1_jac> p1(3);
-    DeviceBuffer<g2_jac> p2(3);
-    fb1.run(kd.get(), 3, p1.get(), s);
-    fb2.run(kd.get() + 3, 3, p2.get(), s);
+    auto gather = [&](fr_t *dst, const fr_t *src, uint64_t count) {
+        NKR_HIP(hipMemcpyAsync(dst, src, count * sizeof(fr_t), hipMemcpyDeviceToDevice, s));
+    };
+    gather(s2.get(), bt.get(), cols);
+    NKR_HIP(hipMemcpyAsync(s2.get() + cols, k2, sizeof(k2), hipMemcpyHostToDevice, s));
+    StreamGuard sg2;
+    NKR_HIP(hipStreamCreateWithFlags(&sg2.s, hipStreamNonBlocking));
+    hipStream_t side = sg2.s;
+    EventGuard ready;
+    NKR_HIP(hipEventCreateWithFlags(&ready.e, hipEventDisableTiming));
+    NKR_HIP(hipEventRecord(ready.e, s));
+    NKR_HIP(hipStreamWaitEvent(side, ready.e, 0));
+    const FixedBaseMul<fq2_t> fb2(g2_generator(), side);
+    fb2.run(s2.get(), n2, out2.get(), side);
+    gather(s1.get(), at.get(), cols);
+    gather(s1.get() + o_b, bt.get(), cols);
+    gather(s1.get() + o_l, l.get(), cols);
+    gather(s1.get() + o_h, h.get(), n);
+    gather(s1.get() + o_ic, ic.get(), pub + 1ull);
+    NKR_HIP(hipMemcpyAsync(s1.get() + o_k1, k1, sizeof(k1), hipMemcpyHostToDevice, s));
+    const FixedBaseMul<fq_t> fb1(g1_generator(), s);
+    fb1.run(s1.get(), n1, out1.get(), s);
+
+    // the host pairs alpha and beta while the GPU works on the queries
+    const fq12_t ab = bn254_pairing(xyzz_to_jacobian_affine(fb1.mul_host(td.alpha)),
+                                    xyzz_to_jacobian_affine(fb2.mul_host(td.beta)));
+    std::memcpy(vk.alpha_g1_beta_g2, &ab, sizeof(ab));
+
+    // alpha, beta, delta in G1; beta, delta, gamma in G2; then the queries
     g1_jac h1[3];
     g2_jac h2[3];
-    NKR_HIP(hipMemcpyAsync(h1, p1.get(), sizeof(h1), hipMemcpyDeviceToHost, s));
-    NKR_HIP(hipMemcpyAsync(h2, p2.get(), sizeof(h2), hipMemcpyDeviceToHost, s));
+    const struct {
+        void *dst;
+        uint64_t at, count;
+    } g1q[5] = {{pk.a_query, 0, cols},
+                {pk.b_g1_query, o_b, cols},
+                {pk.l_query, o_l, cols},
+                {pk.h_query, o_h, n},
+                {vk.ic, o_ic, pub + 1ull}};
+    NKR_HIP(hipMemcpyAsync(h1, out1.get() + o_k1, sizeof(h1), hipMemcpyDeviceToHost, s));
+    for (const auto &q : g1q)
+        NKR_HIP(hipMemcpyAsync(q.dst, out1.get() + q.at, q.count * sizeof(g1_jac), hipMemcpyDeviceToHost, s));
+    NKR_HIP(hipMemcpyAsync(h2, out2.get() + cols, sizeof(h2), hipMemcpyDeviceToHost, side));
+    NKR_HIP(hipMemcpyAsync(pk.b_g2_query, out2.get(), cols * sizeof(g2_jac), hipMemcpyDeviceToHost, side));
     NKR_HIP(hipStreamSynchronize(s));
+    NKR_HIP(hipStreamSynchronize(side));
     std::memcpy(pk.alpha_g1, &h1[0], sizeof(g1_jac));
     std::memcpy(pk.beta_g1, &h1[1], sizeof(g1_jac));
     std::memcpy(pk.delta_g1, &h1[2], sizeof(g1_jac));
@@ -238,8 +268,6 @@ void groth16_keygen(const nkr_g16_circuit &c, const Trapdoors &td, int device, c
     std::memcpy(pk.delta_g2, &h2[1], sizeof(g2_jac));
     std::memcpy(vk.delta_g2, &h2[1], sizeof(g2_jac));
     std::memcpy(vk.gamma_g2, &h2[2], sizeof(g2_jac));
-    const fq12_t ab = bn254_pairing(h1[0], h2[0]);
-    std::memcpy(vk.alpha_g1_beta_g2, &ab, sizeof(ab));
 }
 
 }  // namespace nkr

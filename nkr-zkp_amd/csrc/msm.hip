@@ -1,6 +1,7 @@
 // Pippenger MSM kernels for gfx950 (see msm.h for the design).
 #include "msm.h"
 
+#include "block_inverse.h"
 #include "coop29.h"
 #include "curve29.h"
 
@@ -904,26 +905,23 @@ __global__ __launch_bounds__(256) void k_finite(const g1_jac *__restrict__ a, co
 }
 
 // Base preparation: normalise the reference-layout Jacobian point and store
-// 2^(c*w) * P for every window w (affine, infinity flagged).
+// 2^(c*w) * P for every window w (affine, infinity flagged).  Each window's
+// points share one inversion per workgroup (an inversion of its own cost every
+// point more than twice its c doublings).
+constexpr uint32_t kPrepareThreads = 128;
 template <class F>
-__global__ __launch_bounds__(128) void k_prepare_bases(const Jacobian<F> *__restrict__ in,
-                                                       const uint32_t *__restrict__ perm, uint32_t n, uint32_t c,
-                                                       uint32_t W, Affine<F> *__restrict__ out)
+__global__ __launch_bounds__(kPrepareThreads) void k_prepare_bases(const Jacobian<F> *__restrict__ in,
+                                                                  const uint32_t *__restrict__ perm, uint32_t n,
+                                                                  uint32_t c, uint32_t W, Affine<F> *__restrict__ out)
 {
+    __shared__ fq_t node[2 * kPrepareThreads];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const Jacobian<F> J = in[perm ? perm[i] : i];
-    Affine<F> a;
-    if (!jacobian_to_affine(J, a)) {
-        const Affine<F> inf = affine_infinity<F>();
-        for (uint32_t w = 0; w < W; ++w) out[(size_t)w * n + i] = inf;
-        return;
-    }
-    out[i] = a;
-    Xyzz<F> P = Xyzz<F>::from_affine(a);
-    for (uint32_t w = 1; w < W; ++w) {
-        for (uint32_t t = 0; t < c; ++t) P = xyzz_dbl(P);
-        out[(size_t)w * n + i] = xyzz_to_affine(P);
+    Xyzz<F> P = i < n ? jacobian_to_xyzz(in[perm ? perm[i] : i]) : Xyzz<F>::infinity();
+    for (uint32_t w = 0; w < W; ++w) {
+        if (w)
+            for (uint32_t t = 0; t < c; ++t) P = xyzz_dbl(P);
+        const Affine<F> a = block_to_affine<kPrepareThreads>(P, node);
+        if (i < n) out[(size_t)w * n + i] = a;
     }
 }
 
@@ -1019,8 +1017,8 @@ void MsmBases<F>::prepare(const Jacobian<F> *jacobian, const uint32_t *perm, con
 {
     plan_ = plan;
     pts_.allocate((size_t)plan.W * plan.n);
-    k_prepare_bases<F><<<div_up(plan.n, 128), 128, 0, stream>>>(jacobian, perm, plan.n, plan.c, plan.W,
-                                                                  pts_.get());
+    k_prepare_bases<F><<<div_up(plan.n, kPrepareThreads), kPrepareThreads, 0, stream>>>(jacobian, perm, plan.n, plan.c,
+                                                                                     plan.W, pts_.get());
     NKR_LAUNCH_CHECK();
 }
 
