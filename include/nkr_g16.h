@@ -311,9 +311,8 @@ int nkr_fr_ntt_dev(void *data_dev, uint32_t log_n, int kind, void *stream);    /
 
 /* As nkr_fr_ntt_dev, allocating no device memory: for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  No counterpart in the reference.  The tables and the
- * reordering buffer live in one fixed device array per GPU (64.2 MiB, held
- * until the process ends), so log_n is limited to 1 .. 20; larger sizes fail
+ * forbid hipMalloc).  No counterpart in the reference.  The tables live in
+ * one fixed device array per GPU (32.2 MiB, held until the process ends), so log_n is limited to 1 .. 20; larger sizes fail
  * with an error.  The tables are rebuilt on `stream` by every call.  Every
  * call on one GPU shares that array: calls that overlap on one GPU (other
  * streams, other threads) race and must be serialised by the caller.

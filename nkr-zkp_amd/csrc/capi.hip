@@ -27,19 +27,16 @@ thread_local std::string g_last_error;
 constexpr int kMaxDevices = 16;
 std::mutex g_ntt_mutex;
 nkr::NttDomain *g_ntt_cache[kMaxDevices][29] = {};
-nkr::DeviceBuffer<nkr::fr_t> *g_ntt_scratch[kMaxDevices] = {};
 
 // Device scratch of the allocation-free transform (nkr_fr_ntt_dev_noalloc):
-// the table arena of a 2^20-point domain followed by a 2^20-element buffer
-// for the final reordering -- 2^21 + 6144 elements of 32 B (64.2 MiB), one
-// copy per device for the life of the process.  Host code never names
+// the table arena of a 2^20-point domain -- 2^20 + 6144 elements of 32 B
+// (32.2 MiB), one copy per device for the life of the process.  Host code never names
 // `scratch` in a kernel argument or copy: in host code the name is a stand-in,
 // not a device address.  Each device's address comes from
 // hipGetSymbolAddress (noalloc_scratch) with that device current.
 constexpr uint32_t kNoAllocMaxLog = 20;
 constexpr size_t kNoAllocArenaElems = nkr::NttDomain::standalone_arena_elems(kNoAllocMaxLog);
-constexpr size_t kNoAllocElems = kNoAllocArenaElems + (size_t(1) << kNoAllocMaxLog);
-static __device__ __align__(256) uint4 scratch[kNoAllocElems * sizeof(nkr::fr_t) / sizeof(uint4)];
+static __device__ __align__(256) uint4 scratch[kNoAllocArenaElems * sizeof(nkr::fr_t) / sizeof(uint4)];
 std::mutex g_noalloc_mutex;
 nkr::fr_t *g_noalloc_ptr[kMaxDevices] = {};
 
@@ -554,9 +551,9 @@ int nkr_fr_ntt(void *data, uint32_t log_n, int kind, int device)
         set_device(device);
         NttDomain dom(log_n, nullptr);
         const size_t n = size_t(1) << log_n;
-        DeviceBuffer<fr_t> d(n), scratch(n);
+        DeviceBuffer<fr_t> d(n);
         NKR_HIP(hipMemcpy(d.get(), data, n * sizeof(fr_t), hipMemcpyHostToDevice));
-        dom.standalone(d.get(), scratch.get(), kind, nullptr);
+        dom.standalone(d.get(), kind, nullptr);
         NKR_HIP(hipMemcpy(data, d.get(), n * sizeof(fr_t), hipMemcpyDeviceToHost));
     });
 }
@@ -576,10 +573,7 @@ int nkr_fr_ntt_dev(void *data_dev, uint32_t log_n, int kind, void *stream)
         std::lock_guard<std::mutex> lock(g_ntt_mutex);
         NttDomain *&dom = g_ntt_cache[dev][log_n];
         if (!dom) dom = new NttDomain(log_n, s);
-        DeviceBuffer<fr_t> *&scratch = g_ntt_scratch[dev];
-        if (!scratch) scratch = new DeviceBuffer<fr_t>();
-        scratch->ensure(size_t(1) << log_n);
-        dom->standalone(static_cast<fr_t *>(data_dev), scratch->get(), kind, s);
+        dom->standalone(static_cast<fr_t *>(data_dev), kind, s);
     });
 }
 
@@ -614,7 +608,7 @@ int nkr_fr_ntt_dev_noalloc(void *data_dev, uint32_t log_n, int kind, void *strea
         // Tables are rebuilt on the stream by every call (they are exact, so
         // the results equal nkr_fr_ntt_dev's); nothing needs clearing.
         const NttDomain dom(log_n, kind, arena, s);
-        dom.standalone(static_cast<fr_t *>(data_dev), arena + kNoAllocArenaElems, kind, s);
+        dom.standalone(static_cast<fr_t *>(data_dev), kind, s);
     });
 }
 

@@ -370,15 +370,15 @@ NKR_HD Fp<P> fp29_to_bits(const Fp29<P> &x)
 // 2^29 K p where the textbook one adds 2^29 p, so the eight lower limbs are
 // cleared this way and the top one by the textbook step:
 //   result < sum / 2^261 + (1 + K / 2^29) p.
-// Fq's K is 0x04866389 (0.15 p); Fr's would be 0.5 p, which its lazily
-// reduced transforms have no room for, so Fr keeps the textbook step
-// throughout (result < sum / 2^261 + p).  Fq products in chains on MI355X:
+// Fq's K is 0x04866389 (0.15 p).  Fr's is 0.5 p, which canonical products have
+// no room for, so they keep the textbook step throughout (low = 0, result <
+// sum / 2^261 + p); the transforms, whose values may be larger, take the
+// direct steps.  Fq products in chains on MI355X:
 // 362 against 378 ns per wave and SIMD.
-template <class P, class Terms>
+template <class P, int low = P29<P>::direct_steps(), class Terms>
 NKR_HD Fp29<P> fp29_reduce_terms(const Terms &terms)
 {
     constexpr uint32_t INV = P29<P>::inv();
-    constexpr int low = P29<P>::direct_steps();  // limbs cleared without a multiply
     constexpr typename P29<P>::Limbs direct = P29<P>::direct();
     uint32_t m[9];
     Fp29<P> r;

@@ -19,7 +19,11 @@ __global__ __launch_bounds__(128) void k_hq_scale(const Jacobian<fq_t> *__restri
 {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= (1u << log_n)) return;
-    const fr_t c = fp_from_mont(icoset_rev[rev_bits(k, log_n)]);
+    // the table holds c * 2^261
+    fr_t one = fr_t::zero();
+    one.l[0] = 1;
+    const fr_t c = fp_reduce_once(
+        fp29_to_bits(fp29_mul(fp29_from_bits(icoset_rev[rev_bits(k, log_n)]), fp29_from_bits(one))));
     P[k] = xyzz_mul_u256(jacobian_to_xyzz(in[k]), c.l);
 }
 

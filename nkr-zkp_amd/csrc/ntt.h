@@ -2,7 +2,7 @@
 //
 // A transform of N = 2^n points runs as 1-4 passes.  Each pass performs
 // 2^np-point sub-transforms entirely in LDS (one workgroup holds up to 2048
-// elements = 64 KiB) and multiplies by the inter-pass twiddles omega^(lo*k*2^S)
+// elements = 72 KiB) and multiplies by the inter-pass twiddles omega^(lo*k*2^S)
 // (the four-step factorisation).  A domain that owns its tables holds them
 // whole, one element per position of each twiddled pass (read like the data,
 // one product per element); an arena domain, whose memory is bounded, makes
@@ -13,8 +13,9 @@
 // dit(): bit-reversed order in, natural order out; it is the transpose of
 //        dif() and uses the same twiddles.
 // The Groth16 quotient chain composes the two so that no bit-reversal pass is
-// ever needed; the standalone transforms add one gather pass to return
-// natural order like libfqfft's basic_radix2_domain.
+// ever needed; the standalone transforms reorder in place (in the pass itself
+// when there is only one) to return natural order like libfqfft's
+// basic_radix2_domain.
 #pragma once
 
 #include <vector>
@@ -53,8 +54,9 @@ public:
     size_t size() const { return size_t(1) << log_n_; }
 
     // In-place transforms on device data.  `pre` / `post` are optional
-    // per-position multipliers (indexed by storage position), `post_const` an
-    // optional constant factor applied last.
+    // per-position multipliers (indexed by storage position, in the tables'
+    // 2^261 form), `post_const` an optional constant factor applied last (in
+    // Montgomery form).
     void dif(fr_t *data, bool inverse, const fr_t *pre, const fr_t *post, const fr_t *post_const,
              hipStream_t stream) const;
     void dit(fr_t *data, bool inverse, const fr_t *pre, const fr_t *post, hipStream_t stream) const;
@@ -72,15 +74,16 @@ public:
     // out[i] = in[bitrev(i)] (out of place).
     void bitrev(const fr_t *in, fr_t *out, hipStream_t stream) const;
 
-    // libfqfft semantics, natural order in and out (kind: 0 FFT, 1 iFFT,
-    // 2 cosetFFT, 3 icosetFFT), using `scratch` (n elements) for the final
-    // reordering.
-    void standalone(fr_t *data, fr_t *scratch, int kind, hipStream_t stream) const;
+    // libfqfft semantics, natural order in and out, in place (kind: 0 FFT,
+    // 1 iFFT, 2 cosetFFT, 3 icosetFFT).
+    void standalone(fr_t *data, int kind, hipStream_t stream) const;
 
     // h[i] = (a[i]*b[i] - c[i]) / (g^N - 1) on the coset (divide_by_Z_on_coset).
     void quotient(const fr_t *a, const fr_t *b, const fr_t *c, fr_t *h, hipStream_t stream) const;
 
-    // Tables the prove chain fuses into its passes.
+    // Tables the prove chain fuses into its passes: factors x in the form
+    // x * 2^261 mod r (canonical), as every table of the domain; x * 2^256
+    // times one of them by a product of R = 2^261 is in the data's form.
     const fr_t *coset_rev_scaled() const { return coset_rev_p_; }      // g^rev(j) / N
     const fr_t *icoset_rev_scaled() const { return icoset_rev_p_; }    // g^-rev(j) / N
 
@@ -91,7 +94,7 @@ private:
         unsigned S, np, log_L, log_cols;
     };
     void run(fr_t *data, fr_t *const *batch, uint32_t count, bool dit, bool inverse, const fr_t *pre,
-             const fr_t *post, const fr_t *post_const, hipStream_t stream) const;
+             const fr_t *post, const fr_t *post_const, hipStream_t stream, bool natural_out = false) const;
     // Pass split, constants and table sizes (both constructors).
     void plan(unsigned log_n, const NttShape *shape);
 

@@ -6,6 +6,8 @@
 // 1/N scaling, so outputs equal the reference's element for element.
 #include "ntt.h"
 
+#include "field29.h"
+
 namespace nkr {
 
 namespace {
@@ -38,6 +40,7 @@ struct PassArgs {
     uint32_t has_post_const;
     uint32_t log_n, S, np, log_L, log_cols, log_roots, m_lo;
     uint32_t twiddle;
+    uint32_t natural_out;  // single-pass DIF: element j is stored at bitrev(j)
 };
 
 __device__ __forceinline__ uint32_t brev_bits(uint32_t x, uint32_t bits)
@@ -45,104 +48,132 @@ __device__ __forceinline__ uint32_t brev_bits(uint32_t x, uint32_t bits)
     return bits == 0 ? 0u : (__brev(x) >> (32 - bits));
 }
 
+// Inside a pass every value stays in the 29-bit form (field.h) and is lazily
+// reduced: the canonical residue x 2^256 of the data is taken as it is, and
+// the factors (twiddles, roots, coset powers) are stored as w 2^261, so that a
+// reduced-radix product of the two is (x w) 2^256 with no conversion on either
+// side.  Sums and differences are added limb by limb without carries; a value
+// is carry-normalised when it goes back to LDS.  A pass is bound by the
+// products' multiply-adds, half a product per element and stage.  (On 32-bit
+// limbs each butterfly converted both operands and the product, and each sum
+// and difference was a carry chain and a conditional subtraction: a whole
+// transform of 2^21 took 349 us against 294 now with its reordering, the
+// passes alone 279 against 261, one of 2^11 34.5 against 29.2.)
+using fr29 = Fp29<FrParams>;
+
+// a * b * 2^-261, limbs below 2^29, value below 1.5 r + a b / 2^261.  One
+// operand may have limbs up to 2.5 * 2^30 (a column is at most 9 * 2.5 * 2^59
+// + 9 * 2^58 and a carry, below 2^64); b is a canonical factor.
+__device__ __forceinline__ fr29 mul29(const fr29 &a, const fr29 &b)
+{
+    return fp29_reduce_terms<FrParams, 8>([&](int k, uint64_t &acc) { fp29_column(a, b, k, acc); });
+}
+__device__ __forceinline__ fr29 load29(const fr_t &x) { return fp29_from_bits(x); }
+
+// Limbs below 2^29 (the top one takes what is left), value unchanged.
+__device__ __forceinline__ fr29 normalise29(const fr29 &x)
+{
+    fr29 r;
+    uint32_t c = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t t = x.l[i] + c;
+        r.l[i] = t & kMask29;
+        c = t >> 29;
+    }
+    r.l[8] = x.l[8] + c;
+    return r;
+}
+
+__device__ __forceinline__ fr29 add29(const fr29 &x, const fr29 &y)
+{
+    fr29 r;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) r.l[i] = x.l[i] + y.l[i];
+    return r;
+}
+
+// K r with 2^30 borrowed into every limb from the next, so that limbs up to
+// 2^30 - 2 can be taken from it without a borrow.
+struct Borrowed {
+    uint32_t l[9];
+};
+constexpr Borrowed borrowed(uint32_t K)
+{
+    Borrowed b{};
+    const auto kp = P29<FrParams>::times(K);
+    for (int i = 0; i < 9; ++i) b.l[i] = kp.l[i] + (i < 8 ? (1u << 30) : 0u) - (i > 0 ? 2u : 0u);
+    return b;
+}
+
+// x + K r - y for y below (K - 0.01) r with limbs up to 2^30 - 2; the result's
+// limbs are below x's + 1.5 * 2^30.
+__device__ __forceinline__ fr29 sub29(const fr29 &x, const fr29 &y, const Borrowed &k)
+{
+    fr29 r;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) r.l[i] = x.l[i] + k.l[i] - y.l[i];
+    return r;
+}
+
+// x below 169 r, normalised -> below 1.04 r: the quotient's estimate from the
+// top limb is at most 1 too small and never too large.
+__device__ __forceinline__ fr29 reduce29(const fr29 &x)
+{
+    constexpr uint32_t top = P29<FrParams>::bits(8) + 1;
+    constexpr uint32_t recip = (uint32_t)((1ull << 32) / top);
+    const uint32_t q = (uint32_t)(((uint64_t)x.l[8] * recip) >> 32);
+    fr29 r;
+    int64_t c = 0;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        const int64_t t = (int64_t)x.l[i] - (int64_t)((uint64_t)q * P29<FrParams>::bits(i)) + c;
+        r.l[i] = (uint32_t)t & kMask29;
+        c = t >> 29;
+    }
+    return r;
+}
+
+// The canonical residue of x (below 169 r, normalised).
+__device__ __forceinline__ fr_t canonical29(const fr29 &x) { return fp_reduce_once(fp29_to_bits(reduce29(x))); }
+
+// Product of two factors in the 2^261 form, canonical in that form.
+__device__ __forceinline__ fr_t factor_mul(const fr_t &a, const fr_t &b)
+{
+    return canonical29(mul29(load29(a), load29(b)));
+}
+// x 2^256 -> x 2^261.
+NKR_HD fr_t factor_from_mont(const fr_t &x) { return fp_dbl(fp_dbl(fp_dbl(fp_dbl(fp_dbl(x))))); }
+
 // omega^e from the two-level table.
-__device__ __forceinline__ fr_t tw_pow(const PassArgs &a, uint32_t e)
+__device__ __forceinline__ fr29 tw_pow(const PassArgs &a, uint32_t e)
 {
     const uint32_t lo = e & ((1u << a.m_lo) - 1u);
     const uint32_t hi = e >> a.m_lo;
-    return fp_mul(a.tw_hi[hi], a.tw_lo[lo]);
+    return load29(factor_mul(a.tw_hi[hi], a.tw_lo[lo]));
 }
 
 // The inter-pass twiddle of element j of the sub-transform at column lo:
 // omega^e, e = (lo * bitrev(j)) << S, from the whole table when the domain has
 // one.
-__device__ __forceinline__ fr_t tw_at(const PassArgs &a, uint32_t j, uint32_t lo, uint32_t e)
+__device__ __forceinline__ fr29 tw_at(const PassArgs &a, uint32_t j, uint32_t lo, uint32_t e)
 {
-    return a.tw_full ? a.tw_full[((uint64_t)j << a.log_L) + lo] : tw_pow(a, e);
+    return a.tw_full ? load29(a.tw_full[((uint64_t)j << a.log_L) + lo]) : tw_pow(a, e);
 }
 
-// 2r as eight 32-bit words (r < 2^254, so 2r < 2^255).
-constexpr Fp<FrParams> twice_modulus()
-{
-    Fp<FrParams> t{};
-    uint64_t c = 0;
-    for (int i = 0; i < 8; ++i) {
-        const uint64_t v = 2ull * FrParams::P[i] + c;
-        t.l[i] = (uint32_t)v;
-        c = v >> 32;
-    }
-    return t;
-}
-
-// Lazy reduction: inside a lazily reduced pass every value is kept below 2r
-// (r < 2^254, so 4r < 2^256 and sums of two such values fit the eight words);
-// products skip their final subtraction (below 2r again when the other factor
-// is a canonical twiddle), and the pass stores canonical values.
-
-// x - 2r if x >= 2r, for x < 4r.
-__device__ __forceinline__ fr_t sub_twice_r_if(const fr_t &x)
-{
-    constexpr Fp<FrParams> two_r = twice_modulus();
-    fr_t d;
-    uint32_t borrow = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) d.l[i] = subc32(x.l[i], two_r.l[i], borrow, borrow);
-    fr_t r;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) r.l[i] = borrow ? x.l[i] : d.l[i];
-    return r;
-}
-
-// x + y for x, y < 2r, reduced below 2r.
-__device__ __forceinline__ fr_t add_lazy(const fr_t &x, const fr_t &y)
-{
-    fr_t s;
-    uint32_t carry = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) s.l[i] = addc32(x.l[i], y.l[i], carry, carry);
-    return sub_twice_r_if(s);
-}
-
-// x - y + 2r for x, y < 2r: in (0, 4r), not reduced.
-__device__ __forceinline__ fr_t sub_lazy(const fr_t &x, const fr_t &y)
-{
-    constexpr Fp<FrParams> two_r = twice_modulus();
-    fr_t s;
-    uint32_t carry = 0, borrow = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) s.l[i] = addc32(x.l[i], two_r.l[i], carry, carry);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) s.l[i] = subc32(s.l[i], y.l[i], borrow, borrow);
-    return s;
-}
-
-// Decimation-in-frequency passes run lazily (their butterfly's difference
-// goes straight into the product); decimation-in-time passes stay canonical,
-// since their lazy butterfly needs a second conditional subtraction that
-// costs what the product saves (measured on MI355X).
-template <bool DIT>
-constexpr bool kLazyNtt = !DIT;
-
-// x * w * 2^-256 for x < 4r and a canonical w: below r + x*w/2^256 < 2r
-// (the 29-bit product without its final subtraction).
-__device__ __forceinline__ fr_t mul_lazy(const fr_t &x, const fr_t &w)
-{
-    return fp_mul_r29(x, w);
-}
-
-// LDS tile of n field elements: two planes of 16-byte halves (element i's
-// low half in plane 0, high half in plane 1) so that every access is one
-// 16-byte LDS instruction per half, and within each aligned run of 64
-// elements the 16-element rows are XOR-permuted (row r by 5 * (r mod 4)),
-// which spreads the strided accesses of every radix-4 round over distinct
-// bank groups.
+// LDS tile of n field elements in the 29-bit form: two planes of 16 bytes
+// (limbs 0 .. 3 and 4 .. 7) and one of 4 (limb 8), so that every access is
+// whole LDS instructions, and within each aligned run of 64 elements the
+// 16-element rows are XOR-permuted (row r by 5 * (r mod 4)), which spreads the
+// strided accesses of every radix-4 round over distinct bank groups.
+constexpr uint32_t kTileBytes = 36;  // per element
 __device__ __forceinline__ uint32_t lds_slot(uint32_t i) { return i ^ (5u * ((i >> 4) & 3u)); }
 
-__device__ __forceinline__ fr_t lds_get(const uint4 *tile, uint32_t n, uint32_t i)
+__device__ __forceinline__ fr29 lds_get(const uint4 *tile, uint32_t n, uint32_t i)
 {
     const uint32_t k = lds_slot(i);
     const uint4 a = tile[k], b = tile[n + k];
-    fr_t r;
+    fr29 r;
     r.l[0] = a.x;
     r.l[1] = a.y;
     r.l[2] = a.z;
@@ -151,14 +182,16 @@ __device__ __forceinline__ fr_t lds_get(const uint4 *tile, uint32_t n, uint32_t 
     r.l[5] = b.y;
     r.l[6] = b.z;
     r.l[7] = b.w;
+    r.l[8] = reinterpret_cast<const uint32_t *>(tile + 2 * n)[k];
     return r;
 }
 
-__device__ __forceinline__ void lds_put(uint4 *tile, uint32_t n, uint32_t i, const fr_t &v)
+__device__ __forceinline__ void lds_put(uint4 *tile, uint32_t n, uint32_t i, const fr29 &v)
 {
     const uint32_t k = lds_slot(i);
     tile[k] = make_uint4(v.l[0], v.l[1], v.l[2], v.l[3]);
     tile[n + k] = make_uint4(v.l[4], v.l[5], v.l[6], v.l[7]);
+    reinterpret_cast<uint32_t *>(tile + 2 * n)[k] = v.l[8];
 }
 
 // One round of R consecutive radix-2 stages (t .. t+R-1) on groups of 2^R
@@ -166,11 +199,25 @@ __device__ __forceinline__ void lds_put(uint4 *tile, uint32_t n, uint32_t i, con
 // bits [np-t-R, np-t) that the round's butterflies pair.  The twiddle of the
 // pair (u, u + 2^(R-1-k)) at stage s = t + k is root^((j mod 2^(np-1-s)) * 2^s)
 // for its lower index j, as in the radix-2 DIF recursion.
+//
+// Bounds, in r.  A product comes out below 2.45 as long as its other operand
+// is below 160.  DIF: x[0], which no product touches, is the sum of the whole
+// group; the others are sums of at most 2^(R-1) products.  R <= 2: elements
+// below 2.45 grow to 9.8, 39.2 and 156.8 in three rounds, then x[0] is reduced;
+// from there the largest are sums of two products, 4.9, and grow to 19.6 and
+// 78.4 in two rounds, so x[0] is reduced after rounds 2, 4, 6...  A round that
+// starts below 39.2 takes 40 r for its first stage's differences and 80 r for
+// the second's, which are then below 79.2 and 158.4.  R = 3: x[0] is reduced
+// in every round, elements are below 9.8, sums below 78.4, differences below
+// 119.  DIT: a stage adds at most 4, so 11 stages end below 47 unreduced.
+// Limbs: two stages of sums and differences stay below 3.5 * 2^30, so the
+// third of R = 3 starts from normalised values.
 template <bool DIT, int R, bool LOW0>
 __device__ __forceinline__ void ntt_round(uint4 *smem, uint32_t n, const PassArgs &a, uint32_t t, uint32_t cols,
-                                          uint32_t root_shift)
+                                          uint32_t root_shift, bool reduce)
 {
     constexpr uint32_t G = 1u << R;
+    constexpr Borrowed kBorrow[3] = {borrowed(DIT ? 4 : 40), borrowed(DIT ? 4 : 80), borrowed(DIT ? 4 : 80)};
     const uint32_t low = LOW0 ? 0u : a.np - t - R;
     const uint32_t groups = (1u << (a.np - R)) << a.log_cols;
     for (uint32_t gi = threadIdx.x; gi < groups; gi += blockDim.x) {
@@ -178,7 +225,7 @@ __device__ __forceinline__ void ntt_round(uint4 *smem, uint32_t n, const PassArg
         const uint32_t q = gi >> a.log_cols;
         const uint32_t lo_part = q & ((1u << low) - 1u);
         const uint32_t j0 = ((q >> low) << (a.np - t)) | lo_part;
-        fr_t x[G];
+        fr29 x[G];
 #pragma unroll
         for (uint32_t u = 0; u < G; ++u) x[u] = lds_get(smem, n, (j0 + (u << low)) * cols + c);
 #pragma unroll
@@ -186,46 +233,43 @@ __device__ __forceinline__ void ntt_round(uint4 *smem, uint32_t n, const PassArg
             const int k = DIT ? (R - 1 - kk) : kk;
             const uint32_t s = t + (uint32_t)k;
             const uint32_t hs = 1u << (R - 1 - k);
+            if (kk == 2) {
+#pragma unroll
+                for (uint32_t u = 0; u < G; ++u) x[u] = normalise29(x[u]);
+            }
 #pragma unroll
             for (uint32_t u = 0; u < G; ++u) {
                 if (u & hs) continue;
                 const uint32_t e = (lo_part + ((u & (hs - 1u)) << low)) << s;
-                const fr_t w = a.roots[e << root_shift];
-                const fr_t X = x[u], Y = x[u + hs];
                 // twiddle 1 needs no product.  In the round whose pairs are
                 // adjacent (low = 0, so lo_part = 0) e depends on u alone and
                 // the test folds away; other rounds multiply every pair.
                 const bool one = LOW0 && (u & (hs - 1u)) == 0;
+                const fr29 X = x[u];
+                fr29 Y = x[u + hs];
                 if (!DIT) {
-                    if (kLazyNtt<DIT>) {
-                        x[u] = add_lazy(X, Y);
-                        const fr_t D = sub_lazy(X, Y);
-                        x[u + hs] = one ? sub_twice_r_if(D) : mul_lazy(D, w);
-                    } else {
-                        x[u] = fp_add(X, Y);
-                        const fr_t D = fp_sub(X, Y);
-                        x[u + hs] = one ? D : fp_mul(D, w);
-                    }
+                    const fr29 D = sub29(X, Y, kBorrow[kk]);
+                    x[u] = add29(X, Y);
+                    x[u + hs] = one ? reduce29(normalise29(D)) : mul29(D, load29(a.roots[e << root_shift]));
                 } else {
-                    if (kLazyNtt<DIT>) {
-                        const fr_t wy = one ? Y : mul_lazy(Y, w);
-                        x[u] = add_lazy(X, wy);
-                        x[u + hs] = sub_twice_r_if(sub_lazy(X, wy));
-                    } else {
-                        const fr_t wy = one ? Y : fp_mul(Y, w);
-                        x[u] = fp_add(X, wy);
-                        x[u + hs] = fp_sub(X, wy);
-                    }
+                    Y = one ? reduce29(normalise29(Y)) : mul29(Y, load29(a.roots[e << root_shift]));
+                    x[u] = add29(X, Y);
+                    x[u + hs] = sub29(X, Y, kBorrow[kk]);
                 }
             }
         }
 #pragma unroll
-        for (uint32_t u = 0; u < G; ++u) lds_put(smem, n, (j0 + (u << low)) * cols + c, x[u]);
+        for (uint32_t u = 0; u < G; ++u) {
+            // DIF: odd elements are products (or reduced), normalised already
+            if (DIT || (u & 1u) == 0) x[u] = normalise29(x[u]);
+            if (!DIT && u == 0 && reduce) x[u] = reduce29(x[u]);
+            lds_put(smem, n, (j0 + (u << low)) * cols + c, x[u]);
+        }
     }
 }
 
 // Radix-4 passes are held to 128 registers, four waves per SIMD: as many as
-// the LDS tiles allow (two 64 KiB tiles per CU), at the price of a few spills.
+// the LDS tiles allow (two 72 KiB tiles per CU).
 template <bool DIT, int RMAX>
 __global__ __launch_bounds__(kMaxThreads, RMAX == 2 ? 4 : 1) void k_ntt_pass(PassArgs a)
 {
@@ -251,11 +295,11 @@ __global__ __launch_bounds__(kMaxThreads, RMAX == 2 ? 4 : 1) void k_ntt_pass(Pas
         const uint64_t hi = g >> a.log_L;
         const uint32_t lo = (uint32_t)(g & (L - 1));
         const uint64_t pos = (hi << (a.log_n - a.S)) + ((uint64_t)j << a.log_L) + lo;
-        fr_t v = a.data[pos];
-        if (a.pre) v = kLazyNtt<DIT> ? mul_lazy(v, a.pre[pos]) : fp_mul(v, a.pre[pos]);
+        fr29 v = load29(a.data[pos]);
+        if (a.pre) v = mul29(v, load29(a.pre[pos]));
         if (DIT && a.twiddle) {
             const uint32_t e = (lo * brev_bits(j, a.np)) << a.S;
-            if (e) v = kLazyNtt<DIT> ? mul_lazy(v, tw_at(a, j, lo, e)) : fp_mul(v, tw_at(a, j, lo, e));
+            if (e) v = mul29(v, tw_at(a, j, lo, e));
         }
         lds_put(smem, total, j * cols + c, v);
     }
@@ -266,25 +310,27 @@ __global__ __launch_bounds__(kMaxThreads, RMAX == 2 ? 4 : 1) void k_ntt_pass(Pas
     // visited once per RMAX stages.  DIF rounds run stages t..t+r-1, DIT
     // rounds the same stages in reverse (its transpose).
     const uint32_t root_shift = a.log_roots - a.np;
-    for (uint32_t done = 0; done < a.np;) {
+    uint32_t round = 0;
+    for (uint32_t done = 0; done < a.np; ++round) {
         const uint32_t r = min((uint32_t)RMAX, a.np - done);
         const uint32_t t = DIT ? (a.np - done - r) : done;
         const bool low0 = (a.np - t - r == 0);
+        const bool reduce = RMAX == 3 || (round >= 2 && round % 2 == 0);
         if (r == 3) {
             if (low0)
-                ntt_round<DIT, 3, true>(smem, total, a, t, cols, root_shift);
+                ntt_round<DIT, 3, true>(smem, total, a, t, cols, root_shift, reduce);
             else
-                ntt_round<DIT, 3, false>(smem, total, a, t, cols, root_shift);
+                ntt_round<DIT, 3, false>(smem, total, a, t, cols, root_shift, reduce);
         } else if (r == 2) {
             if (low0)
-                ntt_round<DIT, 2, true>(smem, total, a, t, cols, root_shift);
+                ntt_round<DIT, 2, true>(smem, total, a, t, cols, root_shift, reduce);
             else
-                ntt_round<DIT, 2, false>(smem, total, a, t, cols, root_shift);
+                ntt_round<DIT, 2, false>(smem, total, a, t, cols, root_shift, reduce);
         } else {
             if (low0)
-                ntt_round<DIT, 1, true>(smem, total, a, t, cols, root_shift);
+                ntt_round<DIT, 1, true>(smem, total, a, t, cols, root_shift, reduce);
             else
-                ntt_round<DIT, 1, false>(smem, total, a, t, cols, root_shift);
+                ntt_round<DIT, 1, false>(smem, total, a, t, cols, root_shift, reduce);
         }
         __syncthreads();
         done += r;
@@ -299,21 +345,24 @@ __global__ __launch_bounds__(kMaxThreads, RMAX == 2 ? 4 : 1) void k_ntt_pass(Pas
             j = idx & (G - 1);
             c = idx >> a.np;
         }
+        // a whole transform in one tile may leave in natural order
+        if (a.natural_out) j = brev_bits(j, a.np);
         const uint64_t g = g0 + c;
         const uint64_t hi = g >> a.log_L;
         const uint32_t lo = (uint32_t)(g & (L - 1));
         const uint64_t pos = (hi << (a.log_n - a.S)) + ((uint64_t)j << a.log_L) + lo;
-        fr_t v = lds_get(smem, total, j * cols + c);
+        fr29 v = lds_get(smem, total, j * cols + c);
         if (!DIT && a.twiddle) {
             const uint32_t e = (lo * brev_bits(j, a.np)) << a.S;
-            if (e) v = kLazyNtt<DIT> ? mul_lazy(v, tw_at(a, j, lo, e)) : fp_mul(v, tw_at(a, j, lo, e));
+            if (e) v = mul29(v, tw_at(a, j, lo, e));
         }
-        if (a.post) v = kLazyNtt<DIT> ? mul_lazy(v, a.post[pos]) : fp_mul(v, a.post[pos]);
-        if (a.has_post_const) v = kLazyNtt<DIT> ? mul_lazy(v, a.post_const) : fp_mul(v, a.post_const);
-        a.data[pos] = kLazyNtt<DIT> ? fp_reduce_once(v) : v;
+        if (a.post) v = mul29(v, load29(a.post[pos]));
+        if (a.has_post_const) v = mul29(v, load29(a.post_const));
+        a.data[a.natural_out ? idx : pos] = canonical29(v);
     }
 }
 
+// Tables of factors are in the 2^261 form (factor_from_mont).
 // out[e] = base^e for e < count.
 __global__ void k_pow_table(fr_t *out, fr_t base, uint32_t count)
 {
@@ -325,7 +374,7 @@ __global__ void k_pow_table(fr_t *out, fr_t base, uint32_t count)
         if (x & 1) acc = fp_mul(acc, sq);
         sq = fp_sqr(sq);
     }
-    out[e] = acc;
+    out[e] = factor_from_mont(acc);
 }
 
 // out[j] = base^bitrev(j) * scale for j < 2^log_n.
@@ -339,7 +388,7 @@ __global__ void k_pow_rev_table(fr_t *out, fr_t base, fr_t scale, uint32_t log_n
         if (x & 1) acc = fp_mul(acc, sq);
         sq = fp_sqr(sq);
     }
-    out[j] = acc;
+    out[j] = factor_from_mont(acc);
 }
 
 // out[j] = scale * base^e, e = j (or bitrev(j) when rev), from the two-level
@@ -351,7 +400,7 @@ __global__ void k_pow_two_level(fr_t *out, const fr_t *__restrict__ hi, const fr
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= (1u << log_n)) return;
     const uint32_t e = rev ? brev_bits(j, log_n) : j;
-    fr_t v = fp_mul(hi[e >> m], lo[e & ((1u << m) - 1u)]);
+    fr_t v = factor_mul(hi[e >> m], lo[e & ((1u << m) - 1u)]);
     if (has_scale) v = fp_mul(v, scale);
     out[j] = v;
 }
@@ -365,7 +414,37 @@ __global__ void k_tw_full(fr_t *out, const fr_t *__restrict__ hi, const fr_t *__
     if (i >= (uint64_t(1) << (np + log_L))) return;
     const uint32_t j = (uint32_t)(i >> log_L), lo = (uint32_t)(i & ((1u << log_L) - 1u));
     const uint32_t e = (lo * brev_bits(j, np)) << S;
-    out[i] = fp_mul(hi[e >> m], lo_t[e & ((1u << m) - 1u)]);
+    out[i] = factor_mul(hi[e >> m], lo_t[e & ((1u << m) - 1u)]);
+}
+
+// Bit reversal in place: index = hi | mid | lo with kRevBits-bit hi and lo, and
+// reversed it is rev(lo) | rev(mid) | rev(hi).  The workgroup of mid (mid <=
+// rev(mid)) takes the tiles of mid and rev(mid), each 2^kRevBits runs of as
+// many elements (512 bytes), transposes them in LDS by the reversed hi and lo
+// and exchanges them, so every element is read and written once in long runs.
+// (A gather of single elements into a second array and its copy back took 70
+// us at 2^21; this takes 33, 128 MiB moved.)
+constexpr uint32_t kRevBits = 4;
+__global__ __launch_bounds__(1u << (2 * kRevBits)) void k_bitrev_inplace(fr_t *__restrict__ data, uint32_t log_n)
+{
+    constexpr uint32_t T = 1u << kRevBits;
+    __shared__ fr_t tile[2][T][T + 1];
+    const uint32_t m = log_n - 2 * kRevBits;
+    const uint32_t mid = blockIdx.x, dim = brev_bits(mid, m);
+    if (mid > dim) return;
+    const uint32_t hi = threadIdx.x >> kRevBits, lo = threadIdx.x & (T - 1);
+    const uint64_t row = (uint64_t)hi << (m + kRevBits);
+    fr_t *p0 = data + row + ((uint64_t)mid << kRevBits) + lo, *p1 = data + row + ((uint64_t)dim << kRevBits) + lo;
+    const uint32_t rh = brev_bits(hi, kRevBits), rl = brev_bits(lo, kRevBits);
+    tile[0][rl][rh] = *p0;
+    if (mid != dim) tile[1][rl][rh] = *p1;
+    __syncthreads();
+    if (mid == dim) {
+        *p0 = tile[0][hi][lo];
+    } else {
+        *p0 = tile[1][hi][lo];
+        *p1 = tile[0][hi][lo];
+    }
 }
 
 __global__ void k_bitrev(const fr_t *__restrict__ in, fr_t *__restrict__ out, uint32_t log_n)
@@ -437,6 +516,15 @@ fr_t fr_root_of_unity(unsigned log_n)
     return w;
 }
 
+// A full tile is 72 KiB, above the 64 KiB that a launch gets without asking.
+static void allow_full_tiles()
+{
+    for (const void *k :
+         {reinterpret_cast<const void *>(&k_ntt_pass<false, 2>), reinterpret_cast<const void *>(&k_ntt_pass<true, 2>),
+          reinterpret_cast<const void *>(&k_ntt_pass<false, 3>), reinterpret_cast<const void *>(&k_ntt_pass<true, 3>)})
+        NKR_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kTileBytes << 11)));
+}
+
 void NttDomain::plan(unsigned log_n, const NttShape *shape)
 {
     NKR_REQUIRE(log_n >= 1 && log_n <= kTwoAdicity, "NTT size must be 2^1 .. 2^28");
@@ -452,6 +540,7 @@ void NttDomain::plan(unsigned log_n, const NttShape *shape)
     radix_log_ = shape && shape->radix_log ? shape->radix_log : g_radix_log;
     const unsigned split_policy = shape && shape->split_set ? shape->split_policy : g_split_policy;
     NKR_REQUIRE(lds_log_ == 10 || lds_log_ == 11, "LDS elements per workgroup must be 2^10 or 2^11");
+    if (lds_log_ == 11) allow_full_tiles();
     NKR_REQUIRE(radix_log_ == 2 || radix_log_ == 3, "register radix must be 2^2 or 2^3");
     NKR_REQUIRE(split_policy <= 1, "pass split policy must be 0 (balanced) or 1 (contiguous last)");
     std::vector<unsigned> split;
@@ -579,8 +668,9 @@ NttDomain::NttDomain(unsigned log_n, int kind, fr_t *arena, hipStream_t stream) 
 }
 
 void NttDomain::run(fr_t *data, fr_t *const *batch, uint32_t count, bool dit, bool inverse, const fr_t *pre,
-                    const fr_t *post, const fr_t *post_const, hipStream_t stream) const
+                    const fr_t *post, const fr_t *post_const, hipStream_t stream, bool natural_out) const
 {
+    NKR_REQUIRE(!natural_out || (!dit && passes_.size() == 1), "only a one-pass DIF can leave natural order");
     NKR_REQUIRE(count >= 1 && count <= 65535, "NTT batch must hold 1 .. 65535 transforms");
     const int d = inverse ? 1 : 0;
     NKR_REQUIRE(tw_lo_p_[d], "this transform direction has no tables in this domain");
@@ -598,7 +688,7 @@ void NttDomain::run(fr_t *data, fr_t *const *batch, uint32_t count, bool dit, bo
         a.pre = (k == 0) ? pre : nullptr;
         a.post = (k == P - 1) ? post : nullptr;
         a.has_post_const = (k == P - 1 && post_const) ? 1u : 0u;
-        if (a.has_post_const) a.post_const = *post_const;
+        if (a.has_post_const) a.post_const = factor_from_mont(*post_const);
         a.log_n = log_n_;
         a.S = p.S;
         a.np = p.np;
@@ -607,9 +697,10 @@ void NttDomain::run(fr_t *data, fr_t *const *batch, uint32_t count, bool dit, bo
         a.log_roots = log_roots_;
         a.m_lo = m_lo_;
         a.twiddle = (pi != P - 1) ? 1u : 0u;
+        a.natural_out = natural_out ? 1u : 0u;
         const dim3 blocks((uint32_t)((size_t(1) << (log_n_ - p.np)) >> p.log_cols), count);
         const uint32_t elems = (1u << p.np) << p.log_cols;
-        const size_t lds = size_t(sizeof(fr_t)) * elems;
+        const size_t lds = size_t(kTileBytes) * elems;
         const uint32_t threads = std::min(kMaxThreads, std::max(64u, elems >> radix_log_));
         if (radix_log_ >= 3) {
             if (dit)
@@ -664,18 +755,17 @@ void NttDomain::bitrev(const fr_t *in, fr_t *out, hipStream_t stream) const
     NKR_LAUNCH_CHECK();
 }
 
-void NttDomain::standalone(fr_t *data, fr_t *scratch, int kind, hipStream_t stream) const
+void NttDomain::standalone(fr_t *data, int kind, hipStream_t stream) const
 {
+    NKR_REQUIRE(kind >= 0 && kind <= 3, "unknown transform kind (0 FFT, 1 iFFT, 2 cosetFFT, 3 icosetFFT)");
     NKR_REQUIRE(arena_kind_ < 0 || kind == arena_kind_, "this domain's tables serve another transform kind");
-    switch (kind) {
-    case 0: dif(data, false, nullptr, nullptr, nullptr, stream); break;
-    case 1: dif(data, true, nullptr, nullptr, &n_inv_, stream); break;
-    case 2: dif(data, false, coset_nat_p_, nullptr, nullptr, stream); break;
-    case 3: dif(data, true, nullptr, icoset_rev_p_, nullptr, stream); break;
-    default: throw Error("unknown transform kind (0 FFT, 1 iFFT, 2 cosetFFT, 3 icosetFFT)");
-    }
-    bitrev(data, scratch, stream);
-    NKR_HIP(hipMemcpyAsync(data, scratch, size() * sizeof(fr_t), hipMemcpyDeviceToDevice, stream));
+    const bool one_pass = passes_.size() == 1;
+    run(data, nullptr, 1, false, kind == 1 || kind == 3, kind == 2 ? coset_nat_p_ : nullptr,
+        kind == 3 ? icoset_rev_p_ : nullptr, kind == 1 ? &n_inv_ : nullptr, stream, one_pass);
+    if (one_pass) return;
+    // more than one pass means more than 2^10 elements, so the tiles fit
+    k_bitrev_inplace<<<1u << (log_n_ - 2 * kRevBits), 1u << (2 * kRevBits), 0, stream>>>(data, log_n_);
+    NKR_LAUNCH_CHECK();
 }
 
 void NttDomain::quotient(const fr_t *a, const fr_t *b, const fr_t *c, fr_t *h, hipStream_t stream) const
