@@ -27,10 +27,9 @@
 //               device-to-host copy each.
 //   graphs      a batch of the same contexts in the same order as the
 //               previous call is captured into a HIP graph (one per prover)
-//               and replayed while the composition repeats: the fold levels
-//               are then launched for the capacity's worst case and nothing
-//               is read back mid-sequence.  Any other batch runs eagerly and
-//               drops the graph.
+//               and replayed while the composition repeats (nothing is read
+//               back mid-sequence: every launch is planned on the device).
+//               Any other batch runs eagerly and drops the graph.
 //   host tail   the r,s-only blinding terms while the GPU works, then the
 //               final sums and blinding on a pool of host threads.
 // Each proof's result is bit-identical to proving it alone.

@@ -61,7 +61,7 @@ struct MsmPlan {
     uint32_t c = 0;         // window width in bits
     uint32_t W = 0;         // windows (signed digits), c*W >= 255
     uint32_t B = 0;         // buckets 1..B, B = 2^(c-1)
-    uint32_t piece_lo = 0;  // bounds of the accumulation piece length (max_pieces)
+    uint32_t piece_lo = 0;  // bounds of the accumulation run length (max_pieces)
     uint32_t piece_hi = 0;
 
     // ~3/4 log2 n bits (16 from 2^20 terms up), or c_override when non-zero.
