@@ -1,6 +1,8 @@
 // Batched Groth16 proving on one GPU (see batch.h for the stage plan).
 #include "batch.h"
 
+#include "probe.h"
+
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -54,8 +56,7 @@ BatchProver::BatchProver(int device) : device_(device)
             if (armed) p->release();
         }
     } undo{this};
-    NKR_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
-    NKR_HIP(hipStreamCreateWithFlags(&stream2_, hipStreamNonBlocking));
+    create_overlapping_streams(&stream_, &stream2_);
     NKR_HIP(hipEventCreateWithFlags(&ev_z_, hipEventDisableTiming));
     NKR_HIP(hipEventCreateWithFlags(&ev_wsched_, hipEventDisableTiming));
     NKR_HIP(hipEventCreateWithFlags(&ev_side_, hipEventDisableTiming));

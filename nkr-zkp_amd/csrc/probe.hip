@@ -52,7 +52,70 @@ __global__ void __launch_bounds__(kProbeThreads) k_mul_rate(fr_t *out, uint32_t 
     out[gid] = fp_add(a, b);
 }
 
+// One wave that sleeps for about 4 us per iteration.
+__global__ void k_sleep(uint32_t iters)
+{
+    for (uint32_t i = 0; i < iters; ++i) __builtin_amdgcn_s_sleep(127);
+}
+__global__ void k_nothing() {}
+
 }  // namespace
+
+// The runtime maps a process's streams onto four hardware queues, the least
+// used one at the time of each stream's creation, and streams of one queue run
+// their kernels strictly one after the other.  Which streams share a queue
+// cannot be asked, and a pair created back to back shares one whenever the
+// counts fall so (in some orders of creating and freeing contexts).  So the
+// side stream is tried: while a wave sleeps on the main stream, a kernel on a
+// stream of another queue finishes first.  A rejected candidate is kept until
+// the choice is made, so that the next one gets another queue.  At most 4 x
+// 0.5 ms per context.  (A proof of 64 hashes on a context whose streams shared
+// a queue: 886 us, its G2 chain after its transforms; with the trial 707.)
+void create_overlapping_streams(hipStream_t *main, hipStream_t *side)
+{
+    constexpr int kTries = 4;
+    constexpr uint32_t kSleep = 64;
+    struct Held {
+        hipStream_t rejected[kTries] = {};
+        int n = 0;
+        hipEvent_t main_end = nullptr, side_end = nullptr;
+        ~Held()
+        {
+            for (int i = 0; i < n; ++i) (void)hipStreamDestroy(rejected[i]);
+            if (main_end) (void)hipEventDestroy(main_end);
+            if (side_end) (void)hipEventDestroy(side_end);
+        }
+    } held;
+    NKR_HIP(hipEventCreate(&held.main_end));
+    NKR_HIP(hipEventCreate(&held.side_end));
+    NKR_HIP(hipStreamCreateWithFlags(main, hipStreamNonBlocking));
+    for (int t = 0;; ++t) {
+        NKR_HIP(hipStreamCreateWithFlags(side, hipStreamNonBlocking));
+        // both kernels' first launches (code upload) stay out of the trial
+        k_sleep<<<1, 64, 0, *main>>>(1);
+        NKR_LAUNCH_CHECK();
+        k_nothing<<<1, 64, 0, *side>>>();
+        NKR_LAUNCH_CHECK();
+        NKR_HIP(hipStreamSynchronize(*side));
+        NKR_HIP(hipStreamSynchronize(*main));
+        k_sleep<<<1, 64, 0, *main>>>(kSleep);
+        NKR_LAUNCH_CHECK();
+        NKR_HIP(hipEventRecord(held.main_end, *main));
+        k_nothing<<<1, 64, 0, *side>>>();
+        NKR_LAUNCH_CHECK();
+        NKR_HIP(hipEventRecord(held.side_end, *side));
+        NKR_HIP(hipStreamSynchronize(*side));
+        NKR_HIP(hipStreamSynchronize(*main));
+        // by the device's clock: asking the main stream whether it is done
+        // says no for a while after it is
+        float ahead_ms = 0;
+        NKR_HIP(hipEventElapsedTime(&ahead_ms, held.side_end, held.main_end));
+        if (ahead_ms > 0 || t == kTries - 1) return;
+        held.rejected[held.n++] = *side;
+        *side = nullptr;
+    }
+}
+
 }  // namespace nkr
 
 namespace nkr {

@@ -6,6 +6,7 @@
 
 #include "glv.h"
 #include "hquery.h"
+#include "probe.h"
 #include "setup.h"
 
 namespace nkr {
@@ -94,8 +95,7 @@ Groth16Prover::Groth16Prover(const nkr_g16_circuit &c, const nkr_g16_pk &pk, int
             if (armed) self->release();
         }
     } release_on_throw{this};
-    NKR_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
-    NKR_HIP(hipStreamCreateWithFlags(&stream2_, hipStreamNonBlocking));
+    create_overlapping_streams(&stream_, &stream2_);
     NKR_HIP(hipEventCreateWithFlags(&ev_start_, hipEventDisableTiming));
     NKR_HIP(hipEventCreateWithFlags(&ev_wsched_, hipEventDisableTiming));
 
