@@ -98,7 +98,8 @@ int nkr_g16_ctx_create(const nkr_g16_circuit *circuit, const nkr_g16_pk *pk, int
  *   ntt_lds_log          10 or 11: 2^lds_log elements per transform tile
  *   ntt_radix_log        2 or 3: register radix of the transform rounds
  *   ntt_split_policy     1 + policy: 1 balanced passes, 2 full last pass
- *   msm_target_pieces_log  2^k accumulation pieces per MSM launch, 12..24
+ *   msm_target_pieces_log  2^k accumulation threads per MSM launch, 12..24
+ *                          (19: the library's choice, as nkr_msm_set_shape)
  *   witness_g1_piece_min   shortest piece of the G1 MSMs (the witness ones and
  *                          H share a launch), 1..64 */
 typedef struct {
@@ -333,8 +334,8 @@ int nkr_ntt_set_shape(uint32_t lds_log, uint32_t radix_log, uint32_t split_polic
  * sorted entries of a launch evenly over 2^target_pieces_log threads (10 ..
  * 22); at most complete_lanes_cap lane groups (1, 2, 4, 8 or 16) then sum one
  * bucket's partial sums.  Set while no proof runs.  Results do not depend on
- * either; unset, the library picks the threads by the number of entries and
- * up to 16 lane groups, chosen by measurement. */
+ * either.  The defaults are (19, 16); 19 stands for the library's own choice
+ * of threads by the number of entries, made by measurement. */
 int nkr_msm_set_shape(uint32_t target_pieces_log, uint32_t complete_lanes_cap);
 
 /* y = M * z for one CSR matrix (host memory). */

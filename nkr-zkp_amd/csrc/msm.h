@@ -48,12 +48,12 @@
 namespace nkr {
 
 // Process-wide MSM tuning knobs: the accumulation lanes of a launch
-// (2^target_log, 10 .. 22; until it is set, MsmLanes' own) and the most lane
-// groups that complete one bucket (1 .. 16, a power of two).  Set them before
-// proving, not while proofs run.
+// (2^target_log, 10 .. 22; at kMsmTargetDefault, which it starts at, MsmLanes'
+// own) and the most lane groups that complete one bucket (1 .. 16, a power of
+// two).  Set them before proving, not while proofs run.
 void msm_set_shape(uint32_t target_pieces_log, uint32_t complete_lanes_cap);
-// The lanes of a group's launches: its own rule, or 2^target_log, or (0) the
-// process-wide setting.
+// The lanes of a group's launches (msm_lanes_of) for a target_log, or (0) for
+// the process-wide setting.
 MsmLanes msm_lanes(bool g2, uint32_t target_log = 0, uint32_t piece_min = 1);
 uint32_t msm_complete_lanes_cap();
 

@@ -941,7 +941,7 @@ uint64_t resident_blocks()
     return blocks;
 }
 
-uint32_t g_target_log = 0;  // 0: the group's own lanes
+uint32_t g_target_log = kMsmTargetDefault;
 uint32_t g_lanes_cap = 16;
 
 }  // namespace
@@ -959,12 +959,7 @@ void msm_set_shape(uint32_t target_pieces_log, uint32_t complete_lanes_cap)
 
 MsmLanes msm_lanes(bool g2, uint32_t target_log, uint32_t piece_min)
 {
-    MsmLanes r = g2 ? kMsmLanesG2 : kMsmLanesG1;
-    if (target_log == 0) target_log = g_target_log;
-    if (target_log)
-        for (uint32_t &l : r.lanes) l = 1u << target_log;
-    r.piece_min = std::max(1u, piece_min);
-    return r;
+    return msm_lanes_of(g2, target_log ? target_log : g_target_log, piece_min);
 }
 uint32_t msm_complete_lanes_cap() { return g_lanes_cap; }
 

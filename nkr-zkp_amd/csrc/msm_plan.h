@@ -40,6 +40,19 @@ struct MsmLanes {
 constexpr MsmLanes kMsmLanesG1 = {{1u << 16, 2u << 16, 4u << 16, 6u << 16}, {1u << 22, 1u << 24, 1u << 25}, 1};
 constexpr MsmLanes kMsmLanesG2 = {{1u << 16, 1u << 16, 2u << 16, 4u << 16}, {1u << 19, 1u << 21, 1u << 23}, 1};
 constexpr uint32_t kMsmMaxLanesLog = 19;  // at least log2 of every lane count above
+// The default of the lane setting (2^target_log lanes for every launch): the
+// group's own lanes above.
+constexpr uint32_t kMsmTargetDefault = 19;
+
+// The lanes of a group's launches for a setting of target_log.
+inline MsmLanes msm_lanes_of(bool g2, uint32_t target_log, uint32_t piece_min)
+{
+    MsmLanes r = g2 ? kMsmLanesG2 : kMsmLanesG1;
+    if (target_log != kMsmTargetDefault)
+        for (uint32_t &l : r.lanes) l = 1u << target_log;
+    r.piece_min = std::max(1u, piece_min);
+    return r;
+}
 // Largest bucket count (c <= 16): the histograms and bucket scans hold B
 // counts in one workgroup's LDS (128 KiB of gfx950's 160 KiB).
 constexpr uint32_t kMsmMaxBuckets = 1u << 15;

@@ -3,6 +3,7 @@
 //   plan n c_override target_log piece_lo piece_hi
 //       -> "c W B max_pieces capacity levels" or "error <message>"
 //   folds partials        -> fold levels for one bucket with that many partials
+//   lanes g2 target_log piece_min -> the lane rule: 4 lane counts, 3 limits, minimum
 //   divup a b             -> ceil(a / b) or "error <message>"
 // Errors are reported, never turned into a crash: a zero divisor must raise
 // nkr::Error instead of ending the process with SIGFPE.
@@ -40,6 +41,13 @@ int main()
                 uint64_t k;
                 in >> k;
                 std::printf("%u\n", msm_fold_levels(k));
+            } else if (op == "lanes") {
+                uint64_t g2, tl, pm;
+                in >> g2 >> tl >> pm;
+                const MsmLanes r = msm_lanes_of(g2 != 0, (uint32_t)tl, (uint32_t)pm);
+                for (uint32_t l : r.lanes) std::printf("%u ", l);
+                for (uint64_t b : r.below) std::printf("%llu ", (unsigned long long)b);
+                std::printf("%u\n", r.piece_min);
             } else if (op == "divup") {
                 uint64_t a, b;
                 in >> a >> b;

@@ -86,6 +86,19 @@ def test_fold_levels_and_capacity(plan_bin):
             assert level <= levels and used <= cap, (n, shape)
 
 
+def test_default_target_is_the_groups_own_rule(plan_bin):
+    """The lane setting's default, 19, gives each group its measured rule, so
+    that setting it back restores the default; any other value is 2^value
+    lanes whatever the number of entries."""
+    own = ask(plan_bin, ["lanes 0 19 0", "lanes 1 19 0"])
+    assert own == ["65536 131072 262144 393216 4194304 16777216 33554432 1",
+                   "65536 65536 131072 262144 524288 2097152 8388608 1"]
+    for target in (10, 12, 18, 20, 22, 24):
+        for line in ask(plan_bin, [f"lanes 0 {target} 5", f"lanes 1 {target} 5"]):
+            words = line.split()
+            assert words[:4] == [str(1 << target)] * 4 and words[-1] == "5"
+
+
 def test_zero_divisors_raise_instead_of_crashing(plan_bin):
     out = ask(plan_bin, ["plan 1024 0 19 0 64", "plan 1024 0 19 8 4", "divup 10 0", "divup 10 3",
                          "plan 0 0 19 4 64", "plan 1024 17 19 4 64"])
