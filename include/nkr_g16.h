@@ -156,8 +156,8 @@ int nkr_g16_batch_prove(nkr_g16_batch *batch, const nkr_g16_batch_item *items, u
 int nkr_g16_batch_destroy(nkr_g16_batch *batch);
 /* Launch-sequence reuse (no counterpart in the reference, which launches
  * every kernel of every proof): a batch of the same contexts in the same
- * order as the handle's previous call is captured into a HIP graph on its
- * second occurrence and replayed while the composition repeats (the
+ * order as the handle's previous call, with no nkr_msm_set_shape that changed
+ * anything in between, is captured into a HIP graph on its second occurrence and replayed while the composition repeats (the
  * size-class schedule of that composition); any other batch runs eagerly and
  * drops the graph.  Results are identical either way.  enabled = 0 turns the
  * capture off (and drops a graph); *active tells whether the handle holds a

@@ -26,7 +26,7 @@
 //   bit planes  three batch-wide regions (G1 over the witness, H, G2), one
 //               device-to-host copy each.
 //   graphs      a batch of the same contexts in the same order as the
-//               previous call is captured into a HIP graph (one per prover)
+//               previous call, under the same MSM shape, is captured into a HIP graph (one per prover)
 //               and replayed while the composition repeats (nothing is read
 //               back mid-sequence: every launch is planned on the device).
 //               Any other batch runs eagerly and drops the graph.
@@ -82,10 +82,10 @@ private:
     hipStream_t stream2_ = nullptr;  // witness schedules and G2 MSMs, beside them
     hipEvent_t ev_z_ = nullptr, ev_wsched_ = nullptr, ev_side_ = nullptr;
     std::vector<std::unique_ptr<Slot>> slots_;
-    // the captured launch sequence, the contexts it was captured for, and
-    // the previous call's contexts
+    // the captured launch sequence, the contexts and MSM shape it was captured
+    // for, and those of the previous call
     hipGraphExec_t graph_exec_ = nullptr;
-    std::vector<const void *> graph_key_, last_key_;
+    std::vector<uint64_t> graph_key_, last_key_;
     bool graphs_enabled_ = true;
     MsmScheduleBatch sort_w_, sort_h_;
     MsmBatch<fq_t> batch_g1_;

@@ -145,12 +145,13 @@ void BatchProver::prove(const std::vector<BatchItem> &items)
     while (slots_.size() < K) slots_.push_back(std::make_unique<Slot>());
 
     // Launch-sequence reuse: a batch of the same contexts in the same order as
-    // the previous call (the same sizes, slots and tables) is captured into a
-    // HIP graph on its second occurrence and replayed from then on; any other
-    // batch runs eagerly and drops the graph, since it may move what the
-    // graph's launches refer to.
-    std::vector<const void *> key(K);
-    for (size_t i = 0; i < K; ++i) key[i] = items[i].ctx;
+    // the previous call (the same sizes, slots and tables), under the same
+    // process-wide MSM shape, is captured into a HIP graph on its second
+    // occurrence and replayed from then on; any other batch runs eagerly and
+    // drops the graph, since it may move what the graph's launches refer to.
+    std::vector<uint64_t> key(K + 1);
+    for (size_t i = 0; i < K; ++i) key[i] = reinterpret_cast<uint64_t>(items[i].ctx);
+    key[K] = msm_shape_key();
     const bool replay = graph_exec_ && key == graph_key_;
     const bool capture = !replay && graphs_enabled_ && key == last_key_;
     if (!replay) drop_graph();

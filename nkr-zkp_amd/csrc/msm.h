@@ -38,6 +38,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "curve.h"
@@ -56,6 +57,9 @@ void msm_set_shape(uint32_t target_pieces_log, uint32_t complete_lanes_cap);
 // the process-wide setting.
 MsmLanes msm_lanes(bool g2, uint32_t target_log = 0, uint32_t piece_min = 1);
 uint32_t msm_complete_lanes_cap();
+// Both process-wide knobs in one word: launches captured under one value are
+// not replayed under another.
+uint64_t msm_shape_key();
 
 // Device bytes of one schedule (MsmSchedule) and of one MSM job's partial
 // sums and per-bucket arrays (MsmBatch) for a plan.
@@ -216,10 +220,12 @@ public:
         key_.clear();  // the layout cache refers to the released buffers
     }
 
-    // The jobs' layout is the one the batch's buffers already hold.
+    // The jobs' layout, and the lanes it was sized for, are those the batch's
+    // buffers already hold.
     bool layout_matches(const std::vector<MsmJob<F>> &jobs) const;
 
 private:
+    MsmLanes wanted_lanes() const { return have_lanes_ ? own_lanes_ : msm_lanes(std::is_same<F, fq2_t>::value); }
     void layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream);
     std::vector<const void *> key_;
     uint32_t fold_levels_ = 0;     // 4:1 levels the largest possible bucket needs

@@ -962,6 +962,7 @@ MsmLanes msm_lanes(bool g2, uint32_t target_log, uint32_t piece_min)
     return msm_lanes_of(g2, target_log ? target_log : g_target_log, piece_min);
 }
 uint32_t msm_complete_lanes_cap() { return g_lanes_cap; }
+uint64_t msm_shape_key() { return (uint64_t)g_target_log << 32 | g_lanes_cap; }
 
 uint32_t MsmSchedule::sort_blocks(uint32_t n)
 {
@@ -1127,16 +1128,16 @@ static std::vector<const void *> layout_key(const std::vector<MsmJob<F>> &jobs)
 template <class F>
 bool MsmBatch<F>::layout_matches(const std::vector<MsmJob<F>> &jobs) const
 {
-    return layout_key(jobs) == key_;
+    return layout_key(jobs) == key_ && wanted_lanes() == lanes_;
 }
 
 template <class F>
 void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
 {
+    if (layout_matches(jobs)) return;
     std::vector<const void *> key = layout_key(jobs);
-    const MsmLanes lanes = have_lanes_ ? own_lanes_ : msm_lanes(std::is_same<F, fq2_t>::value);
-    if (key == key_ && lanes == lanes_) return;
-    lanes_ = lanes;
+    key_.clear();  // until the new layout is whole
+    lanes_ = wanted_lanes();
     const uint32_t J = (uint32_t)jobs.size();
     // The pool: a partial per lane and bucket of the launch (k_reduce_plan),
     // then the fold launches' outputs of all jobs; and the per-bucket arrays.

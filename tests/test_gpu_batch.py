@@ -112,6 +112,36 @@ def test_batch_graph_replays_match_plain(mix):
     b.close()
 
 
+@pytest.mark.parametrize("shape", [(12, 16), (20, 16), (19, 2)])
+def test_batch_after_a_change_of_the_msm_shape(mix, shape):
+    """A batch whose contexts repeat but whose process-wide MSM shape changed
+    is laid out again, so it runs eagerly: a layout may not happen inside a
+    capture.  Eager, captured and replayed calls before the change, under the
+    new shape and after the default came back give the plain path's proofs."""
+    _, _, cases = mix
+    rs = circuits.random_scalars(2 * len(cases), 1234)
+    items = [(pv, w, rs[2 * i], rs[2 * i + 1]) for i, (_, pv, _, _, w) in enumerate(cases)]
+    want = [pv.prove_blind(w, r, s) for pv, w, r, s in items]
+    b = N.Batch()
+
+    def graph_after_a_call():
+        for (raw, proof), (raw1, proof1) in zip(b.prove(items), want):
+            assert np.array_equal(raw, raw1) and np.array_equal(proof, proof1)
+        return b.graph_active()
+
+    try:
+        assert not graph_after_a_call()
+        N._check(N.lib().nkr_msm_set_shape(*shape))
+        assert not graph_after_a_call()  # the same contexts, another shape
+        assert graph_after_a_call() and graph_after_a_call()
+        N._check(N.lib().nkr_msm_set_shape(19, 16))
+        assert not graph_after_a_call()  # the graph is dropped with its shape
+        assert graph_after_a_call() and graph_after_a_call()
+    finally:
+        N._check(N.lib().nkr_msm_set_shape(19, 16))
+        b.close()
+
+
 def test_batch_upload_chunk_edges():
     """The batch's packed upload lays witnesses end to end from multiples of
     64 and cuts them into chunks of 2^15 elements: witnesses of 35841 columns
