@@ -38,6 +38,7 @@
 #include <memory>
 #include <vector>
 
+#include "launch_reuse.h"
 #include "msm.h"
 #include "prover.h"
 
@@ -82,10 +83,8 @@ private:
     hipStream_t stream2_ = nullptr;  // witness schedules and G2 MSMs, beside them
     hipEvent_t ev_z_ = nullptr, ev_wsched_ = nullptr, ev_side_ = nullptr;
     std::vector<std::unique_ptr<Slot>> slots_;
-    // the captured launch sequence, the contexts and MSM shape it was captured
-    // for, and those of the previous call
-    hipGraphExec_t graph_exec_ = nullptr;
-    std::vector<uint64_t> graph_key_, last_key_;
+    hipGraphExec_t graph_exec_ = nullptr;  // the captured launch sequence
+    LaunchReuse reuse_;                    // and the calls it stands for
     bool graphs_enabled_ = true;
     MsmScheduleBatch sort_w_, sort_h_;
     MsmBatch<fq_t> batch_g1_;

@@ -71,7 +71,6 @@ BatchProver::~BatchProver()
 void BatchProver::release() noexcept
 {
     drop_graph();
-    last_key_.clear();
     for (hipStream_t *s : {&stream2_, &stream_})
         if (*s) {
             (void)hipStreamSynchronize(*s);
@@ -92,7 +91,7 @@ void BatchProver::drop_graph() noexcept
         (void)hipGraphExecDestroy(graph_exec_);
         graph_exec_ = nullptr;
     }
-    graph_key_.clear();
+    reuse_.dropped();
 }
 
 void BatchProver::set_graphs(bool enabled)
@@ -118,7 +117,7 @@ void BatchProver::trim()
     NKR_HIP(hipStreamSynchronize(stream_));
     NKR_HIP(hipStreamSynchronize(stream2_));
     drop_graph();  // its launches refer to the buffers released here
-    last_key_.clear();
+    reuse_.forget();
     slots_.clear();
     tables_.release();
     planes_w_.release();
@@ -144,18 +143,14 @@ void BatchProver::prove(const std::vector<BatchItem> &items)
     NKR_HIP(hipSetDevice(device_));
     while (slots_.size() < K) slots_.push_back(std::make_unique<Slot>());
 
-    // Launch-sequence reuse: a batch of the same contexts in the same order as
-    // the previous call (the same sizes, slots and tables), under the same
-    // process-wide MSM shape, is captured into a HIP graph on its second
-    // occurrence and replayed from then on; any other batch runs eagerly and
-    // drops the graph, since it may move what the graph's launches refer to.
+    // Launch-sequence reuse (launch_reuse.h): the key is the contexts in their
+    // order (the same sizes, slots and tables) and the process-wide MSM shape.
     std::vector<uint64_t> key(K + 1);
     for (size_t i = 0; i < K; ++i) key[i] = reinterpret_cast<uint64_t>(items[i].ctx);
     key[K] = msm_shape_key();
-    const bool replay = graph_exec_ && key == graph_key_;
-    const bool capture = !replay && graphs_enabled_ && key == last_key_;
+    const LaunchReuse::Mode mode = reuse_.begin(std::move(key), graphs_enabled_);
+    const bool replay = mode == LaunchReuse::Mode::kReplay, capture = mode == LaunchReuse::Mode::kCapture;
     if (!replay) drop_graph();
-    last_key_ = key;
     const bool graph = replay || capture;
 
     // bit planes of every proof in three batch-wide regions (G1 over the
@@ -331,7 +326,7 @@ void BatchProver::prove(const std::vector<BatchItem> &items)
                 graph_exec_ = nullptr;
                 NKR_HIP(ie);
             }
-            graph_key_ = key;
+            reuse_.captured();
             NKR_HIP(hipGraphLaunch(graph_exec_, stream_));
         }
     }
@@ -351,6 +346,7 @@ void BatchProver::prove(const std::vector<BatchItem> &items)
         const Groth16Prover::BlindJob job{it.r, it.s, it.proof_out};
         g.finish_serial(hw + pw_off[i], hh + ph_off[i], h2 + p2_off[i], &job, &pre[i], it.raw_out);
     });
+    reuse_.finish();
 }
 
 }  // namespace nkr
