@@ -146,7 +146,7 @@ void BatchProver::prove(const std::vector<BatchItem> &items)
     // Launch-sequence reuse (launch_reuse.h): the key is the contexts in their
     // order (the same sizes, slots and tables) and the process-wide MSM shape.
     std::vector<uint64_t> key(K + 1);
-    for (size_t i = 0; i < K; ++i) key[i] = reinterpret_cast<uint64_t>(items[i].ctx);
+    for (size_t i = 0; i < K; ++i) key[i] = items[i].ctx->serial();
     key[K] = msm_shape_key();
     const LaunchReuse::Mode mode = reuse_.begin(std::move(key), graphs_enabled_);
     const bool replay = mode == LaunchReuse::Mode::kReplay, capture = mode == LaunchReuse::Mode::kCapture;

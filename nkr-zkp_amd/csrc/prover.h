@@ -54,6 +54,9 @@ public:
 
     uint64_t device_bytes() const;
     int device() const { return device_; }
+    // Never given to another context of the process (an address is, once its
+    // context is gone).
+    uint64_t serial() const { return serial_; }
     // prepared with alpha/beta/delta, which blinding needs
     bool can_blind() const { return have_blind_; }
     hipStream_t stream() const { return stream_; }
@@ -70,6 +73,7 @@ public:
 private:
     void release() noexcept;  // streams, events and pinned memory (destructor, failed constructor)
     int device_;
+    uint64_t serial_;
     hipStream_t stream_ = nullptr;
     uint32_t rows_, cols_, log_n_;
     DeviceBuffer<uint32_t> row_ptr_[3], col_idx_[3], long_rows_[3];

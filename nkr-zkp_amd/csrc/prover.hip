@@ -1,5 +1,6 @@
 #include "prover.h"
 
+#include <atomic>
 #include <chrono>
 #include <cstring>
 #include <exception>
@@ -61,9 +62,13 @@ void check_circuit(const nkr_g16_circuit &c)
     for (int m = 0; m < 3; ++m) NKR_REQUIRE(nnz[m] < (1ull << 32), "matrix has too many non-zeros");
 }
 
+namespace {
+std::atomic<uint64_t> g_next_serial{1};
+}
+
 Groth16Prover::Groth16Prover(const nkr_g16_circuit &c, const nkr_g16_pk &pk, int device,
                              const nkr_g16_tuning *tuning)
-    : device_(device)
+    : device_(device), serial_(g_next_serial.fetch_add(1))
 {
     nkr_g16_tuning tn{};
     if (tuning) tn = *tuning;

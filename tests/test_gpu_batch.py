@@ -142,6 +142,25 @@ def test_batch_after_a_change_of_the_msm_shape(mix, shape):
         b.close()
 
 
+def test_batch_after_a_context_was_replaced():
+    """A context made after another was closed may get its address; a batch
+    that replayed a graph of the old one must not take it for the same."""
+    b = N.Batch()
+    rs = circuits.random_scalars(2, 4321)
+    for seed in range(6):
+        c = circuits.matmul(4, 50 + seed)
+        k = keyed(c, 500 + seed)
+        pv = N.Prover(c, k)
+        for call in range(3):
+            raw, proof = b.prove([(pv, c.witness, rs[0], rs[1])] * 2)[1]
+            raw1, proof1 = pv.prove_blind(c.witness, rs[0], rs[1])
+            assert np.array_equal(raw, raw1) and np.array_equal(proof, proof1), (seed, call)
+            assert N.verify(k, c.witness[1:1 + c.public_inputs], proof), (seed, call)
+            assert b.graph_active() == (call > 0), (seed, call)
+        pv.close()
+    b.close()
+
+
 def test_batch_upload_chunk_edges():
     """The batch's packed upload lays witnesses end to end from multiples of
     64 and cuts them into chunks of 2^15 elements: witnesses of 35841 columns
