@@ -572,7 +572,16 @@ int nkr_fr_ntt_dev(void *data_dev, uint32_t log_n, int kind, void *stream)
         NKR_REQUIRE(dev >= 0 && dev < kMaxDevices, "device index out of range");
         std::lock_guard<std::mutex> lock(g_ntt_mutex);
         NttDomain *&dom = g_ntt_cache[dev][log_n];
-        if (!dom) dom = new NttDomain(log_n, s);
+        if (!dom) {
+            // A domain serves every stream from here on, so its tables are
+            // whole before any call sees it; built on the caller's stream, a
+            // call on another one could read them too early.
+            StreamGuard build;
+            NKR_HIP(hipStreamCreateWithFlags(&build.s, hipStreamNonBlocking));
+            auto made = std::make_unique<NttDomain>(log_n, build.s);
+            NKR_HIP(hipStreamSynchronize(build.s));
+            dom = made.release();
+        }
         dom->standalone(static_cast<fr_t *>(data_dev), kind, s);
     });
 }

@@ -107,14 +107,6 @@ void upload(DeviceBuffer<T> &buf, const T *src, size_t count, hipStream_t stream
 
 fq_t fq_limbs(const uint32_t (&v)[8]) { return fp_to_mont(fq_t{{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]}}); }
 
-struct StreamGuard {
-    hipStream_t s = nullptr;
-    ~StreamGuard()
-    {
-        if (s) (void)hipStreamDestroy(s);
-    }
-};
-
 struct EventGuard {
     hipEvent_t e = nullptr;
     ~EventGuard()

@@ -85,6 +85,18 @@ private:
     size_t count_ = 0;
 };
 
+// A stream owned by one scope.
+struct StreamGuard {
+    hipStream_t s = nullptr;
+    StreamGuard() = default;
+    StreamGuard(const StreamGuard &) = delete;
+    StreamGuard &operator=(const StreamGuard &) = delete;
+    ~StreamGuard()
+    {
+        if (s) (void)hipStreamDestroy(s);
+    }
+};
+
 // Pinned host staging buffer for asynchronous uploads.  `reuse` waits for the
 // upload recorded by `uploaded` before the host writes the buffer again.
 // A short pause for host spin loops.
