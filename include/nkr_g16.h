@@ -100,8 +100,8 @@ int nkr_g16_ctx_create(const nkr_g16_circuit *circuit, const nkr_g16_pk *pk, int
  *   ntt_split_policy     1 + policy: 1 balanced passes, 2 full last pass
  *   msm_target_pieces_log  2^k accumulation threads per MSM launch, 12..24
  *                          (19: the library's choice, as nkr_msm_set_shape)
- *   witness_g1_piece_min   shortest piece of the G1 MSMs (the witness ones and
- *                          H share a launch), 1..64 */
+ *   witness_g1_piece_min   shortest run of entries of a thread in the witness
+ *                          G1 MSMs, 1..64 */
 typedef struct {
     uint32_t witness_window_bits, h_window_bits;
     uint32_t ntt_lds_log, ntt_radix_log, ntt_split_policy;

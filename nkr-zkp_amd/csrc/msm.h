@@ -55,7 +55,7 @@ namespace nkr {
 void msm_set_shape(uint32_t target_pieces_log, uint32_t complete_lanes_cap);
 // The lanes of a group's launches (msm_lanes_of) for a target_log, or (0) for
 // the process-wide setting.
-MsmLanes msm_lanes(bool g2, uint32_t target_log = 0, uint32_t piece_min = 1);
+MsmLanes msm_lanes(bool g2, uint32_t target_log = 0);
 uint32_t msm_complete_lanes_cap();
 // Both process-wide knobs in one word: launches captured under one value are
 // not replayed under another.
@@ -177,6 +177,7 @@ struct MsmJob {
     const MsmBases<F> *bases;
     const MsmSchedule *sched;
     Xyzz<F> *planes;   // device output: c points U_0 .. U_{c-1}
+    uint32_t piece_min = 1;  // shortest run of an accumulation lane of this job
 };
 
 // Runs a batch of MSMs of one group (all with the same window width).

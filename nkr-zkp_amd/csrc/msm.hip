@@ -52,7 +52,7 @@ struct FoldRec {
 // `fold_ctr` are zero between launches; fold_count holds their last values.
 struct ReduceState {
     uint32_t ticket;
-    uint32_t piece;  // entries per accumulation lane
+    uint32_t piece;  // entries per accumulation lane (msm_piece)
     unsigned long long fold_ctr[kMaxFoldLaunches];  // records << 32 | outputs
     unsigned long long fold_count[kMaxFoldLaunches];
 };
@@ -69,6 +69,7 @@ struct JobDev {
     Xyzz<F> *planes;               // c (canonical)
     uint32_t B, c;
     uint32_t b_off;  // buckets of the jobs before this one
+    uint32_t piece_min;
 };
 
 // ------------------------------------------------------------ digit recoding
@@ -320,19 +321,19 @@ __global__ __launch_bounds__(kSortThreads) void k_scatter_batch(const SortJob *_
                   jb.tile_total, jb.block_count, jb.bucket_start, jb.sorted);
 }
 
-// Entries per accumulation lane for E entries in all (MsmLanes).
-__device__ __forceinline__ uint32_t piece_length(uint64_t E, const MsmLanes &r)
+// Accumulation lanes of a job.
+template <class F>
+__device__ __forceinline__ uint32_t job_lanes(const JobDev<F> &jb, uint32_t launch_piece)
 {
-    uint32_t lanes = r.lanes[3];
-    for (int i = 2; i >= 0; --i)
-        if (E < r.below[i]) lanes = r.lanes[i];
-    return (uint32_t)max((uint64_t)r.piece_min, (E + lanes - 1) / lanes);
+    const uint32_t piece = msm_job_piece(launch_piece, jb.piece_min);
+    return (jb.bucket_start[jb.B] + piece - 1) / piece;
 }
 
 // The plan of a batch, from the schedules' bucket starts: one launch before
 // the accumulation instead of several small ones around it.
 //   * the accumulation gives every lane L consecutive entries of a job's
-//     sorted list, L = piece_length of all jobs' entries; a bucket of the
+//     sorted list, L = msm_piece of all jobs' entries or, where that is more,
+//     the job's minimum; a bucket of the
 //     entries [a, b) therefore gets a partial from each of the lanes a / L ..
 //     (b - 1) / L, and lane l's partial of bucket k is number l + k of the job
 //     (two lanes share a bucket, or one lane two buckets, never both), at
@@ -370,13 +371,14 @@ __global__ __launch_bounds__(kPlanThreads) void k_reduce_plan(const JobDev<F> *_
     for (uint32_t i = threadIdx.x; i < J; i += blockDim.x)
         atomicAdd(&entries, (unsigned long long)jobs[i].bucket_start[jobs[i].B]);
     __syncthreads();
-    const uint32_t piece = piece_length(entries, rule);
+    const uint32_t launch_piece = msm_piece(rule, entries);
     __shared__ uint32_t lanes_before;
     if (threadIdx.x == 0) lanes_before = 0;
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < j; i += blockDim.x)
-        atomicAdd(&lanes_before, (jobs[i].bucket_start[jobs[i].B] + piece - 1) / piece);
+        atomicAdd(&lanes_before, job_lanes(jobs[i], launch_piece));
     __syncthreads();
+    const uint32_t piece = msm_job_piece(launch_piece, jb.piece_min);
     uint32_t m = 0;
     if (k < jb.B) {
         const uint32_t beg = jb.bucket_start[k], end = jb.bucket_start[k + 1];
@@ -398,7 +400,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_reduce_plan(const JobDev<F> *_
     // the waves' counts are scanned in LDS
     __shared__ uint32_t count[kCompleteClasses][kPlanThreads / 64], list_at[kCompleteClasses];
     constexpr uint32_t groups = 65536 / Coop<F>::kLanes;
-    const uint32_t serial = 1 + (uint32_t)(3 * (entries / piece + buckets) / (2 * groups));
+    const uint32_t serial = 1 + (uint32_t)(3 * (entries / launch_piece + buckets) / (2 * groups));
     uint32_t c = 0;
     while (c < max_class && (serial << c) < m) ++c;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
@@ -433,8 +435,8 @@ __global__ __launch_bounds__(kPlanThreads) void k_reduce_plan(const JobDev<F> *_
     }
     __syncthreads();
     if (!last) return;
-    if (threadIdx.x == 0) st->piece = piece;
-    group_prefix(J, lane_base, [&](uint32_t i) { return (jobs[i].bucket_start[jobs[i].B] + piece - 1) / piece; });
+    if (threadIdx.x == 0) st->piece = launch_piece;
+    group_prefix(J, lane_base, [&](uint32_t i) { return job_lanes(jobs[i], launch_piece); });
     group_prefix(kCompleteClasses * J, seg_base, [&](uint32_t s) {
         const uint32_t n = atomicExch(&class_count[s], 0u);
         seg_count[s] = n;
@@ -671,7 +673,8 @@ __device__ __forceinline__ void accumulate_body(const JobDev<F> *__restrict__ jo
     const uint32_t j = find_segment(lane_base, J, g);
     const JobDev<F> &jb = jobs[j];
     LaneWords<kLds> lw(words);
-    RunCursor<kLds> c(lw, jb.bucket_start, jb.B, lane_base[j] + jb.b_off, g - lane_base[j], st->piece);
+    RunCursor<kLds> c(lw, jb.bucket_start, jb.B, lane_base[j] + jb.b_off, g - lane_base[j],
+                      msm_job_piece(st->piece, jb.piece_min));
     Stream in(stage[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)], lw, jb.bases, jb.sorted, c.e,
               jb.bucket_start[jb.B]);
     if constexpr (std::is_same<F, fq2_t>::value) {
@@ -957,9 +960,9 @@ void msm_set_shape(uint32_t target_pieces_log, uint32_t complete_lanes_cap)
 }
 
 
-MsmLanes msm_lanes(bool g2, uint32_t target_log, uint32_t piece_min)
+MsmLanes msm_lanes(bool g2, uint32_t target_log)
 {
-    return msm_lanes_of(g2, target_log ? target_log : g_target_log, piece_min);
+    return msm_lanes_of(g2, target_log ? target_log : g_target_log);
 }
 uint32_t msm_complete_lanes_cap() { return g_lanes_cap; }
 uint64_t msm_shape_key() { return (uint64_t)g_target_log << 32 | g_lanes_cap; }
@@ -1121,6 +1124,7 @@ static std::vector<const void *> layout_key(const std::vector<MsmJob<F>> &jobs)
         key.push_back(jb.planes);
         key.push_back(reinterpret_cast<const void *>((uintptr_t)jb.sched->plan().max_entries()));
         key.push_back(reinterpret_cast<const void *>((uintptr_t)jb.sched->plan().B));
+        key.push_back(reinterpret_cast<const void *>((uintptr_t)jb.piece_min));
     }
     return key;
 }
@@ -1191,6 +1195,7 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
         d.B = jb.sched->plan().B;
         d.c = jb.sched->plan().c;
         d.b_off = (uint32_t)b_off[j];
+        d.piece_min = std::max(1u, jb.piece_min);
     }
     std::memcpy(st + jobs_bytes, fold_base_, sizeof(fold_base_));
     // completion lanes: a bucket's lane groups, plus each segment's padding

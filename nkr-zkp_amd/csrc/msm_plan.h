@@ -30,29 +30,44 @@ constexpr uint32_t kMaxFoldLevels = 12;
 struct MsmLanes {
     uint32_t lanes[4];
     uint64_t below[3];
-    uint32_t piece_min;  // shortest run of a lane
     bool operator==(const MsmLanes &o) const
     {
-        return std::equal(lanes, lanes + 4, o.lanes) && std::equal(below, below + 3, o.below) &&
-               piece_min == o.piece_min;
+        return std::equal(lanes, lanes + 4, o.lanes) && std::equal(below, below + 3, o.below);
     }
 };
-constexpr MsmLanes kMsmLanesG1 = {{1u << 16, 2u << 16, 4u << 16, 6u << 16}, {1u << 22, 1u << 24, 1u << 25}, 1};
-constexpr MsmLanes kMsmLanesG2 = {{1u << 16, 1u << 16, 2u << 16, 4u << 16}, {1u << 19, 1u << 21, 1u << 23}, 1};
+constexpr MsmLanes kMsmLanesG1 = {{1u << 16, 2u << 16, 4u << 16, 6u << 16}, {1u << 22, 1u << 24, 1u << 25}};
+constexpr MsmLanes kMsmLanesG2 = {{1u << 16, 1u << 16, 2u << 16, 4u << 16}, {1u << 19, 1u << 21, 1u << 23}};
 constexpr uint32_t kMsmMaxLanesLog = 19;  // at least log2 of every lane count above
 // The default of the lane setting (2^target_log lanes for every launch): the
 // group's own lanes above.
 constexpr uint32_t kMsmTargetDefault = 19;
 
 // The lanes of a group's launches for a setting of target_log.
-inline MsmLanes msm_lanes_of(bool g2, uint32_t target_log, uint32_t piece_min)
+inline MsmLanes msm_lanes_of(bool g2, uint32_t target_log)
 {
     MsmLanes r = g2 ? kMsmLanesG2 : kMsmLanesG1;
     if (target_log != kMsmTargetDefault)
         for (uint32_t &l : r.lanes) l = 1u << target_log;
-    r.piece_min = std::max(1u, piece_min);
     return r;
 }
+
+// The planning kernel's rules (constexpr: host and device run the same code).
+// Lanes of a launch over `entries` entries.
+constexpr uint32_t msm_launch_lanes(const MsmLanes &r, uint64_t entries)
+{
+    uint32_t lanes = r.lanes[3];
+    for (int i = 2; i >= 0; --i)
+        if (entries < r.below[i]) lanes = r.lanes[i];
+    return lanes;
+}
+// Entries per lane of a launch over `entries` entries, and of one of its jobs,
+// whose runs may have a minimum of their own.
+constexpr uint32_t msm_piece(const MsmLanes &r, uint64_t entries)
+{
+    const uint32_t lanes = msm_launch_lanes(r, entries);
+    return entries == 0 ? 1u : (uint32_t)((entries + lanes - 1) / lanes);
+}
+constexpr uint32_t msm_job_piece(uint32_t piece, uint32_t piece_min) { return piece < piece_min ? piece_min : piece; }
 // Largest bucket count (c <= 16): the histograms and bucket scans hold B
 // counts in one workgroup's LDS (128 KiB of gfx950's 160 KiB).
 constexpr uint32_t kMsmMaxBuckets = 1u << 15;

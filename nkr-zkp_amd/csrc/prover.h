@@ -81,6 +81,7 @@ private:
     CsrView views_[3];
     std::unique_ptr<NttDomain> domain_;
     MsmPlan wplan_, bplan_, hplan_;
+    uint32_t witness_piece_min_ = 1;  // shortest run of the witness G1 MSMs' lanes
     // The B query (bs1 and bs2) without its points at infinity: most R1CS
     // variables are in no row of B, and a point at infinity would still cost
     // its digits' sort, its gather and, where another lane of the wave has a

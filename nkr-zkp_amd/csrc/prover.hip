@@ -129,10 +129,11 @@ Groth16Prover::Groth16Prover(const nkr_g16_circuit &c, const nkr_g16_pk &pk, int
     wplan_ = MsmPlan::choose(cols_, tn.witness_window_bits);
     if (wplan_.c > 15) wplan_ = MsmPlan::choose(cols_, 15);
     hplan_ = MsmPlan::choose(rows_, tn.h_window_bits);
-    if (tn.msm_target_pieces_log || tn.witness_g1_piece_min) {
-        batch_g1_.set_lanes(msm_lanes(false, tn.msm_target_pieces_log, tn.witness_g1_piece_min));
+    if (tn.msm_target_pieces_log) {
+        batch_g1_.set_lanes(msm_lanes(false, tn.msm_target_pieces_log));
         batch_g2_.set_lanes(msm_lanes(true, tn.msm_target_pieces_log));
     }
+    witness_piece_min_ = std::max(1u, tn.witness_g1_piece_min);
 
     {
         DeviceBuffer<g1_jac> tmp1(std::max(cols_, rows_));
@@ -486,9 +487,10 @@ void Groth16Prover::run(const fr_t *z, void *raw_out, void *az, void *bz, void *
     // latency-bound reduction levels are paid once for all four.
     hsched_.build(pa_.get(), nullptr, hplan_, s, t);
     NKR_HIP(hipStreamWaitEvent(s, ev_wsched_, 0));
-    batch_g1_.run({MsmJob<fq_t>{&a_, &wsched_, planes1_.get()},
-                   MsmJob<fq_t>{&l_, &wsched_, planes1_.get() + cw},
-                   MsmJob<fq_t>{&b1_, &bsched, planes1_.get() + 2 * cw},
+    const uint32_t pm = witness_piece_min_;
+    batch_g1_.run({MsmJob<fq_t>{&a_, &wsched_, planes1_.get(), pm},
+                   MsmJob<fq_t>{&l_, &wsched_, planes1_.get() + cw, pm},
+                   MsmJob<fq_t>{&b1_, &bsched, planes1_.get() + 2 * cw, pm},
                    MsmJob<fq_t>{&h_, &hsched_, planes1_.get() + planes_g1_witness()}},
                   s, t);
     const size_t n1 = planes_g1_witness() + hplan_.c;

@@ -3,7 +3,9 @@
 //   plan n c_override target_log piece_lo piece_hi
 //       -> "c W B max_pieces capacity levels" or "error <message>"
 //   folds partials        -> fold levels for one bucket with that many partials
-//   lanes g2 target_log piece_min -> the lane rule: 4 lane counts, 3 limits, minimum
+//   lanes g2 target_log   -> the lane rule: 4 lane counts, 3 limits
+//   piece g2 target_log piece_min entries... -> per entry count, the launch's
+//                            entries per lane and those of a job with that minimum
 //   divup a b             -> ceil(a / b) or "error <message>"
 // Errors are reported, never turned into a crash: a zero divisor must raise
 // nkr::Error instead of ending the process with SIGFPE.
@@ -42,12 +44,18 @@ int main()
                 in >> k;
                 std::printf("%u\n", msm_fold_levels(k));
             } else if (op == "lanes") {
-                uint64_t g2, tl, pm;
-                in >> g2 >> tl >> pm;
-                const MsmLanes r = msm_lanes_of(g2 != 0, (uint32_t)tl, (uint32_t)pm);
+                uint64_t g2, tl;
+                in >> g2 >> tl;
+                const MsmLanes r = msm_lanes_of(g2 != 0, (uint32_t)tl);
                 for (uint32_t l : r.lanes) std::printf("%u ", l);
                 for (uint64_t b : r.below) std::printf("%llu ", (unsigned long long)b);
-                std::printf("%u\n", r.piece_min);
+                std::printf("\n");
+            } else if (op == "piece") {
+                uint64_t g2, tl, pm, e;
+                in >> g2 >> tl >> pm;
+                const MsmLanes r = msm_lanes_of(g2 != 0, (uint32_t)tl);
+                while (in >> e) std::printf("%u %u ", msm_piece(r, e), msm_job_piece(msm_piece(r, e), (uint32_t)pm));
+                std::printf("\n");
             } else if (op == "divup") {
                 uint64_t a, b;
                 in >> a >> b;

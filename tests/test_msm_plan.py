@@ -90,13 +90,28 @@ def test_default_target_is_the_groups_own_rule(plan_bin):
     """The lane setting's default, 19, gives each group its measured rule, so
     that setting it back restores the default; any other value is 2^value
     lanes whatever the number of entries."""
-    own = ask(plan_bin, ["lanes 0 19 0", "lanes 1 19 0"])
-    assert own == ["65536 131072 262144 393216 4194304 16777216 33554432 1",
-                   "65536 65536 131072 262144 524288 2097152 8388608 1"]
+    own = [line.split() for line in ask(plan_bin, ["lanes 0 19", "lanes 1 19"])]
+    assert own == ["65536 131072 262144 393216 4194304 16777216 33554432".split(),
+                   "65536 65536 131072 262144 524288 2097152 8388608".split()]
     for target in (10, 12, 18, 20, 22, 24):
-        for line in ask(plan_bin, [f"lanes 0 {target} 5", f"lanes 1 {target} 5"]):
-            words = line.split()
-            assert words[:4] == [str(1 << target)] * 4 and words[-1] == "5"
+        for line in ask(plan_bin, [f"lanes 0 {target}", f"lanes 1 {target}"]):
+            assert line.split()[:4] == [str(1 << target)] * 4
+
+
+def test_a_minimum_binds_its_own_job_only(plan_bin):
+    """Entries per lane of a launch, and of a job with a minimum (the witness
+    MSMs may have one, H, in the same launch, has none); never 0."""
+    rng = np.random.default_rng(3)
+    entries = [0, 1, 65535, 65536, 65537, (1 << 22) - 1, 1 << 22, 1 << 24, (1 << 25) - 1, 1 << 25, 1 << 34]
+    entries += [int(e) for e in 2 ** rng.uniform(0, 33, 20)]
+    lanes = {0: [(1 << 22, 1), (1 << 24, 2), (1 << 25, 4), (1 << 60, 6)],
+             1: [(1 << 21, 1), (1 << 23, 2), (1 << 60, 4)]}
+    for g2 in (0, 1):
+        for minimum in (1, 64):
+            got = list(map(int, ask(plan_bin, [f"piece {g2} 19 {minimum} " + " ".join(map(str, entries))])[0].split()))
+            for e, launch, job in zip(entries, got[::2], got[1::2]):
+                n = 65536 * next(k for below, k in lanes[g2] if e < below)
+                assert launch == max(1, -(-e // n)) and job == max(launch, minimum), (g2, minimum, e)
 
 
 def test_zero_divisors_raise_instead_of_crashing(plan_bin):
