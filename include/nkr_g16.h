@@ -93,7 +93,9 @@ int nkr_g16_ctx_create(const nkr_g16_circuit *circuit, const nkr_g16_pk *pk, int
  * them per (domain size, witness density) by measurement.  No counterpart in
  * the reference (its window and stage choices are fixed,
  * operators/hip/include/msm/msm.hip:25-60).
- *   witness_window_bits  MSM window of the witness MSMs, 2..15
+ *   witness_window_bits  MSM window of the MSMs over all witness columns, 2..15
+ *                          (bs1 and bs2 choose their own where few of the
+ *                          columns occur in B)
  *   h_window_bits        MSM window of the H MSM, 2..16
  *   ntt_lds_log          10 or 11: 2^lds_log elements per transform tile
  *   ntt_radix_log        2 or 3: register radix of the transform rounds

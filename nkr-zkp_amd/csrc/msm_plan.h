@@ -141,6 +141,25 @@ struct MsmPlan {
     }
 };
 
+// The plan of the witness's MSMs over n columns: at most 15 bits, whose
+// schedule is built beside the transforms.
+inline MsmPlan msm_witness_plan(uint32_t n, uint32_t c_override = 0)
+{
+    const MsmPlan p = MsmPlan::choose(n, c_override);
+    return p.c > 15 ? MsmPlan::choose(n, 15) : p;
+}
+
+// The plan of bs1 and bs2 when `finite` of the witness's columns have a finite
+// point: the witness's own, or, where at least a quarter of the columns go, one
+// for the columns that stay.  A width the caller asked for was for all of the
+// columns; these may be a hundredth of them.
+inline MsmPlan msm_b_plan(const MsmPlan &witness, uint32_t finite)
+{
+    const uint32_t n = std::max(1u, finite);  // an MSM has at least one term
+    if (n == witness.n || n > witness.n - witness.n / 4) return witness;
+    return msm_witness_plan(n);
+}
+
 // Partial sums one job needs room for: the level-0 pieces, then each fold
 // level's worst case (a level keeps at most a quarter of the previous one,
 // plus one rounded-up group per bucket).  levels receives the fold levels

@@ -126,8 +126,7 @@ Groth16Prover::Groth16Prover(const nkr_g16_circuit &c, const nkr_g16_pk &pk, int
     domain_ = std::make_unique<NttDomain>(log_n_, stream_, &shape);
     // The witness schedule is sorted on the side stream beside the transforms:
     // at most 15-bit windows, whose 64 KiB histograms share a CU with them.
-    wplan_ = MsmPlan::choose(cols_, tn.witness_window_bits);
-    if (wplan_.c > 15) wplan_ = MsmPlan::choose(cols_, 15);
+    wplan_ = msm_witness_plan(cols_, tn.witness_window_bits);
     hplan_ = MsmPlan::choose(rows_, tn.h_window_bits);
     if (tn.msm_target_pieces_log) {
         batch_g1_.set_lanes(msm_lanes(false, tn.msm_target_pieces_log));
@@ -154,13 +153,8 @@ Groth16Prover::Groth16Prover(const nkr_g16_circuit &c, const nkr_g16_pk &pk, int
             std::vector<uint32_t> terms;
             msm_finite_terms(tmp1.get(), tmp2.get(), cols_, terms, stream_);
             if (terms.empty()) terms.push_back(0);  // an MSM has at least one term
-            bplan_ = wplan_;
-            if (terms.size() <= cols_ - cols_ / 4) {
-                const uint32_t n = (uint32_t)terms.size();
-                bplan_ = MsmPlan::choose(n, tn.witness_window_bits);
-                if (bplan_.c > 15) bplan_ = MsmPlan::choose(n, 15);
-                upload(b_terms_, terms.data(), terms.size(), stream_);
-            }
+            bplan_ = msm_b_plan(wplan_, (uint32_t)terms.size());
+            if (bplan_.n != cols_) upload(b_terms_, terms.data(), terms.size(), stream_);
             b1_.prepare(tmp1.get(), b_terms_.get(), bplan_, stream_);
             b2_.prepare(tmp2.get(), b_terms_.get(), bplan_, stream_);
             NKR_HIP(hipStreamSynchronize(stream_));

@@ -6,6 +6,7 @@
 //   lanes g2 target_log   -> the lane rule: 4 lane counts, 3 limits
 //   piece g2 target_log piece_min entries... -> per entry count, the launch's
 //                            entries per lane and those of a job with that minimum
+//   bplan cols c_override finite -> "n c" of bs1 and bs2
 //   divup a b             -> ceil(a / b) or "error <message>"
 // Errors are reported, never turned into a crash: a zero divisor must raise
 // nkr::Error instead of ending the process with SIGFPE.
@@ -56,6 +57,11 @@ int main()
                 const MsmLanes r = msm_lanes_of(g2 != 0, (uint32_t)tl);
                 while (in >> e) std::printf("%u %u ", msm_piece(r, e), msm_job_piece(msm_piece(r, e), (uint32_t)pm));
                 std::printf("\n");
+            } else if (op == "bplan") {
+                uint64_t cols, c, finite;
+                in >> cols >> c >> finite;
+                const MsmPlan p = msm_b_plan(msm_witness_plan((uint32_t)cols, (uint32_t)c), (uint32_t)finite);
+                std::printf("%u %u\n", p.n, p.c);
             } else if (op == "divup") {
                 uint64_t a, b;
                 in >> a >> b;

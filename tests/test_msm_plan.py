@@ -114,6 +114,29 @@ def test_a_minimum_binds_its_own_job_only(plan_bin):
                 assert launch == max(1, -(-e // n)) and job == max(launch, minimum), (g2, minimum, e)
 
 
+def test_b_query_plan(plan_bin):
+    """bs1 and bs2 use the witness's plan while more than three quarters of the
+    columns are finite, else their own width for what is left, whatever width
+    the witness was given."""
+    n = 1 << 17
+    out = ask(plan_bin, [f"bplan {n} {c} {f}" for c in (0, 13) for f in (n, n - n // 4 + 1, n - n // 4, 1300, 1, 0)]
+              + [f"plan {k} 0 19 4 64" for k in (n, n - n // 4, 1300, 1)])
+    own = [int(line.split()[0]) for line in out[12:]]
+    for c, got in ((own[0], out[:6]), (13, out[6:12])):
+        assert [tuple(map(int, g.split())) for g in got] == \
+            [(n, c), (n, c), (n - n // 4, own[1]), (1300, own[2]), (1, own[3]), (1, own[3])]
+    assert own[2] <= 10
+    # a plan of its own always has fewer terms
+    for cols in (1, 2, 3, 4, 5):
+        for f in range(cols + 1):
+            got, plan = ask(plan_bin, [f"bplan {cols} 9 {f}", f"plan {max(1, f)} 0 19 4 64"])
+            same = max(1, f) == cols or f > cols - cols // 4
+            assert got.split() == ([str(cols), "9"] if same else [str(max(1, f)), plan.split()[0]]), (cols, f)
+    # the witness itself stays at 15 bits
+    assert ask(plan_bin, [f"bplan {1 << 21} 0 {1 << 21}", f"bplan {1 << 22} 0 {1 << 21}"]) == \
+        [f"{1 << 21} 15", f"{1 << 21} 15"]
+
+
 def test_zero_divisors_raise_instead_of_crashing(plan_bin):
     out = ask(plan_bin, ["plan 1024 0 19 0 64", "plan 1024 0 19 8 4", "divup 10 0", "divup 10 3",
                          "plan 0 0 19 4 64", "plan 1024 17 19 4 64"])
