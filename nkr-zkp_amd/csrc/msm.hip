@@ -29,21 +29,13 @@ constexpr uint32_t kTreeThreads = 256;
 // Completion classes: 1, 2, 4, 8 or 16 lane groups per bucket (G2: up to 8,
 // the groups of one wave).
 constexpr uint32_t kCompleteClasses = 5;
-// Partial sums one wave folds into one: three 4:1 levels at once.
-constexpr uint32_t kFoldLevelsPerLaunch = 3;
-constexpr uint32_t kFoldSpan = 64;
-static_assert(kFoldSpan == kMsmFoldIn * kMsmFoldIn * kMsmFoldIn && kFoldSpan <= kMsmCompleteMax, "fold span");
-// Partials of a bucket that are completed without a fold: 8 lane groups sum
-// this many in fewer additions of latency than a fold and a completion.
-constexpr uint32_t kDirectMax = 128;
 constexpr uint32_t kPlanThreads = 1024;
-constexpr uint32_t kMaxFoldLaunches = kMaxFoldLevels / kFoldLevelsPerLaunch;
 // Lane groups of an addition per wave (coop29.h).
 template <class F>
 constexpr uint32_t kWaveGroups = 64 / Coop<F>::kLanes;
 
 // One bucket to fold at one level: its partials at pool[src .. src + cnt)
-// become ceil(cnt / kFoldSpan) sums, the level's outputs `start` ...
+// become ceil(cnt / kMsmFoldSpan) sums, the level's outputs `start` ...
 struct FoldRec {
     uint32_t start, src, cnt;
 };
@@ -53,8 +45,8 @@ struct FoldRec {
 struct ReduceState {
     uint32_t ticket;
     uint32_t piece;  // entries per accumulation lane (msm_piece)
-    unsigned long long fold_ctr[kMaxFoldLaunches];  // records << 32 | outputs
-    unsigned long long fold_count[kMaxFoldLaunches];
+    unsigned long long fold_ctr[kMsmMaxFoldLaunches];  // records << 32 | outputs
+    unsigned long long fold_count[kMsmMaxFoldLaunches];
 };
 
 template <class F>
@@ -338,8 +330,8 @@ __device__ __forceinline__ uint32_t job_lanes(const JobDev<F> &jb, uint32_t laun
 //     (b - 1) / L, and lane l's partial of bucket k is number l + k of the job
 //     (two lanes share a bucket, or one lane two buckets, never both), at
 //     lanes and buckets of the jobs before it in the pool;
-//   * a bucket with more than kDirectMax partials gets a fold record per
-//     level that brings it below (kFoldSpan : 1 each); any bucket's final
+//   * a bucket with more than kMsmDirectMax partials gets a fold record per
+//     level that brings it below (kMsmFoldSpan : 1 each); any bucket's final
 //     partials become reg_start / reg_count;
 //   * completion classes: a bucket with m partials is completed by 2^c lane
 //     groups, the smallest c with m <= serial << c.  With the partials spread
@@ -384,8 +376,8 @@ __global__ __launch_bounds__(kPlanThreads) void k_reduce_plan(const JobDev<F> *_
         const uint32_t beg = jb.bucket_start[k], end = jb.bucket_start[k + 1];
         uint32_t src = lanes_before + jb.b_off + beg / piece + k;
         if (beg < end) m = (end - 1) / piece - beg / piece + 1;
-        for (uint32_t L = 0; m > kDirectMax; ++L) {
-            const uint32_t n = (m + kFoldSpan - 1) / kFoldSpan;
+        for (uint32_t L = 0; msm_folds(m); ++L) {
+            const uint32_t n = (uint32_t)msm_folded(m);
             const unsigned long long at = atomicAdd(&st->fold_ctr[L], (1ull << 32) | n);
             const uint32_t start = (uint32_t)at;
             recs[(size_t)L * rec_cap + (uint32_t)(at >> 32)] = FoldRec{start, src, m};
@@ -442,7 +434,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_reduce_plan(const JobDev<F> *_
         seg_count[s] = n;
         return ((n * Coop<F>::kLanes << (s % kCompleteClasses)) + 63u) & ~63u;
     });
-    if (threadIdx.x < kMaxFoldLaunches) st->fold_count[threadIdx.x] = atomicExch(&st->fold_ctr[threadIdx.x], 0ull);
+    if (threadIdx.x < kMsmMaxFoldLaunches) st->fold_count[threadIdx.x] = atomicExch(&st->fold_ctr[threadIdx.x], 0ull);
 }
 
 // The G2 accumulator of one lane with X and ZZ in registers and Y and ZZZ in
@@ -777,7 +769,7 @@ __device__ __forceinline__ Coop<F> coop_sum(const partial_t<F> *__restrict__ poo
     return acc;
 }
 
-// Fold launch L: a wave sums up to kFoldSpan partials of one record into one
+// Fold launch L: a wave sums up to kMsmFoldSpan partials of one record into one
 // output; 7 (G1) or 10 (G2) additions deep.
 template <class F>
 __global__ __launch_bounds__(256) void k_fold(const ReduceState *__restrict__ st, const FoldRec *__restrict__ recs,
@@ -798,8 +790,8 @@ __global__ __launch_bounds__(256) void k_fold(const ReduceState *__restrict__ st
                 hi = mid;
         }
         const FoldRec r = recs[lo];
-        const uint32_t off = (t - r.start) * kFoldSpan;
-        const uint32_t cnt = min(kFoldSpan, r.cnt - off);
+        const uint32_t off = (t - r.start) * kMsmFoldSpan;
+        const uint32_t cnt = min(kMsmFoldSpan, r.cnt - off);
         const Coop<F> acc =
             coop_reduce(coop_sum<F>(pool, r.src + off, cnt, group, kWaveGroups<F>), kWaveGroups<F>);
         if (group == 0) coop_store<F>(pool, (size_t)out_base + t, acc);
@@ -979,7 +971,7 @@ uint64_t msm_schedule_bytes(const MsmPlan &p)
 }
 
 // Partial sums of all fold launches: a launch turns more than kMsmCompleteMax
-// partials of a bucket into ceil(m / kFoldSpan), fewer than m / 32.
+// partials of a bucket into ceil(m / kMsmFoldSpan), fewer than m / 32.
 static uint64_t fold_outputs(uint64_t partials) { return partials / 32 + 1; }
 // Fold records of one launch: buckets with more than kMsmCompleteMax partials.
 static uint64_t fold_records(uint64_t partials) { return partials / (kMsmCompleteMax + 1) + 1; }
@@ -994,7 +986,7 @@ uint64_t msm_job_bytes(const MsmPlan &p)
     // offsets)
     return msm_partial_capacity(p, partials, nullptr, nullptr) * sizeof(partial_t<F>) +
            (uint64_t)p.B * (3 * sizeof(partial_t<F>) + 8 + 4 * kCompleteClasses) +
-           fold_records(partials) * kMaxFoldLaunches * sizeof(FoldRec) + p.c * sizeof(Xyzz<F>) + 1024;
+           fold_records(partials) * kMsmMaxFoldLaunches * sizeof(FoldRec) + p.c * sizeof(Xyzz<F>) + 1024;
 }
 
 void msm_finite_terms(const g1_jac *a, const g2_jac *b, uint32_t n, std::vector<uint32_t> &terms, hipStream_t stream)
@@ -1156,9 +1148,11 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
         b_off[j + 1] = b_off[j] + p.B;
     }
     lane_bound_ = std::min(entries, max_lanes) + J;
-    fold_levels_ = msm_fold_levels(std::min(entries, max_lanes) + 1);
+    // a bucket has at most a partial per lane of its job
+    fold_launches_ = msm_fold_launches(std::min(entries, max_lanes) + 1);
+    NKR_REQUIRE(fold_launches_ <= kMsmMaxFoldLaunches, "MSM launch with too many lanes to fold");
     uint64_t at = lane_bound_ + b_off[J], outs = at;
-    for (uint32_t L = 0; L < kMaxFoldLaunches; ++L) {
+    for (uint32_t L = 0; L < kMsmMaxFoldLaunches; ++L) {
         fold_base_[L] = (uint32_t)at;
         outs = fold_outputs(outs);
         fold_cap_[L] = outs;
@@ -1207,7 +1201,7 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
     seg_count_.ensure(kCompleteClasses * J);
     class_count_.ensure(kCompleteClasses * J);
     class_list_.ensure(kCompleteClasses * b_off[J]);
-    recs_.ensure(rec_cap_ * kMaxFoldLaunches * sizeof(FoldRec));
+    recs_.ensure(rec_cap_ * kMsmMaxFoldLaunches * sizeof(FoldRec));
     state_.ensure(sizeof(ReduceState));
     jobs_dev_.ensure(table_bytes);
     lane_base_.ensure(J + 1);  // filled on the device per run
@@ -1268,9 +1262,9 @@ void MsmBatch<F>::run(const std::vector<MsmJob<F>> &jobs, hipStream_t stream, St
         timer->begin(kStageFold, stream);
     }
     // as many fold launches as one bucket with every lane's partial would
-    // need (2, or 3 beyond 2^18 lanes): an empty one costs less than the
-    // host's wait for the largest count
-    for (uint32_t L = 0; L * kFoldLevelsPerLaunch < fold_levels_; ++L) {
+    // need (2 from 8193 lanes to 2^19): an empty one costs less than the host's
+    // wait for the largest count
+    for (uint32_t L = 0; L < fold_launches_; ++L) {
         const uint64_t blocks = std::min<uint64_t>(div_up(fold_cap_[L], 4), 1024);
         k_fold<F><<<(uint32_t)blocks, 256, 0, stream>>>(state, recs + (size_t)L * rec_cap_, L, fold_base_[L],
                                                       pool_.get());

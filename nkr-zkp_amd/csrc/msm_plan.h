@@ -72,6 +72,23 @@ constexpr uint32_t msm_job_piece(uint32_t piece, uint32_t piece_min) { return pi
 // counts in one workgroup's LDS (128 KiB of gfx950's 160 KiB).
 constexpr uint32_t kMsmMaxBuckets = 1u << 15;
 
+// Folds: a launch turns the partial sums of every bucket that has more than
+// kMsmDirectMax into one per kMsmFoldSpan.  8 lane groups complete kMsmDirectMax
+// in fewer additions of latency than a fold and a completion take.
+constexpr uint32_t kMsmFoldSpan = 64;
+constexpr uint32_t kMsmDirectMax = 128;
+constexpr uint32_t kMsmMaxFoldLaunches = 4;
+constexpr bool msm_folds(uint64_t partials) { return partials > kMsmDirectMax; }
+constexpr uint64_t msm_folded(uint64_t partials) { return (partials + kMsmFoldSpan - 1) / kMsmFoldSpan; }
+// Fold launches for buckets of at most `partials` partial sums.
+constexpr uint32_t msm_fold_launches(uint64_t partials)
+{
+    uint32_t launches = 0;
+    for (; msm_folds(partials); partials = msm_folded(partials)) ++launches;
+    return launches;
+}
+static_assert(msm_fold_launches((1ull << 24) + 1) <= kMsmMaxFoldLaunches, "the most lanes a launch may have");
+
 // Fold levels (4:1 each) that bring `partials` partial sums of one bucket
 // down to at most kMsmCompleteMax; 0 for an empty or short bucket.
 inline uint32_t msm_fold_levels(uint64_t partials)

@@ -7,6 +7,7 @@
 //   piece g2 target_log piece_min entries... -> per entry count, the launch's
 //                            entries per lane and those of a job with that minimum
 //   bplan cols c_override finite -> "n c" of bs1 and bs2
+//   launches partials     -> fold launches for buckets of at most that many
 //   divup a b             -> ceil(a / b) or "error <message>"
 // Errors are reported, never turned into a crash: a zero divisor must raise
 // nkr::Error instead of ending the process with SIGFPE.
@@ -62,6 +63,10 @@ int main()
                 in >> cols >> c >> finite;
                 const MsmPlan p = msm_b_plan(msm_witness_plan((uint32_t)cols, (uint32_t)c), (uint32_t)finite);
                 std::printf("%u %u\n", p.n, p.c);
+            } else if (op == "launches") {
+                uint64_t k;
+                in >> k;
+                std::printf("%u\n", msm_fold_launches(k));
             } else if (op == "divup") {
                 uint64_t a, b;
                 in >> a >> b;

@@ -137,6 +137,23 @@ def test_b_query_plan(plan_bin):
         [f"{1 << 21} 15", f"{1 << 21} 15"]
 
 
+def test_fold_launches_are_what_the_plan_uses(plan_bin):
+    """The launches issued are those the planning kernel's own fold loop (64:1
+    while a bucket has more than 128 partial sums) can fill, for the largest
+    bucket each lane count allows: two for the default lanes, never an empty
+    third."""
+    def loop(m):
+        n = 0
+        while m > 128:
+            m, n = -(-m // 64), n + 1
+        return n
+    ms = [0, 1, 128, 129, 8192, 8193, (1 << 19), (1 << 19) + 1, (1 << 24) + 1] + \
+        [lanes + 1 for lanes in (65536, 131072, 262144, 393216)]
+    got = list(map(int, ask(plan_bin, [f"launches {m}" for m in ms])))
+    assert got == [loop(m) for m in ms]
+    assert got == [0, 0, 0, 1, 1, 2, 2, 3, 3, 2, 2, 2, 2]
+
+
 def test_zero_divisors_raise_instead_of_crashing(plan_bin):
     out = ask(plan_bin, ["plan 1024 0 19 0 64", "plan 1024 0 19 8 4", "divup 10 0", "divup 10 3",
                          "plan 0 0 19 4 64", "plan 1024 17 19 4 64"])
