@@ -229,15 +229,9 @@ private:
     MsmLanes wanted_lanes() const { return have_lanes_ ? own_lanes_ : msm_lanes(std::is_same<F, fq2_t>::value); }
     void layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream);
     std::vector<const void *> key_;
-    uint32_t fold_launches_ = 0;  // what the largest possible bucket needs
-    uint32_t fold_base_[kMsmMaxFoldLaunches] = {};  // where each fold launch's outputs start in pool_
-    uint64_t fold_cap_[kMsmMaxFoldLaunches] = {};   // and their largest number
-    uint64_t rec_cap_ = 0;                         // fold records of one launch at most
-    uint64_t lane_bound_ = 0;                      // accumulation lanes of all jobs at most
-    uint64_t bucket_total_ = 0;                    // buckets of all jobs
+    MsmSizes sizes_;                 // as of the layout
     MsmLanes lanes_{}, own_lanes_{};               // lanes_: as of the layout
     bool have_lanes_ = false;
-    uint64_t complete_bound_ = 0;                  // completion lanes at most
     DeviceBuffer<uint32_t> seg_base_, seg_count_, class_count_, class_list_, lane_base_;
     DeviceBuffer<uint8_t> jobs_dev_, recs_, state_;
     PinnedStaging<uint8_t> jobs_stage_;

@@ -26,9 +26,6 @@ constexpr uint32_t kScanGroups = 16;
 // LDS per tree workgroup (two buffers of 2^h blocks): two workgroups per CU.
 constexpr size_t kTreeLds = 64 * 1024;
 constexpr uint32_t kTreeThreads = 256;
-// Completion classes: 1, 2, 4, 8 or 16 lane groups per bucket (G2: up to 8,
-// the groups of one wave).
-constexpr uint32_t kCompleteClasses = 5;
 constexpr uint32_t kPlanThreads = 1024;
 // Lane groups of an addition per wave (coop29.h).
 template <class F>
@@ -341,7 +338,7 @@ __device__ __forceinline__ uint32_t job_lanes(const JobDev<F> &jb, uint32_t laun
 //     take several.  An empty bucket's sum is infinity;
 //   * the last workgroup to finish turns the counts into offsets:
 //     lane_base[j] = accumulation lanes of the jobs before j, seg_base[s] =
-//     lanes of the completion segments before s = kCompleteClasses * j + c,
+//     lanes of the completion segments before s = kMsmCompleteClasses * j + c,
 //     each padded to whole waves, and clears the counters for the next launch.
 template <class F>
 __global__ __launch_bounds__(kPlanThreads) void k_reduce_plan(const JobDev<F> *__restrict__ jobs, uint32_t J,
@@ -390,31 +387,31 @@ __global__ __launch_bounds__(kPlanThreads) void k_reduce_plan(const JobDev<F> *_
     }
     // one atomic per workgroup and class: ballots rank the lanes of a wave, and
     // the waves' counts are scanned in LDS
-    __shared__ uint32_t count[kCompleteClasses][kPlanThreads / 64], list_at[kCompleteClasses];
+    __shared__ uint32_t count[kMsmCompleteClasses][kPlanThreads / 64], list_at[kMsmCompleteClasses];
     constexpr uint32_t groups = 65536 / Coop<F>::kLanes;
     const uint32_t serial = 1 + (uint32_t)(3 * (entries / launch_piece + buckets) / (2 * groups));
     uint32_t c = 0;
     while (c < max_class && (serial << c) < m) ++c;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     uint32_t rank = 0;
-    for (uint32_t cc = 0; cc < kCompleteClasses; ++cc) {
+    for (uint32_t cc = 0; cc < kMsmCompleteClasses; ++cc) {
         const uint64_t mask = __ballot(m > 0 && c == cc);
         if (c == cc) rank = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
         if (lane == 0) count[cc][wave] = (uint32_t)__popcll(mask);
     }
     __syncthreads();
-    if (threadIdx.x < kCompleteClasses) {
+    if (threadIdx.x < kMsmCompleteClasses) {
         uint32_t sum = 0;
         for (uint32_t w = 0; w < waves; ++w) {
             const uint32_t n = count[threadIdx.x][w];
             count[threadIdx.x][w] = sum;
             sum += n;
         }
-        if (sum) list_at[threadIdx.x] = atomicAdd(&class_count[kCompleteClasses * j + threadIdx.x], sum);
+        if (sum) list_at[threadIdx.x] = atomicAdd(&class_count[kMsmCompleteClasses * j + threadIdx.x], sum);
     }
     __syncthreads();
     if (m > 0)
-        class_list[((size_t)jb.b_off * kCompleteClasses + (size_t)c * jb.B) + list_at[c] + count[c][wave] + rank] = k;
+        class_list[((size_t)jb.b_off * kMsmCompleteClasses + (size_t)c * jb.B) + list_at[c] + count[c][wave] + rank] = k;
 
     // The last workgroup reads what the others left in the counters, which are
     // only touched by atomics; each of its own has returned here.
@@ -429,10 +426,10 @@ __global__ __launch_bounds__(kPlanThreads) void k_reduce_plan(const JobDev<F> *_
     if (!last) return;
     if (threadIdx.x == 0) st->piece = launch_piece;
     group_prefix(J, lane_base, [&](uint32_t i) { return job_lanes(jobs[i], launch_piece); });
-    group_prefix(kCompleteClasses * J, seg_base, [&](uint32_t s) {
+    group_prefix(kMsmCompleteClasses * J, seg_base, [&](uint32_t s) {
         const uint32_t n = atomicExch(&class_count[s], 0u);
         seg_count[s] = n;
-        return ((n * Coop<F>::kLanes << (s % kCompleteClasses)) + 63u) & ~63u;
+        return ((n * Coop<F>::kLanes << (s % kMsmCompleteClasses)) + 63u) & ~63u;
     });
     if (threadIdx.x < kMsmMaxFoldLaunches) st->fold_count[threadIdx.x] = atomicExch(&st->fold_ctr[threadIdx.x], 0ull);
 }
@@ -811,13 +808,13 @@ __global__ __launch_bounds__(256) void k_complete(const JobDev<F> *__restrict__ 
 #pragma unroll 1
     for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < total; g += gridDim.x * blockDim.x) {
         const uint32_t s = find_segment(seg_base, S, g);
-        const uint32_t j = s / kCompleteClasses, c = s % kCompleteClasses;
+        const uint32_t j = s / kMsmCompleteClasses, c = s % kMsmCompleteClasses;
         const JobDev<F> &jb = jobs[j];
         const uint32_t local = (g - seg_base[s]) / Coop<F>::kLanes;
         const uint32_t idx = local >> c, group = local & ((1u << c) - 1u);
         const bool live = idx < seg_count[s];
         const uint32_t k =
-            live ? class_list[(size_t)jb.b_off * kCompleteClasses + (size_t)c * jb.B + idx] : 0u;
+            live ? class_list[(size_t)jb.b_off * kMsmCompleteClasses + (size_t)c * jb.B + idx] : 0u;
         Coop<F> acc = coop_sum<F>(pool, live ? jb.reg_start[k] : 0u, live ? jb.reg_count[k] : 0u, group, 1u << c);
         acc = coop_reduce(acc, 1u << c);
         if (live && group == 0) coop_store<F>(jb.sums, k, acc);
@@ -970,9 +967,6 @@ uint64_t msm_schedule_bytes(const MsmPlan &p)
     return p.max_entries() * 4 + (uint64_t)p.B * 4 * 2 + blocks * p.B * 4 + 32;
 }
 
-// Partial sums of all fold launches: a launch turns more than kMsmCompleteMax
-// partials of a bucket into ceil(m / kMsmFoldSpan), fewer than m / 32.
-static uint64_t fold_outputs(uint64_t partials) { return partials / 32 + 1; }
 // Fold records of one launch: buckets with more than kMsmCompleteMax partials.
 static uint64_t fold_records(uint64_t partials) { return partials / (kMsmCompleteMax + 1) + 1; }
 
@@ -985,7 +979,7 @@ uint64_t msm_job_bytes(const MsmPlan &p)
     // bit planes; and the job's fixed records (job table, class counters, lane
     // offsets)
     return msm_partial_capacity(p, partials, nullptr, nullptr) * sizeof(partial_t<F>) +
-           (uint64_t)p.B * (3 * sizeof(partial_t<F>) + 8 + 4 * kCompleteClasses) +
+           (uint64_t)p.B * (3 * sizeof(partial_t<F>) + 8 + 4 * kMsmCompleteClasses) +
            fold_records(partials) * kMsmMaxFoldLaunches * sizeof(FoldRec) + p.c * sizeof(Xyzz<F>) + 1024;
 }
 
@@ -1135,11 +1129,9 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
     key_.clear();  // until the new layout is whole
     lanes_ = wanted_lanes();
     const uint32_t J = (uint32_t)jobs.size();
-    // The pool: a partial per lane and bucket of the launch (k_reduce_plan),
-    // then the fold launches' outputs of all jobs; and the per-bucket arrays.
+    // where each job's buckets lie in the per-bucket arrays
     std::vector<uint64_t> b_off(J + 1, 0);
     uint64_t entries = 0;
-    const uint64_t max_lanes = *std::max_element(lanes_.lanes, lanes_.lanes + 4);
     for (uint32_t j = 0; j < J; ++j) {
         const MsmPlan &p = jobs[j].sched->plan();
         NKR_REQUIRE(jobs[j].bases->plan().n == p.n && jobs[j].bases->plan().c == p.c,
@@ -1147,22 +1139,13 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
         entries += p.max_entries();
         b_off[j + 1] = b_off[j] + p.B;
     }
-    lane_bound_ = std::min(entries, max_lanes) + J;
-    // a bucket has at most a partial per lane of its job
-    fold_launches_ = msm_fold_launches(std::min(entries, max_lanes) + 1);
-    NKR_REQUIRE(fold_launches_ <= kMsmMaxFoldLaunches, "MSM launch with too many lanes to fold");
-    uint64_t at = lane_bound_ + b_off[J], outs = at;
-    for (uint32_t L = 0; L < kMsmMaxFoldLaunches; ++L) {
-        fold_base_[L] = (uint32_t)at;
-        outs = fold_outputs(outs);
-        fold_cap_[L] = outs;
-        at += outs;
-    }
-    NKR_REQUIRE(at < (1ull << 32), "MSM partial pool exceeds 32-bit indexing");
-    bucket_total_ = b_off[J];
-    rec_cap_ = fold_records(lane_bound_ + bucket_total_);
+    sizes_ = msm_sizes(J, entries, b_off[J], msm_launch_lanes(lanes_, entries));
+    NKR_REQUIRE(sizes_.pool < (1ull << 32), "MSM partial pool exceeds 32-bit indexing");
+    NKR_REQUIRE(sizes_.complete_lanes < (1ull << 32), "MSM batch too large for 32-bit work indices");
+    uint32_t fold_base[kMsmMaxFoldLaunches];
+    for (uint32_t L = 0; L < kMsmMaxFoldLaunches; ++L) fold_base[L] = (uint32_t)sizes_.fold_base[L];
     // grow-only: a batch whose composition changes from call to call reuses them
-    pool_.ensure(at);
+    pool_.ensure(sizes_.pool);
     sums_.ensure(b_off[J]);
     tree_[0].ensure(b_off[J]);
     tree_[1].ensure(b_off[J]);
@@ -1171,7 +1154,7 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
 
     static_assert(std::is_trivially_copyable<JobDev<F>>::value, "job records are raw-copied");
     const size_t jobs_bytes = (sizeof(JobDev<F>) * J + 15) & ~size_t(15);
-    const size_t table_bytes = jobs_bytes + sizeof(fold_base_);
+    const size_t table_bytes = jobs_bytes + sizeof(fold_base);
     uint8_t *st = jobs_stage_.reuse(table_bytes);
     JobDev<F> *host = reinterpret_cast<JobDev<F> *>(st);
     for (uint32_t j = 0; j < J; ++j) {
@@ -1191,17 +1174,12 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
         d.b_off = (uint32_t)b_off[j];
         d.piece_min = std::max(1u, jb.piece_min);
     }
-    std::memcpy(st + jobs_bytes, fold_base_, sizeof(fold_base_));
-    // completion lanes: a bucket's lane groups, plus each segment's padding
-    complete_bound_ = 0;
-    for (uint32_t j = 0; j < J; ++j)
-        complete_bound_ += (uint64_t)host[j].B * 64 + kCompleteClasses * 64;
-    NKR_REQUIRE(complete_bound_ < (1ull << 32), "MSM batch too large for 32-bit work indices");
-    seg_base_.ensure(kCompleteClasses * J + 1);
-    seg_count_.ensure(kCompleteClasses * J);
-    class_count_.ensure(kCompleteClasses * J);
-    class_list_.ensure(kCompleteClasses * b_off[J]);
-    recs_.ensure(rec_cap_ * kMsmMaxFoldLaunches * sizeof(FoldRec));
+    std::memcpy(st + jobs_bytes, fold_base, sizeof(fold_base));
+    seg_base_.ensure(kMsmCompleteClasses * J + 1);
+    seg_count_.ensure(kMsmCompleteClasses * J);
+    class_count_.ensure(kMsmCompleteClasses * J);
+    class_list_.ensure(kMsmCompleteClasses * b_off[J]);
+    recs_.ensure(sizes_.records * kMsmMaxFoldLaunches * sizeof(FoldRec));
     state_.ensure(sizeof(ReduceState));
     jobs_dev_.ensure(table_bytes);
     lane_base_.ensure(J + 1);  // filled on the device per run
@@ -1245,16 +1223,16 @@ void MsmBatch<F>::run(const std::vector<MsmJob<F>> &jobs, hipStream_t stream, St
 
     uint32_t max_class = 0;
     while ((2u << max_class) <= std::min(msm_complete_lanes_cap(), kWaveGroups<F>)) ++max_class;
-    const uint32_t S = kCompleteClasses * J;
+    const uint32_t S = kMsmCompleteClasses * J;
     const uint32_t plan_threads = std::min<uint32_t>(kPlanThreads, std::max<uint32_t>(256, (Bmax + 63) & ~63u));
     k_reduce_plan<F><<<dim3(div_up(Bmax, plan_threads), J), plan_threads, 0, stream>>>(
-        jd, J, lanes_, (uint32_t)bucket_total_, max_class, state, recs, (uint32_t)rec_cap_, fold_base_dev, class_count_.get(),
+        jd, J, lanes_, (uint32_t)sizes_.buckets, max_class, state, recs, (uint32_t)sizes_.records, fold_base_dev, class_count_.get(),
         class_list_.get(), lane_base_.get(), seg_count_.get(), seg_base_.get());
     NKR_LAUNCH_CHECK();
     // the accumulation stage brackets exactly the k_accumulate launch
     const int acc_stage = std::is_same<F, fq2_t>::value ? kStageAccumulateG2 : kStageAccumulate;
     if (timer) timer->begin(acc_stage, stream);
-    k_accumulate<F><<<(uint32_t)div_up(lane_bound_, kAccThreads), kAccThreads, 0, stream>>>(
+    k_accumulate<F><<<(uint32_t)div_up(sizes_.lanes, kAccThreads), kAccThreads, 0, stream>>>(
         jd, lane_base_.get(), J, state, pool_.get());
     NKR_LAUNCH_CHECK();
     if (timer) {
@@ -1264,14 +1242,14 @@ void MsmBatch<F>::run(const std::vector<MsmJob<F>> &jobs, hipStream_t stream, St
     // as many fold launches as one bucket with every lane's partial would
     // need (2 from 8193 lanes to 2^19): an empty one costs less than the host's
     // wait for the largest count
-    for (uint32_t L = 0; L < fold_launches_; ++L) {
-        const uint64_t blocks = std::min<uint64_t>(div_up(fold_cap_[L], 4), 1024);
-        k_fold<F><<<(uint32_t)blocks, 256, 0, stream>>>(state, recs + (size_t)L * rec_cap_, L, fold_base_[L],
+    for (uint32_t L = 0; L < sizes_.fold_launches; ++L) {
+        const uint64_t blocks = std::min<uint64_t>(div_up(sizes_.fold_cap[L], 4), 1024);
+        k_fold<F><<<(uint32_t)blocks, 256, 0, stream>>>(state, recs + (size_t)L * sizes_.records, L, (uint32_t)sizes_.fold_base[L],
                                                       pool_.get());
         NKR_LAUNCH_CHECK();
     }
     {
-        const uint64_t blocks = std::min<uint64_t>(div_up(complete_bound_, 256), resident_blocks<k_complete<F>>());
+        const uint64_t blocks = std::min<uint64_t>(div_up(sizes_.complete_lanes, 256), resident_blocks<k_complete<F>>());
         k_complete<F><<<(uint32_t)std::max<uint64_t>(blocks, 1), 256, 0, stream>>>(
             jd, pool_.get(), seg_count_.get(), class_list_.get(), seg_base_.get(), S);
     }

@@ -35,8 +35,15 @@ struct MsmLanes {
         return std::equal(lanes, lanes + 4, o.lanes) && std::equal(below, below + 3, o.below);
     }
 };
+// More entries never mean fewer lanes: a bound on the entries bounds the lanes.
+constexpr bool msm_lanes_ascend(const MsmLanes &r)
+{
+    return r.lanes[0] <= r.lanes[1] && r.lanes[1] <= r.lanes[2] && r.lanes[2] <= r.lanes[3] &&
+           r.below[0] <= r.below[1] && r.below[1] <= r.below[2];
+}
 constexpr MsmLanes kMsmLanesG1 = {{1u << 16, 2u << 16, 4u << 16, 6u << 16}, {1u << 22, 1u << 24, 1u << 25}};
 constexpr MsmLanes kMsmLanesG2 = {{1u << 16, 1u << 16, 2u << 16, 4u << 16}, {1u << 19, 1u << 21, 1u << 23}};
+static_assert(msm_lanes_ascend(kMsmLanesG1) && msm_lanes_ascend(kMsmLanesG2), "lane rule");
 constexpr uint32_t kMsmMaxLanesLog = 19;  // at least log2 of every lane count above
 // The default of the lane setting (2^target_log lanes for every launch): the
 // group's own lanes above.
@@ -88,6 +95,50 @@ constexpr uint32_t msm_fold_launches(uint64_t partials)
     return launches;
 }
 static_assert(msm_fold_launches((1ull << 24) + 1) <= kMsmMaxFoldLaunches, "the most lanes a launch may have");
+
+// Completion classes: 1, 2, 4, 8 or 16 lane groups per bucket (G2: up to 8, the
+// groups of one wave), at most 64 lanes.
+constexpr uint32_t kMsmCompleteClasses = 5;
+
+// What the device buffers of a batch of jobs hold at most: the lanes of its
+// accumulation, and from them the partial sums, the folds and the completion.
+struct MsmSizes {
+    uint64_t lanes = 0;    // accumulation lanes
+    uint64_t buckets = 0;  // of all jobs
+    uint32_t fold_launches = 0;
+    // the pool of partial sums: one per (lane, bucket) at slot lane + bucket,
+    // then each fold launch's outputs from fold_base on, fold_cap of them at most
+    uint64_t fold_base[kMsmMaxFoldLaunches] = {}, fold_cap[kMsmMaxFoldLaunches] = {};
+    uint64_t pool = 0;
+    uint64_t records = 0;         // fold records of one launch
+    uint64_t complete_lanes = 0;  // 64 per bucket, and each segment's padding
+};
+// For `jobs` jobs with `buckets` buckets and up to `entries` sorted entries in
+// all, of a launch of `launch_lanes`.  A job's last lane may be a short one, so
+// every job adds one; a bucket has at most a partial per lane of its job.
+inline MsmSizes msm_sizes(uint64_t jobs, uint64_t entries, uint64_t buckets, uint64_t launch_lanes)
+{
+    MsmSizes s;
+    const uint64_t job_lanes = std::min(entries, launch_lanes) + 1;
+    s.lanes = job_lanes - 1 + jobs;
+    s.buckets = buckets;
+    s.fold_launches = msm_fold_launches(job_lanes);
+    NKR_REQUIRE(s.fold_launches <= kMsmMaxFoldLaunches, "MSM launch with too many lanes to fold");
+    // a launch folds buckets of more than kMsmDirectMax partials, to fewer than
+    // a 32nd of them
+    const uint64_t partials = s.lanes + buckets;
+    uint64_t left = partials;
+    s.pool = partials;
+    for (uint32_t L = 0; L < kMsmMaxFoldLaunches; ++L) {
+        left = left / 32 + 1;
+        s.fold_base[L] = s.pool;
+        s.fold_cap[L] = left;
+        s.pool += left;
+    }
+    s.records = partials / (kMsmDirectMax + 1) + 1;
+    s.complete_lanes = (buckets + jobs * kMsmCompleteClasses) * 64;
+    return s;
+}
 
 // Fold levels (4:1 each) that bring `partials` partial sums of one bucket
 // down to at most kMsmCompleteMax; 0 for an empty or short bucket.

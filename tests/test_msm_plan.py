@@ -154,6 +154,72 @@ def test_fold_launches_are_what_the_plan_uses(plan_bin):
     assert got == [0, 0, 0, 1, 1, 2, 2, 3, 3, 2, 2, 2, 2]
 
 
+def spread(rng, shape, entries, B):
+    """Entries per bucket."""
+    if shape == "one":
+        counts = np.zeros(B, dtype=np.int64)
+        counts[rng.integers(B)] = entries
+    elif shape == "uniform":
+        counts = np.full(B, entries // B, dtype=np.int64)
+        counts[: entries % B] += 1
+    elif shape == "singles":
+        counts = np.zeros(B, dtype=np.int64)
+        counts[rng.permutation(B)[: min(B, entries)]] = 1
+    else:
+        counts = rng.multinomial(entries, rng.dirichlet(np.full(B, 0.02)))
+    return counts
+
+
+@pytest.mark.parametrize("g2,target", [(0, 19), (1, 19), (0, 10), (1, 12), (0, 22), (1, 24)])
+def test_buffer_bounds_cover_every_plan(plan_bin, g2, target):
+    """What the layout allocates (msm_sizes, from the most entries its jobs can
+    have) against the plan of a launch: every lane takes an equal run of its
+    job's entries, the partial of lane l and bucket k goes to slot l + k of the
+    job, and buckets of more than 128 partials are folded 64:1 launch by launch.
+    Distributions from one bucket to all, batches of one to five jobs, full and
+    nearly empty ones, at and around the lane rule's limits."""
+    rng = np.random.default_rng(100 * target + g2)
+    batches = [[(1, 8)], [(60000, 256)], [(1 << 21, 4096), (1 << 21, 4096), (9, 16), ((1 << 22) + 7, 1 << 15)],
+               [(1 << 19, 64)] * 5, [((1 << 25) + 1, 1 << 15), (3, 4)], [(5000, 2)] * 3]
+    for jobs in batches:
+        entries, buckets = sum(e for e, _ in jobs), sum(B for _, B in jobs)
+        for shape in ("one", "uniform", "singles", "skewed"):
+            for fill in (1.0, 0.37, 1e-4, 0.0):
+                counts = [spread(rng, shape, int(e * fill), B) for e, B in jobs]
+                E = sum(int(c.sum()) for c in counts)
+                sizes, piece = ask(plan_bin, [f"sizes {g2} {target} {len(jobs)} {entries} {buckets}",
+                                              f"piece {g2} {target} 1 {E}"])
+                lanes_cap, pool, rec_cap, complete, launches, *folds = map(int, sizes.split())
+                p = int(piece.split()[0])
+                base, cap = folds[::2], folds[1::2]
+                lanes_before = b_off = 0
+                ms = []
+                for c in counts:
+                    end = np.cumsum(c)
+                    beg, k = end - c, np.arange(c.size)
+                    first, last = beg // p, np.where(c > 0, (end - 1) // p, -1)
+                    used = c > 0
+                    # slots of one job: a bucket's come after the ones before it
+                    lo, hi = (first + k)[used], (last + k)[used]
+                    assert (lo[1:] > hi[:-1]).all()
+                    lanes = -(-int(end[-1]) // p)
+                    assert hi.size == 0 or hi[-1] < lanes + c.size
+                    assert (hi + lanes_before + b_off < lanes_cap + buckets).all()
+                    lanes_before, b_off = lanes_before + lanes, b_off + c.size
+                    ms.append(np.where(used, last - first + 1, 0))
+                assert lanes_before <= lanes_cap
+                m, issued = np.concatenate(ms), 0
+                while (m > 128).any():
+                    assert issued < launches <= 4
+                    folded = -(-m[m > 128] // 64)
+                    assert folded.size <= rec_cap and folded.sum() <= cap[issued]
+                    assert base[issued] >= lanes_cap + buckets and base[issued] + cap[issued] <= pool
+                    assert issued == 0 or base[issued] >= base[issued - 1] + cap[issued - 1]
+                    m = np.where(m > 128, -(-m // 64), m)
+                    issued += 1
+                assert buckets * 64 + 5 * 64 * len(jobs) == complete
+
+
 def test_zero_divisors_raise_instead_of_crashing(plan_bin):
     out = ask(plan_bin, ["plan 1024 0 19 0 64", "plan 1024 0 19 8 4", "divup 10 0", "divup 10 3",
                          "plan 0 0 19 4 64", "plan 1024 17 19 4 64"])
