@@ -61,11 +61,10 @@ uint32_t msm_complete_lanes_cap();
 // not replayed under another.
 uint64_t msm_shape_key();
 
-// Device bytes of one schedule (MsmSchedule) and of one MSM job's partial
-// sums and per-bucket arrays (MsmBatch) for a plan.
-uint64_t msm_schedule_bytes(const MsmPlan &plan);
+// Device bytes that a request's MSMs of one group add to the MsmBatch that runs
+// them with other requests' (msm_schedule_sizes has a schedule's).
 template <class F>
-uint64_t msm_job_bytes(const MsmPlan &plan);
+uint64_t msm_request_bytes(const std::vector<MsmPlan> &plans);
 
 // Window-shifted affine bases of one proving-key vector.
 template <class F>
@@ -102,9 +101,6 @@ public:
     const MsmPlan &plan() const { return plan_; }
     // Device counter: entries (non-zero digits).
     const uint32_t *totals() const { return bucket_start_.get() + plan_.B; }
-    // Sort workgroups for n scalars (each histograms a contiguous slice).
-    static uint32_t sort_blocks(uint32_t n);
-
     // Device bytes held, and their release (the next prepare reallocates).
     uint64_t device_bytes() const
     {

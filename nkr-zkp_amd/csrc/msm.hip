@@ -16,10 +16,6 @@ namespace nkr {
 namespace {
 
 constexpr uint32_t kEntryMask = 0x7fffffffu;
-// Sort workgroups: about one per CU, each histogramming a contiguous slice of
-// at least kSortMinPerBlock scalars with up to kSortThreads threads.
-constexpr uint32_t kSortBlocksTarget = 256;
-constexpr uint32_t kSortMinPerBlock = 256;
 constexpr uint32_t kSortThreads = 1024;
 // Column scan tile: 64 buckets x kScanGroups row groups per workgroup.
 constexpr uint32_t kScanGroups = 16;
@@ -956,31 +952,21 @@ MsmLanes msm_lanes(bool g2, uint32_t target_log)
 uint32_t msm_complete_lanes_cap() { return g_lanes_cap; }
 uint64_t msm_shape_key() { return (uint64_t)g_target_log << 32 | g_lanes_cap; }
 
-uint32_t MsmSchedule::sort_blocks(uint32_t n)
-{
-    return std::max<uint32_t>(1, std::min<uint32_t>(kSortBlocksTarget, div_up(n, kSortMinPerBlock)));
-}
-
-uint64_t msm_schedule_bytes(const MsmPlan &p)
-{
-    const uint64_t blocks = MsmSchedule::sort_blocks(p.n);
-    return p.max_entries() * 4 + (uint64_t)p.B * 4 * 2 + blocks * p.B * 4 + 32;
-}
-
-// Fold records of one launch: buckets with more than kMsmCompleteMax partials.
-static uint64_t fold_records(uint64_t partials) { return partials / (kMsmCompleteMax + 1) + 1; }
-
 template <class F>
-uint64_t msm_job_bytes(const MsmPlan &p)
+uint64_t msm_request_bytes(const std::vector<MsmPlan> &plans)
 {
-    const uint64_t partials = p.max_pieces(std::max(kMsmMaxLanesLog, g_target_log) - 1);
-    // partial sums and their folds; per bucket: sums and two tree levels,
-    // region start and count, the completion class lists; fold records; the
-    // bit planes; and the job's fixed records (job table, class counters, lane
-    // offsets)
-    return msm_partial_capacity(p, partials, nullptr, nullptr) * sizeof(partial_t<F>) +
-           (uint64_t)p.B * (3 * sizeof(partial_t<F>) + 8 + 4 * kMsmCompleteClasses) +
-           fold_records(partials) * kMsmMaxFoldLaunches * sizeof(FoldRec) + p.c * sizeof(Xyzz<F>) + 1024;
+    uint64_t entries = 0, buckets = 0;
+    for (const MsmPlan &p : plans) {
+        entries += p.max_entries();
+        buckets += p.B;
+    }
+    const MsmLanes rule = msm_lanes(std::is_same<F, fq2_t>::value);
+    const MsmSizes s = msm_sizes(plans.size(), entries, buckets, msm_lane_charge(rule, entries));
+    // partial sums and their folds; per bucket: sums and two tree levels, region
+    // start and count, the completion class lists; fold records; and the fixed
+    // records (job table, class counters, lane offsets, plan state)
+    return s.pool * sizeof(partial_t<F>) + buckets * (3 * sizeof(partial_t<F>) + 8 + 4 * kMsmCompleteClasses) +
+           s.records * kMsmMaxFoldLaunches * sizeof(FoldRec) + 1024 * plans.size();
 }
 
 void msm_finite_terms(const g1_jac *a, const g2_jac *b, uint32_t n, std::vector<uint32_t> &terms, hipStream_t stream)
@@ -1030,14 +1016,14 @@ uint32_t MsmSchedule::prepare(const MsmPlan &plan)
     allow_sort_lds();
     NKR_REQUIRE(plan.B <= kMsmMaxBuckets, "MSM window too wide for the bucket scans");
     plan_ = plan;
-    const uint32_t n = plan.n, B = plan.B;
-    blocks_ = sort_blocks(n);
-    sorted_.ensure(((size_t)n * plan.W + 3) & ~size_t(3));  // read in blocks of four
-    bucket_start_.ensure(B + 1);
-    in_tile_.ensure(B);
-    tile_total_.ensure(div_up(B, 64));
-    block_count_.ensure((size_t)blocks_ * B);
-    return div_up(n, blocks_);
+    blocks_ = msm_sort_blocks(plan.n);
+    const MsmScheduleSizes sizes = msm_schedule_sizes(plan);
+    sorted_.ensure(sizes.sorted);
+    bucket_start_.ensure(sizes.bucket_start);
+    in_tile_.ensure(sizes.in_tile);
+    tile_total_.ensure(sizes.tile_total);
+    block_count_.ensure(sizes.block_count);
+    return div_up(plan.n, blocks_);
 }
 
 void MsmSchedule::build(const fr_t *scalars_mont, const uint32_t *pick, const MsmPlan &plan, hipStream_t stream,
@@ -1320,7 +1306,7 @@ template Jacobian<fq_t> msm_finish(const Xyzz<fq_t> *, uint32_t);
 template Jacobian<fq2_t> msm_finish(const Xyzz<fq2_t> *, uint32_t);
 template Xyzz<fq_t> msm_sum(const Xyzz<fq_t> *, uint32_t);
 template Xyzz<fq2_t> msm_sum(const Xyzz<fq2_t> *, uint32_t);
-template uint64_t msm_job_bytes<fq_t>(const MsmPlan &);
-template uint64_t msm_job_bytes<fq2_t>(const MsmPlan &);
+template uint64_t msm_request_bytes<fq_t>(const std::vector<MsmPlan> &);
+template uint64_t msm_request_bytes<fq2_t>(const std::vector<MsmPlan> &);
 
 }  // namespace nkr

@@ -1,6 +1,6 @@
-// MSM sizing: window choice, piece bounds and the partial-sum capacity of
-// the fold levels.  Host arithmetic only (no HIP), so that a CPU unit test
-// can check every bound the device buffers are sized from.
+// MSM sizing: window choice, accumulation lanes, folds, and the bounds the
+// device buffers are sized from.  No HIP, so that a CPU test can check every
+// one of them; what the planning kernel uses as well is constexpr.
 #pragma once
 
 #include <algorithm>
@@ -10,10 +10,6 @@
 
 namespace nkr {
 
-// Fold fan-in of one level and the completion limit.
-constexpr uint32_t kMsmFoldIn = 4;
-constexpr uint32_t kMsmCompleteMax = 64;
-constexpr uint32_t kMaxFoldLevels = 12;
 // Accumulation lanes.  A batch's E sorted entries (non-zero digits, known on
 // the device) are split evenly: each lane sums ceil(E / lanes) consecutive
 // ones, a serial chain, and leaves about one partial sum to the bucket
@@ -44,7 +40,6 @@ constexpr bool msm_lanes_ascend(const MsmLanes &r)
 constexpr MsmLanes kMsmLanesG1 = {{1u << 16, 2u << 16, 4u << 16, 6u << 16}, {1u << 22, 1u << 24, 1u << 25}};
 constexpr MsmLanes kMsmLanesG2 = {{1u << 16, 1u << 16, 2u << 16, 4u << 16}, {1u << 19, 1u << 21, 1u << 23}};
 static_assert(msm_lanes_ascend(kMsmLanesG1) && msm_lanes_ascend(kMsmLanesG2), "lane rule");
-constexpr uint32_t kMsmMaxLanesLog = 19;  // at least log2 of every lane count above
 // The default of the lane setting (2^target_log lanes for every launch): the
 // group's own lanes above.
 constexpr uint32_t kMsmTargetDefault = 19;
@@ -73,6 +68,21 @@ constexpr uint32_t msm_piece(const MsmLanes &r, uint64_t entries)
 {
     const uint32_t lanes = msm_launch_lanes(r, entries);
     return entries == 0 ? 1u : (uint32_t)((entries + lanes - 1) / lanes);
+}
+// The lanes that a request's jobs, of `entries` entries in all, are charged
+// where launches are shared: for any set of requests at least as many as the
+// launch of all their entries has, though the rule may step up at an entry
+// count that only the sum reaches (a step to `lanes` at `below` entries is paid
+// for by lanes / below an entry).
+constexpr uint64_t msm_lane_charge(const MsmLanes &r, uint64_t entries)
+{
+    uint64_t charge = msm_launch_lanes(r, entries);
+    for (int i = 0; i < 3; ++i)
+        if (r.lanes[i + 1] > r.lanes[i]) {
+            const uint64_t per_lane = r.below[i] / r.lanes[i + 1];
+            charge = std::max(charge, (entries + per_lane - 1) / per_lane);
+        }
+    return std::min(entries, std::min<uint64_t>(charge, r.lanes[3]));
 }
 constexpr uint32_t msm_job_piece(uint32_t piece, uint32_t piece_min) { return piece < piece_min ? piece_min : piece; }
 // Largest bucket count (c <= 16): the histograms and bucket scans hold B
@@ -140,25 +150,11 @@ inline MsmSizes msm_sizes(uint64_t jobs, uint64_t entries, uint64_t buckets, uin
     return s;
 }
 
-// Fold levels (4:1 each) that bring `partials` partial sums of one bucket
-// down to at most kMsmCompleteMax; 0 for an empty or short bucket.
-inline uint32_t msm_fold_levels(uint64_t partials)
-{
-    uint32_t levels = 0;
-    while (partials > kMsmCompleteMax) {
-        partials = (partials + kMsmFoldIn - 1) / kMsmFoldIn;
-        ++levels;
-    }
-    return levels;
-}
-
 struct MsmPlan {
     uint32_t n = 0;         // number of bases / scalars
     uint32_t c = 0;         // window width in bits
     uint32_t W = 0;         // windows (signed digits), c*W >= 255
     uint32_t B = 0;         // buckets 1..B, B = 2^(c-1)
-    uint32_t piece_lo = 0;  // bounds of the accumulation run length (max_pieces)
-    uint32_t piece_hi = 0;
 
     // ~3/4 log2 n bits (16 from 2^20 terms up), or c_override when non-zero.
     static MsmPlan choose(uint32_t n, uint32_t c_override = 0)
@@ -187,8 +183,6 @@ struct MsmPlan {
         p.c = c;
         p.W = (255 + c - 1) / c;
         p.B = 1u << (c - 1);
-        p.piece_lo = 1;
-        p.piece_hi = UINT32_MAX;
         NKR_REQUIRE((uint64_t)p.W * n < (1ull << 31), "MSM too large for 31-bit entry indices");
         return p;
     }
@@ -196,17 +190,6 @@ struct MsmPlan {
     static uint32_t top_bits(uint32_t cc) { return 254 - cc * ((255 + cc - 1) / cc - 1); }
 
     uint64_t max_entries() const { return (uint64_t)n * W; }
-    // Upper bound of level-0 pieces for any scalars when the device targets
-    // 2^target_log pieces: the piece p it picks is piece_hi, or
-    // p >= E / 2^target_log.  Every bucket may add one short piece.
-    uint64_t max_pieces(uint32_t target_log) const
-    {
-        NKR_REQUIRE(piece_lo >= 1 && piece_lo <= piece_hi, "MSM piece bounds must satisfy 1 <= lo <= hi");
-        NKR_REQUIRE(target_log < 40, "MSM target piece count out of range");
-        const uint64_t by_lo = max_entries() / piece_lo;
-        const uint64_t by_target = std::max<uint64_t>(2ull << target_log, max_entries() / piece_hi);
-        return std::min(by_lo, by_target) + B + 1;
-    }
 };
 
 // The plan of the witness's MSMs over n columns: at most 15 bits, whose
@@ -228,31 +211,23 @@ inline MsmPlan msm_b_plan(const MsmPlan &witness, uint32_t finite)
     return msm_witness_plan(n);
 }
 
-// Partial sums one job needs room for: the level-0 pieces, then each fold
-// level's worst case (a level keeps at most a quarter of the previous one,
-// plus one rounded-up group per bucket).  levels receives the fold levels
-// the capacity covers; level_base[L] and level_cap[L] (if non-null,
-// kMaxFoldLevels entries each) the offset and size of level L's output.
-inline uint64_t msm_partial_capacity(const MsmPlan &p, uint64_t pieces, uint32_t *levels, uint64_t *level_base,
-                                     uint64_t *level_cap = nullptr)
+// Sort workgroups: about one per CU, each histogramming a contiguous slice of
+// at least kMsmSortMinPerBlock scalars.
+constexpr uint32_t kMsmSortBlocksTarget = 256;
+constexpr uint32_t kMsmSortMinPerBlock = 256;
+inline uint32_t msm_sort_blocks(uint32_t n)
 {
-    uint64_t cap = pieces, cnt = pieces, base = pieces;
-    uint32_t L = 0;
-    while (cnt > kMsmCompleteMax) {
-        NKR_REQUIRE(L < kMaxFoldLevels, "MSM needs too many fold levels");
-        cnt = (cnt + kMsmFoldIn - 1) / kMsmFoldIn;
-        cap = cap / kMsmFoldIn + p.B + 1;
-        if (level_base) level_base[L] = base;
-        if (level_cap) level_cap[L] = cap;
-        base += cap;
-        ++L;
-    }
-    for (uint32_t k = L; k < kMaxFoldLevels; ++k) {
-        if (level_base) level_base[k] = base;
-        if (level_cap) level_cap[k] = 0;
-    }
-    if (levels) *levels = L;
-    return base;
+    return std::max<uint32_t>(1, std::min<uint32_t>(kMsmSortBlocksTarget, div_up(n, kMsmSortMinPerBlock)));
+}
+// The words of a schedule's buffers.
+struct MsmScheduleSizes {
+    uint64_t sorted, bucket_start, in_tile, tile_total, block_count;
+    uint64_t bytes() const { return 4 * (sorted + bucket_start + in_tile + tile_total + block_count); }
+};
+inline MsmScheduleSizes msm_schedule_sizes(const MsmPlan &p)
+{
+    const uint64_t entries = (p.max_entries() + 3) & ~uint64_t(3);  // read in blocks of four
+    return {entries, uint64_t(p.B) + 1, p.B, div_up(p.B, 64), uint64_t(msm_sort_blocks(p.n)) * p.B};
 }
 
 }  // namespace nkr

@@ -16,9 +16,10 @@ uint64_t Server::request_bytes(const Groth16Prover &g)
     const MsmPlan &w = g.witness_plan(), &b = g.b_plan(), &h = g.h_plan();
     const uint64_t planes =
         (uint64_t)(g.planes_g1_witness() + h.c) * sizeof(Xyzz<fq_t>) + (uint64_t)b.c * sizeof(Xyzz<fq2_t>);
-    const uint64_t own_b = g.own_b_schedule() ? msm_schedule_bytes(b) : 0;
-    return polys + packed + planes + msm_schedule_bytes(w) + own_b + msm_schedule_bytes(h) +
-           2 * msm_job_bytes<fq_t>(w) + msm_job_bytes<fq_t>(b) + msm_job_bytes<fq_t>(h) + msm_job_bytes<fq2_t>(b);
+    const uint64_t schedules = msm_schedule_sizes(w).bytes() + msm_schedule_sizes(h).bytes() +
+                               (g.own_b_schedule() ? msm_schedule_sizes(b).bytes() : 0);
+    return polys + packed + planes + schedules + msm_request_bytes<fq_t>({w, w, b, h}) +
+           msm_request_bytes<fq2_t>({b});
 }
 
 Server::Server(int device, uint32_t workers, uint32_t max_batch, uint64_t work_budget_bytes)

@@ -1,14 +1,13 @@
 // CPU check of the MSM sizing arithmetic (nkr-zkp_amd/csrc/msm_plan.h).
 // stdin: one request per line,
-//   plan n c_override target_log piece_lo piece_hi
-//       -> "c W B max_pieces capacity levels" or "error <message>"
-//   folds partials        -> fold levels for one bucket with that many partials
+//   plan n c_override     -> "c W B" or "error <message>"
+//   schedule n c_override -> the words of a schedule's buffers and their bytes
 //   lanes g2 target_log   -> the lane rule: 4 lane counts, 3 limits
 //   piece g2 target_log piece_min entries... -> per entry count, the launch's
 //                            entries per lane and those of a job with that minimum
 //   bplan cols c_override finite -> "n c" of bs1 and bs2
-//   sizes g2 target_log jobs entries buckets -> the bounds msm_sizes gives a launch
-//                            under that lane rule: lanes pool records complete_lanes
+//   sizes | charge g2 target_log jobs entries buckets -> the bounds msm_sizes gives a
+//                            launch under that lane rule, or a request's share: lanes pool records complete_lanes
 //                            launches, then each fold launch's base and cap
 //   launches partials     -> fold launches for buckets of at most that many
 //   divup a b             -> ceil(a / b) or "error <message>"
@@ -34,20 +33,18 @@ int main()
         in >> op;
         try {
             if (op == "plan") {
-                uint64_t n, c, tl, lo, hi;
-                in >> n >> c >> tl >> lo >> hi;
-                MsmPlan p = MsmPlan::choose((uint32_t)n, (uint32_t)c);
-                p.piece_lo = (uint32_t)lo;
-                p.piece_hi = (uint32_t)hi;
-                const uint64_t pieces = p.max_pieces((uint32_t)tl);
-                uint32_t levels = 0;
-                const uint64_t cap = msm_partial_capacity(p, pieces, &levels, nullptr);
-                std::printf("%u %u %u %llu %llu %u\n", p.c, p.W, p.B, (unsigned long long)pieces,
-                            (unsigned long long)cap, levels);
-            } else if (op == "folds") {
-                uint64_t k;
-                in >> k;
-                std::printf("%u\n", msm_fold_levels(k));
+                uint64_t n, c;
+                in >> n >> c;
+                const MsmPlan p = MsmPlan::choose((uint32_t)n, (uint32_t)c);
+                std::printf("%u %u %u\n", p.c, p.W, p.B);
+            } else if (op == "schedule") {
+                uint64_t n, c;
+                in >> n >> c;
+                const MsmScheduleSizes s = msm_schedule_sizes(MsmPlan::choose((uint32_t)n, (uint32_t)c));
+                std::printf("%llu %llu %llu %llu %llu %llu\n", (unsigned long long)s.sorted,
+                            (unsigned long long)s.bucket_start, (unsigned long long)s.in_tile,
+                            (unsigned long long)s.tile_total, (unsigned long long)s.block_count,
+                            (unsigned long long)s.bytes());
             } else if (op == "lanes") {
                 uint64_t g2, tl;
                 in >> g2 >> tl;
@@ -66,11 +63,12 @@ int main()
                 in >> cols >> c >> finite;
                 const MsmPlan p = msm_b_plan(msm_witness_plan((uint32_t)cols, (uint32_t)c), (uint32_t)finite);
                 std::printf("%u %u\n", p.n, p.c);
-            } else if (op == "sizes") {
+            } else if (op == "sizes" || op == "charge") {
                 uint64_t g2, tl, jobs, entries, buckets;
                 in >> g2 >> tl >> jobs >> entries >> buckets;
                 const MsmLanes r = msm_lanes_of(g2 != 0, (uint32_t)tl);
-                const MsmSizes s = msm_sizes(jobs, entries, buckets, msm_launch_lanes(r, entries));
+                const MsmSizes s = msm_sizes(jobs, entries, buckets,
+                                             op == "sizes" ? msm_launch_lanes(r, entries) : msm_lane_charge(r, entries));
                 std::printf("%llu %llu %llu %llu %u", (unsigned long long)s.lanes, (unsigned long long)s.pool,
                             (unsigned long long)s.records, (unsigned long long)s.complete_lanes, s.fold_launches);
                 for (uint32_t L = 0; L < kMsmMaxFoldLaunches; ++L)

@@ -134,6 +134,27 @@ def test_work_memory_stays_within_the_budget(contexts):
     assert st["proofs"] == len(reqs)
 
 
+def test_a_request_is_charged_what_it_holds():
+    """One worker after one request: the work memory it holds is within the
+    request's charge, and most of it (the MSMs of a request share a launch, so
+    their lanes are charged once)."""
+    c = circuits.matmul(16, 5, wide=True)
+    k = N.setup(c, circuits.random_scalars(5, 99))
+    pv = N.Prover(c, k)
+    need = N.Server.request_bytes(pv)
+    srv = N.Server(workers=1, max_batch=1, budget_bytes=need)
+    try:
+        r, s = circuits.random_scalars(2, 7)
+        (raw, proof), = srv.warm([(pv, c.witness, r, s)])
+        held = srv.memory()["held"]
+    finally:
+        srv.close()
+    raw1, proof1 = pv.prove_blind(c.witness, r, s)
+    pv.close()
+    assert np.array_equal(raw, raw1) and np.array_equal(proof, proof1)
+    assert 0.8 * need < held <= need
+
+
 def test_budget_is_clamped_to_free_device_memory(contexts):
     srv = N.Server(workers=2, max_batch=4, budget_bytes=1 << 60)
     try:

@@ -1,8 +1,9 @@
 """The MSM sizing arithmetic the device buffers are allocated from
-(nkr-zkp_amd/csrc/msm_plan.h), compiled for the CPU: window choice, the
-level-0 piece bound, the fold levels and the partial-sum capacity, including
-schedules with zero entries and invalid piece bounds, which must raise an
-error instead of dividing by zero (SIGFPE)."""
+(nkr-zkp_amd/csrc/msm_plan.h), compiled for the CPU: window choice, the lane
+rule, the bounds of a batch's partial sums and folds against the numbering the
+planning kernel uses, and what a request is charged where launches are shared;
+schedules with zero entries included, and a zero divisor must raise an error
+instead of ending the process (SIGFPE)."""
 import os
 import shutil
 import subprocess
@@ -31,59 +32,14 @@ def ask(binary, lines):
 
 def test_window_choice_covers_the_scalar(plan_bin):
     ns = sorted({1, 2, 3, 5, 7, 100, 1000, 4097} | {1 << k for k in range(0, 25)} | {(1 << k) + 1 for k in range(1, 24)})
-    out = ask(plan_bin, [f"plan {n} 0 19 4 64" for n in ns])
+    out = ask(plan_bin, [f"plan {n} 0" for n in ns])
     for n, line in zip(ns, out):
-        c, W, B, pieces, cap, levels = map(int, line.split())
+        c, W, B = map(int, line.split())
         assert 4 <= c <= 16 and B == 1 << (c - 1)
         assert c * W >= 255 and c * (W - 1) < 255          # W signed digits cover 255 bits, none wasted
         assert 254 - c * (W - 1) >= 4 or c in (4, 16)        # the top window keeps at least 4 bits
         if n >= 1 << 20:
             assert c == 16
-        assert pieces >= B + 1 and cap >= pieces
-
-
-def test_piece_bound_covers_every_split(plan_bin):
-    """The device picks the largest power of two p <= E / 2^target within
-    [lo, hi] (and longer while buckets would keep more than 64 partials);
-    every bucket's run of entries then splits into ceil(count / p) pieces.
-    Worst case over the entry count E and the bucket spread: at most
-    E / p + B pieces, which max_pieces must bound."""
-    rng = np.random.default_rng(7)
-    for n, target in ((1 << 10, 19), (1 << 16, 19), (1 << 20, 19), (1 << 20, 12), (5000, 24)):
-        line = ask(plan_bin, [f"plan {n} 0 {target} 4 64"])[0]
-        c, W, B, pieces, cap, levels = map(int, line.split())
-        for E in [0, 1, B, n * W // 3, n * W] + list(rng.integers(0, n * W + 1, 5)):
-            p = 4
-            while p < 64 and 2 * p <= E >> target:
-                p *= 2
-            assert -(-E // p) + B <= pieces, (n, target, E)
-
-
-def test_fold_levels_and_capacity(plan_bin):
-    """Zero entries need no fold; the partial-sum capacity covers every fold
-    level of any distribution of the level-0 pieces over the buckets (each
-    level writes ceil(k / 4) partials per bucket with k > 64)."""
-    assert ask(plan_bin, ["folds 0", "folds 1", "folds 64", "folds 65", "folds 256", "folds 257", "folds 4096"]) == \
-        ["0", "0", "0", "1", "1", "2", "3"]
-    rng = np.random.default_rng(11)
-    for n in (1 << 12, 1 << 16, 1 << 20):
-        c, W, B, pieces, cap, levels = map(int, ask(plan_bin, [f"plan {n} 0 19 4 64"])[0].split())
-        for shape in ("one", "uniform", "skewed"):
-            total = pieces - B - 1
-            if shape == "one":
-                counts = np.zeros(B, dtype=np.int64)
-                counts[0] = total
-            elif shape == "uniform":
-                counts = np.full(B, total // B, dtype=np.int64)
-            else:
-                counts = rng.multinomial(total, rng.dirichlet(np.full(B, 0.05)))
-            used, level = int(counts.sum()), 0
-            while counts.max() > 64:
-                big = counts > 64
-                counts = np.where(big, -(-counts // 4), counts)
-                used += int(counts[big].sum())
-                level += 1
-            assert level <= levels and used <= cap, (n, shape)
 
 
 def test_default_target_is_the_groups_own_rule(plan_bin):
@@ -120,7 +76,7 @@ def test_b_query_plan(plan_bin):
     the witness was given."""
     n = 1 << 17
     out = ask(plan_bin, [f"bplan {n} {c} {f}" for c in (0, 13) for f in (n, n - n // 4 + 1, n - n // 4, 1300, 1, 0)]
-              + [f"plan {k} 0 19 4 64" for k in (n, n - n // 4, 1300, 1)])
+              + [f"plan {k} 0" for k in (n, n - n // 4, 1300, 1)])
     own = [int(line.split()[0]) for line in out[12:]]
     for c, got in ((own[0], out[:6]), (13, out[6:12])):
         assert [tuple(map(int, g.split())) for g in got] == \
@@ -129,7 +85,7 @@ def test_b_query_plan(plan_bin):
     # a plan of its own always has fewer terms
     for cols in (1, 2, 3, 4, 5):
         for f in range(cols + 1):
-            got, plan = ask(plan_bin, [f"bplan {cols} 9 {f}", f"plan {max(1, f)} 0 19 4 64"])
+            got, plan = ask(plan_bin, [f"bplan {cols} 9 {f}", f"plan {max(1, f)} 0"])
             same = max(1, f) == cols or f > cols - cols // 4
             assert got.split() == ([str(cols), "9"] if same else [str(max(1, f)), plan.split()[0]]), (cols, f)
     # the witness itself stays at 15 bits
@@ -220,12 +176,48 @@ def test_buffer_bounds_cover_every_plan(plan_bin, g2, target):
                 assert buckets * 64 + 5 * 64 * len(jobs) == complete
 
 
-def test_zero_divisors_raise_instead_of_crashing(plan_bin):
-    out = ask(plan_bin, ["plan 1024 0 19 0 64", "plan 1024 0 19 8 4", "divup 10 0", "divup 10 3",
-                         "plan 0 0 19 4 64", "plan 1024 17 19 4 64"])
-    assert out[0].startswith("error MSM piece bounds")
-    assert out[1].startswith("error MSM piece bounds")
-    assert out[2].startswith("error internal sizing error")
-    assert out[3] == "4"
-    assert out[4].startswith("error MSM needs at least one term")
-    assert out[5].startswith("error MSM window")
+@pytest.mark.parametrize("g2", [0, 1])
+@pytest.mark.parametrize("target", [10, 19, 22])
+def test_charges_cover_any_batch(plan_bin, g2, target):
+    """What requests are charged one by one holds the lanes, partial sums and
+    fold records of the batch of all of them, also where only the sum of their
+    entries reaches a step of the lane rule; one request is charged its own
+    launch, or a step that its entries pay for."""
+    rng = np.random.default_rng(target)
+    steps = [1 << k for k in (16, 19, 21, 22, 23, 24, 25)]
+    for trial in range(120):
+        total = int(rng.choice(steps) * rng.choice([0.6, 1, 1.7])) + int(rng.integers(-2, 3))
+        K = int(rng.integers(1, 9))
+        parts = np.maximum(1, rng.multinomial(total, rng.dirichlet(np.full(K, rng.choice([0.1, 5]))))).tolist()
+        buckets = [int(b) for b in 2 ** rng.integers(1, 16, K)]
+        jobs = [int(j) for j in rng.integers(1, 5, K)]
+        out = ask(plan_bin, [f"sizes {g2} {target} {sum(jobs)} {sum(parts)} {sum(buckets)}"] +
+                  [f"charge {g2} {target} {j} {e} {b}" for j, e, b in zip(jobs, parts, buckets)] +
+                  [f"sizes {g2} {target} {j} {e} {b}" for j, e, b in zip(jobs, parts, buckets)])
+        rows = [list(map(int, line.split()))[:3] for line in out]
+        charged = np.array(rows[1:K + 1])
+        assert (charged.sum(axis=0) >= rows[0]).all(), (parts, buckets)
+        alone = np.array(rows[K + 1:])
+        assert (charged >= alone).all()
+        most = {0: (393216, 32), 1: (262144, 16)}[g2] if target == 19 else (1 << target, 1 << 60)
+        for (lanes, _, _), e, j, (own, _, _) in zip(charged, parts, jobs, alone):
+            assert lanes <= min(e, most[0], max(own, -(-e // most[1]))) + j
+
+
+def test_schedule_bytes_count_every_buffer(plan_bin):
+    """The sorted list (whole blocks of four), the bucket starts and the two
+    levels of their prefix, and the sort workgroups' counts."""
+    for n, c in ((1, 4), (5, 7), (255, 0), (257, 8), (65537, 0), (1 << 20, 16)):
+        C, W, B = map(int, ask(plan_bin, [f"plan {n} {c}"])[0].split())
+        blocks = max(1, min(256, -(-n // 256)))
+        words = [-(-n * W // 4) * 4, B + 1, B, -(-B // 64), blocks * B]
+        assert list(map(int, ask(plan_bin, [f"schedule {n} {c}"])[0].split())) == words + [4 * sum(words)]
+
+
+def test_bad_sizes_raise_instead_of_crashing(plan_bin):
+    out = ask(plan_bin, ["divup 10 0", "divup 10 3", "plan 0 0", "plan 1024 17", f"plan {1 << 28} 15"])
+    assert out[0].startswith("error internal sizing error")
+    assert out[1] == "4"
+    assert out[2].startswith("error MSM needs at least one term")
+    assert out[3].startswith("error MSM window")
+    assert out[4].startswith("error MSM too large")
