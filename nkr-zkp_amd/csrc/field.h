@@ -472,12 +472,14 @@ NKR_HD Fp29<P> fp29_mul_add4(const Fp29<P> &a, const Fp29<P> &b, const Fp29<P> &
 
 // x*w*2^-256 mod p (the canonical form's Montgomery product) through the
 // 29-bit product: (32x)*w*2^-261.  x: any 256-bit value; w: below p.  The
-// result is below 1.15p + x*w/2^256 (Fr: p + x*w/2^256), not reduced, in 32-bit
-// limbs; below 2p for a canonical x.
+// result is below p + x*w/2^256 < 2p, not reduced, in 32-bit limbs.  Textbook
+// steps throughout: with direct ones an x near 2^256 could come out above 2p,
+// and one subtraction would not make it canonical.
 template <class P>
 NKR_HD Fp<P> fp_mul_r29(const Fp<P> &x, const Fp<P> &w)
 {
-    return fp29_to_bits(fp29_mul(fp29_from_mont(x), fp29_from_bits(w)));
+    const Fp29<P> a = fp29_from_mont(x), b = fp29_from_bits(w);
+    return fp29_to_bits(fp29_reduce_terms<P, 0>([&](int k, uint64_t &acc) { fp29_column(a, b, k, acc); }));
 }
 
 

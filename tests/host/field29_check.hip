@@ -7,6 +7,8 @@
 //     against 2p), built as x + k*p, gives fp_mul's canonical result;
 //     squarings give fp29_mul(a, a)'s limbs, and a sum of two products with
 //     one reduction the canonical sum;
+//   * the canonical product through the 29-bit form (fp_mul_r29) of any 256-bit
+//     value is below 2p;
 //   * lazy sums and differences: a + b and a + K*p - b are congruent to the
 //     canonical ones;
 //   * mixed addition: chains of xyzz29_add_affine over random bases, repeated
@@ -112,6 +114,26 @@ static void check_field(int n)
     expect(fp29_may_be_zero<P, 10>(z) && fp29_may_be_zero<P, 10>(fp29_sub<P, 1>(z, z)) &&
                fp29_may_be_zero<P, 10>(fp29_sub<P, 5>(z, z)) && fp29_may_be_zero<P, 10>(fp29_sub<P, 9>(z, z)),
            "zero filter on multiples of p", 0);
+}
+
+// x*w*2^-256 for any 256-bit x: below 2p, so that one subtraction makes it
+// canonical, and congruent to the product of the reduced x.
+template <class P>
+static void check_mul_r29(int n)
+{
+    for (int i = 0; i < n; ++i) {
+        Fp<P> x, w = rand_fp<P>();
+        for (int k = 0; k < 8; ++k) x.l[k] = rnd();
+        if (i % 4 != 0) {  // near 2^256, against a factor near p
+            for (int k = 4; k < 8; ++k) x.l[k] = 0xffffffffu;
+            w = Fp<P>::modulus();
+            w.l[0] -= 1 + rnd() % 1000;
+        }
+        Fp<P> r = x;
+        for (int k = 0; k < 5; ++k) r = fp_reduce_once(r);  // 2^256 is below 6p
+        const Fp<P> got = fp_reduce_once(fp_mul_r29(x, w));
+        expect(got == fp_reduce_once(got) && got == fp_mul(r, w), "mul of any 256-bit value", i);
+    }
 }
 
 static Affine<fq_t> random_base(const Affine<fq_t> &g)
@@ -332,6 +354,8 @@ int main()
 {
     check_field<FqParams>(20000);
     check_field<FrParams>(20000);
+    check_mul_r29<FqParams>(4000);
+    check_mul_r29<FrParams>(4000);
     check_madd(200, 80);
     check_add(150, 60);
     check_fq2(5000);
