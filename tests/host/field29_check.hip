@@ -9,6 +9,11 @@
 //     one reduction the canonical sum;
 //   * the canonical product through the 29-bit form (fp_mul_r29) of any 256-bit
 //     value is below 2p;
+//   * products, sums of products and Fq2 products whose inputs are at the top of
+//     what is allowed (145 p^2 in all, in several shapes) come out below 2p;
+//   * the transforms' arithmetic (ntt29.h) at its bounds: products of values near
+//     160 r with limbs near 2.5 * 2^30, reductions near 169 r, differences of
+//     values near K r with limbs up to 2^30 - 2;
 //   * lazy sums and differences: a + b and a + K*p - b are congruent to the
 //     canonical ones;
 //   * mixed addition: chains of xyzz29_add_affine over random bases, repeated
@@ -27,6 +32,7 @@
 #include <vector>
 
 #include "curve29.h"
+#include "ntt29.h"
 
 using namespace nkr;
 
@@ -114,6 +120,172 @@ static void check_field(int n)
     expect(fp29_may_be_zero<P, 10>(z) && fp29_may_be_zero<P, 10>(fp29_sub<P, 1>(z, z)) &&
                fp29_may_be_zero<P, 10>(fp29_sub<P, 5>(z, z)) && fp29_may_be_zero<P, 10>(fp29_sub<P, 9>(z, z)),
            "zero filter on multiples of p", 0);
+}
+
+// K p - 1 - d, the d-th value below K p.
+template <class P, uint32_t K>
+static Fp29<P> below(const Fp<P> &d)
+{
+    Fp29<P> one = Fp29<P>::zero();
+    one.l[0] = 1;
+    return fp29_sub<P, K>(Fp29<P>::zero(), fp29_add(fp29_from_bits(d), one));
+}
+// What below(d) stands for, canonical (the same for every K).
+template <class P>
+static Fp<P> below_residue(const Fp<P> &d)
+{
+    return fp29_to_mont(below<P, 2>(d));
+}
+// The smallest offsets most of the time, any other now and then.
+template <class P>
+static Fp<P> offset(int i)
+{
+    Fp<P> d = Fp<P>::zero();
+    d.l[0] = i < 4 ? i : rnd();
+    return i % 5 == 4 ? rand_fp<P>() : d;
+}
+template <class P, uint32_t K>
+static bool is_below(const Fp29<P> &x)
+{
+    const Fp29<P> y = fp29_sub_if_ge<P, K>(x);
+    bool same = true;
+    for (int k = 0; k < 9; ++k) same = same && x.l[k] == y.l[k];
+    return same;
+}
+template <class P>
+static void expect_product(const Fp29<P> &r, const Fp<P> &want, const char *what, int i)
+{
+    bool limbs = true;
+    for (int k = 0; k < 9; ++k) limbs = limbs && (r.l[k] >> 29) == 0;
+    expect(limbs && is_below<P, 2>(r) && fp29_to_mont(r) == want, what, i);
+}
+
+template <class P, uint32_t A, uint32_t B>
+static void check_product_at(int i)
+{
+    static_assert(A * B <= 145, "allowed");
+    const Fp<P> d = offset<P>(i), e = offset<P>(i + 1);
+    expect_product(fp29_mul(below<P, A>(d), below<P, B>(e)), fp_mul(below_residue<P>(d), below_residue<P>(e)),
+                   "product at 145 p^2", i);
+}
+
+template <class P>
+static void check_bounds(int n)
+{
+    for (int i = 0; i < n; ++i) {
+        check_product_at<P, 145, 1>(i);
+        check_product_at<P, 72, 2>(i);
+        check_product_at<P, 48, 3>(i);
+        check_product_at<P, 36, 4>(i);
+        check_product_at<P, 24, 6>(i);
+        check_product_at<P, 18, 8>(i);
+        check_product_at<P, 12, 12>(i);
+        Fp<P> d[8], r[8];
+        for (int k = 0; k < 8; ++k) {
+            d[k] = offset<P>(i + k);
+            r[k] = below_residue<P>(d[k]);
+        }
+        expect_product(fp29_sqr(below<P, 12>(d[0])), fp_sqr(r[0]), "square at 12p", i);
+        expect_product(fp29_mul_add(below<P, 12>(d[0]), below<P, 6>(d[1]), below<P, 6>(d[2]), below<P, 12>(d[3])),
+                       fp_add(fp_mul(r[0], r[1]), fp_mul(r[2], r[3])), "mul_add at 144 p^2", i);
+        expect_product(fp29_mul_add4(below<P, 6>(d[0]), below<P, 6>(d[1]), below<P, 6>(d[2]), below<P, 6>(d[3]),
+                                     below<P, 4>(d[4]), below<P, 9>(d[5]), below<P, 9>(d[6]), below<P, 4>(d[7])),
+                       fp_add(fp_add(fp_mul(r[0], r[1]), fp_mul(r[2], r[3])),
+                              fp_add(fp_mul(r[4], r[5]), fp_mul(r[6], r[7]))),
+                       "mul_add4 at 144 p^2", i);
+    }
+}
+
+static void check_fq2_bounds(int n)
+{
+    using P = FqParams;
+    for (int i = 0; i < n; ++i) {
+        const fq_t d[4] = {offset<P>(i), offset<P>(i + 1), offset<P>(i + 2), offset<P>(i + 3)};
+        const fq2_t x = {below_residue<P>(d[0]), below_residue<P>(d[1])};
+        const fq2_t y = {below_residue<P>(d[2]), below_residue<P>(d[3])};
+        const fq2_t want = fq2_mul(x, y), sq = fq2_sqr(x);
+        // 36p x 2p with b1 negated by 2p: c1 at 2 * 72; b1 = 0 brings c0 to 36 * 4
+        for (int zero = 0; zero < 2; ++zero) {
+            const Fq2_29<P> a = {below<P, 36>(d[0]), below<P, 36>(d[1])};
+            const Fq2_29<P> b = {below<P, 2>(d[2]), zero ? Fp29<P>::zero() : below<P, 2>(d[3])};
+            const fq2_t w = zero ? fq2_mul(x, {y.c0, fq_t::zero()}) : want;
+            const Fq2_29<P> m = fq2_29_mul<P, 2>(a, b);
+            expect_product(m.c0, w.c0, "fq2 product c0 at its bound", i);
+            expect_product(m.c1, w.c1, "fq2 product c1 at its bound", i);
+        }
+        const Fq2_29<P> s = fq2_29_sqr<P, 6>({below<P, 6>(d[0]), below<P, 6>(d[1])});
+        expect_product(s.c0, sq.c0, "fq2 square c0 at its bound", i);
+        expect_product(s.c1, sq.c1, "fq2 square c1 at its bound", i);
+    }
+}
+
+// The value of x modulo r as a canonical element, through textbook steps.
+static fr_t residue29(const fr29 &x)
+{
+    fr29 one = fr29::zero();
+    one.l[0] = 1;
+    const fr29 n = normalise29(x);
+    const fr29 t = fp29_reduce_terms<FrParams, 0>([&](int k, uint64_t &acc) { fp29_column(n, one, k, acc); });
+    return fp_reduce_once(fp29_to_bits(t));
+}
+static bool equal29(const fr29 &a, const fr29 &b)
+{
+    for (int k = 0; k < 9; ++k)
+        if (a.l[k] != b.l[k]) return false;
+    return true;
+}
+
+template <uint32_t K>
+static void check_sub29(int i)
+{
+    using P = FrParams;
+    constexpr Borrowed bk = borrowed(K);
+    // y: the sum of two values of K/2 r each less a little, so that its limbs
+    // reach 2^30 - 2 and it stays below (K - 0.01) r
+    fr_t d = rand_fp<P>();
+    if (d.l[7] < P::P[7] / 50) d.l[7] += P::P[7] / 50;
+    const fr29 x = i % 2 ? fr29::zero() : below<P, 79>(offset<P>(i)), p = below<P, K / 2>(offset<P>(i)),
+               q = below<P, K / 2>(fp_reduce_once(d));
+    const fr29 y = add29(p, q), r = sub29(x, y, bk);
+    bool limbs = true;
+    for (int k = 0; k < 9; ++k) limbs = limbs && r.l[k] <= x.l[k] + 3u * (1u << 29);
+    const fr29 back = normalise29(add29(normalise29(r), normalise29(y)));
+    expect(limbs && equal29(back, fp29_sub<P, K>(x, fr29::zero())), "sub29 at its bound", i);
+}
+
+static void check_ntt29(int n)
+{
+    using P = FrParams;
+    for (int i = 0; i < n; ++i) {
+        // a: limbs up to 2.5 * 2^30 and a value just below 160 r
+        fr29 a;
+        for (int k = 0; k < 8; ++k) a.l[k] = 5u * (1u << 29) - (i < 3 ? 0u : rnd() % (i % 2 ? 1000 : 1u << 31));
+        a.l[8] = P29<P>::times(160).l[8] - 6 - (i < 3 ? 0u : rnd() % 1000);
+        expect(is_below<P, 160>(normalise29(a)), "the operand is below 160 r", i);
+        const fr_t d = offset<P>(i);
+        const fr29 b = below<P, 1>(d);
+        const fr29 m = mul29(a, b);
+        bool limbs = true;
+        for (int k = 0; k < 9; ++k) limbs = limbs && (m.l[k] >> 29) == 0;
+        // m = a b 2^-261: both sides as canonical Montgomery elements of 2^261
+        const fr29 ra = reduce29(normalise29(a));
+        const fr29 t = fp29_reduce_terms<P, 0>([&](int k, uint64_t &acc) { fp29_column(ra, b, k, acc); });
+        expect(limbs && is_below<P, 5>(fp29_add(m, m)) && residue29(m) == residue29(t), "mul29 at its bound", i);
+
+        const fr29 top = below<P, 169>(d);
+        fr29 r25 = fr29::zero();
+        const fr29 red = reduce29(top);
+        for (int k = 0; k < 25; ++k) r25 = fp29_add(r25, red);
+        expect(is_below<P, 26>(r25) && residue29(red) == residue29(top), "reduce29 near 169 r", i);
+        const fr29 any = fp29_add(below<P, 100>(rand_fp<P>()), fp29_from_mont(rand_fp<P>()));
+        const fr_t c = canonical29(any);
+        expect(c == fp_reduce_once(c) && residue29(load29(c)) == residue29(any), "canonical29", i);
+        check_sub29<4>(i);
+        check_sub29<40>(i);
+        check_sub29<80>(i);
+        const fr_t w = rand_fp<P>(), v = rand_fp<P>();
+        expect(factor_mul(factor_from_mont(w), factor_from_mont(v)) == factor_from_mont(fp_mul(w, v)), "factor_mul", i);
+    }
 }
 
 // x*w*2^-256 for any 256-bit x: below 2p, so that one subtraction makes it
@@ -354,6 +526,10 @@ int main()
 {
     check_field<FqParams>(20000);
     check_field<FrParams>(20000);
+    check_bounds<FqParams>(4000);
+    check_bounds<FrParams>(4000);
+    check_fq2_bounds(4000);
+    check_ntt29(4000);
     check_mul_r29<FqParams>(4000);
     check_mul_r29<FrParams>(4000);
     check_madd(200, 80);
