@@ -1,7 +1,7 @@
 """Autotuner for the per-context choices of the Groth16 backend
 (nkr_g16_tuning in include/nkr_g16.h): MSM window widths of the witness and H
-MSMs, the transform tile, radix and pass split, the MSM piece target and the
-witness G1 piece minimum.  None of them changes a proof, only its time, so
+MSMs, the transform tile, radix and pass split, the MSM's lanes and the
+shortest run of the witness G1 MSMs.  None of them changes a proof, only its time, so
 the tuner checks that every candidate's raw proof equals the default one and
 keeps the fastest.
 
@@ -70,7 +70,7 @@ def knob_alternatives(rows: int, cols: int) -> dict[str, list[int]]:
         "ntt_lds_log": [0, 10],
         "ntt_radix_log": [0, 3],
         "ntt_split_policy": [0, 1],
-        "msm_target_pieces_log": [0, 18, 20],
+        "msm_target_pieces_log": [0, 16, 17, 18, 20],
         "witness_g1_piece_min": [0, 16, 64],
     }
 
