@@ -13,7 +13,7 @@
 //   3. Q = U1 PP, PPP = P PP, ZZ3 = (ZZ1 ZZ2) PP
 //   4. R (Q - X3), S1 PPP, ZZZ3 = (ZZZ1 ZZZ2) PPP (X3 = RR - PPP - 2Q)
 // Operands move between lanes with DPP moves (quad permutes, and for the
-// 8-lane group the half-row mirror).  2.3 us at G1 and 3.4 us at G2 per
+// 8-lane group the half-row mirror).  2.5 us at G1 and 3.8 us at G2 per
 // addition, measured on MI355X.
 //
 // Bounds (p the modulus), closed under the addition and satisfied by the

@@ -1,6 +1,6 @@
 // Mixed XYZZ addition over the reduced-radix field (field29.h), for the MSM
 // bucket accumulation: acc + (x2, y2) with the accumulator kept in 29-bit
-// limbs across a whole piece of a bucket.
+// limbs across a whole run of entries.
 //
 // Bounds (p the modulus; every limb below 2^29):
 //   accumulator  X < 8p, Y < 8p, ZZ < 2p, ZZZ < 2p; infinity is ZZ = 0 exactly

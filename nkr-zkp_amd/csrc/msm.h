@@ -20,7 +20,7 @@
 //      1. accumulate: every lane sums an equally long run of the sorted
 //         entries, one partial sum per bucket it meets (mixed affine
 //         additions into XYZZ);
-//      2. fold: buckets left with more than 64 partial sums (skewed digit
+//      2. fold: buckets left with more than 128 partial sums (skewed digit
 //         distributions, e.g. witnesses that are mostly 0 or 1) are folded
 //         64:1, a wave per sum, until they are not; others are untouched;
 //      3. complete: 1..16 lane groups per bucket, strided partial sums then

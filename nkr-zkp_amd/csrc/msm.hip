@@ -723,7 +723,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 // wave per SIMD; held to two waves, its spills cost less than the second wave
 // gains (G2 accumulation of the dense 2^20 Poseidon-style proof 10.3 -> 8.5
 // ms on MI355X), and with the accumulator's Y and ZZZ in LDS (36 KiB per
-// workgroup) the spills fall from 280 to 80 bytes per lane.
+// workgroup) the spills fell from 280 to 80 bytes per lane (112 with the run's
+// state).
 template <>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_accumulate<fq2_t>(
     const JobDev<fq2_t> *__restrict__ jobs, const uint32_t *__restrict__ lane_base, uint32_t J,

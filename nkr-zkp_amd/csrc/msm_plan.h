@@ -23,6 +23,13 @@ namespace nkr {
 //   than the reduction of their partials costs (10 and 29 us per 65536);
 //   two full rounds of those for the largest, whose last round then ends
 //   early where another stream's kernels took some of the slots.
+// One MSM on MI355X, us, just below and above each limit (2^16, 2^17 and 2^18
+// lanes; 6 * 2^16 in the last figure):
+//   G1  2^22: 561, 541, 553 and 580, 556, 576 (the lines cross above 2^21)
+//       2^24: 1688, 1569, 1556 and 1765, 1642, 1622
+//       2^25: 3202, 2996, 2996 and 3372, 3168, 3125 against 3098
+//   G2  2^21: 759, 794, 840 and 768, 823, 883 (they cross below 2^22: 1230, 1158)
+//       2^23: 2140, 2022, 2033 and 2299, 2160, 2174
 struct MsmLanes {
     uint32_t lanes[4];
     uint64_t below[3];

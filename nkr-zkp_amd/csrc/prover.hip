@@ -477,7 +477,7 @@ void Groth16Prover::run(const fr_t *z, void *raw_out, void *az, void *bz, void *
     planes2_host_.uploaded(stream2_);
 
     // The G1 MSMs ar, bs1, zk (witness) and H as one batch on the main
-    // stream: the witness pieces fill the H accumulation launch, and the
+    // stream: the witness entries fill the H accumulation launch, and the
     // latency-bound reduction levels are paid once for all four.
     hsched_.build(pa_.get(), nullptr, hplan_, s, t);
     NKR_HIP(hipStreamWaitEvent(s, ev_wsched_, 0));
