@@ -172,14 +172,14 @@ int nkr_g16_batch_graph_active(const nkr_g16_batch *batch, int *active);
  * scripts/bench/runner.py:260-355).  Contexts stay resident (keys and NTT
  * tables in HBM); submit() queues a proof and returns a ticket; `workers`
  * threads each own a batch (own streams), and a free worker takes every
- * pending request whose charges fit its share of the work-memory budget, up
+ * pending request whose batch fits its share of the work-memory budget, up
  * to max_batch, so requests arriving while other batches are on the GPU are
  * admitted as workers and memory free up and run alongside them.  The budget
  * is clamped at creation to the device's free memory minus a reserve (the
  * larger of 1 GiB and 1/32 of the device) and split equally between the
- * workers; each request is charged nkr_g16_server_request_bytes of its
- * context, and a request larger than one worker's share is rejected by
- * submit.  A worker releases its grow-only work buffers whenever keeping them
+ * workers.  A request alone needs nkr_g16_server_request_bytes of its context
+ * (a batch at most about the sum: its MSMs share their launches), and one
+ * larger than a worker's share is rejected by submit.  A worker releases its grow-only work buffers whenever keeping them
  * would exceed its share, so the work memory held by all workers stays within
  * the budget.  A request that cannot be proved (its context lacks the
  * blinding elements) fails alone: its wait() reports the error and the rest
@@ -202,8 +202,8 @@ int nkr_g16_server_wait(nkr_g16_server *server, uint64_t ticket, double *latency
  * buffers), so that its work buffers are already sized for such requests
  * instead of growing on the first one, which would then pay the device
  * allocations.  Waits until no batch is in flight; requests submitted
- * meanwhile wait for it.  count <= max_batch and the items' request bytes
- * must fit one worker's share.  Not concurrently with another warm-up or
+ * meanwhile wait for it.  count <= max_batch and the items' batch must fit one
+ * worker's share.  Not concurrently with another warm-up or
  * with nkr_g16_server_destroy. */
 int nkr_g16_server_warm(nkr_g16_server *server, const nkr_g16_batch_item *items, uint64_t count);
 int nkr_g16_server_request_bytes(const nkr_g16_ctx *ctx, uint64_t *bytes);

@@ -61,10 +61,10 @@ uint32_t msm_complete_lanes_cap();
 // not replayed under another.
 uint64_t msm_shape_key();
 
-// Device bytes that a request's MSMs of one group add to the MsmBatch that runs
-// them with other requests' (msm_schedule_sizes has a schedule's).
+// Device bytes of an MsmBatch that runs jobs of these totals
+// (msm_schedule_sizes has a schedule's).
 template <class F>
-uint64_t msm_request_bytes(const std::vector<MsmPlan> &plans);
+uint64_t msm_batch_bytes(const MsmTotals &jobs);
 
 // Window-shifted affine bases of one proving-key vector.
 template <class F>

@@ -960,20 +960,15 @@ uint32_t msm_complete_lanes_cap() { return g_lanes_cap; }
 uint64_t msm_shape_key() { return (uint64_t)g_target_log << 32 | g_lanes_cap; }
 
 template <class F>
-uint64_t msm_request_bytes(const std::vector<MsmPlan> &plans)
+uint64_t msm_batch_bytes(const MsmTotals &jobs)
 {
-    uint64_t entries = 0, buckets = 0;
-    for (const MsmPlan &p : plans) {
-        entries += p.max_entries();
-        buckets += p.B;
-    }
-    const MsmLanes rule = msm_lanes(std::is_same<F, fq2_t>::value);
-    const MsmSizes s = msm_sizes(plans.size(), entries, buckets, msm_lane_charge(rule, entries));
+    if (jobs.jobs == 0) return 0;
+    const MsmSizes s = jobs.sizes(msm_lanes(std::is_same<F, fq2_t>::value));
     // partial sums and their folds; per bucket: sums and two tree levels, region
     // start and count, the completion class lists; fold records; and the fixed
     // records (job table, class counters, lane offsets, plan state)
-    return s.pool * sizeof(partial_t<F>) + buckets * (3 * sizeof(partial_t<F>) + 8 + 4 * kMsmCompleteClasses) +
-           s.records * kMsmMaxFoldLaunches * sizeof(FoldRec) + 1024 * plans.size();
+    return s.pool * sizeof(partial_t<F>) + s.buckets * (3 * sizeof(partial_t<F>) + 8 + 4 * kMsmCompleteClasses) +
+           s.records * kMsmMaxFoldLaunches * sizeof(FoldRec) + 1024 * jobs.jobs;
 }
 
 void msm_finite_terms(const g1_jac *a, const g2_jac *b, uint32_t n, std::vector<uint32_t> &terms, hipStream_t stream)
@@ -1124,15 +1119,15 @@ void MsmBatch<F>::layout(const std::vector<MsmJob<F>> &jobs, hipStream_t stream)
     const uint32_t J = (uint32_t)jobs.size();
     // where each job's buckets lie in the per-bucket arrays
     std::vector<uint64_t> b_off(J + 1, 0);
-    uint64_t entries = 0;
+    MsmTotals totals;
     for (uint32_t j = 0; j < J; ++j) {
         const MsmPlan &p = jobs[j].sched->plan();
         NKR_REQUIRE(jobs[j].bases->plan().n == p.n && jobs[j].bases->plan().c == p.c,
                     "MSM bases and schedule disagree");
-        entries += p.max_entries();
+        totals.add(p);
         b_off[j + 1] = b_off[j] + p.B;
     }
-    sizes_ = msm_sizes(J, entries, b_off[J], msm_launch_lanes(lanes_, entries));
+    sizes_ = totals.sizes(lanes_);
     NKR_REQUIRE(sizes_.pool < (1ull << 32), "MSM partial pool exceeds 32-bit indexing");
     NKR_REQUIRE(sizes_.complete_lanes < (1ull << 32), "MSM batch too large for 32-bit work indices");
     uint32_t fold_base[kMsmMaxFoldLaunches];
@@ -1313,7 +1308,7 @@ template Jacobian<fq_t> msm_finish(const Xyzz<fq_t> *, uint32_t);
 template Jacobian<fq2_t> msm_finish(const Xyzz<fq2_t> *, uint32_t);
 template Xyzz<fq_t> msm_sum(const Xyzz<fq_t> *, uint32_t);
 template Xyzz<fq2_t> msm_sum(const Xyzz<fq2_t> *, uint32_t);
-template uint64_t msm_request_bytes<fq_t>(const std::vector<MsmPlan> &);
-template uint64_t msm_request_bytes<fq2_t>(const std::vector<MsmPlan> &);
+template uint64_t msm_batch_bytes<fq_t>(const MsmTotals &);
+template uint64_t msm_batch_bytes<fq2_t>(const MsmTotals &);
 
 }  // namespace nkr

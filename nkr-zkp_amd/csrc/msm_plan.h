@@ -76,21 +76,6 @@ constexpr uint32_t msm_piece(const MsmLanes &r, uint64_t entries)
     const uint32_t lanes = msm_launch_lanes(r, entries);
     return entries == 0 ? 1u : (uint32_t)((entries + lanes - 1) / lanes);
 }
-// The lanes that a request's jobs, of `entries` entries in all, are charged
-// where launches are shared: for any set of requests at least as many as the
-// launch of all their entries has, though the rule may step up at an entry
-// count that only the sum reaches (a step to `lanes` at `below` entries is paid
-// for by lanes / below an entry).
-constexpr uint64_t msm_lane_charge(const MsmLanes &r, uint64_t entries)
-{
-    uint64_t charge = msm_launch_lanes(r, entries);
-    for (int i = 0; i < 3; ++i)
-        if (r.lanes[i + 1] > r.lanes[i]) {
-            const uint64_t per_lane = r.below[i] / r.lanes[i + 1];
-            charge = std::max(charge, (entries + per_lane - 1) / per_lane);
-        }
-    return std::min(entries, std::min<uint64_t>(charge, r.lanes[3]));
-}
 constexpr uint32_t msm_job_piece(uint32_t piece, uint32_t piece_min) { return piece < piece_min ? piece_min : piece; }
 // Largest bucket count (c <= 16): the histograms and bucket scans hold B
 // counts in one workgroup's LDS (128 KiB of gfx950's 160 KiB).
@@ -217,6 +202,28 @@ inline MsmPlan msm_b_plan(const MsmPlan &witness, uint32_t finite)
     if (n == witness.n || n > witness.n - witness.n / 4) return witness;
     return msm_witness_plan(n);
 }
+
+// What the sizes of a batch's jobs of one group depend on; the totals of several
+// batches add up to those of their union.
+struct MsmTotals {
+    uint64_t jobs = 0, entries = 0, buckets = 0;
+    void add(const MsmPlan &p)
+    {
+        ++jobs;
+        entries += p.max_entries();
+        buckets += p.B;
+    }
+    void add(const MsmTotals &o)
+    {
+        jobs += o.jobs;
+        entries += o.entries;
+        buckets += o.buckets;
+    }
+    MsmSizes sizes(const MsmLanes &rule) const
+    {
+        return msm_sizes(jobs, entries, buckets, msm_launch_lanes(rule, entries));
+    }
+};
 
 // Sort workgroups: about one per CU, each histogramming a contiguous slice of
 // at least kMsmSortMinPerBlock scalars.

@@ -11,12 +11,12 @@
 //
 // Device memory: the work budget is clamped at creation to the device's
 // free memory minus a reserve (the larger of 1 GiB and 1/32 of the device),
-// and each worker gets an equal share of it.  A request is charged the device
-// bytes its batch slot needs (witness, three domain polynomials, the two
-// digit schedules, MSM partial sums and per-bucket arrays); a worker admits
-// requests while their charges fit its share, and a request larger than a
-// share is rejected at submission.  A worker's batch prover keeps its
-// buffers between batches (they only grow), so before a batch whose charges
+// and each worker gets an equal share of it.  A batch needs what each request's
+// slot holds (witness, three domain polynomials, the digit schedules) and the
+// partial sums and per-bucket arrays of its joint MSM launches; a worker admits
+// requests while their batch fits its share, and a request larger than a share
+// by itself is rejected at submission.  A worker's batch prover keeps its
+// buffers between batches (they only grow), so before a batch whose bytes
 // would take it over its share, and after any batch that left it above its
 // share, the worker releases them: the work memory all workers hold stays
 // within the budget.
@@ -62,13 +62,13 @@ public:
     // buffers already have the size those requests need; otherwise a worker
     // grows them on its first such request, which then pays the device
     // allocations.  Waits until no batch is in flight; requests submitted
-    // meanwhile wait for the warm-up.  The items' charges must fit one
+    // meanwhile wait for the warm-up.  The items' batch must fit one
     // worker's share and max_batch; calls must not overlap each other or the
     // server's destruction.
     void warm(const std::vector<BatchItem> &items);
 
-    // Device bytes a request on this context is charged at admission.
-    static uint64_t request_bytes(const Groth16Prover &ctx);
+    // Device bytes of a batch of one request on this context.
+    static uint64_t request_bytes(const Groth16Prover &ctx) { return Work(ctx).bytes(); }
 
     struct Stats {
         uint64_t batches = 0, proofs = 0, max_batch_seen = 0, peak_work_bytes = 0;
@@ -83,10 +83,21 @@ public:
     Memory memory() const;
 
 private:
+    // What a batch of requests needs: bytes that add up request by request, and
+    // the MSM jobs, which share one launch per group (its lanes, and with them
+    // most of a small request's bytes, do not add up).
+    struct Work {
+        uint64_t own = 0;
+        MsmTotals g1, g2;
+        Work() = default;
+        explicit Work(const Groth16Prover &ctx);
+        Work with(const Work &o) const;
+        uint64_t bytes() const;
+    };
     struct Request {
         uint64_t ticket;
         BatchItem item;
-        uint64_t bytes;
+        Work work;
         std::chrono::steady_clock::time_point t_submit;
     };
     struct Done {

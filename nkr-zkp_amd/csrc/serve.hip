@@ -6,7 +6,7 @@
 
 namespace nkr {
 
-uint64_t Server::request_bytes(const Groth16Prover &g)
+Server::Work::Work(const Groth16Prover &g)
 {
     const uint64_t polys = (uint64_t)g.cols() * sizeof(fr_t) + 3ull * g.rows() * sizeof(fr_t);
     // the packed witness on the device (every value, at worst) and its masks,
@@ -18,9 +18,21 @@ uint64_t Server::request_bytes(const Groth16Prover &g)
         (uint64_t)(g.planes_g1_witness() + h.c) * sizeof(Xyzz<fq_t>) + (uint64_t)b.c * sizeof(Xyzz<fq2_t>);
     const uint64_t schedules = msm_schedule_sizes(w).bytes() + msm_schedule_sizes(h).bytes() +
                                (g.own_b_schedule() ? msm_schedule_sizes(b).bytes() : 0);
-    return polys + packed + planes + schedules + msm_request_bytes<fq_t>({w, w, b, h}) +
-           msm_request_bytes<fq2_t>({b});
+    own = polys + packed + planes + schedules;
+    for (const MsmPlan *p : {&w, &w, &b, &h}) g1.add(*p);
+    g2.add(b);
 }
+
+Server::Work Server::Work::with(const Work &o) const
+{
+    Work sum = *this;
+    sum.own += o.own;
+    sum.g1.add(o.g1);
+    sum.g2.add(o.g2);
+    return sum;
+}
+
+uint64_t Server::Work::bytes() const { return own + msm_batch_bytes<fq_t>(g1) + msm_batch_bytes<fq2_t>(g2); }
 
 Server::Server(int device, uint32_t workers, uint32_t max_batch, uint64_t work_budget_bytes)
     : device_(device), max_batch_(max_batch)
@@ -57,7 +69,8 @@ uint64_t Server::submit(Groth16Prover *ctx, const void *witness, const fr_t &r, 
 {
     NKR_REQUIRE(ctx && witness && raw_out && proof_out, "null request member");
     NKR_REQUIRE(ctx->device() == device_, "context prepared on another device");
-    const uint64_t bytes = request_bytes(*ctx);
+    const Work work(*ctx);
+    const uint64_t bytes = work.bytes();
     NKR_REQUIRE(bytes <= share_, "request needs " + std::to_string(bytes) +
                                      " bytes of work memory, more than a worker's share of " +
                                      std::to_string(share_) + " (a budget of " + std::to_string(budget_) +
@@ -67,7 +80,7 @@ uint64_t Server::submit(Groth16Prover *ctx, const void *witness, const fr_t &r, 
     Request q;
     q.ticket = next_ticket_++;
     q.item = BatchItem{ctx, witness, r, s, raw_out, proof_out};
-    q.bytes = bytes;
+    q.work = work;
     q.t_submit = std::chrono::steady_clock::now();
     pending_.push_back(q);
     done_[q.ticket] = Done{};
@@ -91,13 +104,14 @@ void Server::warm(const std::vector<BatchItem> &items)
 {
     NKR_REQUIRE(!items.empty(), "nothing to warm with");
     NKR_REQUIRE(items.size() <= max_batch_, "more warm-up items than max_batch");
-    uint64_t bytes = 0;
+    Work work;
     for (const BatchItem &it : items) {
         NKR_REQUIRE(it.ctx && it.witness && it.raw_out && it.proof_out, "null warm-up item member");
         NKR_REQUIRE(it.ctx->device() == device_, "context prepared on another device");
         NKR_REQUIRE(it.ctx->can_blind(), "the context was prepared without alpha/beta/delta, which blinding needs");
-        bytes += request_bytes(*it.ctx);
+        work = work.with(Work(*it.ctx));
     }
+    const uint64_t bytes = work.bytes();
     NKR_REQUIRE(bytes <= share_, "warm-up items need " + std::to_string(bytes) +
                                      " bytes of work memory, more than a worker's share of " +
                                      std::to_string(share_));
@@ -199,15 +213,19 @@ void Server::worker_loop(uint32_t index)
     BatchProver &prover = *provers_[index];
     for (;;) {
         std::vector<Request> batch;
+        Work work;
         uint64_t bytes = 0;
         {
             std::unique_lock<std::mutex> lk(mu_);
-            // admit pending requests in arrival order while their charges fit
-            // this worker's share (every request fits a share: submit checks)
+            // admit pending requests in arrival order while their batch fits
+            // this worker's share (every request alone does: submit checks)
             cv_work_.wait(lk, [&] { return (!pending_.empty() && !warming_) || stop_; });
             if (stop_ && pending_.empty()) return;
-            while (!pending_.empty() && batch.size() < max_batch_ && bytes + pending_.front().bytes <= share_) {
-                bytes += pending_.front().bytes;
+            while (!pending_.empty() && batch.size() < max_batch_) {
+                const Work more = work.with(pending_.front().work);
+                if (more.bytes() > share_) break;
+                work = more;
+                bytes = more.bytes();
                 batch.push_back(pending_.front());
                 pending_.pop_front();
             }
@@ -219,7 +237,7 @@ void Server::worker_loop(uint32_t index)
             stats_.max_batch_seen = std::max<uint64_t>(stats_.max_batch_seen, batch.size());
         }
         // The prover's buffers from earlier batches stay unless this batch's
-        // charges would take it over the share.
+        // bytes would take it over the share.
         std::vector<std::string> errors(batch.size());
         uint64_t held = 0;
         try {

@@ -6,8 +6,8 @@
 //   piece g2 target_log piece_min entries... -> per entry count, the launch's
 //                            entries per lane and those of a job with that minimum
 //   bplan cols c_override finite -> "n c" of bs1 and bs2
-//   sizes | charge g2 target_log jobs entries buckets -> the bounds msm_sizes gives a
-//                            launch under that lane rule, or a request's share: lanes pool records complete_lanes
+//   sizes g2 target_log jobs entries buckets -> the bounds msm_sizes gives a launch
+//                            under that lane rule: lanes pool records complete_lanes
 //                            launches, then each fold launch's base and cap
 //   launches partials     -> fold launches for buckets of at most that many
 //   divup a b             -> ceil(a / b) or "error <message>"
@@ -63,12 +63,13 @@ int main()
                 in >> cols >> c >> finite;
                 const MsmPlan p = msm_b_plan(msm_witness_plan((uint32_t)cols, (uint32_t)c), (uint32_t)finite);
                 std::printf("%u %u\n", p.n, p.c);
-            } else if (op == "sizes" || op == "charge") {
+            } else if (op == "sizes") {
                 uint64_t g2, tl, jobs, entries, buckets;
                 in >> g2 >> tl >> jobs >> entries >> buckets;
                 const MsmLanes r = msm_lanes_of(g2 != 0, (uint32_t)tl);
-                const MsmSizes s = msm_sizes(jobs, entries, buckets,
-                                             op == "sizes" ? msm_launch_lanes(r, entries) : msm_lane_charge(r, entries));
+                MsmTotals totals;
+                totals.add(MsmTotals{jobs, entries, buckets});
+                const MsmSizes s = totals.sizes(r);
                 std::printf("%llu %llu %llu %llu %u", (unsigned long long)s.lanes, (unsigned long long)s.pool,
                             (unsigned long long)s.records, (unsigned long long)s.complete_lanes, s.fold_launches);
                 for (uint32_t L = 0; L < kMsmMaxFoldLaunches; ++L)

@@ -134,25 +134,32 @@ def test_work_memory_stays_within_the_budget(contexts):
     assert st["proofs"] == len(reqs)
 
 
-def test_a_request_is_charged_what_it_holds():
-    """One worker after one request: the work memory it holds is within the
-    request's charge, and most of it (the MSMs of a request share a launch, so
-    their lanes are charged once)."""
-    c = circuits.matmul(16, 5, wide=True)
+def test_work_bytes_are_what_a_batch_holds():
+    """One worker after one request and after eight in one batch: the work
+    memory it holds is within what the batch is admitted with, and most of it.
+    The MSMs of a batch share their launches: eight 2^10 requests together stay
+    below the lane rule's first step, so that they need one request's G1 lanes
+    and, in all, about twice its bytes (added up it would be eight times)."""
+    c = circuits.matmul(8, 5, wide=True)
+    assert c.rows == 1 << 10
     k = N.setup(c, circuits.random_scalars(5, 99))
     pv = N.Prover(c, k)
     need = N.Server.request_bytes(pv)
-    srv = N.Server(workers=1, max_batch=1, budget_bytes=need)
-    try:
-        r, s = circuits.random_scalars(2, 7)
-        (raw, proof), = srv.warm([(pv, c.witness, r, s)])
-        held = srv.memory()["held"]
-    finally:
-        srv.close()
-    raw1, proof1 = pv.prove_blind(c.witness, r, s)
+    rs = circuits.random_scalars(16, 7)
+    items = [(pv, c.witness, rs[2 * i], rs[2 * i + 1]) for i in range(8)]
+    want = [pv.prove_blind(w, r, s) for _, w, r, s in items]
+    for count, share in ((1, need), (8, 3 * need)):
+        srv = N.Server(workers=1, max_batch=8, budget_bytes=share)
+        try:
+            outs = srv.warm(items[:count])
+            held = srv.memory()["held"]
+        finally:
+            srv.close()
+        for (raw, proof), (raw1, proof1) in zip(outs, want):
+            assert np.array_equal(raw, raw1) and np.array_equal(proof, proof1)
+        assert held <= share and held > 0.8 * need
+        assert count > 1 or held <= need
     pv.close()
-    assert np.array_equal(raw, raw1) and np.array_equal(proof, proof1)
-    assert 0.8 * need < held <= need
 
 
 def test_budget_is_clamped_to_free_device_memory(contexts):

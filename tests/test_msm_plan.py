@@ -1,9 +1,9 @@
 """The MSM sizing arithmetic the device buffers are allocated from
 (nkr-zkp_amd/csrc/msm_plan.h), compiled for the CPU: window choice, the lane
 rule, the bounds of a batch's partial sums and folds against the numbering the
-planning kernel uses, and what a request is charged where launches are shared;
-schedules with zero entries included, and a zero divisor must raise an error
-instead of ending the process (SIGFPE)."""
+planning kernel uses, and the schedules' buffers; schedules with zero entries
+included, and a zero divisor must raise an error instead of ending the process
+(SIGFPE)."""
 import os
 import shutil
 import subprocess
@@ -174,34 +174,6 @@ def test_buffer_bounds_cover_every_plan(plan_bin, g2, target):
                     m = np.where(m > 128, -(-m // 64), m)
                     issued += 1
                 assert buckets * 64 + 5 * 64 * len(jobs) == complete
-
-
-@pytest.mark.parametrize("g2", [0, 1])
-@pytest.mark.parametrize("target", [10, 19, 22])
-def test_charges_cover_any_batch(plan_bin, g2, target):
-    """What requests are charged one by one holds the lanes, partial sums and
-    fold records of the batch of all of them, also where only the sum of their
-    entries reaches a step of the lane rule; one request is charged its own
-    launch, or a step that its entries pay for."""
-    rng = np.random.default_rng(target)
-    steps = [1 << k for k in (16, 19, 21, 22, 23, 24, 25)]
-    for trial in range(120):
-        total = int(rng.choice(steps) * rng.choice([0.6, 1, 1.7])) + int(rng.integers(-2, 3))
-        K = int(rng.integers(1, 9))
-        parts = np.maximum(1, rng.multinomial(total, rng.dirichlet(np.full(K, rng.choice([0.1, 5]))))).tolist()
-        buckets = [int(b) for b in 2 ** rng.integers(1, 16, K)]
-        jobs = [int(j) for j in rng.integers(1, 5, K)]
-        out = ask(plan_bin, [f"sizes {g2} {target} {sum(jobs)} {sum(parts)} {sum(buckets)}"] +
-                  [f"charge {g2} {target} {j} {e} {b}" for j, e, b in zip(jobs, parts, buckets)] +
-                  [f"sizes {g2} {target} {j} {e} {b}" for j, e, b in zip(jobs, parts, buckets)])
-        rows = [list(map(int, line.split()))[:3] for line in out]
-        charged = np.array(rows[1:K + 1])
-        assert (charged.sum(axis=0) >= rows[0]).all(), (parts, buckets)
-        alone = np.array(rows[K + 1:])
-        assert (charged >= alone).all()
-        most = {0: (393216, 32), 1: (262144, 16)}[g2] if target == 19 else (1 << target, 1 << 60)
-        for (lanes, _, _), e, j, (own, _, _) in zip(charged, parts, jobs, alone):
-            assert lanes <= min(e, most[0], max(own, -(-e // most[1]))) + j
 
 
 def test_schedule_bytes_count_every_buffer(plan_bin):
